@@ -28,36 +28,47 @@ namespace fvmi {
 //  * reciprocal: v_rcp_f32 (1 ulp) refined by one Newton step with FMA,
 //    y = y0 + y0 (1 - b y0), which rounds to the correctly rounded 1/b;
 //  * quotient: q0 = a y, the exact remainder r = a - b q0 by FMA, and
-//    q = q0 + r y: correctly rounded when y is (Markstein's theorem); a zero
-//    quotient is q0 itself, whose sign is that of a b (q0 + r y would turn
-//    -0 into +0, and the sign of a zero reaches copysign in the WAF limiter);
-//  * square root: v_sqrt_f32 (1 ulp) and its two neighbours, the one whose
-//    residual x - s s' changes sign chosen by two FMAs.
+//    q = q0 + r y: correctly rounded when y is (Markstein's theorem).  A zero
+//    quotient needs care only for its sign, which q0 has and q0 + r y may turn
+//    from -0 into +0: div_rn puts it back with one v_bfi (the sign of a zero
+//    reaches copysign in the WAF limiter), quot_rn leaves it (no other scheme
+//    reads a zero's sign, and its values are equal either way);
+//  * square root: s = x y with y = v_rsq_f32(x), and s + (x - s^2) y/2 with
+//    both products in FMAs.  The argument of v_rsq is x + 2^-126, x itself for
+//    every x above 2^-101, so that the square root of a zero is zero.
 // Checked against the IEEE sequences on every mantissa of [1, 2) (reciprocal)
 // and [1, 4) (square root) and on random quotients, and in every exact-
-// arithmetic test, which compare the fields bitwise with the float32 oracle.
+// arithmetic test, which compare the fields with the float32 oracle for
+// equality.  The exact kernels are bound by VALU issue, so their time follows
+// the instruction count: with the quotient at 6 and the square root at 6
+// instructions (8 and 9 before, signs and neighbours chosen by compares) and
+// the limiter of minmod_slope2, KP07_dimsplit went from 480 to 343
+// instructions a row and from 222 to 184 us per 4096^2 substep, HLL2 from 274
+// to 219, Euler from 275 to 231 and WAF (no limited slopes) from 315 to 298.
 __device__ __forceinline__ float rcp_rn(float b) {
     const float y = __builtin_amdgcn_rcpf(b);
     return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
 }
+__device__ __forceinline__ float quot_rn(float a, float b) {
+    const float y = rcp_rn(b);
+    const float q = a * y;
+    return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+}
 __device__ __forceinline__ float div_rn(float a, float b) {
     const float y = rcp_rn(b);
     const float q = a * y;
-    const float qc = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
-    return q == 0.0f ? q : qc;
+    return __builtin_copysignf(__builtin_fmaf(__builtin_fmaf(-b, q, a), y, q), q);
 }
 __device__ __forceinline__ float sqrt_rn(float x) {
-    const float s = __builtin_amdgcn_sqrtf(x);
-    const float dn = __uint_as_float(__float_as_uint(s) - 1u);
-    const float up = __uint_as_float(__float_as_uint(s) + 1u);
-    float r = (__builtin_fmaf(-dn, s, x) <= 0.0f) ? dn : s;
-    r = (__builtin_fmaf(-up, s, x) > 0.0f) ? up : r;
-    return r;
+    const float y = __builtin_amdgcn_rsqf(x + 0x1p-126f);
+    const float s = x * y;
+    return __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
 }
 
 struct MathExact {
     static constexpr bool exact = true;
     __device__ static __forceinline__ float div(float a, float b) { return div_rn(a, b); }
+    __device__ static __forceinline__ float quot(float a, float b) { return quot_rn(a, b); }
     __device__ static __forceinline__ float sqrt(float x) { return sqrt_rn(x); }
     __device__ static __forceinline__ float rcp(float x) { return rcp_rn(x); }
 };
@@ -66,6 +77,7 @@ struct MathFast {
     static constexpr bool exact = false;
     __device__ static __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
     __device__ static __forceinline__ float div(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
+    __device__ static __forceinline__ float quot(float a, float b) { return div(a, b); }
     __device__ static __forceinline__ float sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 };
 
@@ -73,21 +85,18 @@ struct MathFast {
 // Limiters: GPUSimulators/cuda/limiters.h, common.h
 // ---------------------------------------------------------------------------
 
-// minmodSlope, limiters.h:31-41, in the reference's operation order (exact
-// policy).  The fast policy evaluates the same minmod as
-// med3(med3(b, f, 0), c, 0) -- the inner median is 0 unless b and f share a
-// sign, and then c shares it too -- in its scaled form (reconstruct in
-// fv_substep.h, half_slope in fv_unsplit.h).
-template <class M>
-__device__ __forceinline__ float minmod_slope(float left, float center, float right, float theta) {
-    static_assert(M::exact, "the fast policy uses the scaled med3 form");
-    const float backward = (center - left) * theta;
-    const float central = (right - left) * 0.5f;
-    const float forward = (right - center) * theta;
-    const float sb = __builtin_copysignf(1.0f, backward);
-    const float sc = __builtin_copysignf(1.0f, central);
-    const float sf = __builtin_copysignf(1.0f, forward);
-    return 0.25f * sb * (sb + sc) * (sc + sf) * fminf(fminf(fabsf(backward), fabsf(central)), fabsf(forward));
+// Twice the slope of minmodSlope (limiters.h:31-41) in exact arithmetic, from
+// the differences b2 = (center - left) 2 theta, f2 = (right - center) 2 theta
+// and cd = right - left, twice the reference's backward, forward and central
+// ones (scaling by two is exact, and commutes with their roundings).  The
+// reference's sign products 0.25 sb (sb + sc) (sc + sf) are the common sign or
+// zero, so its value is the median form: the inner median is zero unless b2
+// and f2 share a sign, and then cd shares it (the float differences keep the
+// order of the operands).  2 instructions where the sign products take 10.
+// The fast policy evaluates the same minmod in a scaled form (reconstruct_fast
+// in fv_substep.h, half_slope in fv_unsplit.h).
+__device__ __forceinline__ float minmod_slope2(float b2, float cd, float f2) {
+    return __builtin_amdgcn_fmed3f(__builtin_amdgcn_fmed3f(b2, f2, 0.0f), cd, 0.0f);
 }
 
 // generalized_minmod, limiters.h:100-102
@@ -99,7 +108,7 @@ __device__ __forceinline__ float generalized_minmod(float r, float theta) {
 template <class M>
 __device__ __forceinline__ float desingularize(float x, float eps) {
     return __builtin_copysignf(1.0f, x) *
-           fmaxf(fabsf(x), fminf(M::div(x * x, 2.0f * eps) + 0.5f * eps, eps));
+           fmaxf(fabsf(x), fminf(M::quot(x * x, 2.0f * eps) + 0.5f * eps, eps));
 }
 
 // limiterToWAFLimiter, SWECommon.h:109-111
@@ -111,13 +120,13 @@ __device__ __forceinline__ float limiter_to_waf(float r, float c) {
 // Shallow water: GPUSimulators/cuda/SWECommon.h
 // ---------------------------------------------------------------------------
 
-// F_func, SWECommon.h:29-37
-template <class M>
+// F_func, SWECommon.h:29-37.  SignedZero: F[2] keeps the sign of a zero (WAF).
+template <class M, bool SignedZero = false>
 __device__ __forceinline__ void swe_F(const float q[3], float g, float F[3]) {
     if constexpr (M::exact) {
         F[0] = q[1];
-        F[1] = M::div(q[1] * q[1], q[0]) + 0.5f * g * q[0] * q[0];
-        F[2] = M::div(q[1] * q[2], q[0]);
+        F[1] = M::quot(q[1] * q[1], q[0]) + 0.5f * g * q[0] * q[0];
+        F[2] = SignedZero ? M::div(q[1] * q[2], q[0]) : M::quot(q[1] * q[2], q[0]);
     } else {
         const float u = q[1] * M::rcp(q[0]);
         F[0] = q[1];
@@ -132,17 +141,17 @@ __device__ __forceinline__ void swe_cu_flux(const float qm[3], const float qp[3]
     if constexpr (M::exact) {
         float Fp[3], Fm[3];
         swe_F<M>(qp, g, Fp);
-        const float up = M::div(qp[1], qp[0]);
+        const float up = M::quot(qp[1], qp[0]);
         const float cp = M::sqrt(g * qp[0]);
         swe_F<M>(qm, g, Fm);
-        const float um = M::div(qm[1], qm[0]);
+        const float um = M::quot(qm[1], qm[0]);
         const float cm = M::sqrt(g * qm[0]);
         const float am = fminf(fminf(um - cm, up - cp), 0.0f);
         const float ap = fmaxf(fmaxf(um + cm, up + cp), 0.0f);
         const float apam = ap * am;
         const float den = ap - am;
 #pragma unroll
-        for (int k = 0; k < 3; ++k) out[k] = M::div((ap * Fm[k] - am * Fp[k]) + apam * (qp[k] - qm[k]), den);
+        for (int k = 0; k < 3; ++k) out[k] = M::quot((ap * Fm[k] - am * Fp[k]) + apam * (qp[k] - qm[k]), den);
     } else {
         const float ip = M::rcp(qp[0]);
         const float im = M::rcp(qm[0]);
@@ -166,17 +175,17 @@ __device__ __forceinline__ void swe_hll_flux(const float ql[3], const float qr[3
     const float h_l = ql[0], h_r = qr[0];
     float u_l, u_r;
     if constexpr (M::exact) {
-        u_l = M::div(ql[1], h_l);
-        u_r = M::div(qr[1], h_r);
+        u_l = M::quot(ql[1], h_l);
+        u_r = M::quot(qr[1], h_r);
     } else {
         u_l = ql[1] * M::rcp(h_l);
         u_r = qr[1] * M::rcp(h_r);
     }
     const float c_l = M::sqrt(g * h_l);
     const float c_r = M::sqrt(g * h_r);
-    const float h_dag = 0.5f * (h_l + h_r) - M::div(0.25f * (u_r - u_l) * (h_l + h_r), c_l + c_r);
-    const float q_l_tmp = M::sqrt(0.5f * M::div((h_dag + h_l) * h_dag, h_l * h_l));
-    const float q_r_tmp = M::sqrt(0.5f * M::div((h_dag + h_r) * h_dag, h_r * h_r));
+    const float h_dag = 0.5f * (h_l + h_r) - M::quot(0.25f * (u_r - u_l) * (h_l + h_r), c_l + c_r);
+    const float q_l_tmp = M::sqrt(0.5f * M::quot((h_dag + h_l) * h_dag, h_l * h_l));
+    const float q_r_tmp = M::sqrt(0.5f * M::quot((h_dag + h_r) * h_dag, h_r * h_r));
     const float q_l = (h_dag > h_l) ? q_l_tmp : 1.0f;
     const float q_r = (h_dag > h_r) ? q_r_tmp : 1.0f;
     const float S_l = u_l - c_l * q_l;
@@ -189,7 +198,7 @@ __device__ __forceinline__ void swe_hll_flux(const float ql[3], const float qr[3
         const float den = S_r - S_l;
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-            const float star = M::div(S_r * F_l[k] - S_l * F_r[k] + srsl * (qr[k] - ql[k]), den);
+            const float star = M::quot(S_r * F_l[k] - S_l * F_r[k] + srsl * (qr[k] - ql[k]), den);
             out[k] = (S_l >= 0.0f) ? F_l[k] : ((S_r <= 0.0f) ? F_r[k] : star);
         }
     } else {
@@ -209,7 +218,7 @@ __device__ __forceinline__ float compute_h_star(float h_l, float h_r, float u_l,
     (void)h_l;
     (void)h_r;
     const float h_tmp = 0.5f * (c_l + c_r) + 0.25f * (u_l - u_r);
-    return M::div(h_tmp * h_tmp, g);
+    return M::quot(h_tmp * h_tmp, g);
 }
 
 // ---------------------------------------------------------------------------
@@ -311,8 +320,8 @@ __device__ __forceinline__ void waf_flux_core(const WafCell& L, const WafCell& R
     const float q_l1[3] = {L.h, L.hu, L.hv};
     const float q_r1[3] = {R.h, R.hu, R.hv};
     if constexpr (M::exact) {
-        const float q_l_tmp = M::div(M::sqrt(0.5f * ((h_dag + h_l) * h_dag)), h_l);
-        const float q_r_tmp = M::div(M::sqrt(0.5f * ((h_dag + h_r) * h_dag)), h_r);
+        const float q_l_tmp = M::quot(M::sqrt(0.5f * ((h_dag + h_l) * h_dag)), h_l);
+        const float q_r_tmp = M::quot(M::sqrt(0.5f * ((h_dag + h_r) * h_dag)), h_r);
         const float q_l = (h_dag > h_l) ? q_l_tmp : 1.0f;
         const float q_r = (h_dag > h_r) ? q_r_tmp : 1.0f;
         const float S_l = u_l - c_l * q_l;
@@ -324,8 +333,8 @@ __device__ __forceinline__ void waf_flux_core(const WafCell& L, const WafCell& R
         const float Q_star_l[3] = {s_l * 1.0f, s_l * S_star, s_l * v_l};
         const float Q_star_r[3] = {s_r * 1.0f, s_r * S_star, s_r * v_r};
         float F_1[3], F_4[3], F_2[3], F_3[3];
-        swe_F<M>(q_l1, g, F_1);
-        swe_F<M>(q_r1, g, F_4);
+        swe_F<M, true>(q_l1, g, F_1);
+        swe_F<M, true>(q_r1, g, F_4);
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             F_2[k] = F_1[k] + S_l * (Q_star_l[k] - q_l1[k]);
@@ -335,9 +344,9 @@ __device__ __forceinline__ void waf_flux_core(const WafCell& L, const WafCell& R
         const float c_2 = M::div(S_star * dt, d);
         const float c_3 = M::div(S_r * dt, d);
         // desingularize((c_1 > 0) ? h_dag_l - h_l2 : h_dag_r - h_r) / desingularize(h_dag - h_l), ...
-        const float r_1 = M::div((c_1 > 0.0f) ? Dl.d1 : Dr.d1, D.d1);
-        const float r_2 = M::div((c_2 > 0.0f) ? Dl.d2 : Dr.d2, D.d2);
-        const float r_3 = M::div((c_3 > 0.0f) ? Dl.d3 : Dr.d3, D.d3);
+        const float r_1 = M::quot((c_1 > 0.0f) ? Dl.d1 : Dr.d1, D.d1);
+        const float r_2 = M::quot((c_2 > 0.0f) ? Dl.d2 : Dr.d2, D.d2);
+        const float r_3 = M::quot((c_3 > 0.0f) ? Dl.d3 : Dr.d3, D.d3);
         const float A_1 = __builtin_copysignf(1.0f, c_1) * limiter_to_waf(generalized_minmod(r_1, 1.9f), c_1);
         const float A_2 = __builtin_copysignf(1.0f, c_2) * limiter_to_waf(generalized_minmod(r_2, 1.9f), c_2);
         const float A_3 = __builtin_copysignf(1.0f, c_3) * limiter_to_waf(generalized_minmod(r_3, 1.9f), c_3);
@@ -390,15 +399,15 @@ template <class M>
 __device__ __forceinline__ float swe_cell_dt(const float q[3], float dx, float dy, float g) {
     if constexpr (M::exact) {
         const float h = q[0];
-        const float u = M::div(q[1], h);
-        const float v = M::div(q[2], h);
-        const float max_u = M::div(dx, fabsf(u) + M::sqrt(g * h));
-        const float max_v = M::div(dy, fabsf(v) + M::sqrt(g * h));
+        const float u = M::quot(q[1], h);
+        const float v = M::quot(q[2], h);
+        const float max_u = M::quot(dx, fabsf(u) + M::sqrt(g * h));
+        const float max_v = M::quot(dy, fabsf(v) + M::sqrt(g * h));
         return fminf(max_u, max_v);
     } else {
         const float ih = M::rcp(q[0]);
         const float c = M::sqrt(g * q[0]);
-        return fminf(M::div(dx, fabsf(q[1] * ih) + c), M::div(dy, fabsf(q[2] * ih) + c));
+        return fminf(M::quot(dx, fabsf(q[1] * ih) + c), M::quot(dy, fabsf(q[2] * ih) + c));
     }
 }
 
@@ -409,13 +418,13 @@ __device__ __forceinline__ float swe_cell_dt(const float q[3], float dx, float d
 // pressure, EulerCommon.h:83-90
 template <class M>
 __device__ __forceinline__ float euler_pressure(const float q[4], float gamma) {
-    return (gamma - 1.0f) * (q[3] - M::div(0.5f * (q[1] * q[1] + q[2] * q[2]), q[0]));
+    return (gamma - 1.0f) * (q[3] - M::quot(0.5f * (q[1] * q[1] + q[2] * q[2]), q[0]));
 }
 
 // F_func, EulerCommon.h:93-109.  P is a pressure.
 template <class M>
 __device__ __forceinline__ void euler_F(const float q[4], float P, float F[4]) {
-    const float u = M::div(q[1], q[0]);
+    const float u = M::quot(q[1], q[0]);
     F[0] = q[1];
     F[1] = q[1] * u + P;
     F[2] = q[2] * u;
@@ -426,15 +435,15 @@ __device__ __forceinline__ void euler_F(const float q[4], float P, float F[4]) {
 template <class M>
 __device__ __forceinline__ void euler_hll_flux(const float ql[4], const float qr[4], float gamma, float out[4]) {
     const float h_l = ql[0], h_r = qr[0];
-    const float u_l = M::div(ql[1], h_l);
-    const float u_r = M::div(qr[1], h_r);
+    const float u_l = M::quot(ql[1], h_l);
+    const float u_r = M::quot(qr[1], h_r);
     const float P_l = euler_pressure<M>(ql, gamma);
     const float P_r = euler_pressure<M>(qr, gamma);
-    const float c_l = M::sqrt(M::div(gamma * P_l, ql[0]));
-    const float c_r = M::sqrt(M::div(gamma * P_r, qr[0]));
-    const float h_dag = 0.5f * (h_l + h_r) - M::div(0.25f * (u_r - u_l) * (h_l + h_r), c_l + c_r);
-    const float q_l_tmp = M::sqrt(0.5f * M::div((h_dag + h_l) * h_dag, h_l * h_l));
-    const float q_r_tmp = M::sqrt(0.5f * M::div((h_dag + h_r) * h_dag, h_r * h_r));
+    const float c_l = M::sqrt(M::quot(gamma * P_l, ql[0]));
+    const float c_r = M::sqrt(M::quot(gamma * P_r, qr[0]));
+    const float h_dag = 0.5f * (h_l + h_r) - M::quot(0.25f * (u_r - u_l) * (h_l + h_r), c_l + c_r);
+    const float q_l_tmp = M::sqrt(0.5f * M::quot((h_dag + h_l) * h_dag, h_l * h_l));
+    const float q_r_tmp = M::sqrt(0.5f * M::quot((h_dag + h_r) * h_dag, h_r * h_r));
     const float q_l = (h_dag > h_l) ? q_l_tmp : 1.0f;
     const float q_r = (h_dag > h_r) ? q_r_tmp : 1.0f;
     const float S_l = u_l - c_l * q_l;
@@ -447,7 +456,7 @@ __device__ __forceinline__ void euler_hll_flux(const float ql[4], const float qr
         const float den = S_r - S_l;
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            const float star = M::div(S_r * F_l[k] - S_l * F_r[k] + srsl * (qr[k] - ql[k]), den);
+            const float star = M::quot(S_r * F_l[k] - S_l * F_r[k] + srsl * (qr[k] - ql[k]), den);
             out[k] = (S_l >= 0.0f) ? F_l[k] : ((S_r <= 0.0f) ? F_r[k] : star);
         }
     } else {
@@ -466,19 +475,19 @@ __device__ __forceinline__ void euler_cu_flux(const float qm[4], const float qp[
     const float Pp = euler_pressure<M>(qp, gamma);
     float Fp[4], Fm[4];
     euler_F<M>(qp, Pp, Fp);
-    const float up = M::div(qp[1], qp[0]);
-    const float cp = M::sqrt(M::div(gamma * Pp, qp[0]));
+    const float up = M::quot(qp[1], qp[0]);
+    const float cp = M::sqrt(M::quot(gamma * Pp, qp[0]));
     const float Pm = euler_pressure<M>(qm, gamma);
     euler_F<M>(qm, Pm, Fm);
-    const float um = M::div(qm[1], qm[0]);
-    const float cm = M::sqrt(M::div(gamma * Pm, qm[0]));
+    const float um = M::quot(qm[1], qm[0]);
+    const float cm = M::sqrt(M::quot(gamma * Pm, qm[0]));
     const float am = fminf(fminf(um - cm, up - cp), 0.0f);
     const float ap = fmaxf(fmaxf(um + cm, up + cp), 0.0f);
     const float apam = ap * am;
     if constexpr (M::exact) {
         const float den = ap - am;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) out[k] = M::div((ap * Fm[k] - am * Fp[k]) + apam * (qp[k] - qm[k]), den);
+        for (int k = 0; k < 4; ++k) out[k] = M::quot((ap * Fm[k] - am * Fp[k]) + apam * (qp[k] - qm[k]), den);
     } else {
         const float iden = M::rcp(ap - am);
 #pragma unroll
@@ -490,10 +499,10 @@ __device__ __forceinline__ void euler_cu_flux(const float qm[4], const float qp[
 template <class M>
 __device__ __forceinline__ float euler_cell_dt(const float q[4], float dx, float dy, float gamma) {
     const float rho = q[0];
-    const float u = M::div(q[1], rho);
-    const float v = M::div(q[2], rho);
-    const float max_u = M::div(dx, fabsf(u) + M::sqrt(gamma * rho));
-    const float max_v = M::div(dy, fabsf(v) + M::sqrt(gamma * rho));
+    const float u = M::quot(q[1], rho);
+    const float v = M::quot(q[2], rho);
+    const float max_u = M::quot(dx, fabsf(u) + M::sqrt(gamma * rho));
+    const float max_v = M::quot(dy, fabsf(v) + M::sqrt(gamma * rho));
     return fminf(max_u, max_v);
 }
 

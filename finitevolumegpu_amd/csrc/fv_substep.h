@@ -90,6 +90,7 @@ struct SubstepArgs {
     float half_theta;  // theta / 2
     float inv_2theta;  // 1 / (2 theta), 0 for theta <= 0
     float g_theta;     // g theta
+    float two_theta;   // 2 theta (exact policy)
 };
 
 // Rows per segment of the equal-segment plan: at most waves_per_simd waves on
@@ -113,11 +114,12 @@ __host__ __device__ inline int balanced_segment_rows(int rows, int strips, int c
     return seg1 < kMinSegRowsSmall ? kMinSegRowsSmall : seg1;
 }
 
-// the slope constants of the fast policy from g and theta
+// the slope constants from g and theta
 __host__ __device__ inline void set_slope_constants(SubstepArgs& a) {
     a.half_theta = 0.5f * a.theta;
     a.inv_2theta = a.theta > 0.0f ? 0.5f / a.theta : 0.0f;
     a.g_theta = a.g * a.theta;
+    a.two_theta = 2.0f * a.theta;
 }
 
 struct AxisMap {
@@ -425,19 +427,28 @@ __device__ __forceinline__ void reconstruct_fast(B b, F f, const float c[S::NV],
     }
 }
 
-// Reconstruction + half-step predictor of one cell (computeFluxF, SWE2D_KP07_dimsplit.cu:42-58):
-// slope from (l, c, r); returns the predicted left-face (qbl) and right-face (qbr) states.
-template <class S, class M>
-__device__ __forceinline__ void reconstruct(const float l[S::NV], const float c[S::NV], const float r[S::NV],
-                                            const SubstepArgs& a, float kk, float qbl[S::NV], float qbr[S::NV]) {
+// Difference of two neighbouring values as the limiter takes it: times
+// 2 theta in the exact policy (minmod_slope2 in fv_math.h).
+template <class M>
+__device__ __forceinline__ float limiter_diff(float lo, float hi, const SubstepArgs& a) {
+    return M::exact ? (hi - lo) * a.two_theta : hi - lo;
+}
+
+// Reconstruction + half-step predictor of one cell (computeFluxF, SWE2D_KP07_dimsplit.cu:42-58)
+// from its backward and forward differences b(k), f(k) (limiter_diff) and, in
+// the exact policy, cd(k) = right - left; returns the predicted left-face
+// (qbl) and right-face (qbr) states.
+template <class S, class M, class B, class F, class D2>
+__device__ __forceinline__ void reconstruct(B b, F f, D2 cd, const float c[S::NV], const SubstepArgs& a, float kk,
+                                            float qbl[S::NV], float qbr[S::NV]) {
     constexpr int NV = S::NV;
     if constexpr (M::exact) {
         float QL[NV], QR[NV], D[NV];
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
-            const float s = minmod_slope<M>(l[k], c[k], r[k], a.theta);
-            QL[k] = c[k] - 0.5f * s;
-            QR[k] = c[k] + 0.5f * s;
+            const float s2 = minmod_slope2(b(k), cd(k), f(k));  // twice the slope
+            QL[k] = __builtin_fmaf(-0.25f, s2, c[k]);           // c - 0.5 s, rounded once
+            QR[k] = __builtin_fmaf(0.25f, s2, c[k]);
         }
         S::pred_diff(QL, QR, a, D);
 #pragma unroll
@@ -446,16 +457,17 @@ __device__ __forceinline__ void reconstruct(const float l[S::NV], const float c[
             qbr[k] = QR[k] + kk * D[k];
         }
     } else {
-        reconstruct_fast<S>([&](int k) { return c[k] - l[k]; }, [&](int k) { return r[k] - c[k]; }, c, a, kk, qbl,
-                            qbr);
+        reconstruct_fast<S>(b, f, c, a, kk, qbl, qbr);
     }
 }
 
-// evolveF/evolveG, common.h:450, 471; dtd = dt/d (fast policy only)
-template <class M>
+// evolveF/evolveG, common.h:450, 471; dtd = dt/d (fast policy only).
+// SignedZero: the increment keeps the sign of a zero (WAF).
+template <class M, bool SignedZero = false>
 __device__ __forceinline__ float evolve(float q, float f_in, float f_out, float dt, float d, float dtd) {
     if constexpr (M::exact) {
-        return q + M::div((f_in - f_out) * dt, d);
+        const float df = (f_in - f_out) * dt;
+        return q + (SignedZero ? M::div(df, d) : M::quot(df, d));
     } else {
         return q + (f_in - f_out) * dtd;
     }
@@ -483,6 +495,14 @@ __device__ __forceinline__ void x_sweep_row(float (&q)[S::kC][S::NV], const Subs
     if constexpr (S::kSlopes) {
         const float kk = M::exact ? M::div(a.dt, 2.0f * a.dx) : 0.5f * a.dtdx;
         float qbl[C][NV], qbr[C][NV];
+        // exact policy: each scaled difference once, the left neighbour's through DPP
+        float f[C][NV];
+        if constexpr (M::exact) {
+#pragma unroll
+            for (int c = 0; c < C; ++c)
+#pragma unroll
+                for (int k = 0; k < NV; ++k) f[c][k] = limiter_diff<M>(q[c][k], right_of<C, NV>(q, c, k), a);
+        }
 #pragma unroll
         for (int c = 0; c < C; ++c) {
             float l[NV], r[NV];
@@ -491,7 +511,12 @@ __device__ __forceinline__ void x_sweep_row(float (&q)[S::kC][S::NV], const Subs
                 l[k] = left_of<C, NV>(q, c, k);
                 r[k] = right_of<C, NV>(q, c, k);
             }
-            reconstruct<S, M>(l, q[c], r, a, kk, qbl[c], qbr[c]);
+            if constexpr (M::exact)
+                reconstruct<S, M>([&](int k) { return left_of<C, NV>(f, c, k); }, [&](int k) { return f[c][k]; },
+                                  [&](int k) { return r[k] - l[k]; }, q[c], a, kk, qbl[c], qbr[c]);
+            else
+                reconstruct_fast<S>([&](int k) { return q[c][k] - l[k]; }, [&](int k) { return r[k] - q[c][k]; },
+                                    q[c], a, kk, qbl[c], qbr[c]);
         }
 #pragma unroll
         for (int c = 0; c < C; ++c) {
@@ -527,7 +552,7 @@ __device__ __forceinline__ void x_sweep_row(float (&q)[S::kC][S::NV], const Subs
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
             const float Fl = left_of<C, NV>(F, c, k);
-            q[c][k] = evolve<M>(q[c][k], Fl, F[c][k], a.dt, a.dx, a.dtdx);
+            q[c][k] = evolve<M, !S::kSlopes>(q[c][k], Fl, F[c][k], a.dt, a.dx, a.dtdx);
         }
     }
 }
@@ -700,8 +725,8 @@ __device__ __forceinline__ void slope_row(const SubstepArgs& a, const Strip<S::k
                                           float (&g)[S::kC][S::NV], float (&dq)[S::kC][S::NV], int r, bool emit,
                                           float& dt_min) {
     // w0, w1: rows r-2, r-1 (already x swept when XFirst); w2: raw row r on entry.
-    // dq (fast policy): y-order difference row r-1 minus row r-2 on entry, row r
-    // minus row r-1 on exit.
+    // dq (unless the fast policy's kCarryDiff is off): y-order limiter_diff of
+    // rows r-2 and r-1 on entry, of rows r-1 and r on exit.
     constexpr int NV = S::NV;
     constexpr int C = S::kC;
     if constexpr (XFirst) x_sweep_row<S, M>(w2, a);
@@ -712,14 +737,15 @@ __device__ __forceinline__ void slope_row(const SubstepArgs& a, const Strip<S::k
         to_y<NV>(w0[c], y0);
         to_y<NV>(w1[c], y1);
         to_y<NV>(w2[c], y2);
-        if constexpr (M::exact || !S::kCarryDiff) {
-            reconstruct<S, M>(y0, y1, y2, a, kky, qbb, qbt_next);  // faces of row r-1
+        if constexpr (!M::exact && !S::kCarryDiff) {
+            reconstruct_fast<S>([&](int k) { return y1[k] - y0[k]; }, [&](int k) { return y2[k] - y1[k]; }, y1, a,
+                                kky, qbb, qbt_next);  // faces of row r-1
         } else {
             float f[NV];
 #pragma unroll
-            for (int k = 0; k < NV; ++k) f[k] = y2[k] - y1[k];
-            reconstruct_fast<S>([&](int k) { return dq[c][k]; }, [&](int k) { return f[k]; }, y1, a, kky, qbb,
-                                qbt_next);  // faces of row r-1
+            for (int k = 0; k < NV; ++k) f[k] = limiter_diff<M>(y1[k], y2[k], a);
+            reconstruct<S, M>([&](int k) { return dq[c][k]; }, [&](int k) { return f[k]; },
+                              [&](int k) { return y2[k] - y0[k]; }, y1, a, kky, qbb, qbt_next);  // faces of row r-1
 #pragma unroll
             for (int k = 0; k < NV; ++k) dq[c][k] = f[k];
         }
@@ -788,7 +814,7 @@ __device__ __forceinline__ void waf_row(const SubstepArgs& a, const Strip<S::kC>
             float y1[3];
             to_y<3>(w1[c], y1);
 #pragma unroll
-            for (int k = 0; k < 3; ++k) y1[k] = evolve<M>(y1[k], g[c][k], G[k], a.dt, a.dy, a.dtdy);
+            for (int k = 0; k < 3; ++k) y1[k] = evolve<M, true>(y1[k], g[c][k], G[k], a.dt, a.dy, a.dtdy);
             to_y<3>(y1, outq[c]);
         }
         hd[c] = hd_r;
@@ -838,12 +864,13 @@ __device__ __forceinline__ float march_slopes(const SubstepArgs& a, const Strip<
         to_y<NV>(ring[0][c], y0);
         to_y<NV>(ring[1][c], y1);
         to_y<NV>(ring[2][c], y2);
-        reconstruct<S, M>(y0, y1, y2, a, kky, qbb, P[c]);  // faces of row 1
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
-            dq[c][k] = y2[k] - y1[k];
+            dq[c][k] = limiter_diff<M>(y1[k], y2[k], a);
             G[c][k] = 0.0f;
         }
+        reconstruct<S, M>([&](int k) { return limiter_diff<M>(y0[k], y1[k], a); }, [&](int k) { return dq[c][k]; },
+                          [&](int k) { return y2[k] - y0[k]; }, y1, a, kky, qbb, P[c]);  // faces of row 1
     }
     ys[(3 + PF) % N] = load_row_raw<C, NV, S::kPinRows, Edge>(a, st, min(3 + PF, last), ring[(3 + PF) % N]);
     use_row<C, NV, S::kPinRows>(st, ys[3 % N], ring[3 % N]);

@@ -52,6 +52,7 @@ struct UnsplitArgs {
     float hg, sqrt_g, inv_dx, inv_dy, dtdx, dtdy;
     float lxf_kx, lxf_ky, lf_kx, lf_ky, lw_kx, lw_ky;
     float half_theta, inv_2theta;  // theta/2 and 1/(2 theta) (0 for theta <= 0), KP07
+    float two_theta;               // 2 theta, KP07 in exact arithmetic
 };
 
 // Half the limited slope, s/2, of a cell with neighbours l and r.  Fast form:
@@ -60,7 +61,7 @@ struct UnsplitArgs {
 template <class M>
 __device__ __forceinline__ float half_slope(float l, float c, float r, const UnsplitArgs& a) {
     if constexpr (M::exact) {
-        return 0.5f * minmod_slope<M>(l, c, r, a.theta);
+        return 0.25f * minmod_slope2((c - l) * a.two_theta, r - l, (r - c) * a.two_theta);
     } else {
         const float b = c - l, f = r - c;
         return a.half_theta *
@@ -80,7 +81,7 @@ __device__ __forceinline__ void lxf_2d_flux(const float ql[3], const float qr[3]
     float Fl[3], Fr[3];
     swe_F<M>(ql, g, Fl);
     swe_F<M>(qr, g, Fr);
-    if constexpr (M::exact) k = M::div(d, 4.0f * dt);
+    if constexpr (M::exact) k = M::quot(d, 4.0f * dt);
 #pragma unroll
     for (int i = 0; i < 3; ++i) out[i] = 0.5f * (Fl[i] + Fr[i]) + k * (ql[i] - qr[i]);
 }
@@ -94,8 +95,8 @@ __device__ __forceinline__ void force_1d_flux(const float ql[3], const float qr[
     swe_F<M>(ql, g, Fl);
     swe_F<M>(qr, g, Fr);
     if constexpr (M::exact) {
-        klf = M::div(d, 2.0f * dt);
-        klw = M::div(dt, 2.0f * d);
+        klf = M::quot(d, 2.0f * dt);
+        klw = M::quot(dt, 2.0f * d);
     }
 #pragma unroll
     for (int i = 0; i < 3; ++i) q[i] = 0.5f * (ql[i] + qr[i]) + klw * (Fl[i] - Fr[i]);
@@ -286,7 +287,7 @@ __device__ __forceinline__ void swap_tn(const float (&q)[3], float (&o)[3]) {
 template <class M>
 __device__ __forceinline__ float u_update(float q, float fl, float fr, float gs, float gn, const UnsplitArgs& a) {
     if constexpr (M::exact)
-        return q + (M::div((fl - fr) * a.dt, a.dx) + M::div((gs - gn) * a.dt, a.dy));
+        return q + (M::quot((fl - fr) * a.dt, a.dx) + M::quot((gs - gn) * a.dt, a.dy));
     else
         return q + ((fl - fr) * a.dtdx + (gs - gn) * a.dtdy);
 }
