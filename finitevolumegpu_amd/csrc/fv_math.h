@@ -42,7 +42,7 @@ namespace fvmi {
 // equality.  The exact kernels are bound by VALU issue, so their time follows
 // the instruction count: with the quotient at 6 and the square root at 6
 // instructions (8 and 9 before, signs and neighbours chosen by compares) and
-// the limiter of minmod_slope2, KP07_dimsplit went from 480 to 343
+// the limiter of minmod_slope, KP07_dimsplit went from 480 to 343
 // instructions a row and from 222 to 184 us per 4096^2 substep, HLL2 from 274
 // to 219, Euler from 275 to 231 and WAF (no limited slopes) from 315 to 298.
 __device__ __forceinline__ float rcp_rn(float b) {
@@ -85,18 +85,18 @@ struct MathFast {
 // Limiters: GPUSimulators/cuda/limiters.h, common.h
 // ---------------------------------------------------------------------------
 
-// Twice the slope of minmodSlope (limiters.h:31-41) in exact arithmetic, from
-// the differences b2 = (center - left) 2 theta, f2 = (right - center) 2 theta
-// and cd = right - left, twice the reference's backward, forward and central
-// ones (scaling by two is exact, and commutes with their roundings).  The
-// reference's sign products 0.25 sb (sb + sc) (sc + sf) are the common sign or
-// zero, so its value is the median form: the inner median is zero unless b2
-// and f2 share a sign, and then cd shares it (the float differences keep the
-// order of the operands).  2 instructions where the sign products take 10.
+// minmodSlope (limiters.h:31-41) in exact arithmetic, from the reference's
+// backward, central and forward differences.  Its sign products 0.25 sb
+// (sb + sc) (sc + sf) are the common sign or zero, so its value is the median
+// form: the inner median is zero unless b and f share a sign, and then c shares
+// it (the float differences keep the order of the operands).  2 instructions
+// where the sign products take 10.  No factor of two is moved between the
+// differences and the slope: that would round differently where they are
+// denormal, as at the foot of a wave that decays into still water.
 // The fast policy evaluates the same minmod in a scaled form (reconstruct_fast
 // in fv_substep.h, half_slope in fv_unsplit.h).
-__device__ __forceinline__ float minmod_slope2(float b2, float cd, float f2) {
-    return __builtin_amdgcn_fmed3f(__builtin_amdgcn_fmed3f(b2, f2, 0.0f), cd, 0.0f);
+__device__ __forceinline__ float minmod_slope(float b, float c, float f) {
+    return __builtin_amdgcn_fmed3f(__builtin_amdgcn_fmed3f(b, f, 0.0f), c, 0.0f);
 }
 
 // generalized_minmod, limiters.h:100-102

@@ -90,7 +90,6 @@ struct SubstepArgs {
     float half_theta;  // theta / 2
     float inv_2theta;  // 1 / (2 theta), 0 for theta <= 0
     float g_theta;     // g theta
-    float two_theta;   // 2 theta (exact policy)
 };
 
 // Rows per segment of the equal-segment plan: at most waves_per_simd waves on
@@ -119,7 +118,6 @@ __host__ __device__ inline void set_slope_constants(SubstepArgs& a) {
     a.half_theta = 0.5f * a.theta;
     a.inv_2theta = a.theta > 0.0f ? 0.5f / a.theta : 0.0f;
     a.g_theta = a.g * a.theta;
-    a.two_theta = 2.0f * a.theta;
 }
 
 struct AxisMap {
@@ -428,10 +426,10 @@ __device__ __forceinline__ void reconstruct_fast(B b, F f, const float c[S::NV],
 }
 
 // Difference of two neighbouring values as the limiter takes it: times
-// 2 theta in the exact policy (minmod_slope2 in fv_math.h).
+// theta in the exact policy (minmod_slope in fv_math.h).
 template <class M>
 __device__ __forceinline__ float limiter_diff(float lo, float hi, const SubstepArgs& a) {
-    return M::exact ? (hi - lo) * a.two_theta : hi - lo;
+    return M::exact ? (hi - lo) * a.theta : hi - lo;
 }
 
 // Reconstruction + half-step predictor of one cell (computeFluxF, SWE2D_KP07_dimsplit.cu:42-58)
@@ -446,9 +444,9 @@ __device__ __forceinline__ void reconstruct(B b, F f, D2 cd, const float c[S::NV
         float QL[NV], QR[NV], D[NV];
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
-            const float s2 = minmod_slope2(b(k), cd(k), f(k));  // twice the slope
-            QL[k] = __builtin_fmaf(-0.25f, s2, c[k]);           // c - 0.5 s, rounded once
-            QR[k] = __builtin_fmaf(0.25f, s2, c[k]);
+            const float hs = 0.5f * minmod_slope(b(k), 0.5f * cd(k), f(k));
+            QL[k] = c[k] - hs;
+            QR[k] = c[k] + hs;
         }
         S::pred_diff(QL, QR, a, D);
 #pragma unroll

@@ -52,7 +52,6 @@ struct UnsplitArgs {
     float hg, sqrt_g, inv_dx, inv_dy, dtdx, dtdy;
     float lxf_kx, lxf_ky, lf_kx, lf_ky, lw_kx, lw_ky;
     float half_theta, inv_2theta;  // theta/2 and 1/(2 theta) (0 for theta <= 0), KP07
-    float two_theta;               // 2 theta, KP07 in exact arithmetic
 };
 
 // Half the limited slope, s/2, of a cell with neighbours l and r.  Fast form:
@@ -61,7 +60,7 @@ struct UnsplitArgs {
 template <class M>
 __device__ __forceinline__ float half_slope(float l, float c, float r, const UnsplitArgs& a) {
     if constexpr (M::exact) {
-        return 0.25f * minmod_slope2((c - l) * a.two_theta, r - l, (r - c) * a.two_theta);
+        return 0.5f * minmod_slope((c - l) * a.theta, 0.5f * (r - l), (r - c) * a.theta);
     } else {
         const float b = c - l, f = r - c;
         return a.half_theta *

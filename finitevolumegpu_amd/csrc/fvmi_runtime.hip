@@ -319,7 +319,6 @@ int run_unsplit(int scheme, UnsplitArgs& a, int gc, const fvmi_launch_t* launch,
     a.dtdy = a.dt / a.dy;
     a.half_theta = 0.5f * a.theta;
     a.inv_2theta = a.theta > 0.0f ? 0.5f / a.theta : 0.0f;
-    a.two_theta = 2.0f * a.theta;
     if (centred) {
         a.lxf_kx = a.dx / (4.0f * a.dt);
         a.lxf_ky = a.dy / (4.0f * a.dt);
