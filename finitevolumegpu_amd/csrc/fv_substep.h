@@ -44,13 +44,13 @@ constexpr int kLanes = 64;
 // lanes at each end that hold the strip's 2-column x halo are not written:
 // halo_lanes<C>() of them, leaving strip_cols<C>() output columns (60 for one
 // column per lane, 124 for two).
-template <int C>
+template <int C, int Halo = 2>
 __host__ __device__ constexpr int halo_lanes() {
-    return (2 + C - 1) / C;
+    return (Halo + C - 1) / C;
 }
-template <int C>
+template <int C, int Halo = 2>
 __host__ __device__ constexpr int strip_cols() {
-    return (kLanes - 2 * halo_lanes<C>()) * C;
+    return (kLanes - 2 * halo_lanes<C, Halo>()) * C;
 }
 
 struct SubstepArgs {
@@ -64,6 +64,7 @@ struct SubstepArgs {
     float* out[4];
     int out_pitch[4];
     float* cfl;  // two-slot CFL buffer: a step-1 launch minimises slot 1, every launch resets slot 1-step; may be null
+    int cfl_slot;  // whole-step launch: the slot it minimises (it resets the other)
     // Work decomposition: the sub-area is cut into strips of strip_cols columns and every
     // strip into `segs_per_strip` segments of `seg_rows` rows (the last one
     // shorter), one per wavefront.  Segment j starts at the same row in every
@@ -130,7 +131,9 @@ struct AxisMap {
 // array are clamped as readBlock does (those lanes/rows are never stored).
 // GC ghost cells a side: ghost k < GC mirrors cell 2*GC-1-k (bc*Reflective,
 // common.h:133-239, for any gc), periodic wraps by n.
-template <int GC>
+// Deep: two more images a side (k from -GC to n + 3 GC - 1) on periodic edges;
+// elsewhere those indices read some cell of the array.
+template <int GC, bool Deep = false>
 __device__ __forceinline__ AxisMap map_axis_gc(int k, int n, int bc_lo, int bc_hi) {
     if (k < GC) {
         if (bc_lo == BC_PERIODIC) return {k + n, false};
@@ -139,17 +142,14 @@ __device__ __forceinline__ AxisMap map_axis_gc(int k, int n, int bc_lo, int bc_h
         return {k, false};
     }
     if (k >= n + GC) {
-        if (k > n + 2 * GC - 1) k = n + 2 * GC - 1;
+        const int k_max = n + 2 * GC - 1 + (Deep && bc_hi == BC_PERIODIC ? 2 : 0);
+        if (k > k_max) k = k_max;
         if (bc_hi == BC_PERIODIC) return {k - n, false};
         if (bc_hi == BC_REFLECTIVE) return {2 * (n + GC) - 1 - k, true};
         if (bc_hi == BC_OUTFLOW) return {n + GC - 1, false};
         return {k, false};
     }
     return {k, false};
-}
-
-__device__ __forceinline__ AxisMap map_axis(int k, int n, int bc_lo, int bc_hi) {
-    return map_axis_gc<2>(k, n, bc_lo, bc_hi);
 }
 
 // The same map along y in affine, branch-free form for the row march (the row
@@ -160,7 +160,7 @@ __device__ __forceinline__ AxisMap map_axis(int k, int n, int bc_lo, int bc_hi) 
 struct RowMap {
     int lo_a, lo_b, hi_a, hi_b;
     int n_gc;   // n + GC, the first ghost row of the high side
-    int k_max;  // n + 2 GC - 1, the last padded row
+    int k_max;  // n + 2 GC - 1, the last padded row (Deep, periodic: two more images)
     unsigned lo_sign, hi_sign;
 };
 
@@ -181,13 +181,13 @@ __device__ __forceinline__ void row_map_side(int bc, int n, bool hi, int& a, int
     }
 }
 
-template <int GC>
+template <int GC, bool Deep = false>
 __device__ __forceinline__ RowMap make_row_map(int n, int bc_lo, int bc_hi) {
     RowMap m;
     row_map_side<GC>(bc_lo, n, false, m.lo_a, m.lo_b, m.lo_sign);
     row_map_side<GC>(bc_hi, n, true, m.hi_a, m.hi_b, m.hi_sign);
     m.n_gc = n + GC;
-    m.k_max = n + 2 * GC - 1;
+    m.k_max = n + 2 * GC - 1 + (Deep && bc_hi == BC_PERIODIC ? 2 : 0);
     return m;
 }
 
@@ -227,6 +227,86 @@ __device__ __forceinline__ WafCell waf_shift_right(const WafCell& p) {
     r.c = from_right(p.c);
     r.ih = from_right(p.ih);
     return r;
+}
+
+// Cross-lane operations on N values at once, as one run of DPP instructions: a
+// lone one among other VALU instructions costs several times its place in a
+// run (see FVMI_TRANS_RUN in fv_fast.h).  s_nop 1: a DPP operand that the
+// instruction before has written needs two wait states, which the compiler
+// does not see inside the block.  Lane 0 (63) takes 0 for its missing
+// neighbour.
+#define FVMI_DPP_MOV(o, x, ctrl) "v_mov_b32_dpp %" #o ", %" #x " " ctrl " row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+#define FVMI_DPP_SUB(o, x, y, ctrl) \
+    "v_sub_f32_dpp %" #o ", %" #x ", %" #y " " ctrl " row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+#define FVMI_OUT3 "=&v"(o[0]), "=&v"(o[1]), "=&v"(o[2])
+#define FVMI_OUT4 FVMI_OUT3, "=&v"(o[3])
+#define FVMI_OUT6 FVMI_OUT4, "=&v"(o[4]), "=&v"(o[5])
+#define FVMI_OUT8 FVMI_OUT6, "=&v"(o[6]), "=&v"(o[7])
+#define FVMI_IN3(v) "v"(v[0]), "v"(v[1]), "v"(v[2])
+#define FVMI_IN4(v) FVMI_IN3(v), "v"(v[3])
+#define FVMI_IN6(v) FVMI_IN4(v), "v"(v[4]), "v"(v[5])
+#define FVMI_IN8(v) FVMI_IN6(v), "v"(v[6]), "v"(v[7])
+#define FVMI_DPP_MOV_RUN(name, ctrl) \
+    template <int N> \
+    __device__ __forceinline__ void name(const float (&x)[N], float (&o)[N]) { \
+        static_assert(N == 3 || N == 4 || N == 6 || N == 8, "runs of 3, 4, 6 or 8"); \
+        if constexpr (N == 3) \
+            asm("s_nop 1\n\t" \
+                FVMI_DPP_MOV(0, 3, ctrl) FVMI_DPP_MOV(1, 4, ctrl) FVMI_DPP_MOV(2, 5, ctrl) \
+                : FVMI_OUT3 : FVMI_IN3(x)); \
+        if constexpr (N == 4) \
+            asm("s_nop 1\n\t" \
+                FVMI_DPP_MOV(0, 4, ctrl) FVMI_DPP_MOV(1, 5, ctrl) FVMI_DPP_MOV(2, 6, ctrl) \
+                FVMI_DPP_MOV(3, 7, ctrl) \
+                : FVMI_OUT4 : FVMI_IN4(x)); \
+        if constexpr (N == 6) \
+            asm("s_nop 1\n\t" \
+                FVMI_DPP_MOV(0, 6, ctrl) FVMI_DPP_MOV(1, 7, ctrl) FVMI_DPP_MOV(2, 8, ctrl) \
+                FVMI_DPP_MOV(3, 9, ctrl) FVMI_DPP_MOV(4, 10, ctrl) FVMI_DPP_MOV(5, 11, ctrl) \
+                : FVMI_OUT6 : FVMI_IN6(x)); \
+        if constexpr (N == 8) \
+            asm("s_nop 1\n\t" \
+                FVMI_DPP_MOV(0, 8, ctrl) FVMI_DPP_MOV(1, 9, ctrl) FVMI_DPP_MOV(2, 10, ctrl) \
+                FVMI_DPP_MOV(3, 11, ctrl) FVMI_DPP_MOV(4, 12, ctrl) FVMI_DPP_MOV(5, 13, ctrl) \
+                FVMI_DPP_MOV(6, 14, ctrl) FVMI_DPP_MOV(7, 15, ctrl) \
+                : FVMI_OUT8 : FVMI_IN8(x)); \
+    }
+#define FVMI_DPP_SUB_RUN(name, ctrl) \
+    template <int N> \
+    __device__ __forceinline__ void name(const float (&x)[N], const float (&y)[N], float (&o)[N]) { \
+        static_assert(N == 3 || N == 4 || N == 6 || N == 8, "runs of 3, 4, 6 or 8"); \
+        if constexpr (N == 3) \
+            asm("s_nop 1\n\t" \
+                FVMI_DPP_SUB(0, 3, 6, ctrl) FVMI_DPP_SUB(1, 4, 7, ctrl) FVMI_DPP_SUB(2, 5, 8, ctrl) \
+                : FVMI_OUT3 : FVMI_IN3(x), FVMI_IN3(y)); \
+        if constexpr (N == 4) \
+            asm("s_nop 1\n\t" \
+                FVMI_DPP_SUB(0, 4, 8, ctrl) FVMI_DPP_SUB(1, 5, 9, ctrl) FVMI_DPP_SUB(2, 6, 10, ctrl) \
+                FVMI_DPP_SUB(3, 7, 11, ctrl) \
+                : FVMI_OUT4 : FVMI_IN4(x), FVMI_IN4(y)); \
+        if constexpr (N == 6) \
+            asm("s_nop 1\n\t" \
+                FVMI_DPP_SUB(0, 6, 12, ctrl) FVMI_DPP_SUB(1, 7, 13, ctrl) FVMI_DPP_SUB(2, 8, 14, ctrl) \
+                FVMI_DPP_SUB(3, 9, 15, ctrl) FVMI_DPP_SUB(4, 10, 16, ctrl) FVMI_DPP_SUB(5, 11, 17, ctrl) \
+                : FVMI_OUT6 : FVMI_IN6(x), FVMI_IN6(y)); \
+        if constexpr (N == 8) \
+            asm("s_nop 1\n\t" \
+                FVMI_DPP_SUB(0, 8, 16, ctrl) FVMI_DPP_SUB(1, 9, 17, ctrl) FVMI_DPP_SUB(2, 10, 18, ctrl) \
+                FVMI_DPP_SUB(3, 11, 19, ctrl) FVMI_DPP_SUB(4, 12, 20, ctrl) FVMI_DPP_SUB(5, 13, 21, ctrl) \
+                FVMI_DPP_SUB(6, 14, 22, ctrl) FVMI_DPP_SUB(7, 15, 23, ctrl) \
+                : FVMI_OUT8 : FVMI_IN8(x), FVMI_IN8(y)); \
+    }
+FVMI_DPP_MOV_RUN(all_from_left, "wave_shr:1")    // o = x of lane - 1
+FVMI_DPP_MOV_RUN(all_from_right, "wave_shl:1")   // o = x of lane + 1
+FVMI_DPP_SUB_RUN(left_minus_all, "wave_shr:1")   // o = x of lane - 1, minus y
+FVMI_DPP_SUB_RUN(right_minus_all, "wave_shl:1")  // o = x of lane + 1, minus y
+
+// the WafCell of lane+1
+__device__ __forceinline__ WafCell waf_from_right(const WafCell& p) {
+    const float x[6] = {p.h, p.hu, p.hv, p.u, p.v, p.c};
+    float o[6];
+    all_from_right<6>(x, o);
+    return {o[0], o[1], o[2], o[3], o[4], o[5], from_right(p.ih)};
 }
 
 __device__ __forceinline__ float wave_min(float v) {
@@ -290,10 +370,10 @@ struct SweBase {
         for (int k = 0; k < 3; ++k) D[k] = FL[k] - FR[k];
     }
     // fast policy: faces QL/QR = c -/+ (theta/2) m of the cell c with limited
-    // slope m (in units of theta)
-    __device__ static void pred_diff_fast(const float QL[3], const float QR[3], const float c[3], const float m[3],
-                                          const SubstepArgs& a, float D[3]) {
-        fast::swe_pred_diff(QL, QR, c[0], m[0], a.g_theta, D);
+    // slope m (in units of theta), r = 1/(QL0 QR0)
+    __device__ static void pred_diff_fast(const float QL[3], const float QR[3], float r, const float c[3],
+                                          const float m[3], const SubstepArgs& a, float D[3]) {
+        fast::swe_pred_diff(QL, QR, r, c[0], m[0], a.g_theta, D);
     }
     __device__ static float cell_dt(const float q[3], const SubstepArgs& a) { return swe_cell_dt<M>(q, a.dx, a.dy, a.g); }
     __device__ static float cell_rate(const float q[3], const SubstepArgs& a) {
@@ -301,34 +381,56 @@ struct SweBase {
     }
 };
 
-template <class M>
+// Cols: columns per lane.  flux_x / flux_y take the interfaces of a lane's
+// columns at once.
+template <class M, int Cols = FVMI_SWE_COLS>
 struct SweKP07 : SweBase<M> {
+    using Pair = SweKP07<M, 2>;  // two rows side by side (Rows of x_sweep_row)
     static constexpr int kPrefetch = FVMI_SWE_PREFETCH;
     static constexpr bool kSlopes = true;
-    static constexpr int kC = FVMI_SWE_COLS;  // columns per lane
-    __device__ static void flux(const float l[3], const float r[3], const SubstepArgs& a, float o[3]) {
-        if constexpr (M::exact)
-            swe_cu_flux<M>(l, r, a.g, o);
-        else
-            fast::swe_cu_flux(l, r, a.hg, a.sqrt_g, o);
+    static constexpr int kC = Cols;
+    __device__ static void flux(const float (&l)[kC][3], const float (&r)[kC][3], const SubstepArgs& a,
+                                float (&o)[kC][3]) {
+        if constexpr (M::exact) {
+#pragma unroll
+            for (int c = 0; c < kC; ++c) swe_cu_flux<M>(l[c], r[c], a.g, o[c]);
+        } else {
+            fast::swe_cu_flux<kC>(l, r, a.hg, a.sqrt_g, o);
+        }
     }
-    __device__ static void flux_x(const float l[3], const float r[3], const SubstepArgs& a, float o[3]) { flux(l, r, a, o); }
-    __device__ static void flux_y(const float l[3], const float r[3], const SubstepArgs& a, float o[3]) { flux(l, r, a, o); }
+    __device__ static void flux_x(const float (&l)[kC][3], const float (&r)[kC][3], const SubstepArgs& a,
+                                  float (&o)[kC][3]) {
+        flux(l, r, a, o);
+    }
+    __device__ static void flux_y(const float (&l)[kC][3], const float (&r)[kC][3], const SubstepArgs& a,
+                                  float (&o)[kC][3]) {
+        flux(l, r, a, o);
+    }
 };
 
-template <class M>
+template <class M, int Cols = FVMI_SWE_COLS>
 struct SweHLL2 : SweBase<M> {
+    using Pair = SweHLL2<M, 2>;  // two rows side by side (Rows of x_sweep_row)
     static constexpr int kPrefetch = FVMI_SWE_PREFETCH;
     static constexpr bool kSlopes = true;
-    static constexpr int kC = FVMI_SWE_COLS;  // columns per lane
-    __device__ static void flux(const float l[3], const float r[3], const SubstepArgs& a, float o[3]) {
-        if constexpr (M::exact)
-            swe_hll_flux<M>(l, r, a.g, o);
-        else
-            fast::swe_hll_flux(l, r, a.hg, a.sqrt_g, o);
+    static constexpr int kC = Cols;
+    __device__ static void flux(const float (&l)[kC][3], const float (&r)[kC][3], const SubstepArgs& a,
+                                float (&o)[kC][3]) {
+        if constexpr (M::exact) {
+#pragma unroll
+            for (int c = 0; c < kC; ++c) swe_hll_flux<M>(l[c], r[c], a.g, o[c]);
+        } else {
+            fast::swe_hll_flux<kC>(l, r, a.hg, a.sqrt_g, o);
+        }
     }
-    __device__ static void flux_x(const float l[3], const float r[3], const SubstepArgs& a, float o[3]) { flux(l, r, a, o); }
-    __device__ static void flux_y(const float l[3], const float r[3], const SubstepArgs& a, float o[3]) { flux(l, r, a, o); }
+    __device__ static void flux_x(const float (&l)[kC][3], const float (&r)[kC][3], const SubstepArgs& a,
+                                  float (&o)[kC][3]) {
+        flux(l, r, a, o);
+    }
+    __device__ static void flux_y(const float (&l)[kC][3], const float (&r)[kC][3], const SubstepArgs& a,
+                                  float (&o)[kC][3]) {
+        flux(l, r, a, o);
+    }
 };
 
 template <class M>
@@ -339,14 +441,15 @@ struct SweWAF : SweBase<M> {
     static constexpr int kC = 1;  // columns per lane (its march needs the registers of two)
 };
 
-template <class M>
+template <class M, int Cols = (M::exact ? 1 : 2)>
 struct EulerKP07 {
+    using Pair = EulerKP07<M, 2>;
     static constexpr int NV = 4;
     static constexpr bool kSlopes = true;
     // columns per lane: two in fast arithmetic (8-byte accesses: 8192^2 step
     // 1.263 -> 1.157 ms); the exact arithmetic's division sequences need the
     // registers of the second column
-    static constexpr int kC = M::exact ? 1 : 2;
+    static constexpr int kC = Cols;
     static constexpr bool kEuler = true;
     static constexpr bool kPinRows = false;
     static constexpr bool kCarryDiff = false;
@@ -359,23 +462,29 @@ struct EulerKP07 {
 #pragma unroll
         for (int k = 0; k < 4; ++k) D[k] = FL[k] - FR[k];
     }
-    __device__ static void pred_diff_fast(const float QL[4], const float QR[4], const float c[4], const float m[4],
-                                          const SubstepArgs& a, float D[4]) {
+    __device__ static void pred_diff_fast(const float QL[4], const float QR[4], float r, const float c[4],
+                                          const float m[4], const SubstepArgs& a, float D[4]) {
         (void)c;
         (void)m;
-        fast::euler_pred_diff(QL, QR, a.gamma, D);
+        fast::euler_pred_diff(QL, QR, r, a.gamma, D);
     }
-    __device__ static void flux_x(const float l[4], const float r[4], const SubstepArgs& a, float o[4]) {
-        if constexpr (M::exact)
-            euler_hll_flux<M>(l, r, a.gamma, o);
-        else
-            fast::euler_hll_flux(l, r, a.gamma, o);
+    __device__ static void flux_x(const float (&l)[kC][4], const float (&r)[kC][4], const SubstepArgs& a,
+                                  float (&o)[kC][4]) {
+        if constexpr (M::exact) {
+#pragma unroll
+            for (int c = 0; c < kC; ++c) euler_hll_flux<M>(l[c], r[c], a.gamma, o[c]);
+        } else {
+            fast::euler_hll_flux<kC>(l, r, a.gamma, o);
+        }
     }
-    __device__ static void flux_y(const float l[4], const float r[4], const SubstepArgs& a, float o[4]) {
-        if constexpr (M::exact)
-            euler_cu_flux<M>(l, r, a.gamma, o);
-        else
-            fast::euler_cu_flux(l, r, a.gamma, o);
+    __device__ static void flux_y(const float (&l)[kC][4], const float (&r)[kC][4], const SubstepArgs& a,
+                                  float (&o)[kC][4]) {
+        if constexpr (M::exact) {
+#pragma unroll
+            for (int c = 0; c < kC; ++c) euler_cu_flux<M>(l[c], r[c], a.gamma, o[c]);
+        } else {
+            fast::euler_cu_flux<kC>(l, r, a.gamma, o);
+        }
     }
     __device__ static float cell_dt(const float q[4], const SubstepArgs& a) {
         return euler_cell_dt<M>(q, a.dx, a.dy, a.gamma);
@@ -398,30 +507,40 @@ __device__ __forceinline__ void to_y(const float q[NV], float o[NV]) {
     if constexpr (NV == 4) o[3] = q[3];
 }
 
-// Fast-policy reconstruction + half-step predictor of one cell from its
-// backward and forward differences, b(k) = c - l and f(k) = r - c of variable
-// k (callables, so that each difference is formed where it is used):
+// Fast-policy reconstruction + half-step predictor of a lane's cells from
+// their backward and forward differences, b(c, k) = q - l and f(c, k) = r - q
+// of variable k (callables, so that each difference is formed where it is used):
 //   minmod(theta b, (b + f)/2, theta f) = theta minmod(b, (b + f)/(2 theta), f)
-// for theta > 0, so each neighbour enters once (a cross-lane operand in the x
-// sweep) and the y sweep reuses the forward difference of one row as the
-// backward difference of the next.
+// for theta > 0, so each neighbour enters once and the y sweep reuses the
+// forward difference of one row as the backward difference of the next.
 template <class S, class B, class F>
-__device__ __forceinline__ void reconstruct_fast(B b, F f, const float c[S::NV], const SubstepArgs& a, float kk,
-                                                 float qbl[S::NV], float qbr[S::NV]) {
+__device__ __forceinline__ void reconstruct_fast(B b, F f, const float (&q)[S::kC][S::NV], const SubstepArgs& a,
+                                                 float kk, float (&qbl)[S::kC][S::NV], float (&qbr)[S::kC][S::NV]) {
     constexpr int NV = S::NV;
-    float QL[NV], QR[NV], D[NV], m[NV];
+    constexpr int C = S::kC;
+    float QL[C][NV], QR[C][NV], m[C][NV], p[C], r[C];
 #pragma unroll
-    for (int k = 0; k < NV; ++k) {
-        const float bk = b(k), fk = f(k);
-        m[k] = __builtin_amdgcn_fmed3f(__builtin_amdgcn_fmed3f(bk, fk, 0.0f), (bk + fk) * a.inv_2theta, 0.0f);
-        QL[k] = __builtin_fmaf(-a.half_theta, m[k], c[k]);
-        QR[k] = __builtin_fmaf(a.half_theta, m[k], c[k]);
+    for (int c = 0; c < C; ++c) {
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+            const float bk = b(c, k), fk = f(c, k);
+            m[c][k] =
+                __builtin_amdgcn_fmed3f(__builtin_amdgcn_fmed3f(bk, fk, 0.0f), (bk + fk) * a.inv_2theta, 0.0f);
+            QL[c][k] = __builtin_fmaf(-a.half_theta, m[c][k], q[c][k]);
+            QR[c][k] = __builtin_fmaf(a.half_theta, m[c][k], q[c][k]);
+        }
+        p[c] = QL[c][0] * QR[c][0];
     }
-    S::pred_diff_fast(QL, QR, c, m, a, D);
+    fast::rcp_all<C>(p, r);
 #pragma unroll
-    for (int k = 0; k < NV; ++k) {
-        qbl[k] = QL[k] + kk * D[k];
-        qbr[k] = QR[k] + kk * D[k];
+    for (int c = 0; c < C; ++c) {
+        float D[NV];
+        S::pred_diff_fast(QL[c], QR[c], r[c], q[c], m[c], a, D);
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+            qbl[c][k] = QL[c][k] + kk * D[k];
+            qbr[c][k] = QR[c][k] + kk * D[k];
+        }
     }
 }
 
@@ -432,127 +551,127 @@ __device__ __forceinline__ float limiter_diff(float lo, float hi, const SubstepA
     return M::exact ? (hi - lo) * a.theta : hi - lo;
 }
 
-// Reconstruction + half-step predictor of one cell (computeFluxF, SWE2D_KP07_dimsplit.cu:42-58)
-// from its backward and forward differences b(k), f(k) (limiter_diff) and, in
-// the exact policy, cd(k) = right - left; returns the predicted left-face
-// (qbl) and right-face (qbr) states.
+// Reconstruction + half-step predictor of a lane's cells (computeFluxF,
+// SWE2D_KP07_dimsplit.cu:42-58) from their backward and forward differences
+// b(c, k), f(c, k) (limiter_diff) and, in the exact policy, cd(c, k) = right -
+// left; gives the predicted left-face (qbl) and right-face (qbr) states.
 template <class S, class M, class B, class F, class D2>
-__device__ __forceinline__ void reconstruct(B b, F f, D2 cd, const float c[S::NV], const SubstepArgs& a, float kk,
-                                            float qbl[S::NV], float qbr[S::NV]) {
+__device__ __forceinline__ void reconstruct(B b, F f, D2 cd, const float (&q)[S::kC][S::NV], const SubstepArgs& a,
+                                            float kk, float (&qbl)[S::kC][S::NV], float (&qbr)[S::kC][S::NV]) {
     constexpr int NV = S::NV;
     if constexpr (M::exact) {
-        float QL[NV], QR[NV], D[NV];
 #pragma unroll
-        for (int k = 0; k < NV; ++k) {
-            const float hs = 0.5f * minmod_slope(b(k), 0.5f * cd(k), f(k));
-            QL[k] = c[k] - hs;
-            QR[k] = c[k] + hs;
-        }
-        S::pred_diff(QL, QR, a, D);
+        for (int c = 0; c < S::kC; ++c) {
+            float QL[NV], QR[NV], D[NV];
 #pragma unroll
-        for (int k = 0; k < NV; ++k) {
-            qbl[k] = QL[k] + kk * D[k];
-            qbr[k] = QR[k] + kk * D[k];
+            for (int k = 0; k < NV; ++k) {
+                const float hs = 0.5f * minmod_slope(b(c, k), 0.5f * cd(c, k), f(c, k));
+                QL[k] = q[c][k] - hs;
+                QR[k] = q[c][k] + hs;
+            }
+            S::pred_diff(QL, QR, a, D);
+#pragma unroll
+            for (int k = 0; k < NV; ++k) {
+                qbl[c][k] = QL[k] + kk * D[k];
+                qbr[c][k] = QR[k] + kk * D[k];
+            }
         }
     } else {
-        reconstruct_fast<S>(b, f, c, a, kk, qbl, qbr);
+        reconstruct_fast<S>(b, f, q, a, kk, qbl, qbr);
     }
 }
 
-// evolveF/evolveG, common.h:450, 471; dtd = dt/d (fast policy only).
-// SignedZero: the increment keeps the sign of a zero (WAF).
+// evolveF/evolveG, common.h:450, 471: q plus the flux difference df = f_in -
+// f_out times dt/d; dtd = dt/d (fast policy only).  SignedZero: the increment
+// keeps the sign of a zero (WAF).
 template <class M, bool SignedZero = false>
-__device__ __forceinline__ float evolve(float q, float f_in, float f_out, float dt, float d, float dtd) {
+__device__ __forceinline__ float evolve(float q, float df, float dt, float d, float dtd) {
     if constexpr (M::exact) {
-        const float df = (f_in - f_out) * dt;
-        return q + (SignedZero ? M::div(df, d) : M::quot(df, d));
+        return q + (SignedZero ? M::div(df * dt, d) : M::quot(df * dt, d));
     } else {
-        return q + (f_in - f_out) * dtd;
+        return q + df * dtd;
     }
 }
 
-// Neighbours across a row held C columns per lane: column c of this lane's
-// left neighbour is column c - 1 here, or for c = 0 column C - 1 of lane - 1;
-// the right one column c + 1, or for c = C - 1 column 0 of lane + 1.
-template <int C, int NV>
-__device__ __forceinline__ float left_of(const float (&x)[C][NV], int c, int k) {
-    return c > 0 ? x[c - 1][k] : from_left(x[C - 1][k]);
-}
-template <int C, int NV>
-__device__ __forceinline__ float right_of(const float (&x)[C][NV], int c, int k) {
-    return c < C - 1 ? x[c + 1][k] : from_right(x[0][k]);
-}
-
-// x sweep of one padded row held across the 64 lanes, C columns per lane
-// (valid on the strip's output columns).
-template <class S, class M>
+// x sweep of rows held across the 64 lanes (valid on the strip's output
+// columns).  q[c]: column c of the lane's C columns of one row, or, with Rows,
+// the lane's column of row c of C independent rows swept side by side.  The
+// cross-lane operations and the transcendentals of all C come in runs.
+template <class S, class M, bool Rows = false>
 __device__ __forceinline__ void x_sweep_row(float (&q)[S::kC][S::NV], const SubstepArgs& a) {
     constexpr int NV = S::NV;
     constexpr int C = S::kC;
+    // values that cross a lane's ends: the first and last column of each row
+    constexpr int E = Rows ? C : 1;
+    constexpr int N = E * NV;
+    const auto first = [](const float (&x)[C][NV], float (&o)[N]) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) o[i] = x[Rows ? i / NV : 0][i % NV];
+    };
+    const auto last = [](const float (&x)[C][NV], float (&o)[N]) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) o[i] = x[Rows ? i / NV : C - 1][i % NV];
+    };
+    const auto end = [](const float (&x)[N], int c, int k) { return x[(Rows ? c : 0) * NV + k]; };
     float F[C][NV];
     if constexpr (S::kSlopes) {
         const float kk = M::exact ? M::div(a.dt, 2.0f * a.dx) : 0.5f * a.dtdx;
         float qbl[C][NV], qbr[C][NV];
-        // exact policy: each scaled difference once, the left neighbour's through DPP
-        float f[C][NV];
+        float q_first[N], q_last[N], d_hi[N], d_lo[N];
+        first(q, q_first);
+        last(q, q_last);
+        right_minus_all<N>(q_first, q_last, d_hi);  // forward difference of the last column
         if constexpr (M::exact) {
+            static_assert(Rows || C == 1, "exact arithmetic marches one column per lane");
+            float q_lo[N], cd[N];
+            all_from_left<N>(q_last, q_lo);
+            right_minus_all<N>(q_first, q_lo, cd);
 #pragma unroll
-            for (int c = 0; c < C; ++c)
-#pragma unroll
-                for (int k = 0; k < NV; ++k) f[c][k] = limiter_diff<M>(q[c][k], right_of<C, NV>(q, c, k), a);
+            for (int i = 0; i < N; ++i) d_hi[i] *= a.theta;  // limiter_diff
+            all_from_left<N>(d_hi, d_lo);
+            reconstruct<S, M>([&](int c, int k) { return end(d_lo, c, k); },
+                              [&](int c, int k) { return end(d_hi, c, k); },
+                              [&](int c, int k) { return end(cd, c, k); }, q, a, kk, qbl, qbr);
+        } else {
+            all_from_left<N>(d_hi, d_lo);  // backward difference of the first column
+            const auto f = [&](int c, int k) { return Rows || c == C - 1 ? end(d_hi, c, k) : q[c + 1][k] - q[c][k]; };
+            const auto b = [&](int c, int k) { return Rows || c == 0 ? end(d_lo, c, k) : q[c][k] - q[c - 1][k]; };
+            reconstruct_fast<S>(b, f, q, a, kk, qbl, qbr);
         }
+        float qbl_first[N], qbl_hi[N], qr[C][NV];  // qr: left faces of the right neighbours
+        first(qbl, qbl_first);
+        all_from_right<N>(qbl_first, qbl_hi);
 #pragma unroll
-        for (int c = 0; c < C; ++c) {
-            float l[NV], r[NV];
+        for (int c = 0; c < C; ++c)
 #pragma unroll
-            for (int k = 0; k < NV; ++k) {
-                l[k] = left_of<C, NV>(q, c, k);
-                r[k] = right_of<C, NV>(q, c, k);
-            }
-            if constexpr (M::exact)
-                reconstruct<S, M>([&](int k) { return left_of<C, NV>(f, c, k); }, [&](int k) { return f[c][k]; },
-                                  [&](int k) { return r[k] - l[k]; }, q[c], a, kk, qbl[c], qbr[c]);
-            else
-                reconstruct_fast<S>([&](int k) { return q[c][k] - l[k]; }, [&](int k) { return r[k] - q[c][k]; },
-                                    q[c], a, kk, qbl[c], qbr[c]);
-        }
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-            float qbl_r[NV];
-#pragma unroll
-            for (int k = 0; k < NV; ++k) qbl_r[k] = right_of<C, NV>(qbl, c, k);
-            S::flux_x(qbr[c], qbl_r, a, F[c]);  // interface (c, c+1)
-        }
+            for (int k = 0; k < NV; ++k) qr[c][k] = Rows || c == C - 1 ? end(qbl_hi, c, k) : qbl[c + 1][k];
+        S::flux_x(qbr, qr, a, F);  // interfaces (c, c+1)
     } else {
-        // WAF: each column's cell quantities, and the h* and limiter
-        // denominators of its right interface, once; the neighbours' through DPP
-        WafCell P[C], R[C];
-        float hd[C];
-        WafDen D[C];
-#pragma unroll
-        for (int c = 0; c < C; ++c) P[c] = waf_cell<M>(q[c], a.g, a.sqrt_g);
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-            R[c] = c < C - 1 ? P[c + 1] : waf_shift_right(P[0]);
-            hd[c] = waf_hstar<M>(P[c], R[c], a.g, a.inv_g);
-            D[c] = waf_den<M>(P[c], R[c], hd[c]);
-        }
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-            const WafDen Dl = c > 0 ? D[c - 1]
-                                    : WafDen{from_left(D[C - 1].d1), from_left(D[C - 1].d2), from_left(D[C - 1].d3)};
-            const WafDen Dr = c < C - 1 ? D[c + 1] : WafDen{from_right(D[0].d1), from_right(D[0].d2), from_right(D[0].d3)};
-            waf_flux_core<M>(P[c], R[c], Dl, D[c], Dr, hd[c], a.g, a.hg, a.dx, a.dt, a.dtdx, F[c]);
-        }
+        // WAF: the cell's quantities, and the h* and limiter denominators of
+        // its right interface, once; the neighbours' through DPP
+        static_assert(C == 1, "WAF marches one column per lane");
+        const WafCell P = waf_cell<M>(q[0], a.g, a.sqrt_g);
+        const WafCell R = waf_from_right(P);
+        const float hd = waf_hstar<M>(P, R, a.g, a.inv_g);
+        const WafDen D = waf_den<M>(P, R, hd);
+        const float d[3] = {D.d1, D.d2, D.d3};
+        float dl[3], dr[3];
+        all_from_left<3>(d, dl);
+        all_from_right<3>(d, dr);
+        waf_flux_core<M>(P, R, WafDen{dl[0], dl[1], dl[2]}, D, WafDen{dr[0], dr[1], dr[2]}, hd, a.g, a.hg, a.dx, a.dt,
+                         a.dtdx, F[0]);
     }
+    float F_first[N], F_last[N], dF[N];
+    first(F, F_first);
+    last(F, F_last);
+    left_minus_all<N>(F_last, F_first, dF);
 #pragma unroll
-    for (int c = 0; c < C; ++c) {
+    for (int c = 0; c < C; ++c)
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
-            const float Fl = left_of<C, NV>(F, c, k);
-            q[c][k] = evolve<M, !S::kSlopes>(q[c][k], Fl, F[c][k], a.dt, a.dx, a.dtdx);
+            const float df = Rows || c == 0 ? end(dF, c, k) : F[c - 1][k] - F[c][k];
+            q[c][k] = evolve<M, !S::kSlopes>(q[c][k], df, a.dt, a.dx, a.dtdx);
         }
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -671,7 +790,7 @@ __device__ __forceinline__ void use_row(const Strip<C>& st, unsigned ysign, floa
 
 template <int C, int NV, bool Edge = false>
 __device__ __forceinline__ void store_row(const SubstepArgs& a, const Strip<C>& st, int r, const float (&q)[C][NV]) {
-    const int prow = __builtin_amdgcn_readfirstlane(st.row0 + r - 2);
+    const int prow = __builtin_amdgcn_readfirstlane(st.row0 + r);
     // every lane stores; the halo lanes' offset is out of range and the
     // hardware drops their writes (no branch around the stores)
 #pragma unroll
@@ -715,65 +834,116 @@ __device__ __forceinline__ void accumulate_cfl(const float (&q)[S::kC][S::NV], c
 // One row step of the y sweep for slope schemes.  Loop-carried state (per
 // column): qbt, the predicted top face of row r-2, and g, the flux through its
 // bottom interface; both are replaced by the values of row r-1 (in place:
-// reads precede writes).
+// reads precede writes).  w0, w1, w2: rows r-2, r-1, r (x swept when the x
+// sweep comes first).  dq (unless the fast policy's kCarryDiff is off):
+// y-order limiter_diff of rows r-2 and r-1 on entry, of rows r-1 and r on exit.
+// With `emit`, outq is row r-2 after the y sweep.
+template <class S, class M>
+__device__ __forceinline__ void y_sweep_step(const SubstepArgs& a, float kky, const float (&w0)[S::kC][S::NV],
+                                             const float (&w1)[S::kC][S::NV], const float (&w2)[S::kC][S::NV],
+                                             float (&qbt)[S::kC][S::NV], float (&g)[S::kC][S::NV],
+                                             float (&dq)[S::kC][S::NV], bool emit, float (&outq)[S::kC][S::NV]) {
+    constexpr int NV = S::NV;
+    constexpr int C = S::kC;
+    float y0[C][NV], y1[C][NV], y2[C][NV], qbb[C][NV], qbt_next[C][NV], G[C][NV];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        to_y<NV>(w0[c], y0[c]);
+        to_y<NV>(w1[c], y1[c]);
+        to_y<NV>(w2[c], y2[c]);
+    }
+    if constexpr (!M::exact && !S::kCarryDiff) {
+        reconstruct_fast<S>([&](int c, int k) { return y1[c][k] - y0[c][k]; },
+                            [&](int c, int k) { return y2[c][k] - y1[c][k]; }, y1, a, kky, qbb,
+                            qbt_next);  // faces of row r-1
+    } else {
+        float f[C][NV];
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+            for (int k = 0; k < NV; ++k) f[c][k] = limiter_diff<M>(y1[c][k], y2[c][k], a);
+        reconstruct<S, M>([&](int c, int k) { return dq[c][k]; }, [&](int c, int k) { return f[c][k]; },
+                          [&](int c, int k) { return y2[c][k] - y0[c][k]; }, y1, a, kky, qbb,
+                          qbt_next);  // faces of row r-1
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+            for (int k = 0; k < NV; ++k) dq[c][k] = f[c][k];
+    }
+    S::flux_y(qbt, qbb, a, G);  // interface (r-2, r-1)
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        if (emit) {
+#pragma unroll
+            for (int k = 0; k < NV; ++k) y0[c][k] = evolve<M>(y0[c][k], g[c][k] - G[c][k], a.dt, a.dy, a.dtdy);
+            to_y<NV>(y0[c], outq[c]);
+        }
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+            qbt[c][k] = qbt_next[c][k];
+            g[c][k] = G[c][k];
+        }
+    }
+}
+
+// The y sweep's carried state from the first three rows of a march: the faces
+// of row 1 (its top face in qbt) and its difference to row 2.
+template <class S, class M>
+__device__ __forceinline__ void y_sweep_begin(const SubstepArgs& a, float kky, const float (&w0)[S::kC][S::NV],
+                                              const float (&w1)[S::kC][S::NV], const float (&w2)[S::kC][S::NV],
+                                              float (&qbt)[S::kC][S::NV], float (&g)[S::kC][S::NV],
+                                              float (&dq)[S::kC][S::NV]) {
+    constexpr int NV = S::NV;
+    constexpr int C = S::kC;
+    float y0[C][NV], y1[C][NV], y2[C][NV], qbb[C][NV];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        to_y<NV>(w0[c], y0[c]);
+        to_y<NV>(w1[c], y1[c]);
+        to_y<NV>(w2[c], y2[c]);
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+            dq[c][k] = limiter_diff<M>(y1[c][k], y2[c][k], a);
+            g[c][k] = 0.0f;
+        }
+    }
+    reconstruct<S, M>([&](int c, int k) { return limiter_diff<M>(y0[c][k], y1[c][k], a); },
+                      [&](int c, int k) { return dq[c][k]; },
+                      [&](int c, int k) { return y2[c][k] - y0[c][k]; }, y1, a, kky, qbb, qbt);
+}
+
+// gravity source after both sweeps of a substep, EE2D_KP07_dimsplit.cu:197-205
+template <class S>
+__device__ __forceinline__ void gravity_source(const SubstepArgs& a, float (&q)[S::kC][S::NV]) {
+    if constexpr (S::kEuler) {
+        if (a.g > 0.0f) {
+#pragma unroll
+            for (int c = 0; c < S::kC; ++c) {
+                const float rho_v = q[c][2];
+                q[c][2] -= a.g * q[c][0] * a.dt;
+                q[c][3] -= a.g * rho_v * a.dt;
+            }
+        }
+    }
+}
+
+// One row of a substep's march: the x and y sweeps in the substep's order,
+// gravity, store and CFL of row r-2.  w2 holds raw row r on entry.
 template <class S, class M, bool XFirst, bool Edge>
 __device__ __forceinline__ void slope_row(const SubstepArgs& a, const Strip<S::kC>& st, float kky,
                                           const float (&w0)[S::kC][S::NV], const float (&w1)[S::kC][S::NV],
                                           float (&w2)[S::kC][S::NV], float (&qbt)[S::kC][S::NV],
                                           float (&g)[S::kC][S::NV], float (&dq)[S::kC][S::NV], int r, bool emit,
                                           float& dt_min) {
-    // w0, w1: rows r-2, r-1 (already x swept when XFirst); w2: raw row r on entry.
-    // dq (unless the fast policy's kCarryDiff is off): y-order limiter_diff of
-    // rows r-2 and r-1 on entry, of rows r-1 and r on exit.
     constexpr int NV = S::NV;
     constexpr int C = S::kC;
     if constexpr (XFirst) x_sweep_row<S, M>(w2, a);
     float outq[C][NV];
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-        float y0[NV], y1[NV], y2[NV], qbb[NV], qbt_next[NV];
-        to_y<NV>(w0[c], y0);
-        to_y<NV>(w1[c], y1);
-        to_y<NV>(w2[c], y2);
-        if constexpr (!M::exact && !S::kCarryDiff) {
-            reconstruct_fast<S>([&](int k) { return y1[k] - y0[k]; }, [&](int k) { return y2[k] - y1[k]; }, y1, a,
-                                kky, qbb, qbt_next);  // faces of row r-1
-        } else {
-            float f[NV];
-#pragma unroll
-            for (int k = 0; k < NV; ++k) f[k] = limiter_diff<M>(y1[k], y2[k], a);
-            reconstruct<S, M>([&](int k) { return dq[c][k]; }, [&](int k) { return f[k]; },
-                              [&](int k) { return y2[k] - y0[k]; }, y1, a, kky, qbb, qbt_next);  // faces of row r-1
-#pragma unroll
-            for (int k = 0; k < NV; ++k) dq[c][k] = f[k];
-        }
-        float G[NV];
-        S::flux_y(qbt[c], qbb, a, G);  // interface (r-2, r-1)
-        if (emit) {
-#pragma unroll
-            for (int k = 0; k < NV; ++k) y0[k] = evolve<M>(y0[k], g[c][k], G[k], a.dt, a.dy, a.dtdy);
-            to_y<NV>(y0, outq[c]);  // row r-2 after the y sweep
-        }
-#pragma unroll
-        for (int k = 0; k < NV; ++k) {
-            qbt[c][k] = qbt_next[k];
-            g[c][k] = G[k];
-        }
-    }
+    y_sweep_step<S, M>(a, kky, w0, w1, w2, qbt, g, dq, emit, outq);
     if (emit) {
         if constexpr (!XFirst) x_sweep_row<S, M>(outq, a);
-        if constexpr (S::kEuler) {
-            // gravity source, EE2D_KP07_dimsplit.cu:197-205
-            if (a.g > 0.0f) {
-#pragma unroll
-                for (int c = 0; c < C; ++c) {
-                    const float rho_v = outq[c][2];
-                    outq[c][2] -= a.g * outq[c][0] * a.dt;
-                    outq[c][3] -= a.g * rho_v * a.dt;
-                }
-            }
-        }
-        store_row<C, NV, Edge>(a, st, r, outq);
+        gravity_source<S>(a, outq);
+        store_row<C, NV, Edge>(a, st, r - 2, outq);
         // the CFL minimum is taken after the y-then-x substep only: it is what
         // computeDt reads after a full step (the last launch's values)
         if constexpr (!XFirst) accumulate_cfl<S, M>(outq, a, st, dt_min);
@@ -812,7 +982,7 @@ __device__ __forceinline__ void waf_row(const SubstepArgs& a, const Strip<S::kC>
             float y1[3];
             to_y<3>(w1[c], y1);
 #pragma unroll
-            for (int k = 0; k < 3; ++k) y1[k] = evolve<M, true>(y1[k], g[c][k], G[k], a.dt, a.dy, a.dtdy);
+            for (int k = 0; k < 3; ++k) y1[k] = evolve<M, true>(y1[k], g[c][k] - G[k], a.dt, a.dy, a.dtdy);
             to_y<3>(y1, outq[c]);
         }
         hd[c] = hd_r;
@@ -823,7 +993,7 @@ __device__ __forceinline__ void waf_row(const SubstepArgs& a, const Strip<S::kC>
     }
     if (emit) {
         if constexpr (!XFirst) x_sweep_row<S, M>(outq, a);
-        store_row<C, 3, Edge>(a, st, r, outq);
+        store_row<C, 3, Edge>(a, st, r - 2, outq);
         // the CFL minimum is taken after the y-then-x substep only: it is what
         // computeDt reads after a full step (the last launch's values)
         if constexpr (!XFirst) accumulate_cfl<S, M>(outq, a, st, dt_min);
@@ -856,20 +1026,7 @@ __device__ __forceinline__ float march_slopes(const SubstepArgs& a, const Strip<
         x_sweep_row<S, M>(ring[1], a);
         x_sweep_row<S, M>(ring[2], a);
     }
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-        float y0[NV], y1[NV], y2[NV], qbb[NV];
-        to_y<NV>(ring[0][c], y0);
-        to_y<NV>(ring[1][c], y1);
-        to_y<NV>(ring[2][c], y2);
-#pragma unroll
-        for (int k = 0; k < NV; ++k) {
-            dq[c][k] = limiter_diff<M>(y1[k], y2[k], a);
-            G[c][k] = 0.0f;
-        }
-        reconstruct<S, M>([&](int k) { return limiter_diff<M>(y0[k], y1[k], a); }, [&](int k) { return dq[c][k]; },
-                          [&](int k) { return y2[k] - y0[k]; }, y1, a, kky, qbb, P[c]);  // faces of row 1
-    }
+    y_sweep_begin<S, M>(a, kky, ring[0], ring[1], ring[2], P, G, dq);  // faces of row 1
     ys[(3 + PF) % N] = load_row_raw<C, NV, S::kPinRows, Edge>(a, st, min(3 + PF, last), ring[(3 + PF) % N]);
     use_row<C, NV, S::kPinRows>(st, ys[3 % N], ring[3 % N]);
     slope_row<S, M, XFirst, Edge>(a, st, kky, ring[1], ring[2], ring[3 % N], P, G, dq, 3, false, dt_min);
@@ -954,20 +1111,22 @@ __device__ __forceinline__ float march_waf(const SubstepArgs& a, const Strip<S::
     return dt_min;
 }
 
-template <class S, class M>
+// Halo: cells of halo a side, 2 for a substep and 4 for a whole step.
+template <class S, class M, int Halo = 2>
 __device__ __forceinline__ void setup_strip(const SubstepArgs& a, Strip<S::kC>& st, int lane, int strip_x, int row_in,
                                             int count) {
     constexpr int C = S::kC;
-    constexpr int H = halo_lanes<C>();
+    constexpr int H = halo_lanes<C, Halo>();
+    constexpr bool Deep = Halo > 2;
     st.lane = lane;
-    const int wstart = a.x0 + strip_cols<C>() * strip_x + 2 - H * C;  // padded column of lane 0, column 0
-    st.row0 = __builtin_amdgcn_readfirstlane(a.y0 + row_in);         // padded row of r = 0
-    st.r_end = __builtin_amdgcn_readfirstlane(count + 4);            // output rows r = 4 .. count+3
-    st.ymap = make_row_map<2>(a.ny, (a.bc >> 16) & 0xF, (a.bc >> 24) & 0xF);
+    const int wstart = a.x0 + strip_cols<C, Halo>() * strip_x + 2 - H * C;    // padded column of lane 0, column 0
+    st.row0 = __builtin_amdgcn_readfirstlane(a.y0 + row_in + 2 - Halo);       // padded row of r = 0
+    st.r_end = __builtin_amdgcn_readfirstlane(count + 2 * Halo);              // output rows r = 2 Halo .. r_end-1
+    st.ymap = make_row_map<2, Deep>(a.ny, (a.bc >> 16) & 0xF, (a.bc >> 24) & 0xF);
 #pragma unroll
     for (int c = 0; c < C; ++c) {
         st.col[c] = wstart + C * lane + c;
-        const AxisMap mx = map_axis(st.col[c], a.nx, a.bc & 0xF, (a.bc >> 8) & 0xF);
+        const AxisMap mx = map_axis_gc<2, Deep>(st.col[c], a.nx, a.bc & 0xF, (a.bc >> 8) & 0xF);
         st.lane_off[c] = mx.idx * (int)sizeof(float);
         st.xsign[c] = mx.mirrored ? 0x80000000u : 0u;
         st.lane_out[c] = lane >= H && lane < kLanes - H && st.col[c] < a.x1 + 2;

@@ -111,6 +111,12 @@ __device__ __forceinline__ void force_1d_flux(const float ql[3], const float qr[
 // Scheme policies
 // ---------------------------------------------------------------------------
 
+// a state as the array of one column that the fast fluxes take
+__device__ __forceinline__ const float (&one_column(const float* q))[1][3] {
+    return *reinterpret_cast<const float(*)[1][3]>(q);
+}
+__device__ __forceinline__ float (&one_column(float* q))[1][3] { return *reinterpret_cast<float(*)[1][3]>(q); }
+
 template <class M>
 struct UnsplitBase {
     __device__ static float cell_dt(const float q[3], const UnsplitArgs& a) {
@@ -141,7 +147,7 @@ struct SweHLL1 : UnsplitBase<M> {
         if constexpr (M::exact)
             swe_hll_flux<M>(l, r, a.g, o);
         else
-            fast::swe_hll_flux(l, r, a.hg, a.sqrt_g, o);
+            fast::swe_hll_flux<1>(one_column(l), one_column(r), a.hg, a.sqrt_g, one_column(o));
     }
     __device__ static void flux_y(const float l[3], const float r[3], const UnsplitArgs& a, float o[3]) {
         flux_x(l, r, a, o);
@@ -168,7 +174,7 @@ struct SweKP07U : UnsplitBase<M> {
         if constexpr (M::exact)
             swe_cu_flux<M>(l, r, a.g, o);
         else
-            fast::swe_cu_flux(l, r, a.hg, a.sqrt_g, o);
+            fast::swe_cu_flux<1>(one_column(l), one_column(r), a.hg, a.sqrt_g, one_column(o));
     }
 };
 
@@ -281,14 +287,14 @@ __device__ __forceinline__ void swap_tn(const float (&q)[3], float (&o)[3]) {
     o[2] = q[1];
 }
 
-// q + ((fl - fr) dt / dx + (gs - gn) dt / dy), the unsplit update of
-// SWE2D_LxF.cu:147-152 and SWE2D_KP07.cu:190-195
+// q + (df dt / dx + dg dt / dy) with the flux differences df = fl - fr, dg = gs
+// - gn: the unsplit update of SWE2D_LxF.cu:147-152 and SWE2D_KP07.cu:190-195
 template <class M>
-__device__ __forceinline__ float u_update(float q, float fl, float fr, float gs, float gn, const UnsplitArgs& a) {
+__device__ __forceinline__ float u_update(float q, float df, float dg, const UnsplitArgs& a) {
     if constexpr (M::exact)
-        return q + (M::quot((fl - fr) * a.dt, a.dx) + M::quot((gs - gn) * a.dt, a.dy));
+        return q + (M::quot(df * a.dt, a.dx) + M::quot(dg * a.dt, a.dy));
     else
-        return q + ((fl - fr) * a.dtdx + (gs - gn) * a.dtdy);
+        return q + (df * a.dtdx + dg * a.dtdy);
 }
 
 // ---------------------------------------------------------------------------
@@ -300,8 +306,7 @@ __device__ __forceinline__ float u_update(float q, float fl, float fr, float gs,
 template <class S, class M>
 __device__ __forceinline__ void x_fluxes_first_order(const float (&q)[3], const UnsplitArgs& a, float (&F)[3]) {
     float r[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) r[k] = from_right(q[k]);
+    all_from_right<3>(q, r);
     S::flux_x(q, r, a, F);
 }
 
@@ -309,13 +314,16 @@ __device__ __forceinline__ void x_fluxes_first_order(const float (&q)[3], const 
 // central-upwind flux at (c, c+1) (SWE2D_KP07.cu:30-56, 103-115)
 template <class S, class M>
 __device__ __forceinline__ void x_fluxes_kp07(const float (&q)[3], const UnsplitArgs& a, float (&F)[3]) {
-    float qm[3], qp[3];
+    float l[3], r[3], qm[3], bot[3], qp[3];
+    all_from_left<3>(q, l);
+    all_from_right<3>(q, r);
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        const float hs = half_slope<M>(from_left(q[k]), q[k], from_right(q[k]), a);
-        qm[k] = q[k] + hs;               // right face of cell c
-        qp[k] = from_right(q[k] - hs);   // left face of cell c + 1
+        const float hs = half_slope<M>(l[k], q[k], r[k], a);
+        qm[k] = q[k] + hs;   // right face of cell c
+        bot[k] = q[k] - hs;  // left face of cell c
     }
+    all_from_right<3>(bot, qp);  // of cell c + 1
     S::flux(qm, qp, a, F);
 }
 
@@ -338,10 +346,11 @@ template <class S, class M>
 __device__ __forceinline__ void gc1_row(const UnsplitArgs& a, const UStrip<1>& st, const float (&w0)[3],
                                         float (&w1)[3], float (&g)[3], int r, bool emit, float& acc) {
     if constexpr (S::kind == KIND_SPLIT1) {
-        float F[3];
+        float F[3], dF[3];
         x_fluxes_first_order<S, M>(w1, a, F);
+        left_minus_all<3>(F, F, dF);
 #pragma unroll
-        for (int k = 0; k < 3; ++k) w1[k] = evolve<M>(w1[k], from_left(F[k]), F[k], a.dt, a.dx, a.dtdx);
+        for (int k = 0; k < 3; ++k) w1[k] = evolve<M>(w1[k], dF[k], a.dt, a.dx, a.dtdx);
     }
     float G[3];
     y_flux<S>(w0, w1, a, G);
@@ -349,12 +358,13 @@ __device__ __forceinline__ void gc1_row(const UnsplitArgs& a, const UStrip<1>& s
         float out[3];
         if constexpr (S::kind == KIND_SPLIT1) {
 #pragma unroll
-            for (int k = 0; k < 3; ++k) out[k] = evolve<M>(w0[k], g[k], G[k], a.dt, a.dy, a.dtdy);
+            for (int k = 0; k < 3; ++k) out[k] = evolve<M>(w0[k], g[k] - G[k], a.dt, a.dy, a.dtdy);
         } else {
-            float F[3];
+            float F[3], dF[3];
             x_fluxes_first_order<S, M>(w0, a, F);
+            left_minus_all<3>(F, F, dF);
 #pragma unroll
-            for (int k = 0; k < 3; ++k) out[k] = u_update<M>(w0[k], from_left(F[k]), F[k], g[k], G[k], a);
+            for (int k = 0; k < 3; ++k) out[k] = u_update<M>(w0[k], dF[k], g[k] - G[k], a);
         }
         u_store<1>(a, st, st.row0 + r - 1, out, out);
         u_cfl<S, M>(out, a, st.lane_out, acc);
@@ -387,10 +397,11 @@ __device__ __forceinline__ void kp07u_row(const UnsplitArgs& a, const UStrip<2>&
         swap_tn(o, G);
     }
     if (emit) {
-        float F[3], out[3];
+        float F[3], dF[3], out[3];
         x_fluxes_kp07<S, M>(w0, a, F);
+        left_minus_all<3>(F, F, dF);
 #pragma unroll
-        for (int k = 0; k < 3; ++k) out[k] = u_update<M>(w0[k], from_left(F[k]), F[k], g[k], G[k], a);
+        for (int k = 0; k < 3; ++k) out[k] = u_update<M>(w0[k], dF[k], g[k] - G[k], a);
         u_store<2, Stage2>(a, st, st.row0 + r - 2, out, old);
         u_cfl<S, M>(out, a, st.lane_out, acc);  // before the RK2 average, as writeCfl reads the tile
     }
@@ -418,10 +429,11 @@ __device__ __forceinline__ float march_gc1(const UnsplitArgs& a, const UStrip<1>
     u_use<1>(st, ys[0], ring[0]);
     u_use<1>(st, ys[1], ring[1]);
     if constexpr (S::kind == KIND_SPLIT1) {
-        float F[3];
+        float F[3], dF[3];
         x_fluxes_first_order<S, M>(ring[0], a, F);
+        left_minus_all<3>(F, F, dF);
 #pragma unroll
-        for (int k = 0; k < 3; ++k) ring[0][k] = evolve<M>(ring[0][k], from_left(F[k]), F[k], a.dt, a.dx, a.dtdx);
+        for (int k = 0; k < 3; ++k) ring[0][k] = evolve<M>(ring[0][k], dF[k], a.dt, a.dx, a.dtdx);
     }
 #pragma unroll
     for (int k = 0; k < 3; ++k) G[k] = 0.0f;
