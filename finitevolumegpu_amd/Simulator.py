@@ -198,6 +198,7 @@ def resolve_math(scheme, math):
         raise ValueError("math must be 'fast', 'exact' or None")
     return math
 
+
 class DimsplitSimulator(BaseSimulator):
     """Shared body of the four dimensionally split scheme wrappers."""
 
@@ -227,19 +228,66 @@ class DimsplitSimulator(BaseSimulator):
         ptr = ctypes.c_void_p()
         _lib.call("fvmi_malloc", ctypes.byref(ptr), 8)
         self.cfl_data = ptr
+        self.cfl_last = 1  # slot of the latest minimum (slot 1 for a substep, either for a whole step)
+        self.cfl_free = 0  # slot known to hold +inf
         init = np.array([np.inf, cfl_host], dtype=np.float32)
         _lib.call("fvmi_memcpy_async", self.cfl_data, init.ctypes.data, 8, _lib.MEMCPY_HTOD, self.stream.handle)
         self.stream.synchronize()
+        self._step_buffer = ctypes.create_string_buffer(ctypes.sizeof(_lib.StepArgs))
+        self._step_out = (ctypes.c_int * 2)()  # buffer of the new state, slot of its CFL minimum
+        self._step_out_ptr = ctypes.addressof(self._step_out)
+        # step() is one library call unless a subclass brings its own substeps
+        self._whole_step = all(
+            getattr(type(self), name).__module__.partition(".")[0] == __name__.partition(".")[0]
+            for name in ("substep", "substepDimsplit", "_launch", "_field_args", "cfl_pointer"))
 
     def cfl_pointer(self):
         return self.cfl_data.value
+
+    def step(self, dt):
+        """One full step as one library call (fvmi_dimsplit_step), with the
+        results of the two substeps of BaseSimulator.step."""
+        if not self._whole_step or "substep" in self.__dict__:
+            super().step(dt)
+            return
+        self._step_both(dt, self.boundary_conditions)
+        self.t += float(dt)
+        self.nt += 1
+
+    def _step_both(self, dt, boundary_conditions):
+        """Both substeps of one step under ``boundary_conditions``."""
+        cfl = self.cfl_pointer() or 0
+        fields = []
+        pitches = []
+        for state in (self.u0, self.u1):
+            arrays = state.gpu_variables
+            fields += [v.ptr.value or 0 for v in arrays] + [0] * (4 - len(arrays))
+            pitches += [v.pitch for v in arrays] + [0] * (4 - len(arrays))
+        _lib.STEP_PACK.pack_into(self._step_buffer, 0, _lib.SCHEME_IDS[self.scheme], self.nx, self.ny,
+                                 boundary_conditions, self.dx, self.dy, np.float32(dt * 0.5), self.g,
+                                 getattr(self, "theta", 0.0), getattr(self, "gamma", 0.0), *fields, *pitches,
+                                 cfl, self.cfl_free)
+        out = self._step_out
+        _lib.call("fvmi_dimsplit_step", self._step_buffer, self.launch, self._step_out_ptr, self._step_out_ptr + 4,
+                  self.stream.handle)
+        if out[0]:
+            self.u0, self.u1 = self.u1, self.u0
+        if cfl:
+            self.cfl_last = out[1]
+            self.cfl_free = 1 - out[1]
 
     def substep(self, dt, step_number):
         self.substepDimsplit(dt * 0.5, step_number)
 
     def substepDimsplit(self, dt, substep):
         self._launch(np.float32(dt), int(substep), self.u0, self.u1, self.cfl_pointer())
+        self._note_substep(substep)
         self.u0, self.u1 = self.u1, self.u0
+
+    def _note_substep(self, substep):
+        """A substep launch resets slot 1 - substep; substep 1 minimises slot 1."""
+        self.cfl_last = 1
+        self.cfl_free = 1 - int(substep)
 
     def _field_args(self, state):
         args = []
@@ -260,7 +308,7 @@ class DimsplitSimulator(BaseSimulator):
         _lib.call("fvmi_memcpy_async", host.ctypes.data, self.cfl_data, 8, _lib.MEMCPY_DTOH, self.stream.handle)
         self.stream.synchronize()
         # float32 minimum promoted to double as the reference's 0-d array times 0.5
-        return float(host[1]) * 0.5
+        return float(host[self.cfl_last]) * 0.5
 
     def __del__(self):
         ptr = getattr(self, "cfl_data", None)

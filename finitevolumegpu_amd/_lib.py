@@ -6,6 +6,7 @@ There is no fallback: if the shared library is missing or cannot be loaded,
 
 import ctypes
 import os
+import struct
 
 import numpy as np
 
@@ -35,6 +36,19 @@ class RegionCopy(ctypes.Structure):
     """fvmi_region_copy_t"""
     _fields_ = [("src", c_void_p), ("dst", c_void_p), ("src_pitch", c_int), ("dst_pitch", c_int),
                 ("width", c_int), ("height", c_int)]
+
+
+class StepArgs(ctypes.Structure):
+    """fvmi_step_t"""
+    _fields_ = [("scheme", c_int), ("nx", c_int), ("ny", c_int), ("boundary_conditions", c_int),
+                ("dx", c_float), ("dy", c_float), ("dt", c_float), ("g", c_float), ("theta", c_float),
+                ("gamma", c_float), ("state", (c_void_p * 4) * 2), ("pitch", (c_int * 4) * 2),
+                ("cfl", c_void_p), ("cfl_slot", c_int)]
+
+
+# fvmi_step_t as one pack: the fields in order, state pointers and pitches of
+# both buffers (native alignment)
+STEP_PACK = struct.Struct("@4i6f8P8iPi")
 
 
 class Instance(ctypes.Structure):
@@ -123,6 +137,7 @@ SIGNATURES = {
                                + [c_void_p, c_int] * 6 + [c_void_p, c_int, P(LaunchConfig), c_void_p]),
     "fvmi_swe_kp07_substep": (c_int, [c_int, c_int, c_float, c_float, c_float, c_float, c_float, c_int, c_int]
                               + [c_void_p, c_int] * 6 + [c_void_p, c_int, P(LaunchConfig), c_void_p]),
+    "fvmi_dimsplit_step": (c_int, [c_void_p, P(LaunchConfig), c_void_p, c_void_p, c_void_p]),
     "fvmi_halo_copy_periodic_x": (c_int, [c_int, c_int, c_int, P(c_void_p), P(c_int), c_void_p]),
     "fvmi_halo_exchange_periodic": (c_int, [c_int, c_int, c_int, P(c_void_p), P(c_int), c_int, c_int, c_void_p]),
     "fvmi_field_stats": (c_int, [c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p]),

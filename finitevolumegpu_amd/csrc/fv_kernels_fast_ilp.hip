@@ -19,6 +19,16 @@ hipError_t launch_substep_fast_ilp(int scheme, const SubstepArgs& a, int grid, h
             return hipErrorInvalidValue;
     }
 }
+hipError_t launch_step_fast_ilp(int scheme, const SubstepArgs& a, int grid, hipStream_t stream) {
+    switch (scheme) {
+        case SCHEME_KP07:
+            return launch_step_scheme<StepKP07, MathFast>(a, grid, stream);
+        case SCHEME_HLL2:
+            return launch_step_scheme<StepHLL2, MathFast>(a, grid, stream);
+        default:
+            return hipErrorInvalidValue;
+    }
+}
 hipError_t launch_ensemble_fast_ilp(int scheme, const EnsembleArgs& e, int grid, hipStream_t stream) {
     switch (scheme) {
         case SCHEME_KP07:

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include "fv_ensemble.h"
+#include "fv_step.h"
 #include "fv_substep.h"
 
 namespace fvmi {
@@ -25,6 +26,31 @@ inline int scheme_cols_per_lane(int scheme, int math) {
 inline int scheme_strip_cols(int scheme, int math) {
     return scheme_cols_per_lane(scheme, math) == 2 ? strip_cols<2>() : strip_cols<1>();
 }
+
+// The whole-step kernels (one column per lane).
+using StepKP07 = SweKP07<MathFast, 1>;
+using StepHLL2 = SweHLL2<MathFast, 1>;
+using StepEuler = EulerKP07<MathFast, 1>;
+
+// Whether a whole step of this grid is one launch (fv_step.h).  Fast arithmetic
+// only: the exact kernels and WAF are bound by VALU issue already as substeps
+// (4096^2: 184 us for KP07_dimsplit, 260 for WAF, against 79 us for their
+// bytes), so that the wider halo would cost more than the memory passes saved.
+inline bool step_is_fused(int scheme, int math, const SubstepArgs& a) {
+    if (math == FVMI_MATH_EXACT || scheme == SCHEME_WAF) return false;
+    if (a.nx < kStepMinSide || a.ny < kStepMinSide) return false;
+    if (a.seg_rows > 0 && a.seg_rows < kStepMinSegRows) return false;
+    const int w = a.bc & 0xF, e = (a.bc >> 8) & 0xF, s = (a.bc >> 16) & 0xF, n = (a.bc >> 24) & 0xF;
+    if (w == BC_DIRICHLET || e == BC_DIRICHLET || s == BC_DIRICHLET || n == BC_DIRICHLET) return false;
+    // a periodic edge opposite to another kind wraps to cells whose own
+    // neighbours are that kind's ghosts, which the images marched along are not
+    return (w == BC_PERIODIC) == (e == BC_PERIODIC) && (s == BC_PERIODIC) == (n == BC_PERIODIC);
+}
+
+// Segments of a whole step re-sweep about 4 rows' worth of halo, twice a
+// substep's: at least 40 rows where the grid has them (HLL2 2047^2 step of one
+// simulator 93 us with 24, 81 with 40; of three in turn 57.7 and 55.0).
+constexpr int kStepMinSeg = 40;
 
 // Fills the decomposition fields of `a` (sub-area, launch shape, device size)
 // and returns the grid size to launch.  seg_rows == 0 picks the shape:
@@ -102,6 +128,12 @@ hipError_t launch_substep(int scheme, SubstepArgs a, int grid, hipStream_t strea
 }
 
 template <class S, class M>
+hipError_t launch_step_scheme(const SubstepArgs& a, int grid, hipStream_t stream) {
+    hipLaunchKernelGGL((step_kernel<S, M>), dim3(grid), dim3(kLanes * a.waves_per_block), 0, stream, a);
+    return hipGetLastError();
+}
+
+template <class S, class M>
 hipError_t launch_ensemble_scheme(const EnsembleArgs& e, int grid, hipStream_t stream) {
     hipLaunchKernelGGL((ensemble_substep_kernel<S, M>), dim3(grid), dim3(kLanes * e.waves_per_block), 0, stream, e);
     return hipGetLastError();
@@ -136,6 +168,8 @@ hipError_t launch_substep_exact(int scheme, const SubstepArgs& a, int grid, hipS
 hipError_t launch_substep_fast(int scheme, const SubstepArgs& a, int grid, hipStream_t stream);
 // KP07_dimsplit and HLL2 in fast arithmetic, single grid and ensemble
 // (fv_kernels_fast_ilp.hip, built with the ILP-maximising scheduler)
+hipError_t launch_step_fast(int scheme, const SubstepArgs& a, int grid, hipStream_t stream);
+hipError_t launch_step_fast_ilp(int scheme, const SubstepArgs& a, int grid, hipStream_t stream);
 hipError_t launch_substep_fast_ilp(int scheme, const SubstepArgs& a, int grid, hipStream_t stream);
 hipError_t launch_ensemble_fast_ilp(int scheme, const EnsembleArgs& e, int grid, hipStream_t stream);
 

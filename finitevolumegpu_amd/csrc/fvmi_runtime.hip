@@ -84,7 +84,8 @@ int fill_launch(const fvmi_launch_t* l, SubstepArgs& a, int* math) {
     return FVMI_OK;
 }
 
-int run_substep(int scheme, SubstepArgs& a, int nvars, const fvmi_launch_t* launch, void* stream) {
+// Checks a launch's arguments and fills the fields of `a` that follow from them.
+int check_substep(int scheme, SubstepArgs& a, int nvars, const fvmi_launch_t* launch, int* math_out) {
     if (a.nx < 2 || a.ny < 2) return fail(FVMI_ERR_INVALID, "grid %dx%d too small (need nx, ny >= 2)", a.nx, a.ny);
     if ((size_t)(a.ny + 4) * (size_t)(a.nx + 4) > (size_t)1 << 30)
         return fail(FVMI_ERR_INVALID, "grid %dx%d too large", a.nx, a.ny);
@@ -128,6 +129,13 @@ int run_substep(int scheme, SubstepArgs& a, int nvars, const fvmi_launch_t* laun
     a.dtdx = a.dt / a.dx;
     a.dtdy = a.dt / a.dy;
     set_slope_constants(a);
+    *math_out = math;
+    return FVMI_OK;
+}
+
+int run_substep(int scheme, SubstepArgs& a, int nvars, const fvmi_launch_t* launch, void* stream) {
+    int math = 0;
+    if (int rc = check_substep(scheme, a, nvars, launch, &math)) return rc;
     a.strip_cols = scheme_strip_cols(scheme, math);
     // WAF keeps equal segments: the round-weighted plan made it 3 % slower
     const int grid = plan_substep(a, current_cu_count(), scheme != SCHEME_WAF);
@@ -645,6 +653,46 @@ int fvmi_euler_kp07_dimsplit_substep(int nx, int ny, float dx, float dy, float d
     a.cfl = cfl;
     a.x0 = x0, a.y0 = y0, a.x1 = x1, a.y1 = y1;
     return run_substep(SCHEME_EULER, a, 4, launch, stream);
+}
+
+int fvmi_dimsplit_step(const fvmi_step_t* p, const fvmi_launch_t* launch, int* state_out, int* cfl_slot_out,
+                       void* stream) {
+    if (!p || !state_out || !cfl_slot_out) return fail(FVMI_ERR_INVALID, "NULL argument");
+    if (p->scheme < SCHEME_KP07 || p->scheme > SCHEME_EULER)
+        return fail(FVMI_ERR_INVALID, "unknown scheme %d", p->scheme);
+    if (p->cfl_slot != 0 && p->cfl_slot != 1) return fail(FVMI_ERR_INVALID, "cfl_slot must be 0 or 1");
+    const int nvars = p->scheme == SCHEME_EULER ? 4 : 3;
+    auto args = [&](int from, int step) {
+        SubstepArgs a{};
+        a.nx = p->nx, a.ny = p->ny, a.dx = p->dx, a.dy = p->dy, a.dt = p->dt;
+        a.g = p->g, a.theta = p->theta, a.gamma = p->gamma;
+        a.step = step, a.bc = p->boundary_conditions;
+        for (int k = 0; k < nvars; ++k) {
+            a.in[k] = p->state[from][k], a.in_pitch[k] = p->pitch[from][k];
+            a.out[k] = p->state[1 - from][k], a.out_pitch[k] = p->pitch[1 - from][k];
+        }
+        a.cfl = p->cfl;
+        return a;
+    };
+    int math = 0;
+    SubstepArgs a = args(0, 0);
+    if (int rc = check_substep(p->scheme, a, nvars, launch, &math)) return rc;
+    if (!step_is_fused(p->scheme, math, a)) {
+        if (int rc = run_substep(p->scheme, a, nvars, launch, stream)) return rc;
+        SubstepArgs b = args(1, 1);
+        if (int rc = run_substep(p->scheme, b, nvars, launch, stream)) return rc;
+        *state_out = 0;
+        *cfl_slot_out = 1;
+        return FVMI_OK;
+    }
+    a.cfl_slot = p->cfl_slot;
+    a.strip_cols = strip_cols<1, kStepHalo>();
+    const int grid = plan_substep(a, current_cu_count(), true, 4, kStepMinSeg);
+    hipError_t e = launch_step_fast(p->scheme, a, grid, (hipStream_t)stream);
+    if (e != hipSuccess) return hip_fail(e, "step launch");
+    *state_out = 1;
+    *cfl_slot_out = p->cfl_slot;
+    return FVMI_OK;
 }
 
 int fvmi_halo_exchange_periodic(int nx, int ny, int nvars, float* const* fields, const int* pitches, int wrap_x,

@@ -188,6 +188,42 @@ int fvmi_euler_kp07_dimsplit_substep(int nx, int ny, float dx, float dy, float d
                                      float* cfl, int x0, int y0, int x1, int y1, const fvmi_launch_t* launch,
                                      void* stream);
 
+/* One full step of a dimensionally split scheme (SchemeId of
+ * fvmi_ensemble_substep): substep 0 (x then y) and substep 1 (y then x), each
+ * of length `dt`, as BaseSimulator.step runs them (Simulator.py:220-228).
+ * state[0] holds the fields on entry (rho or h, the two momenta, E for Euler),
+ * with pitches in bytes; on return *state_out (0 or 1) says which of the two
+ * buffers the new state is in.  The interior of the other one is then either
+ * the state before the step or the one between the substeps.
+ *
+ * The KP07_dimsplit, HLL2 and Euler steps in fast arithmetic are one launch
+ * that reads and writes the state once (grids of at least 8 x 8 cells, no
+ * Dirichlet edge, no periodic edge opposite to another kind, tile_rows 0 or at
+ * least 4); every other step is the two substep launches.  The fields and the CFL minimum are the same either way.
+ *
+ * cfl (may be NULL): two floats, of which slot `cfl_slot` holds +inf on entry.
+ * On return the CFL minimum of the new state is in slot *cfl_slot_out and the
+ * other slot holds +inf (pass it to the next step). */
+typedef struct fvmi_step {
+    int scheme;
+    int nx;
+    int ny;
+    int boundary_conditions;
+    float dx;
+    float dy;
+    float dt;
+    float g;
+    float theta;
+    float gamma;
+    float* state[2][4];
+    int pitch[2][4];
+    float* cfl;
+    int cfl_slot;
+} fvmi_step_t;
+
+int fvmi_dimsplit_step(const fvmi_step_t* p, const fvmi_launch_t* launch, int* state_out, int* cfl_slot_out,
+                       void* stream);
+
 /* One-rank stand-in for MPISimulator.full_exchange's east/west leg
  * (MPISimulator.py:283-295, 440-480) with a periodic-x neighbour: for each of
  * the `nvars` fields copy padded columns [nx, nx+2) -> [0, 2) and

@@ -1,0 +1,170 @@
+"""Simulator.step (one library call, one launch for the slope schemes in fast
+arithmetic) against its two substeps run one by one: the fields and the CFL
+minimum are equal bitwise.  Sizes at the edges of a strip of the whole-step
+march (56 output columns, 120 with two columns per lane), smallest sides,
+segments as short as they may be, and every kind of edge."""
+
+import itertools
+
+import numpy as np
+import pytest
+
+from oracle import fv_oracle as O
+from tests._cases import make_gpu_sim, state
+
+pytestmark = pytest.mark.gpu
+
+R, P, F, D = O.REFLECTIVE, O.PERIODIC, O.OUTFLOW, O.DIRICHLET
+
+BOUNDARIES = {
+    "reflective": O.pack_bc(R, R, R, R),
+    "periodic": O.pack_bc(P, P, P, P),
+    "outflow": O.pack_bc(F, F, F, F),
+    "mixed": O.pack_bc(R, F, F, R),
+    "channel": O.pack_bc(F, R, P, P),
+}
+
+SIZES = [(8, 8), (9, 11), (55, 12), (56, 8), (57, 30), (59, 9), (60, 64), (113, 65), (120, 17), (121, 40), (123, 8),
+         (241, 133)]
+
+CASES = [("kp07_dimsplit", "fast"), ("hll2", "fast"), ("ee2d_kp07_dimsplit", "fast"),
+         ("ee2d_kp07_dimsplit", "exact"), ("waf", "exact")]
+
+
+def run_pair(ctx, scheme, nx, ny, bc, math, steps=3, **kw):
+    fields = state(scheme, nx, ny, seed=nx + 7 * ny)
+    a = make_gpu_sim(ctx, scheme, fields, nx, ny, 1.0, 1.0, bc, math=math, **kw)
+    b = make_gpu_sim(ctx, scheme, fields, nx, ny, 1.0, 1.0, bc, math=math, **kw)
+    dt = np.float32(0.05) if scheme == "ee2d_kp07_dimsplit" else np.float32(0.9 * a.computeDt())
+    for n in range(steps):
+        a.step(dt)
+        for i in range(2):
+            b.substep(dt, i)
+        assert a.computeDt() == b.computeDt(), (n, a.computeDt(), b.computeDt())
+        for k, (x, y) in enumerate(zip(a.download(), b.download())):
+            assert np.array_equal(x, y), (n, k, np.argwhere(x != y)[:5].tolist())
+    return a, b, dt
+
+
+@pytest.mark.parametrize("bc", sorted(BOUNDARIES))
+@pytest.mark.parametrize("scheme,math", CASES)
+def test_step_equals_its_substeps(ctx, scheme, math, bc):
+    sizes = SIZES if math == "fast" else SIZES[-2:]
+    for nx, ny in sizes:
+        print("case step", scheme, math, bc, nx, ny, flush=True)
+        run_pair(ctx, scheme, nx, ny, BOUNDARIES[bc], math)
+
+
+@pytest.mark.parametrize("scheme", ["kp07_dimsplit", "ee2d_kp07_dimsplit"])
+def test_step_with_every_combination_of_edges(ctx, scheme):
+    """All 256 combinations of the four edge kinds, those that take one launch
+    and those that take two."""
+    nx, ny = 61, 18
+    frame = (1.05, 0.01, -0.01, 6.5)
+    fields = state(scheme, nx, ny, seed=4)
+    pads = []
+    for k, f in enumerate(fields):
+        pad = np.full((ny + 4, nx + 4), frame[k], dtype=np.float32)
+        pad[2:-2, 2:-2] = f
+        pads.append(pad)
+    print("case step edges", scheme, flush=True)
+    for code in itertools.product((D, P, R, F), repeat=4):
+        out = []
+        for whole in (True, False):
+            sim = make_gpu_sim(ctx, scheme, fields, nx, ny, 1.0, 1.0, O.pack_bc(*code))
+            for buf in (sim.u0, sim.u1):  # ghost memory that Dirichlet edges read
+                for k, pad in enumerate(pads):
+                    buf[k].upload(sim.stream, pad, extent=[0, 0, nx + 4, ny + 4])
+            if whole:
+                sim.step(np.float32(0.04))
+            else:
+                sim.substep(np.float32(0.04), 0)
+                sim.substep(np.float32(0.04), 1)
+            out.append(sim.download() + [np.float32(sim.computeDt())])
+        assert all(np.array_equal(x, y) for x, y in zip(*out)), code
+
+
+@pytest.mark.parametrize("scheme", ["kp07_dimsplit", "ee2d_kp07_dimsplit"])
+@pytest.mark.parametrize("tile_rows,waves", [(4, 4), (5, 1), (9, 2), (3, 4), (64, 3)])
+def test_step_of_any_launch_shape(ctx, scheme, tile_rows, waves):
+    for nx, ny in ((70, 45), (250, 61)):
+        print("case step shape", scheme, nx, ny, tile_rows, waves, flush=True)
+        run_pair(ctx, scheme, nx, ny, BOUNDARIES["mixed"], "fast", tile_rows=tile_rows, waves_per_block=waves)
+
+
+@pytest.mark.parametrize("scheme,nx,ny", [("kp07_dimsplit", 4096, 2050), ("hll2", 2300, 4095),
+                                          ("ee2d_kp07_dimsplit", 3001, 4032)])
+@pytest.mark.parametrize("bc", ["mixed", "periodic"])
+def test_step_with_the_round_weighted_split(ctx, scheme, nx, ny, bc):
+    print("case step rounds", scheme, nx, ny, bc, flush=True)
+    run_pair(ctx, scheme, nx, ny, BOUNDARIES[bc], "fast", steps=2)
+
+
+def test_step_and_substeps_in_turn(ctx):
+    """Whole steps and single substeps of one simulator, in any order, leave
+    the CFL minimum of the last step and the same state."""
+    a, b, dt = run_pair(ctx, "kp07_dimsplit", 64, 40, BOUNDARIES["reflective"], "fast")
+    for whole in (False, True, True, False, True):
+        if whole:
+            a.step(dt)
+        else:
+            a.substep(dt, 0)
+            a.substep(dt, 1)
+        b.substep(dt, 0)
+        b.substep(dt, 1)
+        assert a.computeDt() == b.computeDt()
+    assert all(np.array_equal(x, y) for x, y in zip(a.download(), b.download()))
+
+
+def test_dirichlet_edges_read_both_buffers(ctx):
+    """A Dirichlet edge reads each substep's own input buffer, so its step
+    takes the substep launches: different ghost values in the two buffers."""
+    nx, ny = 70, 50
+    bc = O.pack_bc(D, R, R, D)
+    sims = [make_gpu_sim(ctx, "kp07_dimsplit", state("kp07_dimsplit", nx, ny, 5), nx, ny, 1.0, 1.0, bc)
+            for _ in range(2)]
+    for sim in sims:
+        for j, buf in enumerate((sim.u0, sim.u1)):
+            for k, v in enumerate((1.0 + 0.1 * j, 0.02 * j, -0.01)):
+                pad = np.full((ny + 4, nx + 4), v, dtype=np.float32)
+                pad[2:-2, 2:-2] = buf[k].download(sim.stream)
+                buf[k].upload(sim.stream, pad, extent=[0, 0, nx + 4, ny + 4])
+    for _ in range(4):
+        sims[0].step(np.float32(0.08))
+        for i in range(2):
+            sims[1].substep(np.float32(0.08), i)
+    assert all(np.array_equal(x, y) for x, y in zip(sims[0].download(), sims[1].download()))
+    assert sims[0].computeDt() == sims[1].computeDt()
+
+
+def test_subclass_with_its_own_substep_is_called(ctx):
+    from finitevolumegpu_amd.KP07_dimsplit import KP07_dimsplit
+
+    class Counting(KP07_dimsplit):
+        calls = 0
+
+        def substep(self, dt, step_number):
+            self.calls += 1
+            super().substep(dt, step_number)
+
+    sim = Counting(ctx, *state("kp07_dimsplit", 32, 32, 1), 32, 32, 1.0, 1.0, 9.81)
+    sim.step(np.float32(0.05))
+    assert sim.calls == 2
+
+
+@pytest.mark.parametrize("math", ["fast", "exact"])
+def test_mpi_step_equals_exchange_between_substeps(ctx, math):
+    from finitevolumegpu_amd.MPISimulator import MPISimulator
+    nx, ny = 130, 75
+    sims = [MPISimulator(make_gpu_sim(ctx, "ee2d_kp07_dimsplit", state("ee2d_kp07_dimsplit", nx, ny, 2), nx, ny, 1.0,
+                                      1.0, BOUNDARIES["channel"], math=math)) for _ in range(2)]
+    dt = np.float32(0.05)
+    for _ in range(3):
+        sims[0].step(dt)
+        for i in range(2):
+            sims[1].substep(dt, i)
+        padded = [[v.download(s.stream, extent=[0, 0, nx + 4, ny + 4]) for v in s.getOutput().gpu_variables]
+                  for s in sims]
+        assert all(np.array_equal(x, y) for x, y in zip(*padded))
+    assert sims[0].computeDt() == sims[1].computeDt()
+    assert sims[0].profiling_data_mpi["n_time_steps"] == sims[1].profiling_data_mpi["n_time_steps"]
