@@ -12,35 +12,14 @@
 
 #include <hip/hip_runtime.h>
 
+#include "fv_math.h"
+
 namespace fvmi {
 namespace fast {
 
 __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ __forceinline__ float rsq(float x) { return __builtin_amdgcn_rsqf(x); }
 __device__ __forceinline__ float sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
-
-// One transcendental of several values, issued as one run: a lone one among
-// other VALU instructions costs two to three times its place in a run (the two
-// waves that a SIMD issues from in turn fall out of step at each change).
-// s_nop: a transcendental's result may not be read by the next instruction,
-// which the compiler does not see inside the block.
-#define FVMI_TRANS_RUN(name, one, op)                                                                                    \
-    template <int N>                                                                                                \
-    __device__ __forceinline__ void name(const float (&x)[N], float (&r)[N]) {                                      \
-        static_assert(N == 1 || N == 2 || N == 4, "runs of 1, 2 or 4");                                             \
-        if constexpr (N == 1)                                                                                       \
-            r[0] = one(x[0]);                                                                                       \
-        else if constexpr (N == 2)                                                                                  \
-            asm(op " %0, %2\n\t" op " %1, %3\n\ts_nop 0" : "=&v"(r[0]), "=v"(r[1]) : "v"(x[0]), "v"(x[1]));       \
-        else                                                                                                        \
-            asm(op " %0, %4\n\t" op " %1, %5\n\t" op " %2, %6\n\t" op " %3, %7\n\ts_nop 0"                       \
-                : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=v"(r[3])                                                 \
-                : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]));                                                      \
-    }
-FVMI_TRANS_RUN(rcp_all, rcp, "v_rcp_f32")
-FVMI_TRANS_RUN(rsq_all, rsq, "v_rsq_f32")
-FVMI_TRANS_RUN(sqrt_all, sqrt, "v_sqrt_f32")
-#undef FVMI_TRANS_RUN
 
 // Predictor difference F(QL) - F(QR) of the SWE flux (SWECommon.h:29-37), one
 // reciprocal r = 1/(QL0 QR0) for both faces.  The faces are h0 -/+ (theta/2) m0

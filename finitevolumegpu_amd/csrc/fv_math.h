@@ -21,6 +21,33 @@
 
 namespace fvmi {
 
+// One transcendental of several values, issued as one run: a lone one among
+// other VALU instructions costs two to three times its place in a run (the two
+// waves that a SIMD issues from in turn fall out of step at each change).
+// s_nop: a transcendental's result may not be read by the next instruction,
+// which the compiler does not see inside the block.
+#define FVMI_TRANS_RUN(name, one, op)                                                                                    \
+    template <int N>                                                                                                \
+    __device__ __forceinline__ void name(const float (&x)[N], float (&r)[N]) {                                      \
+        static_assert(N >= 1 && N <= 4, "runs of 1 to 4");                                                          \
+        if constexpr (N == 1)                                                                                       \
+            r[0] = one(x[0]);                                                                                       \
+        else if constexpr (N == 2)                                                                                  \
+            asm(op " %0, %2\n\t" op " %1, %3\n\ts_nop 0" : "=&v"(r[0]), "=v"(r[1]) : "v"(x[0]), "v"(x[1]));       \
+        else if constexpr (N == 3)                                                                                  \
+            asm(op " %0, %3\n\t" op " %1, %4\n\t" op " %2, %5\n\ts_nop 0"                                        \
+                : "=&v"(r[0]), "=&v"(r[1]), "=v"(r[2])                                                              \
+                : "v"(x[0]), "v"(x[1]), "v"(x[2]));                                                                 \
+        else                                                                                                        \
+            asm(op " %0, %4\n\t" op " %1, %5\n\t" op " %2, %6\n\t" op " %3, %7\n\ts_nop 0"                       \
+                : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=v"(r[3])                                                 \
+                : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]));                                                      \
+    }
+FVMI_TRANS_RUN(rcp_all, __builtin_amdgcn_rcpf, "v_rcp_f32")
+FVMI_TRANS_RUN(rsq_all, __builtin_amdgcn_rsqf, "v_rsq_f32")
+FVMI_TRANS_RUN(sqrt_all, __builtin_amdgcn_sqrtf, "v_sqrt_f32")
+#undef FVMI_TRANS_RUN
+
 // Correctly rounded float32 division and square root in fewer instructions
 // than the compiler's general IEEE sequences, for operands in the normal range
 // (no scaling for denormal or overflowing intermediates, no special-case
@@ -49,20 +76,41 @@ __device__ __forceinline__ float rcp_rn(float b) {
     const float y = __builtin_amdgcn_rcpf(b);
     return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
 }
-__device__ __forceinline__ float quot_rn(float a, float b) {
-    const float y = rcp_rn(b);
+// a / b with y = rcp_rn(b) known
+__device__ __forceinline__ float quot_rn(float a, float b, float y) {
     const float q = a * y;
     return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
 }
-__device__ __forceinline__ float div_rn(float a, float b) {
-    const float y = rcp_rn(b);
+__device__ __forceinline__ float div_rn(float a, float b, float y) {
     const float q = a * y;
     return __builtin_copysignf(__builtin_fmaf(__builtin_fmaf(-b, q, a), y, q), q);
 }
+__device__ __forceinline__ float quot_rn(float a, float b) { return quot_rn(a, b, rcp_rn(b)); }
+__device__ __forceinline__ float div_rn(float a, float b) { return div_rn(a, b, rcp_rn(b)); }
 __device__ __forceinline__ float sqrt_rn(float x) {
     const float y = __builtin_amdgcn_rsqf(x + 0x1p-126f);
     const float s = x * y;
     return __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
+}
+// the same of N values, their v_rcp / v_rsq in one run
+template <int N>
+__device__ __forceinline__ void rcp_rn_all(const float (&b)[N], float (&r)[N]) {
+    float y[N];
+    rcp_all<N>(b, y);
+#pragma unroll
+    for (int i = 0; i < N; ++i) r[i] = __builtin_fmaf(__builtin_fmaf(-b[i], y[i], 1.0f), y[i], y[i]);
+}
+template <int N>
+__device__ __forceinline__ void sqrt_rn_all(const float (&x)[N], float (&r)[N]) {
+    float b[N], y[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) b[i] = x[i] + 0x1p-126f;
+    rsq_all<N>(b, y);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const float s = x[i] * y[i];
+        r[i] = __builtin_fmaf(__builtin_fmaf(-s, s, x[i]), 0.5f * y[i], s);
+    }
 }
 
 struct MathExact {
@@ -107,8 +155,7 @@ __device__ __forceinline__ float generalized_minmod(float r, float theta) {
 // desingularize, common.h:81-83
 template <class M>
 __device__ __forceinline__ float desingularize(float x, float eps) {
-    return __builtin_copysignf(1.0f, x) *
-           fmaxf(fabsf(x), fminf(M::quot(x * x, 2.0f * eps) + 0.5f * eps, eps));
+    return __builtin_copysignf(fmaxf(fabsf(x), fminf(M::quot(x * x, 2.0f * eps) + 0.5f * eps, eps)), x);
 }
 
 // limiterToWAFLimiter, SWECommon.h:109-111
@@ -120,13 +167,13 @@ __device__ __forceinline__ float limiter_to_waf(float r, float c) {
 // Shallow water: GPUSimulators/cuda/SWECommon.h
 // ---------------------------------------------------------------------------
 
-// F_func, SWECommon.h:29-37.  SignedZero: F[2] keeps the sign of a zero (WAF).
-template <class M, bool SignedZero = false>
+// F_func, SWECommon.h:29-37
+template <class M>
 __device__ __forceinline__ void swe_F(const float q[3], float g, float F[3]) {
     if constexpr (M::exact) {
         F[0] = q[1];
         F[1] = M::quot(q[1] * q[1], q[0]) + 0.5f * g * q[0] * q[0];
-        F[2] = SignedZero ? M::div(q[1] * q[2], q[0]) : M::quot(q[1] * q[2], q[0]);
+        F[2] = M::quot(q[1] * q[2], q[0]);
     } else {
         const float u = q[1] * M::rcp(q[0]);
         F[0] = q[1];
@@ -135,79 +182,53 @@ __device__ __forceinline__ void swe_F(const float q[3], float g, float F[3]) {
     }
 }
 
+// The fluxes below are the exact policy's (the fast one's are in fv_fast.h).
+
 // CentralUpwindFlux, SWECommon.h:228-241.  qm = left state, qp = right state.
-template <class M>
 __device__ __forceinline__ void swe_cu_flux(const float qm[3], const float qp[3], float g, float out[3]) {
-    if constexpr (M::exact) {
-        float Fp[3], Fm[3];
-        swe_F<M>(qp, g, Fp);
-        const float up = M::quot(qp[1], qp[0]);
-        const float cp = M::sqrt(g * qp[0]);
-        swe_F<M>(qm, g, Fm);
-        const float um = M::quot(qm[1], qm[0]);
-        const float cm = M::sqrt(g * qm[0]);
-        const float am = fminf(fminf(um - cm, up - cp), 0.0f);
-        const float ap = fmaxf(fmaxf(um + cm, up + cp), 0.0f);
-        const float apam = ap * am;
-        const float den = ap - am;
+    const float h[2] = {qm[0], qp[0]}, gh[2] = {g * qm[0], g * qp[0]};
+    float y[2], c[2];
+    rcp_rn_all<2>(h, y);
+    sqrt_rn_all<2>(gh, c);
+    const float um = quot_rn(qm[1], qm[0], y[0]), up = quot_rn(qp[1], qp[0], y[1]);
+    const float Fm[3] = {qm[1], quot_rn(qm[1] * qm[1], qm[0], y[0]) + 0.5f * g * qm[0] * qm[0],
+                         quot_rn(qm[1] * qm[2], qm[0], y[0])};
+    const float Fp[3] = {qp[1], quot_rn(qp[1] * qp[1], qp[0], y[1]) + 0.5f * g * qp[0] * qp[0],
+                         quot_rn(qp[1] * qp[2], qp[0], y[1])};
+    const float am = fminf(fminf(um - c[0], up - c[1]), 0.0f);
+    const float ap = fmaxf(fmaxf(um + c[0], up + c[1]), 0.0f);
+    const float apam = ap * am;
+    const float den = ap - am, iden = rcp_rn(den);
 #pragma unroll
-        for (int k = 0; k < 3; ++k) out[k] = M::quot((ap * Fm[k] - am * Fp[k]) + apam * (qp[k] - qm[k]), den);
-    } else {
-        const float ip = M::rcp(qp[0]);
-        const float im = M::rcp(qm[0]);
-        const float up = qp[1] * ip, um = qm[1] * im;
-        const float cp = M::sqrt(g * qp[0]), cm = M::sqrt(g * qm[0]);
-        const float hg = 0.5f * g;
-        const float Fp[3] = {qp[1], qp[1] * up + hg * qp[0] * qp[0], qp[2] * up};
-        const float Fm[3] = {qm[1], qm[1] * um + hg * qm[0] * qm[0], qm[2] * um};
-        const float am = fminf(fminf(um - cm, up - cp), 0.0f);
-        const float ap = fmaxf(fmaxf(um + cm, up + cp), 0.0f);
-        const float apam = ap * am;
-        const float iden = M::rcp(ap - am);
-#pragma unroll
-        for (int k = 0; k < 3; ++k) out[k] = ((ap * Fm[k] - am * Fp[k]) + apam * (qp[k] - qm[k])) * iden;
-    }
+    for (int k = 0; k < 3; ++k) out[k] = quot_rn((ap * Fm[k] - am * Fp[k]) + apam * (qp[k] - qm[k]), den, iden);
 }
 
 // HLL_flux (SWE), SWECommon.h:274-313
-template <class M>
 __device__ __forceinline__ void swe_hll_flux(const float ql[3], const float qr[3], float g, float out[3]) {
     const float h_l = ql[0], h_r = qr[0];
-    float u_l, u_r;
-    if constexpr (M::exact) {
-        u_l = M::quot(ql[1], h_l);
-        u_r = M::quot(qr[1], h_r);
-    } else {
-        u_l = ql[1] * M::rcp(h_l);
-        u_r = qr[1] * M::rcp(h_r);
-    }
-    const float c_l = M::sqrt(g * h_l);
-    const float c_r = M::sqrt(g * h_r);
-    const float h_dag = 0.5f * (h_l + h_r) - M::quot(0.25f * (u_r - u_l) * (h_l + h_r), c_l + c_r);
-    const float q_l_tmp = M::sqrt(0.5f * M::quot((h_dag + h_l) * h_dag, h_l * h_l));
-    const float q_r_tmp = M::sqrt(0.5f * M::quot((h_dag + h_r) * h_dag, h_r * h_r));
+    const float h[2] = {h_l, h_r}, gh[2] = {g * h_l, g * h_r};
+    float y[2], c[2];
+    rcp_rn_all<2>(h, y);
+    sqrt_rn_all<2>(gh, c);
+    const float u_l = quot_rn(ql[1], h_l, y[0]), u_r = quot_rn(qr[1], h_r, y[1]);
+    const float c_l = c[0], c_r = c[1];
+    const float h_dag = 0.5f * (h_l + h_r) - quot_rn(0.25f * (u_r - u_l) * (h_l + h_r), c_l + c_r);
+    const float q_l_tmp = sqrt_rn(0.5f * quot_rn((h_dag + h_l) * h_dag, h_l * h_l));
+    const float q_r_tmp = sqrt_rn(0.5f * quot_rn((h_dag + h_r) * h_dag, h_r * h_r));
     const float q_l = (h_dag > h_l) ? q_l_tmp : 1.0f;
     const float q_r = (h_dag > h_r) ? q_r_tmp : 1.0f;
     const float S_l = u_l - c_l * q_l;
     const float S_r = u_r + c_r * q_r;
-    float F_l[3], F_r[3];
-    swe_F<M>(ql, g, F_l);
-    swe_F<M>(qr, g, F_r);
+    const float F_l[3] = {ql[1], quot_rn(ql[1] * ql[1], h_l, y[0]) + 0.5f * g * h_l * h_l,
+                          quot_rn(ql[1] * ql[2], h_l, y[0])};
+    const float F_r[3] = {qr[1], quot_rn(qr[1] * qr[1], h_r, y[1]) + 0.5f * g * h_r * h_r,
+                          quot_rn(qr[1] * qr[2], h_r, y[1])};
     const float srsl = S_r * S_l;
-    if constexpr (M::exact) {
-        const float den = S_r - S_l;
+    const float den = S_r - S_l, iden = rcp_rn(den);
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const float star = M::quot(S_r * F_l[k] - S_l * F_r[k] + srsl * (qr[k] - ql[k]), den);
-            out[k] = (S_l >= 0.0f) ? F_l[k] : ((S_r <= 0.0f) ? F_r[k] : star);
-        }
-    } else {
-        const float iden = M::rcp(S_r - S_l);
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const float star = (S_r * F_l[k] - S_l * F_r[k] + srsl * (qr[k] - ql[k])) * iden;
-            out[k] = (S_l >= 0.0f) ? F_l[k] : ((S_r <= 0.0f) ? F_r[k] : star);
-        }
+    for (int k = 0; k < 3; ++k) {
+        const float star = quot_rn(S_r * F_l[k] - S_l * F_r[k] + srsl * (qr[k] - ql[k]), den, iden);
+        out[k] = (S_l >= 0.0f) ? F_l[k] : ((S_r <= 0.0f) ? F_r[k] : star);
     }
 }
 
@@ -232,38 +253,34 @@ __device__ __forceinline__ float compute_h_star(float h_l, float h_r, float u_l,
 struct WafCell {
     float h, hu, hv;  // state in sweep order (depth, normal, tangential momentum)
     float u, v, c;    // normal and tangential velocity, sqrt(g h)
-    float ih;         // 1/h (fast policy only)
+    float ih;         // 1/h
+    float f1, f2;     // fluxes of the normal and tangential momentum (that of h is hu)
 };
 
+// hg = g/2
 template <class M>
-__device__ __forceinline__ WafCell waf_cell(const float q[3], float g, float sqrt_g) {
+__device__ __forceinline__ WafCell waf_cell(const float q[3], float g, float hg, float sqrt_g) {
     WafCell p;
     p.h = q[0];
     p.hu = q[1];
     p.hv = q[2];
     if constexpr (M::exact) {
-        p.u = M::div(q[1], q[0]);
-        p.v = M::div(q[2], q[0]);
-        p.c = M::sqrt(g * q[0]);
-        p.ih = 0.0f;
+        p.ih = rcp_rn(p.h);
+        p.u = div_rn(p.hu, p.h, p.ih);
+        p.v = div_rn(p.hv, p.h, p.ih);
+        p.c = M::sqrt(g * p.h);
+        p.f1 = quot_rn(p.hu * p.hu, p.h, p.ih) + hg * p.h * p.h;
+        p.f2 = div_rn(p.hu * p.hv, p.h, p.ih);
     } else {
-        const float s = __builtin_amdgcn_rsqf(q[0]);
+        const float s = __builtin_amdgcn_rsqf(p.h);
         p.ih = s * s;
-        p.u = q[1] * p.ih;
-        p.v = q[2] * p.ih;
-        p.c = sqrt_g * q[0] * s;
+        p.u = p.hu * p.ih;
+        p.v = p.hv * p.ih;
+        p.c = sqrt_g * p.h * s;
+        p.f1 = p.hu * p.u + hg * p.h * p.h;
+        p.f2 = p.hv * p.u;
     }
     return p;
-}
-
-// the cell seen by the other sweep direction (normal and tangential swapped)
-__device__ __forceinline__ WafCell waf_transpose(const WafCell& p) {
-    WafCell t = p;
-    t.hu = p.hv;
-    t.hv = p.hu;
-    t.u = p.v;
-    t.v = p.u;
-    return t;
 }
 
 // computeHStar (SWECommon.h:114-121) of the interface between l and r
@@ -314,42 +331,49 @@ __device__ __forceinline__ WafDen waf_den(const WafCell& l, const WafCell& r, fl
 // the interfaces to its left (Dl) and right (Dr).  dtd = dt / d (fast policy).
 template <class M>
 __device__ __forceinline__ void waf_flux_core(const WafCell& L, const WafCell& R, const WafDen& Dl, const WafDen& D,
-                                              const WafDen& Dr, float h_dag, float g, float hg, float d, float dt,
-                                              float dtd, float out[3]) {
+                                              const WafDen& Dr, float h_dag, float d, float dt, float dtd,
+                                              float out[3]) {
     const float h_l = L.h, h_r = R.h, u_l = L.u, u_r = R.u, v_l = L.v, v_r = R.v, c_l = L.c, c_r = R.c;
     const float q_l1[3] = {L.h, L.hu, L.hv};
     const float q_r1[3] = {R.h, R.hu, R.hv};
+    const float F_1[3] = {L.hu, L.f1, L.f2};
+    const float F_4[3] = {R.hu, R.f1, R.f2};
     if constexpr (M::exact) {
-        const float q_l_tmp = M::quot(M::sqrt(0.5f * ((h_dag + h_l) * h_dag)), h_l);
-        const float q_r_tmp = M::quot(M::sqrt(0.5f * ((h_dag + h_r) * h_dag)), h_r);
-        const float q_l = (h_dag > h_l) ? q_l_tmp : 1.0f;
-        const float q_r = (h_dag > h_r) ? q_r_tmp : 1.0f;
+        const float q_arg[2] = {0.5f * ((h_dag + h_l) * h_dag), 0.5f * ((h_dag + h_r) * h_dag)};
+        float q_tmp[2];
+        sqrt_rn_all<2>(q_arg, q_tmp);
+        const float q_l = (h_dag > h_l) ? quot_rn(q_tmp[0], h_l, L.ih) : 1.0f;
+        const float q_r = (h_dag > h_r) ? quot_rn(q_tmp[1], h_r, R.ih) : 1.0f;
         const float S_l = u_l - c_l * q_l;
         const float S_r = u_r + c_r * q_r;
-        const float S_star = M::div(S_l * h_r * (u_r - S_r) - S_r * h_l * (u_l - S_l),
-                                    h_r * (u_r - S_r) - h_l * (u_l - S_l));
-        const float s_l = M::div(h_l * (S_l - u_l), S_l - S_star);
-        const float s_r = M::div(h_r * (S_r - u_r), S_r - S_star);
+        const float dl = h_l * (u_l - S_l), dr = h_r * (u_r - S_r);
+        const float S_star = M::div(S_l * h_r * (u_r - S_r) - S_r * h_l * (u_l - S_l), dr - dl);
+        const float e[2] = {S_l - S_star, S_r - S_star};
+        float ie[2];
+        rcp_rn_all<2>(e, ie);
+        const float s_l = div_rn(-dl, e[0], ie[0]);  // h_l (S_l - u_l) / (S_l - S_star)
+        const float s_r = div_rn(-dr, e[1], ie[1]);
         const float Q_star_l[3] = {s_l * 1.0f, s_l * S_star, s_l * v_l};
         const float Q_star_r[3] = {s_r * 1.0f, s_r * S_star, s_r * v_r};
-        float F_1[3], F_4[3], F_2[3], F_3[3];
-        swe_F<M, true>(q_l1, g, F_1);
-        swe_F<M, true>(q_r1, g, F_4);
+        float F_2[3], F_3[3];
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             F_2[k] = F_1[k] + S_l * (Q_star_l[k] - q_l1[k]);
             F_3[k] = F_4[k] + S_r * (Q_star_r[k] - q_r1[k]);
         }
-        const float c_1 = M::div(S_l * dt, d);
-        const float c_2 = M::div(S_star * dt, d);
-        const float c_3 = M::div(S_r * dt, d);
+        // Courant numbers; a zero one has the sign of its numerator
+        const float p_1 = S_l * dt, p_2 = S_star * dt, p_3 = S_r * dt;
+        const float c_1 = M::quot(p_1, d), c_2 = M::quot(p_2, d), c_3 = M::quot(p_3, d);
         // desingularize((c_1 > 0) ? h_dag_l - h_l2 : h_dag_r - h_r) / desingularize(h_dag - h_l), ...
-        const float r_1 = M::quot((c_1 > 0.0f) ? Dl.d1 : Dr.d1, D.d1);
-        const float r_2 = M::quot((c_2 > 0.0f) ? Dl.d2 : Dr.d2, D.d2);
-        const float r_3 = M::quot((c_3 > 0.0f) ? Dl.d3 : Dr.d3, D.d3);
-        const float A_1 = __builtin_copysignf(1.0f, c_1) * limiter_to_waf(generalized_minmod(r_1, 1.9f), c_1);
-        const float A_2 = __builtin_copysignf(1.0f, c_2) * limiter_to_waf(generalized_minmod(r_2, 1.9f), c_2);
-        const float A_3 = __builtin_copysignf(1.0f, c_3) * limiter_to_waf(generalized_minmod(r_3, 1.9f), c_3);
+        const float den[3] = {D.d1, D.d2, D.d3};
+        float iden[3];
+        rcp_rn_all<3>(den, iden);
+        const float r_1 = quot_rn((c_1 > 0.0f) ? Dl.d1 : Dr.d1, D.d1, iden[0]);
+        const float r_2 = quot_rn((c_2 > 0.0f) ? Dl.d2 : Dr.d2, D.d2, iden[1]);
+        const float r_3 = quot_rn((c_3 > 0.0f) ? Dl.d3 : Dr.d3, D.d3, iden[2]);
+        const float A_1 = __builtin_copysignf(1.0f, p_1) * limiter_to_waf(generalized_minmod(r_1, 1.9f), c_1);
+        const float A_2 = __builtin_copysignf(1.0f, p_2) * limiter_to_waf(generalized_minmod(r_2, 1.9f), c_2);
+        const float A_3 = __builtin_copysignf(1.0f, p_3) * limiter_to_waf(generalized_minmod(r_3, 1.9f), c_3);
 #pragma unroll
         for (int k = 0; k < 3; ++k)
             out[k] = 0.5f * (F_1[k] + F_4[k]) -
@@ -367,8 +391,6 @@ __device__ __forceinline__ void waf_flux_core(const WafCell& L, const WafCell& R
         const float ie = M::rcp(el * er);
         const float s_l = -dl * (er * ie);  // h_l (S_l - u_l) / (S_l - S_star)
         const float s_r = -dr * (el * ie);  // h_r (S_r - u_r) / (S_r - S_star)
-        const float F_1[3] = {L.hu, L.hu * u_l + hg * h_l * h_l, L.hv * u_l};
-        const float F_4[3] = {R.hu, R.hu * u_r + hg * h_r * h_r, R.hv * u_r};
         const float Qsl[3] = {s_l, s_l * S_star, s_l * v_l};
         const float Qsr[3] = {s_r, s_r * S_star, s_r * v_r};
         const float c_1 = S_l * dtd, c_2 = S_star * dtd, c_3 = S_r * dtd;
@@ -415,12 +437,6 @@ __device__ __forceinline__ float swe_cell_dt(const float q[3], float dx, float d
 // Euler: GPUSimulators/cuda/EulerCommon.h
 // ---------------------------------------------------------------------------
 
-// pressure, EulerCommon.h:83-90
-template <class M>
-__device__ __forceinline__ float euler_pressure(const float q[4], float gamma) {
-    return (gamma - 1.0f) * (q[3] - M::quot(0.5f * (q[1] * q[1] + q[2] * q[2]), q[0]));
-}
-
 // F_func, EulerCommon.h:93-109.  P is a pressure.
 template <class M>
 __device__ __forceinline__ void euler_F(const float q[4], float P, float F[4]) {
@@ -431,68 +447,62 @@ __device__ __forceinline__ void euler_F(const float q[4], float P, float F[4]) {
     F[3] = u * (q[3] + P);
 }
 
+// 1/rho, normal velocity, pressure, sound speed and flux of the two states of an
+// interface (pressure EulerCommon.h:83-90, F_func :93-109)
+__device__ __forceinline__ void euler_states(const float ql[4], const float qr[4], float gamma, float u[2], float c[2],
+                                             float F_l[4], float F_r[4]) {
+    const float rho[2] = {ql[0], qr[0]};
+    float y[2], P[2], cc[2];
+    rcp_rn_all<2>(rho, y);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const float* q = i ? qr : ql;
+        float* F = i ? F_r : F_l;
+        u[i] = quot_rn(q[1], q[0], y[i]);
+        P[i] = (gamma - 1.0f) * (q[3] - quot_rn(0.5f * (q[1] * q[1] + q[2] * q[2]), q[0], y[i]));
+        cc[i] = quot_rn(gamma * P[i], q[0], y[i]);
+        F[0] = q[1];
+        F[1] = q[1] * u[i] + P[i];
+        F[2] = q[2] * u[i];
+        F[3] = u[i] * (q[3] + P[i]);
+    }
+    float s[2];
+    sqrt_rn_all<2>(cc, s);
+    c[0] = s[0];
+    c[1] = s[1];
+}
+
 // HLL_flux (Euler), EulerCommon.h:117-160
-template <class M>
 __device__ __forceinline__ void euler_hll_flux(const float ql[4], const float qr[4], float gamma, float out[4]) {
     const float h_l = ql[0], h_r = qr[0];
-    const float u_l = M::quot(ql[1], h_l);
-    const float u_r = M::quot(qr[1], h_r);
-    const float P_l = euler_pressure<M>(ql, gamma);
-    const float P_r = euler_pressure<M>(qr, gamma);
-    const float c_l = M::sqrt(M::quot(gamma * P_l, ql[0]));
-    const float c_r = M::sqrt(M::quot(gamma * P_r, qr[0]));
-    const float h_dag = 0.5f * (h_l + h_r) - M::quot(0.25f * (u_r - u_l) * (h_l + h_r), c_l + c_r);
-    const float q_l_tmp = M::sqrt(0.5f * M::quot((h_dag + h_l) * h_dag, h_l * h_l));
-    const float q_r_tmp = M::sqrt(0.5f * M::quot((h_dag + h_r) * h_dag, h_r * h_r));
+    float u[2], c[2], F_l[4], F_r[4];
+    euler_states(ql, qr, gamma, u, c, F_l, F_r);
+    const float h_dag = 0.5f * (h_l + h_r) - quot_rn(0.25f * (u[1] - u[0]) * (h_l + h_r), c[0] + c[1]);
+    const float q_l_tmp = sqrt_rn(0.5f * quot_rn((h_dag + h_l) * h_dag, h_l * h_l));
+    const float q_r_tmp = sqrt_rn(0.5f * quot_rn((h_dag + h_r) * h_dag, h_r * h_r));
     const float q_l = (h_dag > h_l) ? q_l_tmp : 1.0f;
     const float q_r = (h_dag > h_r) ? q_r_tmp : 1.0f;
-    const float S_l = u_l - c_l * q_l;
-    const float S_r = u_r + c_r * q_r;
-    float F_l[4], F_r[4];
-    euler_F<M>(ql, P_l, F_l);
-    euler_F<M>(qr, P_r, F_r);
+    const float S_l = u[0] - c[0] * q_l;
+    const float S_r = u[1] + c[1] * q_r;
     const float srsl = S_r * S_l;
-    if constexpr (M::exact) {
-        const float den = S_r - S_l;
+    const float den = S_r - S_l, iden = rcp_rn(den);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const float star = M::quot(S_r * F_l[k] - S_l * F_r[k] + srsl * (qr[k] - ql[k]), den);
-            out[k] = (S_l >= 0.0f) ? F_l[k] : ((S_r <= 0.0f) ? F_r[k] : star);
-        }
-    } else {
-        const float iden = M::rcp(S_r - S_l);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const float star = (S_r * F_l[k] - S_l * F_r[k] + srsl * (qr[k] - ql[k])) * iden;
-            out[k] = (S_l >= 0.0f) ? F_l[k] : ((S_r <= 0.0f) ? F_r[k] : star);
-        }
+    for (int k = 0; k < 4; ++k) {
+        const float star = quot_rn(S_r * F_l[k] - S_l * F_r[k] + srsl * (qr[k] - ql[k]), den, iden);
+        out[k] = (S_l >= 0.0f) ? F_l[k] : ((S_r <= 0.0f) ? F_r[k] : star);
     }
 }
 
 // CentralUpwindFlux (Euler), EulerCommon.h:171-187
-template <class M>
 __device__ __forceinline__ void euler_cu_flux(const float qm[4], const float qp[4], float gamma, float out[4]) {
-    const float Pp = euler_pressure<M>(qp, gamma);
-    float Fp[4], Fm[4];
-    euler_F<M>(qp, Pp, Fp);
-    const float up = M::quot(qp[1], qp[0]);
-    const float cp = M::sqrt(M::quot(gamma * Pp, qp[0]));
-    const float Pm = euler_pressure<M>(qm, gamma);
-    euler_F<M>(qm, Pm, Fm);
-    const float um = M::quot(qm[1], qm[0]);
-    const float cm = M::sqrt(M::quot(gamma * Pm, qm[0]));
-    const float am = fminf(fminf(um - cm, up - cp), 0.0f);
-    const float ap = fmaxf(fmaxf(um + cm, up + cp), 0.0f);
+    float u[2], c[2], Fm[4], Fp[4];
+    euler_states(qm, qp, gamma, u, c, Fm, Fp);
+    const float am = fminf(fminf(u[0] - c[0], u[1] - c[1]), 0.0f);
+    const float ap = fmaxf(fmaxf(u[0] + c[0], u[1] + c[1]), 0.0f);
     const float apam = ap * am;
-    if constexpr (M::exact) {
-        const float den = ap - am;
+    const float den = ap - am, iden = rcp_rn(den);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) out[k] = M::quot((ap * Fm[k] - am * Fp[k]) + apam * (qp[k] - qm[k]), den);
-    } else {
-        const float iden = M::rcp(ap - am);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) out[k] = ((ap * Fm[k] - am * Fp[k]) + apam * (qp[k] - qm[k])) * iden;
-    }
+    for (int k = 0; k < 4; ++k) out[k] = quot_rn((ap * Fm[k] - am * Fp[k]) + apam * (qp[k] - qm[k]), den, iden);
 }
 
 // writeCfl per-cell value (Euler), EulerCommon.h:41-49: sqrt(gamma*rho) as written

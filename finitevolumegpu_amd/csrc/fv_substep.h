@@ -303,10 +303,11 @@ FVMI_DPP_SUB_RUN(right_minus_all, "wave_shl:1")  // o = x of lane + 1, minus y
 
 // the WafCell of lane+1
 __device__ __forceinline__ WafCell waf_from_right(const WafCell& p) {
-    const float x[6] = {p.h, p.hu, p.hv, p.u, p.v, p.c};
-    float o[6];
+    const float x[6] = {p.h, p.hu, p.hv, p.u, p.v, p.c}, y[3] = {p.ih, p.f1, p.f2};
+    float o[6], w[3];
     all_from_right<6>(x, o);
-    return {o[0], o[1], o[2], o[3], o[4], o[5], from_right(p.ih)};
+    all_from_right<3>(y, w);
+    return {o[0], o[1], o[2], o[3], o[4], o[5], w[0], w[1], w[2]};
 }
 
 __device__ __forceinline__ float wave_min(float v) {
@@ -393,7 +394,7 @@ struct SweKP07 : SweBase<M> {
                                 float (&o)[kC][3]) {
         if constexpr (M::exact) {
 #pragma unroll
-            for (int c = 0; c < kC; ++c) swe_cu_flux<M>(l[c], r[c], a.g, o[c]);
+            for (int c = 0; c < kC; ++c) swe_cu_flux(l[c], r[c], a.g, o[c]);
         } else {
             fast::swe_cu_flux<kC>(l, r, a.hg, a.sqrt_g, o);
         }
@@ -418,7 +419,7 @@ struct SweHLL2 : SweBase<M> {
                                 float (&o)[kC][3]) {
         if constexpr (M::exact) {
 #pragma unroll
-            for (int c = 0; c < kC; ++c) swe_hll_flux<M>(l[c], r[c], a.g, o[c]);
+            for (int c = 0; c < kC; ++c) swe_hll_flux(l[c], r[c], a.g, o[c]);
         } else {
             fast::swe_hll_flux<kC>(l, r, a.hg, a.sqrt_g, o);
         }
@@ -472,7 +473,7 @@ struct EulerKP07 {
                                   float (&o)[kC][4]) {
         if constexpr (M::exact) {
 #pragma unroll
-            for (int c = 0; c < kC; ++c) euler_hll_flux<M>(l[c], r[c], a.gamma, o[c]);
+            for (int c = 0; c < kC; ++c) euler_hll_flux(l[c], r[c], a.gamma, o[c]);
         } else {
             fast::euler_hll_flux<kC>(l, r, a.gamma, o);
         }
@@ -481,7 +482,7 @@ struct EulerKP07 {
                                   float (&o)[kC][4]) {
         if constexpr (M::exact) {
 #pragma unroll
-            for (int c = 0; c < kC; ++c) euler_cu_flux<M>(l[c], r[c], a.gamma, o[c]);
+            for (int c = 0; c < kC; ++c) euler_cu_flux(l[c], r[c], a.gamma, o[c]);
         } else {
             fast::euler_cu_flux<kC>(l, r, a.gamma, o);
         }
@@ -531,7 +532,7 @@ __device__ __forceinline__ void reconstruct_fast(B b, F f, const float (&q)[S::k
         }
         p[c] = QL[c][0] * QR[c][0];
     }
-    fast::rcp_all<C>(p, r);
+    rcp_all<C>(p, r);
 #pragma unroll
     for (int c = 0; c < C; ++c) {
         float D[NV];
@@ -650,7 +651,7 @@ __device__ __forceinline__ void x_sweep_row(float (&q)[S::kC][S::NV], const Subs
         // WAF: the cell's quantities, and the h* and limiter denominators of
         // its right interface, once; the neighbours' through DPP
         static_assert(C == 1, "WAF marches one column per lane");
-        const WafCell P = waf_cell<M>(q[0], a.g, a.sqrt_g);
+        const WafCell P = waf_cell<M>(q[0], a.g, a.hg, a.sqrt_g);
         const WafCell R = waf_from_right(P);
         const float hd = waf_hstar<M>(P, R, a.g, a.inv_g);
         const WafDen D = waf_den<M>(P, R, hd);
@@ -658,8 +659,8 @@ __device__ __forceinline__ void x_sweep_row(float (&q)[S::kC][S::NV], const Subs
         float dl[3], dr[3];
         all_from_left<3>(d, dl);
         all_from_right<3>(d, dr);
-        waf_flux_core<M>(P, R, WafDen{dl[0], dl[1], dl[2]}, D, WafDen{dr[0], dr[1], dr[2]}, hd, a.g, a.hg, a.dx, a.dt,
-                         a.dtdx, F[0]);
+        waf_flux_core<M>(P, R, WafDen{dl[0], dl[1], dl[2]}, D, WafDen{dr[0], dr[1], dr[2]}, hd, a.dx, a.dt, a.dtdx,
+                         F[0]);
     }
     float F_first[N], F_last[N], dF[N];
     first(F, F_first);
@@ -971,13 +972,12 @@ __device__ __forceinline__ void waf_row(const SubstepArgs& a, const Strip<S::kC>
         {
             float y3[3];
             to_y<3>(w3[c], y3);
-            c3[c] = waf_cell<M>(y3, a.g, a.sqrt_g);
+            c3[c] = waf_cell<M>(y3, a.g, a.hg, a.sqrt_g);
         }
         const float hd_r = waf_hstar<M>(c2[c], c3[c], a.g, a.inv_g);  // interface (r-1, r)
         const WafDen Dn = waf_den<M>(c2[c], c3[c], hd_r);
         float G[3];
-        waf_flux_core<M>(c1[c], c2[c], dd[0][c], dd[1][c], Dn, hd[c], a.g, a.hg, a.dy, a.dt, a.dtdy,
-                         G);  // interface (r-2, r-1)
+        waf_flux_core<M>(c1[c], c2[c], dd[0][c], dd[1][c], Dn, hd[c], a.dy, a.dt, a.dtdy, G);  // interface (r-2, r-1)
         if (emit) {
             float y1[3];
             to_y<3>(w1[c], y1);
@@ -1076,7 +1076,7 @@ __device__ __forceinline__ float march_waf(const SubstepArgs& a, const Strip<S::
         for (int c = 0; c < C; ++c) {
             float y[3];
             to_y<3>(ring[m][c], y);
-            cell[m][c] = waf_cell<M>(y, a.g, a.sqrt_g);
+            cell[m][c] = waf_cell<M>(y, a.g, a.hg, a.sqrt_g);
         }
     }
 #pragma unroll

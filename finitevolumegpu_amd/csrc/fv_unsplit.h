@@ -145,7 +145,7 @@ struct SweHLL1 : UnsplitBase<M> {
     static constexpr int kind = KIND_SPLIT1;
     __device__ static void flux_x(const float l[3], const float r[3], const UnsplitArgs& a, float o[3]) {
         if constexpr (M::exact)
-            swe_hll_flux<M>(l, r, a.g, o);
+            swe_hll_flux(l, r, a.g, o);
         else
             fast::swe_hll_flux<1>(one_column(l), one_column(r), a.hg, a.sqrt_g, one_column(o));
     }
@@ -172,7 +172,7 @@ struct SweKP07U : UnsplitBase<M> {
     static constexpr int kind = KIND_KP07U;
     __device__ static void flux(const float l[3], const float r[3], const UnsplitArgs& a, float o[3]) {
         if constexpr (M::exact)
-            swe_cu_flux<M>(l, r, a.g, o);
+            swe_cu_flux(l, r, a.g, o);
         else
             fast::swe_cu_flux<1>(one_column(l), one_column(r), a.hg, a.sqrt_g, one_column(o));
     }
