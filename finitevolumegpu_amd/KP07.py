@@ -5,7 +5,7 @@ GPUSimulators/cuda/SWE2D_KP07.cu)."""
 import numpy as np
 
 from . import _lib
-from .Simulator import BoundaryCondition, UnsplitSimulator, swe_initial_cfl
+from .Simulator import BoundaryCondition, UnsplitSimulator, _library_methods, _StepCall, swe_initial_cfl
 
 
 def stepOrderToCodedInt(step, order):
@@ -33,6 +33,22 @@ class KP07(UnsplitSimulator):
         self.dt_factor = 0.5 ** (order - 1)
         self._init_unsplit([h0, hu0, hv0], swe_initial_cfl(h0, hu0, hv0, self.dx, self.dy, g),
                            tile_rows, waves_per_block, math, xcd_remap)
+        # a second-order step is one library call unless a subclass brings its own substeps
+        self._step_call = _StepCall()
+        self._whole_step = order == 2 and _library_methods(self, ("substep", "_launch", "_field_args", "cfl_pointer"))
+
+    def step(self, dt):
+        """One full step; with two stages as one library call
+        (fvmi_swe_kp07_rk2_step) with the results of the two substeps."""
+        if not self._whole_step or self.num_substeps != 2 or "substep" in self.__dict__:
+            super().step(dt)
+            return
+        in_other, self.cfl_last = self._step_call("fvmi_swe_kp07_rk2_step", self, 0, dt, self.boundary_conditions,
+                                                  1 - self.cfl_last)
+        if in_other:
+            self.u0, self.u1 = self.u1, self.u0
+        self.t += float(dt)
+        self.nt += 1
 
     def substepRK(self, dt, substep):
         self.substep(dt, substep)

@@ -199,6 +199,36 @@ def resolve_math(scheme, math):
     return math
 
 
+class _StepCall:
+    """Calls a whole-step entry point of the library (fvmi_step_t) for a
+    simulator's current buffers and parameters."""
+
+    def __init__(self):
+        self.args = ctypes.create_string_buffer(ctypes.sizeof(_lib.StepArgs))
+        self.out = (ctypes.c_int * 2)()  # buffer of the new state, slot of its CFL minimum
+        self.out_ptr = ctypes.addressof(self.out)
+
+    def __call__(self, name, sim, scheme, dt, boundary_conditions, cfl_slot):
+        """Returns (state is in u1, CFL slot)."""
+        fields = []
+        pitches = []
+        for state in (sim.u0, sim.u1):
+            arrays = state.gpu_variables
+            fields += [v.ptr.value or 0 for v in arrays] + [0] * (4 - len(arrays))
+            pitches += [v.pitch for v in arrays] + [0] * (4 - len(arrays))
+        _lib.STEP_PACK.pack_into(self.args, 0, scheme, sim.nx, sim.ny, boundary_conditions, sim.dx, sim.dy,
+                                 np.float32(dt), sim.g, getattr(sim, "theta", 0.0), getattr(sim, "gamma", 0.0),
+                                 *fields, *pitches, sim.cfl_pointer() or 0, cfl_slot)
+        _lib.call(name, self.args, sim.launch, self.out_ptr, self.out_ptr + 4, sim.stream.handle)
+        return bool(self.out[0]), self.out[1]
+
+
+def _library_methods(sim, names):
+    """Whether the class of ``sim`` has the package's own methods of these names."""
+    package = __name__.partition(".")[0]
+    return all(getattr(type(sim), name).__module__.partition(".")[0] == package for name in names)
+
+
 class DimsplitSimulator(BaseSimulator):
     """Shared body of the four dimensionally split scheme wrappers."""
 
@@ -233,13 +263,10 @@ class DimsplitSimulator(BaseSimulator):
         init = np.array([np.inf, cfl_host], dtype=np.float32)
         _lib.call("fvmi_memcpy_async", self.cfl_data, init.ctypes.data, 8, _lib.MEMCPY_HTOD, self.stream.handle)
         self.stream.synchronize()
-        self._step_buffer = ctypes.create_string_buffer(ctypes.sizeof(_lib.StepArgs))
-        self._step_out = (ctypes.c_int * 2)()  # buffer of the new state, slot of its CFL minimum
-        self._step_out_ptr = ctypes.addressof(self._step_out)
+        self._step_call = _StepCall()
         # step() is one library call unless a subclass brings its own substeps
-        self._whole_step = all(
-            getattr(type(self), name).__module__.partition(".")[0] == __name__.partition(".")[0]
-            for name in ("substep", "substepDimsplit", "_launch", "_field_args", "cfl_pointer"))
+        self._whole_step = _library_methods(self, ("substep", "substepDimsplit", "_launch", "_field_args",
+                                                   "cfl_pointer"))
 
     def cfl_pointer(self):
         return self.cfl_data.value
@@ -256,25 +283,13 @@ class DimsplitSimulator(BaseSimulator):
 
     def _step_both(self, dt, boundary_conditions):
         """Both substeps of one step under ``boundary_conditions``."""
-        cfl = self.cfl_pointer() or 0
-        fields = []
-        pitches = []
-        for state in (self.u0, self.u1):
-            arrays = state.gpu_variables
-            fields += [v.ptr.value or 0 for v in arrays] + [0] * (4 - len(arrays))
-            pitches += [v.pitch for v in arrays] + [0] * (4 - len(arrays))
-        _lib.STEP_PACK.pack_into(self._step_buffer, 0, _lib.SCHEME_IDS[self.scheme], self.nx, self.ny,
-                                 boundary_conditions, self.dx, self.dy, np.float32(dt * 0.5), self.g,
-                                 getattr(self, "theta", 0.0), getattr(self, "gamma", 0.0), *fields, *pitches,
-                                 cfl, self.cfl_free)
-        out = self._step_out
-        _lib.call("fvmi_dimsplit_step", self._step_buffer, self.launch, self._step_out_ptr, self._step_out_ptr + 4,
-                  self.stream.handle)
-        if out[0]:
+        in_other, slot = self._step_call("fvmi_dimsplit_step", self, _lib.SCHEME_IDS[self.scheme], dt * 0.5,
+                                         boundary_conditions, self.cfl_free)
+        if in_other:
             self.u0, self.u1 = self.u1, self.u0
-        if cfl:
-            self.cfl_last = out[1]
-            self.cfl_free = 1 - out[1]
+        if self.cfl_pointer():
+            self.cfl_last = slot
+            self.cfl_free = 1 - slot
 
     def substep(self, dt, step_number):
         self.substepDimsplit(dt * 0.5, step_number)

@@ -4,6 +4,7 @@
 // scheduler: KP07_dimsplit 4 % faster, its ensemble 6 %; WAF and LxF 2 % with
 // the pinned row march.  The Euler kernels are in fv_kernels_fast.hip.
 #include "fv_launch.h"
+#include "fv_rk2.h"
 #include "fv_unsplit.h"
 
 namespace fvmi {
@@ -40,6 +41,10 @@ hipError_t launch_ensemble_fast_ilp(int scheme, const EnsembleArgs& e, int grid,
         default:
             return hipErrorInvalidValue;
     }
+}
+hipError_t launch_rk2_step(const SubstepArgs& a, int grid, hipStream_t stream) {
+    hipLaunchKernelGGL((rk2_kernel<MathFast>), dim3(grid), dim3(kLanes * a.waves_per_block), 0, stream, a);
+    return hipGetLastError();
 }
 hipError_t launch_unsplit_fast(int scheme, const UnsplitArgs& a, int grid, hipStream_t stream) {
     return launch_unsplit<MathFast>(scheme, a, grid, stream);

@@ -32,12 +32,8 @@ using StepKP07 = SweKP07<MathFast, 1>;
 using StepHLL2 = SweHLL2<MathFast, 1>;
 using StepEuler = EulerKP07<MathFast, 1>;
 
-// Whether a whole step of this grid is one launch (fv_step.h).  Fast arithmetic
-// only: the exact kernels and WAF are bound by VALU issue already as substeps
-// (4096^2: 184 us for KP07_dimsplit, 260 for WAF, against 79 us for their
-// bytes), so that the wider halo would cost more than the memory passes saved.
-inline bool step_is_fused(int scheme, int math, const SubstepArgs& a) {
-    if (math == FVMI_MATH_EXACT || scheme == SCHEME_WAF) return false;
+// Whether a whole step of this grid can be one launch (fv_step.h, fv_rk2.h).
+inline bool step_grid_fits(const SubstepArgs& a) {
     if (a.nx < kStepMinSide || a.ny < kStepMinSide) return false;
     if (a.seg_rows > 0 && a.seg_rows < kStepMinSegRows) return false;
     const int w = a.bc & 0xF, e = (a.bc >> 8) & 0xF, s = (a.bc >> 16) & 0xF, n = (a.bc >> 24) & 0xF;
@@ -45,6 +41,13 @@ inline bool step_is_fused(int scheme, int math, const SubstepArgs& a) {
     // a periodic edge opposite to another kind wraps to cells whose own
     // neighbours are that kind's ghosts, which the images marched along are not
     return (w == BC_PERIODIC) == (e == BC_PERIODIC) && (s == BC_PERIODIC) == (n == BC_PERIODIC);
+}
+
+// Whether a dimensionally split step is.  Fast arithmetic only: the exact kernels and WAF are bound by VALU issue already as substeps
+// (4096^2: 184 us for KP07_dimsplit, 260 for WAF, against 79 us for their
+// bytes), so that the wider halo would cost more than the memory passes saved.
+inline bool step_is_fused(int scheme, int math, const SubstepArgs& a) {
+    return math != FVMI_MATH_EXACT && scheme != SCHEME_WAF && step_grid_fits(a);
 }
 
 // Segments of a whole step re-sweep about 4 rows' worth of halo, twice a
@@ -170,6 +173,7 @@ hipError_t launch_substep_fast(int scheme, const SubstepArgs& a, int grid, hipSt
 // (fv_kernels_fast_ilp.hip, built with the ILP-maximising scheduler)
 hipError_t launch_step_fast(int scheme, const SubstepArgs& a, int grid, hipStream_t stream);
 hipError_t launch_step_fast_ilp(int scheme, const SubstepArgs& a, int grid, hipStream_t stream);
+hipError_t launch_rk2_step(const SubstepArgs& a, int grid, hipStream_t stream);  // fast arithmetic
 hipError_t launch_substep_fast_ilp(int scheme, const SubstepArgs& a, int grid, hipStream_t stream);
 hipError_t launch_ensemble_fast_ilp(int scheme, const EnsembleArgs& e, int grid, hipStream_t stream);
 

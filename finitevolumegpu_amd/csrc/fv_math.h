@@ -29,8 +29,15 @@ namespace fvmi {
 #define FVMI_TRANS_RUN(name, one, op)                                                                                    \
     template <int N>                                                                                                \
     __device__ __forceinline__ void name(const float (&x)[N], float (&r)[N]) {                                      \
-        static_assert(N >= 1 && N <= 4, "runs of 1 to 4");                                                          \
-        if constexpr (N == 1)                                                                                       \
+        static_assert((N >= 1 && N <= 4) || N == 8, "runs of 1 to 4, or two of 4");                                 \
+        if constexpr (N == 8) {                                                                                     \
+            const float xa[4] = {x[0], x[1], x[2], x[3]}, xb[4] = {x[4], x[5], x[6], x[7]};                         \
+            float ra[4], rb[4];                                                                                     \
+            name<4>(xa, ra);                                                                                        \
+            name<4>(xb, rb);                                                                                        \
+            r[0] = ra[0], r[1] = ra[1], r[2] = ra[2], r[3] = ra[3];                                                 \
+            r[4] = rb[0], r[5] = rb[1], r[6] = rb[2], r[7] = rb[3];                                                 \
+        } else if constexpr (N == 1)                                                                                \
             r[0] = one(x[0]);                                                                                       \
         else if constexpr (N == 2)                                                                                  \
             asm(op " %0, %2\n\t" op " %1, %3\n\ts_nop 0" : "=&v"(r[0]), "=v"(r[1]) : "v"(x[0]), "v"(x[1]));       \

@@ -89,10 +89,10 @@ __device__ __forceinline__ void setup_edge(const SubstepArgs& a, const Strip<1>&
 __device__ __forceinline__ bool needs_edge(const StepEdge& e) { return e.fix_x || e.fix_lo || e.hi_row != kNoRow; }
 
 // Ghost columns of a middle row: each takes its source column's values.
-template <class S>
-__device__ __forceinline__ void fill_ghost_columns(const StepEdge& e, float (&q)[1][S::NV]) {
+template <int NV>
+__device__ __forceinline__ void fill_ghost_columns(const StepEdge& e, float (&q)[1][NV]) {
 #pragma unroll
-    for (int k = 0; k < S::NV; ++k) {
+    for (int k = 0; k < NV; ++k) {
         int w = __builtin_amdgcn_ds_bpermute(e.src_addr, __float_as_int(q[0][k]));
         if (k == 1) w ^= (int)e.xsign;
         q[0][k] = __int_as_float(w);
@@ -100,14 +100,30 @@ __device__ __forceinline__ void fill_ghost_columns(const StepEdge& e, float (&q)
 }
 
 // A ghost row from an interior row: a mirroring edge flips the y momentum.
-template <class S>
-__device__ __forceinline__ void copy_ghost_row(int kind, const float (&src)[1][S::NV], float (&q)[1][S::NV]) {
+template <int NV>
+__device__ __forceinline__ void copy_ghost_row(int kind, const float (&src)[1][NV], float (&q)[1][NV]) {
     const unsigned sign = kind == BC_REFLECTIVE ? 0x80000000u : 0u;
 #pragma unroll
-    for (int k = 0; k < S::NV; ++k) {
+    for (int k = 0; k < NV; ++k) {
         const unsigned w = __float_as_uint(src[0][k]);
         q[0][k] = __uint_as_float(k == 2 ? w ^ sign : w);
     }
+}
+
+// Middle row `row` (padded) if it is a ghost row of a filled high edge, from
+// the rows one, two and three before it.
+template <int NV>
+__device__ __forceinline__ void fill_ghost_row(const StepEdge& e, int row, const float (&back1)[1][NV],
+                                               const float (&back2)[1][NV], const float (&back3)[1][NV],
+                                               float (&q)[1][NV]) {
+    const int ghost = __builtin_amdgcn_readfirstlane(row - e.hi_row);
+    if (ghost < 0) return;
+    if (ghost == 0)  // from the last interior row, both kinds
+        copy_ghost_row<NV>(e.hi_kind, back1, q);
+    else if (e.hi_kind == BC_REFLECTIVE)  // from the interior row before it
+        copy_ghost_row<NV>(e.hi_kind, back3, q);
+    else  // outflow: the last interior row again
+        copy_ghost_row<NV>(e.hi_kind, back2, q);
 }
 
 // Edge waves (and segments of one row): the four sweeps of an iteration one
@@ -143,17 +159,9 @@ __device__ __forceinline__ float march_step_edge(const SubstepArgs& a, const Str
         float q[1][NV];
         y_sweep_step<S, M>(a, kky, w[(u + 1) % 3], w[(u + 2) % 3], w[u], P, G, dq, true, q);
         gravity_source<S>(a, q);
-        if (e.fix_x) fill_ghost_columns<S>(e, q);
-        const int s = (u + 1) % 3;  // slot of row r-2; row r-3 is in slot u, row r-4 in (u + 2) % 3
-        const int ghost = __builtin_amdgcn_readfirstlane(st.row0 + r - 2 - e.hi_row);
-        if (ghost >= 0) {
-            if (ghost == 0)  // the last interior row, both kinds
-                copy_ghost_row<S>(e.hi_kind, m[u], q);
-            else if (e.hi_kind == BC_REFLECTIVE)  // the interior row before it, row r-5, still in this slot
-                copy_ghost_row<S>(e.hi_kind, m[s], q);
-            else  // outflow: the last interior row, row r-4
-                copy_ghost_row<S>(e.hi_kind, m[(u + 2) % 3], q);
-        }
+        if (e.fix_x) fill_ghost_columns<NV>(e, q);
+        const int s = (u + 1) % 3;  // slot of row r-2; row r-3 is in slot u, row r-4 in (u + 2) % 3, row r-5 still in s
+        fill_ghost_row<NV>(e, st.row0 + r - 2, m[u], m[(u + 2) % 3], m[s], q);
         copy(q, m[s]);
     };
     // y sweep of the middle rows r-4 .. r-2, x sweep and store of row r-4
@@ -194,11 +202,11 @@ __device__ __forceinline__ float march_step_edge(const SubstepArgs& a, const Str
     // rows 2 and 3 are the ghost rows of a low edge: from rows 4 and 5
     if (e.fix_lo) {
         float g0[1][NV];
-        copy_ghost_row<S>(e.lo_kind, m[1], m[0]);
+        copy_ghost_row<NV>(e.lo_kind, m[1], m[0]);
         if (e.lo_kind == BC_REFLECTIVE)
-            copy_ghost_row<S>(e.lo_kind, m[2], g0);
+            copy_ghost_row<NV>(e.lo_kind, m[2], g0);
         else
-            copy_ghost_row<S>(e.lo_kind, m[1], g0);
+            copy_ghost_row<NV>(e.lo_kind, m[1], g0);
         y_sweep_begin<S, M>(a, kky, g0, m[0], m[1], P2, G2, dq2);
     }
     finish(1, 7, false);  // flux (3, 4) of the middle rows

@@ -57,8 +57,8 @@ struct UnsplitArgs {
 // Half the limited slope, s/2, of a cell with neighbours l and r.  Fast form:
 // minmod(theta b, (b + f)/2, theta f) = theta minmod(b, (b + f)/(2 theta), f)
 // for theta > 0 (b, f the backward and forward differences).
-template <class M>
-__device__ __forceinline__ float half_slope(float l, float c, float r, const UnsplitArgs& a) {
+template <class M, class Args>
+__device__ __forceinline__ float half_slope(float l, float c, float r, const Args& a) {
     if constexpr (M::exact) {
         return 0.5f * minmod_slope((c - l) * a.theta, 0.5f * (r - l), (r - c) * a.theta);
     } else {
@@ -289,8 +289,8 @@ __device__ __forceinline__ void swap_tn(const float (&q)[3], float (&o)[3]) {
 
 // q + (df dt / dx + dg dt / dy) with the flux differences df = fl - fr, dg = gs
 // - gn: the unsplit update of SWE2D_LxF.cu:147-152 and SWE2D_KP07.cu:190-195
-template <class M>
-__device__ __forceinline__ float u_update(float q, float df, float dg, const UnsplitArgs& a) {
+template <class M, class Args>
+__device__ __forceinline__ float u_update(float q, float df, float dg, const Args& a) {
     if constexpr (M::exact)
         return q + (M::quot(df * a.dt, a.dx) + M::quot(dg * a.dt, a.dy));
     else

@@ -655,6 +655,31 @@ int fvmi_euler_kp07_dimsplit_substep(int nx, int ny, float dx, float dy, float d
     return run_substep(SCHEME_EULER, a, 4, launch, stream);
 }
 
+namespace {
+
+// The arguments of a launch that reads buffer `from` of a step and writes the other.
+SubstepArgs step_args(const fvmi_step_t* p, int nvars, int from, int step) {
+    SubstepArgs a{};
+    a.nx = p->nx, a.ny = p->ny, a.dx = p->dx, a.dy = p->dy, a.dt = p->dt;
+    a.g = p->g, a.theta = p->theta, a.gamma = p->gamma;
+    a.step = step, a.bc = p->boundary_conditions;
+    for (int k = 0; k < nvars; ++k) {
+        a.in[k] = p->state[from][k], a.in_pitch[k] = p->pitch[from][k];
+        a.out[k] = p->state[1 - from][k], a.out_pitch[k] = p->pitch[1 - from][k];
+    }
+    a.cfl = p->cfl;
+    return a;
+}
+
+// Plans a launch of a whole step; returns its grid.
+int plan_step(SubstepArgs& a, int cfl_slot) {
+    a.cfl_slot = cfl_slot;
+    a.strip_cols = strip_cols<1, kStepHalo>();
+    return plan_substep(a, current_cu_count(), true, 4, kStepMinSeg);
+}
+
+}  // namespace
+
 int fvmi_dimsplit_step(const fvmi_step_t* p, const fvmi_launch_t* launch, int* state_out, int* cfl_slot_out,
                        void* stream) {
     if (!p || !state_out || !cfl_slot_out) return fail(FVMI_ERR_INVALID, "NULL argument");
@@ -662,33 +687,49 @@ int fvmi_dimsplit_step(const fvmi_step_t* p, const fvmi_launch_t* launch, int* s
         return fail(FVMI_ERR_INVALID, "unknown scheme %d", p->scheme);
     if (p->cfl_slot != 0 && p->cfl_slot != 1) return fail(FVMI_ERR_INVALID, "cfl_slot must be 0 or 1");
     const int nvars = p->scheme == SCHEME_EULER ? 4 : 3;
-    auto args = [&](int from, int step) {
-        SubstepArgs a{};
-        a.nx = p->nx, a.ny = p->ny, a.dx = p->dx, a.dy = p->dy, a.dt = p->dt;
-        a.g = p->g, a.theta = p->theta, a.gamma = p->gamma;
-        a.step = step, a.bc = p->boundary_conditions;
-        for (int k = 0; k < nvars; ++k) {
-            a.in[k] = p->state[from][k], a.in_pitch[k] = p->pitch[from][k];
-            a.out[k] = p->state[1 - from][k], a.out_pitch[k] = p->pitch[1 - from][k];
-        }
-        a.cfl = p->cfl;
-        return a;
-    };
     int math = 0;
-    SubstepArgs a = args(0, 0);
+    SubstepArgs a = step_args(p, nvars, 0, 0);
     if (int rc = check_substep(p->scheme, a, nvars, launch, &math)) return rc;
     if (!step_is_fused(p->scheme, math, a)) {
         if (int rc = run_substep(p->scheme, a, nvars, launch, stream)) return rc;
-        SubstepArgs b = args(1, 1);
+        SubstepArgs b = step_args(p, nvars, 1, 1);
         if (int rc = run_substep(p->scheme, b, nvars, launch, stream)) return rc;
         *state_out = 0;
         *cfl_slot_out = 1;
         return FVMI_OK;
     }
-    a.cfl_slot = p->cfl_slot;
-    a.strip_cols = strip_cols<1, kStepHalo>();
-    const int grid = plan_substep(a, current_cu_count(), true, 4, kStepMinSeg);
+    const int grid = plan_step(a, p->cfl_slot);
     hipError_t e = launch_step_fast(p->scheme, a, grid, (hipStream_t)stream);
+    if (e != hipSuccess) return hip_fail(e, "step launch");
+    *state_out = 1;
+    *cfl_slot_out = p->cfl_slot;
+    return FVMI_OK;
+}
+
+int fvmi_swe_kp07_rk2_step(const fvmi_step_t* p, const fvmi_launch_t* launch, int* state_out, int* cfl_slot_out,
+                           void* stream) {
+    if (!p || !state_out || !cfl_slot_out) return fail(FVMI_ERR_INVALID, "NULL argument");
+    if (p->cfl_slot != 0 && p->cfl_slot != 1) return fail(FVMI_ERR_INVALID, "cfl_slot must be 0 or 1");
+    int math = 0;
+    SubstepArgs a = step_args(p, 3, 0, 0);
+    if (int rc = check_substep(SCHEME_KP07, a, 3, launch, &math)) return rc;
+    if (math == FVMI_MATH_EXACT || !step_grid_fits(a)) {
+        for (int stage = 0; stage < 2; ++stage) {
+            const int slot = stage == 0 ? p->cfl_slot : 1 - p->cfl_slot;
+            if (int rc = fvmi_swe_kp07_substep(
+                    p->nx, p->ny, p->dx, p->dy, p->dt, p->g, p->theta, (stage << 16) | 2, p->boundary_conditions,
+                    p->state[stage][0], p->pitch[stage][0], p->state[stage][1], p->pitch[stage][1],
+                    p->state[stage][2], p->pitch[stage][2], p->state[1 - stage][0], p->pitch[1 - stage][0],
+                    p->state[1 - stage][1], p->pitch[1 - stage][1], p->state[1 - stage][2], p->pitch[1 - stage][2],
+                    p->cfl, slot, launch, stream))
+                return rc;
+        }
+        *state_out = 0;
+        *cfl_slot_out = 1 - p->cfl_slot;
+        return FVMI_OK;
+    }
+    const int grid = plan_step(a, p->cfl_slot);
+    hipError_t e = launch_rk2_step(a, grid, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "step launch");
     *state_out = 1;
     *cfl_slot_out = p->cfl_slot;

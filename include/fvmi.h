@@ -224,6 +224,14 @@ typedef struct fvmi_step {
 int fvmi_dimsplit_step(const fvmi_step_t* p, const fvmi_launch_t* launch, int* state_out, int* cfl_slot_out,
                        void* stream);
 
+/* One full step of the unsplit KP07 scheme with its two Runge-Kutta stages (the
+ * second one averaged with the state before the step), both of length `dt`;
+ * `scheme` and `gamma` are not read.  One launch in fast arithmetic under the
+ * conditions above, else fvmi_swe_kp07_substep twice; same results and outputs
+ * as fvmi_dimsplit_step. */
+int fvmi_swe_kp07_rk2_step(const fvmi_step_t* p, const fvmi_launch_t* launch, int* state_out, int* cfl_slot_out,
+                           void* stream);
+
 /* One-rank stand-in for MPISimulator.full_exchange's east/west leg
  * (MPISimulator.py:283-295, 440-480) with a periodic-x neighbour: for each of
  * the `nvars` fields copy padded columns [nx, nx+2) -> [0, 2) and

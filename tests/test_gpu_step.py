@@ -1,5 +1,5 @@
-"""Simulator.step (one library call, one launch for the slope schemes in fast
-arithmetic) against its two substeps run one by one: the fields and the CFL
+"""Simulator.step (one library call, one launch for the slope schemes and the
+two-stage KP07 in fast arithmetic) against its two substeps run one by one: the fields and the CFL
 minimum are equal bitwise.  Sizes at the edges of a strip of the whole-step
 march (56 output columns, 120 with two columns per lane), smallest sides,
 segments as short as they may be, and every kind of edge."""
@@ -27,14 +27,23 @@ BOUNDARIES = {
 SIZES = [(8, 8), (9, 11), (55, 12), (56, 8), (57, 30), (59, 9), (60, 64), (113, 65), (120, 17), (121, 40), (123, 8),
          (241, 133)]
 
-CASES = [("kp07_dimsplit", "fast"), ("hll2", "fast"), ("ee2d_kp07_dimsplit", "fast"),
-         ("ee2d_kp07_dimsplit", "exact"), ("waf", "exact")]
+CASES = [("kp07_dimsplit", "fast"), ("hll2", "fast"), ("ee2d_kp07_dimsplit", "fast"), ("kp07", "fast"),
+         ("ee2d_kp07_dimsplit", "exact"), ("waf", "exact"), ("kp07", "exact")]
+
+
+def make(ctx, scheme, fields, nx, ny, bc, math="fast", **kw):
+    if scheme != "kp07":  # the unsplit scheme, two Runge-Kutta stages
+        return make_gpu_sim(ctx, scheme, fields, nx, ny, 1.0, 1.0, bc, math=math, **kw)
+    from finitevolumegpu_amd.KP07 import KP07
+    from finitevolumegpu_amd.Simulator import BoundaryCondition
+    return KP07(ctx, *fields, nx, ny, 1.0, 1.0, 9.81, boundary_conditions=BoundaryCondition(
+        BoundaryCondition.getTypes(bc)), math=math, **kw)
 
 
 def run_pair(ctx, scheme, nx, ny, bc, math, steps=3, **kw):
     fields = state(scheme, nx, ny, seed=nx + 7 * ny)
-    a = make_gpu_sim(ctx, scheme, fields, nx, ny, 1.0, 1.0, bc, math=math, **kw)
-    b = make_gpu_sim(ctx, scheme, fields, nx, ny, 1.0, 1.0, bc, math=math, **kw)
+    a = make(ctx, scheme, fields, nx, ny, bc, math, **kw)
+    b = make(ctx, scheme, fields, nx, ny, bc, math, **kw)
     dt = np.float32(0.05) if scheme == "ee2d_kp07_dimsplit" else np.float32(0.9 * a.computeDt())
     for n in range(steps):
         a.step(dt)
@@ -55,7 +64,7 @@ def test_step_equals_its_substeps(ctx, scheme, math, bc):
         run_pair(ctx, scheme, nx, ny, BOUNDARIES[bc], math)
 
 
-@pytest.mark.parametrize("scheme", ["kp07_dimsplit", "ee2d_kp07_dimsplit"])
+@pytest.mark.parametrize("scheme", ["kp07_dimsplit", "ee2d_kp07_dimsplit", "kp07"])
 def test_step_with_every_combination_of_edges(ctx, scheme):
     """All 256 combinations of the four edge kinds, those that take one launch
     and those that take two."""
@@ -71,7 +80,7 @@ def test_step_with_every_combination_of_edges(ctx, scheme):
     for code in itertools.product((D, P, R, F), repeat=4):
         out = []
         for whole in (True, False):
-            sim = make_gpu_sim(ctx, scheme, fields, nx, ny, 1.0, 1.0, O.pack_bc(*code))
+            sim = make(ctx, scheme, fields, nx, ny, O.pack_bc(*code))
             for buf in (sim.u0, sim.u1):  # ghost memory that Dirichlet edges read
                 for k, pad in enumerate(pads):
                     buf[k].upload(sim.stream, pad, extent=[0, 0, nx + 4, ny + 4])
@@ -84,7 +93,7 @@ def test_step_with_every_combination_of_edges(ctx, scheme):
         assert all(np.array_equal(x, y) for x, y in zip(*out)), code
 
 
-@pytest.mark.parametrize("scheme", ["kp07_dimsplit", "ee2d_kp07_dimsplit"])
+@pytest.mark.parametrize("scheme", ["kp07_dimsplit", "ee2d_kp07_dimsplit", "kp07"])
 @pytest.mark.parametrize("tile_rows,waves", [(4, 4), (5, 1), (9, 2), (3, 4), (64, 3)])
 def test_step_of_any_launch_shape(ctx, scheme, tile_rows, waves):
     for nx, ny in ((70, 45), (250, 61)):
@@ -93,7 +102,7 @@ def test_step_of_any_launch_shape(ctx, scheme, tile_rows, waves):
 
 
 @pytest.mark.parametrize("scheme,nx,ny", [("kp07_dimsplit", 4096, 2050), ("hll2", 2300, 4095),
-                                          ("ee2d_kp07_dimsplit", 3001, 4032)])
+                                          ("ee2d_kp07_dimsplit", 3001, 4032), ("kp07", 3000, 4000)])
 @pytest.mark.parametrize("bc", ["mixed", "periodic"])
 def test_step_with_the_round_weighted_split(ctx, scheme, nx, ny, bc):
     print("case step rounds", scheme, nx, ny, bc, flush=True)
