@@ -740,13 +740,12 @@ __device__ __forceinline__ void apply_signs(const Strip<C>& st, unsigned ysign, 
 // Issues the loads of padded row r and returns the sign-bit mask of its y
 // momentum.  Pinned: the raw words are returned and use_row applies the mirror
 // signs at the row's first use; otherwise they are applied here.
-template <int C, int NV, bool Pinned, bool Edge = false>
-__device__ __forceinline__ unsigned load_row_raw(const SubstepArgs& a, const Strip<C>& st, int r,
-                                                 float (&v)[C][NV]) {
+template <int C, int NV, bool Pinned, bool Edge = false, int GC = 2, class Args>
+__device__ __forceinline__ unsigned load_row_raw(const Args& a, const Strip<C>& st, int r, float (&v)[C][NV]) {
     // Row offsets are wave-uniform (SGPR soffset); the lane adds its column
     // offset (VGPR voffset): no per-lane address arithmetic.
     unsigned ysign;
-    const int row = map_row<2>(st.ymap, __builtin_amdgcn_readfirstlane(st.row0 + r), ysign);
+    const int row = map_row<GC>(st.ymap, __builtin_amdgcn_readfirstlane(st.row0 + r), ysign);
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
         const int soff = row * a.in_pitch[k];
@@ -756,8 +755,9 @@ __device__ __forceinline__ unsigned load_row_raw(const SubstepArgs& a, const Str
         } else {
             static_assert(C == 2, "one or two columns per lane");
             const fvmi_v2u x = __builtin_amdgcn_raw_buffer_load_b64(st.rin[k], st.pair_off, soff, 0);
-            unsigned w0 = st.pair_rev ? x.y : x.x;
-            unsigned w1 = st.pair_rev ? x.x : x.y;
+            // (with one ghost cell a side no pair is reversed)
+            unsigned w0 = GC > 1 && st.pair_rev ? x.y : x.x;
+            unsigned w1 = GC > 1 && st.pair_rev ? x.x : x.y;
             if constexpr (Edge) {
                 const unsigned f0 = __builtin_amdgcn_raw_buffer_load_b32(st.rin[k], st.fix_off[0], soff, 0);
                 const unsigned f1 = __builtin_amdgcn_raw_buffer_load_b32(st.rin[k], st.fix_off[1], soff, 0);
@@ -789,8 +789,8 @@ __device__ __forceinline__ void use_row(const Strip<C>& st, unsigned ysign, floa
     }
 }
 
-template <int C, int NV, bool Edge = false>
-__device__ __forceinline__ void store_row(const SubstepArgs& a, const Strip<C>& st, int r, const float (&q)[C][NV]) {
+template <int C, int NV, bool Edge = false, class Args>
+__device__ __forceinline__ void store_row(const Args& a, const Strip<C>& st, int r, const float (&q)[C][NV]) {
     const int prow = __builtin_amdgcn_readfirstlane(st.row0 + r);
     // every lane stores; the halo lanes' offset is out of range and the
     // hardware drops their writes (no branch around the stores)
@@ -1111,31 +1111,25 @@ __device__ __forceinline__ float march_waf(const SubstepArgs& a, const Strip<S::
     return dt_min;
 }
 
-// Halo: cells of halo a side, 2 for a substep and 4 for a whole step.
-template <class S, class M, int Halo = 2>
-__device__ __forceinline__ void setup_strip(const SubstepArgs& a, Strip<S::kC>& st, int lane, int strip_x, int row_in,
-                                            int count) {
-    constexpr int C = S::kC;
-    constexpr int H = halo_lanes<C, Halo>();
-    constexpr bool Deep = Halo > 2;
+// The column constants of a strip whose lane 0, column 0 is padded column
+// `wstart`; H lanes at each end are halo, and only columns [lo, hi) are written.
+template <int C, int GC, bool Deep>
+__device__ __forceinline__ void setup_columns(Strip<C>& st, int lane, int wstart, int H, int nx, int bc, int lo,
+                                              int hi) {
     st.lane = lane;
-    const int wstart = a.x0 + strip_cols<C, Halo>() * strip_x + 2 - H * C;    // padded column of lane 0, column 0
-    st.row0 = __builtin_amdgcn_readfirstlane(a.y0 + row_in + 2 - Halo);       // padded row of r = 0
-    st.r_end = __builtin_amdgcn_readfirstlane(count + 2 * Halo);              // output rows r = 2 Halo .. r_end-1
-    st.ymap = make_row_map<2, Deep>(a.ny, (a.bc >> 16) & 0xF, (a.bc >> 24) & 0xF);
 #pragma unroll
     for (int c = 0; c < C; ++c) {
         st.col[c] = wstart + C * lane + c;
-        const AxisMap mx = map_axis_gc<2, Deep>(st.col[c], a.nx, a.bc & 0xF, (a.bc >> 8) & 0xF);
+        const AxisMap mx = map_axis_gc<GC, Deep>(st.col[c], nx, bc & 0xF, (bc >> 8) & 0xF);
         st.lane_off[c] = mx.idx * (int)sizeof(float);
         st.xsign[c] = mx.mirrored ? 0x80000000u : 0u;
-        st.lane_out[c] = lane >= H && lane < kLanes - H && st.col[c] < a.x1 + 2;
+        st.lane_out[c] = lane >= H && lane < kLanes - H && st.col[c] >= lo && st.col[c] < hi;
     }
     if constexpr (C == 1) {
         st.store_off = st.lane_out[0] ? st.col[0] * (int)sizeof(float) : kMaskedOffset;
     } else {
         const int o0 = st.lane_off[0], o1 = st.lane_off[1];
-        const bool fwd = o1 == o0 + 4, rev = o1 == o0 - 4;
+        const bool fwd = o1 == o0 + 4, rev = GC > 1 && o1 == o0 - 4;
         const int base = rev ? o1 : o0;
         st.pair_rev = rev;
         st.lane_fix = !(fwd || rev) || (base & 7) != 0;
@@ -1150,11 +1144,31 @@ __device__ __forceinline__ void setup_strip(const SubstepArgs& a, Strip<S::kC>& 
         st.single_off[1] = (!full && st.lane_out[1]) ? s0 + 4 : kMaskedOffset;
         st.wave_single = __builtin_amdgcn_ballot_w64(!full && (st.lane_out[0] || st.lane_out[1])) != 0;
     }
+}
+
+// The fields' buffer descriptors, of `rows` padded rows each.
+template <int NV, int C, class Args>
+__device__ __forceinline__ void setup_fields(const Args& a, Strip<C>& st, int rows) {
 #pragma unroll
-    for (int k = 0; k < S::NV; ++k) {
-        st.rin[k] = field_rsrc(a.in[k], (unsigned)(a.ny + 4) * (unsigned)a.in_pitch[k]);
-        st.rout[k] = field_rsrc(a.out[k], (unsigned)(a.ny + 4) * (unsigned)a.out_pitch[k]);
+    for (int k = 0; k < NV; ++k) {
+        st.rin[k] = field_rsrc(a.in[k], (unsigned)rows * (unsigned)a.in_pitch[k]);
+        st.rout[k] = field_rsrc(a.out[k], (unsigned)rows * (unsigned)a.out_pitch[k]);
     }
+}
+
+// Halo: cells of halo a side, 2 for a substep and 4 for a whole step.
+template <class S, class M, int Halo = 2>
+__device__ __forceinline__ void setup_strip(const SubstepArgs& a, Strip<S::kC>& st, int lane, int strip_x, int row_in,
+                                            int count) {
+    constexpr int C = S::kC;
+    constexpr int H = halo_lanes<C, Halo>();
+    constexpr bool Deep = Halo > 2;
+    st.row0 = __builtin_amdgcn_readfirstlane(a.y0 + row_in + 2 - Halo);  // padded row of r = 0
+    st.r_end = __builtin_amdgcn_readfirstlane(count + 2 * Halo);         // output rows r = 2 Halo .. r_end-1
+    st.ymap = make_row_map<2, Deep>(a.ny, (a.bc >> 16) & 0xF, (a.bc >> 24) & 0xF);
+    const int first = a.x0 + strip_cols<C, Halo>() * strip_x + 2;  // padded column of the first output
+    setup_columns<C, 2, Deep>(st, lane, first - H * C, H, a.nx, a.bc, first, a.x1 + 2);
+    setup_fields<S::NV>(a, st, a.ny + 4);
 }
 
 // The march of one segment: sweep order by step, and the edge variant only

@@ -14,7 +14,7 @@
 // Work split and addressing as the dimensionally split kernel (fv_substep.h):
 // a wavefront owns a strip of 64 - 2*GC columns (lane c = padded column
 // 62*s + c for GC = 1, 60*s + c for GC = 2; the GC lanes at each edge are the
-// x halo) and marches down a segment of rows; x neighbours come through DPP
+// x halo), or for GC = 1 on large grids of 124 columns, two per lane, and marches down a segment of rows; x neighbours come through DPP
 // row moves, y neighbours from a register ring of rows.
 #pragma once
 
@@ -35,6 +35,7 @@ struct UnsplitArgs {
     float* out[3];
     int out_pitch[3];
     float* cfl;  // two floats, may be null
+    int cols;  // columns per lane: two for the one-ghost-cell schemes on 8-byte aligned fields, else one
     int seg_rows;
     int segs_per_strip;
     int strips_x;
@@ -127,15 +128,22 @@ struct UnsplitBase {
     }
 };
 
+// flux_x / flux_y take the interfaces of a lane's C columns at once.
 template <class M>
 struct SweLxF : UnsplitBase<M> {
     static constexpr int GC = 1;
     static constexpr int kind = KIND_LXF;
-    __device__ static void flux_x(const float l[3], const float r[3], const UnsplitArgs& a, float o[3]) {
-        lxf_2d_flux<M>(l, r, a.g, a.dx, a.dt, a.lxf_kx, o);
+    template <int C>
+    __device__ static void flux_x(const float (&l)[C][3], const float (&r)[C][3], const UnsplitArgs& a,
+                                  float (&o)[C][3]) {
+#pragma unroll
+        for (int c = 0; c < C; ++c) lxf_2d_flux<M>(l[c], r[c], a.g, a.dx, a.dt, a.lxf_kx, o[c]);
     }
-    __device__ static void flux_y(const float l[3], const float r[3], const UnsplitArgs& a, float o[3]) {
-        lxf_2d_flux<M>(l, r, a.g, a.dy, a.dt, a.lxf_ky, o);
+    template <int C>
+    __device__ static void flux_y(const float (&l)[C][3], const float (&r)[C][3], const UnsplitArgs& a,
+                                  float (&o)[C][3]) {
+#pragma unroll
+        for (int c = 0; c < C; ++c) lxf_2d_flux<M>(l[c], r[c], a.g, a.dy, a.dt, a.lxf_ky, o[c]);
     }
 };
 
@@ -143,14 +151,20 @@ template <class M>
 struct SweHLL1 : UnsplitBase<M> {
     static constexpr int GC = 1;
     static constexpr int kind = KIND_SPLIT1;
-    __device__ static void flux_x(const float l[3], const float r[3], const UnsplitArgs& a, float o[3]) {
-        if constexpr (M::exact)
-            swe_hll_flux(l, r, a.g, o);
-        else
-            fast::swe_hll_flux<1>(one_column(l), one_column(r), a.hg, a.sqrt_g, one_column(o));
+    template <int C>
+    __device__ static void flux_x(const float (&l)[C][3], const float (&r)[C][3], const UnsplitArgs& a,
+                                  float (&o)[C][3]) {
+        if constexpr (M::exact) {
+#pragma unroll
+            for (int c = 0; c < C; ++c) swe_hll_flux(l[c], r[c], a.g, o[c]);
+        } else {
+            fast::swe_hll_flux<C>(l, r, a.hg, a.sqrt_g, o);
+        }
     }
-    __device__ static void flux_y(const float l[3], const float r[3], const UnsplitArgs& a, float o[3]) {
-        flux_x(l, r, a, o);
+    template <int C>
+    __device__ static void flux_y(const float (&l)[C][3], const float (&r)[C][3], const UnsplitArgs& a,
+                                  float (&o)[C][3]) {
+        flux_x<C>(l, r, a, o);
     }
 };
 
@@ -158,11 +172,17 @@ template <class M>
 struct SweFORCE : UnsplitBase<M> {
     static constexpr int GC = 1;
     static constexpr int kind = KIND_SPLIT1;
-    __device__ static void flux_x(const float l[3], const float r[3], const UnsplitArgs& a, float o[3]) {
-        force_1d_flux<M>(l, r, a.g, a.dx, a.dt, a.lf_kx, a.lw_kx, o);
+    template <int C>
+    __device__ static void flux_x(const float (&l)[C][3], const float (&r)[C][3], const UnsplitArgs& a,
+                                  float (&o)[C][3]) {
+#pragma unroll
+        for (int c = 0; c < C; ++c) force_1d_flux<M>(l[c], r[c], a.g, a.dx, a.dt, a.lf_kx, a.lw_kx, o[c]);
     }
-    __device__ static void flux_y(const float l[3], const float r[3], const UnsplitArgs& a, float o[3]) {
-        force_1d_flux<M>(l, r, a.g, a.dy, a.dt, a.lf_ky, a.lw_ky, o);
+    template <int C>
+    __device__ static void flux_y(const float (&l)[C][3], const float (&r)[C][3], const UnsplitArgs& a,
+                                  float (&o)[C][3]) {
+#pragma unroll
+        for (int c = 0; c < C; ++c) force_1d_flux<M>(l[c], r[c], a.g, a.dy, a.dt, a.lf_ky, a.lw_ky, o[c]);
     }
 };
 
@@ -179,52 +199,32 @@ struct SweKP07U : UnsplitBase<M> {
 };
 
 // ---------------------------------------------------------------------------
-// Strip addressing for GC ghost cells
+// Strip addressing (Strip, load_row_raw, use_row, store_row of fv_substep.h)
 // ---------------------------------------------------------------------------
 
-template <int GC>
-struct UStrip {
-    int col;       // padded column of this lane
-    int row0;      // padded row of r = 0
-    int r_end;     // rows r in [0, r_end)
-    int lane_off;    // byte offset of this lane's column (after the boundary map)
-    unsigned xsign;  // sign-bit mask of the x momentum (mirrored ghost column)
-    bool lane_out;
-    int store_off;  // byte offset of the column for writing lanes, kMaskedOffset for the others
-    RowMap ymap;
-    __amdgpu_buffer_rsrc_t rin[3], rout[3];
-};
+// Columns of a strip of C columns per lane.  One ghost cell: 62 with one column
+// (lane 1 of strip 0 holds padded column 1), 124 with two (lane 1 holds columns
+// 0 and 1, so that pairs sit at 8-byte offsets; column 0 is not written).
+template <int GC, int C>
+__host__ __device__ constexpr int u_strip_cols() {
+    return strip_cols<C, GC>();
+}
+// first padded column in the output lanes of strip 0
+template <int GC, int C>
+__host__ __device__ constexpr int u_first_col() {
+    return GC == 1 && C == 2 ? 0 : GC;
+}
 
-template <int GC>
-__device__ __forceinline__ void u_setup(const UnsplitArgs& a, UStrip<GC>& st, int lane, int strip_x, int row_in,
+template <int GC, int C>
+__device__ __forceinline__ void u_setup(const UnsplitArgs& a, Strip<C>& st, int lane, int strip_x, int row_in,
                                         int count) {
-    constexpr int W = kLanes - 2 * GC;
-    st.col = W * strip_x + lane;
+    constexpr int H = halo_lanes<C, GC>();
     st.row0 = __builtin_amdgcn_readfirstlane(row_in);  // padded row of the first row read
     st.r_end = __builtin_amdgcn_readfirstlane(count + 2 * GC);
     st.ymap = make_row_map<GC>(a.ny, (a.bc >> 16) & 0xF, (a.bc >> 24) & 0xF);
-    const AxisMap mx = map_axis_gc<GC>(st.col, a.nx, a.bc & 0xF, (a.bc >> 8) & 0xF);
-    st.lane_off = mx.idx * (int)sizeof(float);
-    st.xsign = mx.mirrored ? 0x80000000u : 0u;
-    st.lane_out = lane >= GC && lane < GC + W && st.col < a.nx + GC;
-    st.store_off = st.lane_out ? st.col * (int)sizeof(float) : kMaskedOffset;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        st.rin[k] = field_rsrc(a.in[k], (unsigned)(a.ny + 2 * GC) * (unsigned)a.in_pitch[k]);
-        st.rout[k] = field_rsrc(a.out[k], (unsigned)(a.ny + 2 * GC) * (unsigned)a.out_pitch[k]);
-    }
-}
-
-// Issues the loads of padded row r (raw words) and returns the sign-bit mask
-// of its y momentum; u_use applies the mirror signs at the row's first use.
-template <int GC>
-__device__ __forceinline__ unsigned u_load(const UnsplitArgs& a, const UStrip<GC>& st, int r, float (&v)[3]) {
-    unsigned ysign;
-    const int row = map_row<GC>(st.ymap, __builtin_amdgcn_readfirstlane(st.row0 + r), ysign);
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-        v[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(st.rin[k], st.lane_off, row * a.in_pitch[k], 0));
-    return ysign;
+    const int first = u_first_col<GC, C>() + u_strip_cols<GC, C>() * strip_x;
+    setup_columns<C, GC, false>(st, lane, first - H * C, H, a.nx, a.bc, GC, a.nx + GC);
+    setup_fields<3>(a, st, a.ny + 2 * GC);
 }
 
 // Values first used here: an empty volatile statement hands them on, so the
@@ -236,34 +236,11 @@ __device__ __forceinline__ void u_pin(float (&v)[3]) {
     for (int k = 0; k < 3; ++k) asm volatile("" : "+v"(v[k]));
 }
 
-// First use of a row loaded by u_load: pinned, then x mirrors flip the x
-// momentum and y mirrors the y momentum.
-template <int GC>
-__device__ __forceinline__ void u_use(const UStrip<GC>& st, unsigned ysign, float (&v)[3]) {
-    u_pin(v);
-    v[1] = __uint_as_float(__float_as_uint(v[1]) ^ st.xsign);
-    v[2] = __uint_as_float(__float_as_uint(v[2]) ^ ysign);
-}
-
-// Output row `prow` (padded): the stored state, or for the second RK2 stage
-// 0.5 (old + q) with `old` the output buffer's value (SWE2D_KP07.cu:205-209),
-// read ahead by u_load_old.  Every lane stores; the halo lanes' offset is out
-// of range (kMaskedOffset), so the hardware drops their writes (and returns 0
-// for their reads).
-template <int GC, bool Avg = false>
-__device__ __forceinline__ void u_store(const UnsplitArgs& a, const UStrip<GC>& st, int prow, const float (&q)[3],
-                                        const float (&old)[3]) {
-    const int row = __builtin_amdgcn_readfirstlane(prow);
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        const float v = Avg ? 0.5f * (old[k] + q[k]) : q[k];
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), st.rout[k], st.store_off, row * a.out_pitch[k], 0);
-    }
-}
-
-// the output buffer's row `prow` (padded), for the second RK2 stage
-template <int GC>
-__device__ __forceinline__ void u_load_old(const UnsplitArgs& a, const UStrip<GC>& st, int prow, float (&old)[3]) {
+// Output row `prow` (padded) of the second RK2 stage, 0.5 (old + q) with `old`
+// the output buffer's value (SWE2D_KP07.cu:205-209), read ahead by u_load_old.
+// Every lane stores; the halo lanes' offset is out of range (kMaskedOffset), so
+// the hardware drops their writes (and returns 0 for their reads).
+__device__ __forceinline__ void u_load_old(const UnsplitArgs& a, const Strip<1>& st, int prow, float (&old)[3]) {
     const int row = __builtin_amdgcn_readfirstlane(prow);
 #pragma unroll
     for (int k = 0; k < 3; ++k)
@@ -301,13 +278,33 @@ __device__ __forceinline__ float u_update(float q, float df, float dg, const Arg
 // Row steps
 // ---------------------------------------------------------------------------
 
-// x fluxes of one row held across the lanes: F[k] through the interface
-// (c, c+1) of this lane's column c.
-template <class S, class M>
-__device__ __forceinline__ void x_fluxes_first_order(const float (&q)[3], const UnsplitArgs& a, float (&F)[3]) {
-    float r[3];
-    all_from_right<3>(q, r);
-    S::flux_x(q, r, a, F);
+// x fluxes of one row held across the lanes, C columns each: F[c] through the
+// right interface of column c; dF[c] = left flux minus right flux of column c.
+template <class S, int C>
+__device__ __forceinline__ void x_flux_differences(const float (&q)[C][3], const UnsplitArgs& a, float (&dF)[C][3]) {
+    float right[C][3], F[C][3];
+    all_from_right<3>(q[0], right[C - 1]);
+#pragma unroll
+    for (int c = 0; c < C - 1; ++c)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) right[c][k] = q[c + 1][k];
+    S::template flux_x<C>(q, right, a, F);
+    left_minus_all<3>(F[C - 1], F[0], dF[0]);
+#pragma unroll
+    for (int c = 1; c < C; ++c)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) dF[c][k] = F[c - 1][k] - F[c][k];
+}
+
+// x sweep of a row of a split first-order scheme
+template <class S, class M, int C>
+__device__ __forceinline__ void x_sweep_first_order(float (&q)[C][3], const UnsplitArgs& a) {
+    float dF[C][3];
+    x_flux_differences<S, C>(q, a, dF);
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) q[c][k] = evolve<M>(q[c][k], dF[c][k], a.dt, a.dx, a.dtdx);
 }
 
 // x fluxes of KP07: minmod slope along the row, face values Q -+ slope/2,
@@ -327,50 +324,52 @@ __device__ __forceinline__ void x_fluxes_kp07(const float (&q)[3], const Unsplit
     S::flux(qm, qp, a, F);
 }
 
-// y flux between two rows (lower = row r, upper = row r+1): the flux
+// y fluxes between two rows (lower = row r, upper = row r+1): the flux
 // functions see (h, hv, hu) and the result is swapped back
-template <class S>
-__device__ __forceinline__ void y_flux(const float (&lo)[3], const float (&hi)[3], const UnsplitArgs& a,
-                                       float (&G)[3]) {
-    float l[3], h[3], o[3];
-    swap_tn(lo, l);
-    swap_tn(hi, h);
-    S::flux_y(l, h, a, o);
-    swap_tn(o, G);
+template <class S, int C>
+__device__ __forceinline__ void y_fluxes(const float (&lo)[C][3], const float (&hi)[C][3], const UnsplitArgs& a,
+                                         float (&G)[C][3]) {
+    float l[C][3], h[C][3], o[C][3];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        swap_tn(lo[c], l[c]);
+        swap_tn(hi[c], h[c]);
+    }
+    S::template flux_y<C>(l, h, a, o);
+#pragma unroll
+    for (int c = 0; c < C; ++c) swap_tn(o[c], G[c]);
 }
 
 // One step of the one-ghost-cell march: w0 = row r-1 (x-evolved for the split
 // schemes), w1 = raw row r on entry (x-evolved here for the split schemes);
 // g = flux (r-2, r-1) on entry, (r-1, r) on return; emits row r-1.
-template <class S, class M>
-__device__ __forceinline__ void gc1_row(const UnsplitArgs& a, const UStrip<1>& st, const float (&w0)[3],
-                                        float (&w1)[3], float (&g)[3], int r, bool emit, float& acc) {
-    if constexpr (S::kind == KIND_SPLIT1) {
-        float F[3], dF[3];
-        x_fluxes_first_order<S, M>(w1, a, F);
-        left_minus_all<3>(F, F, dF);
-#pragma unroll
-        for (int k = 0; k < 3; ++k) w1[k] = evolve<M>(w1[k], dF[k], a.dt, a.dx, a.dtdx);
-    }
-    float G[3];
-    y_flux<S>(w0, w1, a, G);
+template <class S, class M, int C, bool Edge>
+__device__ __forceinline__ void gc1_row(const UnsplitArgs& a, const Strip<C>& st, const float (&w0)[C][3],
+                                        float (&w1)[C][3], float (&g)[C][3], int r, bool emit, float& acc) {
+    if constexpr (S::kind == KIND_SPLIT1) x_sweep_first_order<S, M, C>(w1, a);
+    float G[C][3];
+    y_fluxes<S, C>(w0, w1, a, G);
     if (emit) {
-        float out[3];
-        if constexpr (S::kind == KIND_SPLIT1) {
+        float out[C][3], dF[C][3];
+        if constexpr (S::kind != KIND_SPLIT1) x_flux_differences<S, C>(w0, a, dF);
 #pragma unroll
-            for (int k = 0; k < 3; ++k) out[k] = evolve<M>(w0[k], g[k] - G[k], a.dt, a.dy, a.dtdy);
-        } else {
-            float F[3], dF[3];
-            x_fluxes_first_order<S, M>(w0, a, F);
-            left_minus_all<3>(F, F, dF);
+        for (int c = 0; c < C; ++c)
 #pragma unroll
-            for (int k = 0; k < 3; ++k) out[k] = u_update<M>(w0[k], dF[k], g[k] - G[k], a);
-        }
-        u_store<1>(a, st, st.row0 + r - 1, out, out);
-        u_cfl<S, M>(out, a, st.lane_out, acc);
+            for (int k = 0; k < 3; ++k) {
+                const float dG = g[c][k] - G[c][k];
+                if constexpr (S::kind == KIND_SPLIT1)
+                    out[c][k] = evolve<M>(w0[c][k], dG, a.dt, a.dy, a.dtdy);
+                else
+                    out[c][k] = u_update<M>(w0[c][k], dF[c][k], dG, a);
+            }
+        store_row<C, 3, Edge>(a, st, r - 1, out);
+#pragma unroll
+        for (int c = 0; c < C; ++c) u_cfl<S, M>(out[c], a, st.lane_out[c], acc);
     }
 #pragma unroll
-    for (int k = 0; k < 3; ++k) g[k] = G[k];
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) g[c][k] = G[c][k];
 }
 
 // One step of the KP07 march: w0, w1, w2 = raw rows r-2, r-1, r; top = top
@@ -378,7 +377,7 @@ __device__ __forceinline__ void gc1_row(const UnsplitArgs& a, const UStrip<1>& s
 // (r-2, r-1) on return; emits row r-2 (Stage2: averaged with `old`, the output
 // buffer's row r-2).
 template <class S, class M, bool Stage2>
-__device__ __forceinline__ void kp07u_row(const UnsplitArgs& a, const UStrip<2>& st, const float (&w0)[3],
+__device__ __forceinline__ void kp07u_row(const UnsplitArgs& a, const Strip<1>& st, const float (&w0)[3],
                                           const float (&w1)[3], const float (&w2)[3], const float (&old)[3],
                                           float (&top)[3], float (&g)[3], int r, bool emit, float& acc) {
     float bot[3], top_next[3];
@@ -402,8 +401,11 @@ __device__ __forceinline__ void kp07u_row(const UnsplitArgs& a, const UStrip<2>&
         left_minus_all<3>(F, F, dF);
 #pragma unroll
         for (int k = 0; k < 3; ++k) out[k] = u_update<M>(w0[k], dF[k], g[k] - G[k], a);
-        u_store<2, Stage2>(a, st, st.row0 + r - 2, out, old);
-        u_cfl<S, M>(out, a, st.lane_out, acc);  // before the RK2 average, as writeCfl reads the tile
+        float v[1][3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) v[0][k] = Stage2 ? 0.5f * (old[k] + out[k]) : out[k];
+        store_row<1, 3>(a, st, r - 2, v);
+        u_cfl<S, M>(out, a, st.lane_out[0], acc);  // before the RK2 average, as writeCfl reads the tile
     }
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -416,33 +418,31 @@ __device__ __forceinline__ void kp07u_row(const UnsplitArgs& a, const UStrip<2>&
 // Marches (row m of a segment in ring slot m % N; see march_slopes)
 // ---------------------------------------------------------------------------
 
-template <class S, class M>
-__device__ __forceinline__ float march_gc1(const UnsplitArgs& a, const UStrip<1>& st) {
+template <class S, class M, int C, bool Edge>
+__device__ __forceinline__ float march_gc1(const UnsplitArgs& a, const Strip<C>& st) {
     constexpr int PF = kRowPrefetch;
     constexpr int N = PF + 2;  // rows r-1, r and PF rows in flight
     float acc = M::exact ? __builtin_inff() : 0.0f;
-    float ring[N][3], G[3];
+    float ring[N][C][3], G[C][3];
     unsigned ys[N];  // y-momentum sign mask of each slot's row
     const int last = st.r_end - 1;  // r_end >= 3
+    auto load = [&](int slot, int m) { ys[slot] = load_row_raw<C, 3, true, Edge, 1>(a, st, min(m, last), ring[slot]); };
+    auto use = [&](int slot) { use_row<C, 3, true>(st, ys[slot], ring[slot]); };
 #pragma unroll
-    for (int m = 0; m < N; ++m) ys[m] = u_load<1>(a, st, min(m, last), ring[m]);
-    u_use<1>(st, ys[0], ring[0]);
-    u_use<1>(st, ys[1], ring[1]);
-    if constexpr (S::kind == KIND_SPLIT1) {
-        float F[3], dF[3];
-        x_fluxes_first_order<S, M>(ring[0], a, F);
-        left_minus_all<3>(F, F, dF);
+    for (int m = 0; m < N; ++m) load(m, m);
+    use(0);
+    use(1);
+    if constexpr (S::kind == KIND_SPLIT1) x_sweep_first_order<S, M, C>(ring[0], a);
 #pragma unroll
-        for (int k = 0; k < 3; ++k) ring[0][k] = evolve<M>(ring[0][k], dF[k], a.dt, a.dx, a.dtdx);
-    }
+    for (int c = 0; c < C; ++c)
 #pragma unroll
-    for (int k = 0; k < 3; ++k) G[k] = 0.0f;
+        for (int k = 0; k < 3; ++k) G[c][k] = 0.0f;
     // the prologue holds rows 0 .. 1+PF, all that step 1 and its prefetch need
-    gc1_row<S, M>(a, st, ring[0], ring[1], G, 1, false, acc);  // flux (0, 1)
+    gc1_row<S, M, C, Edge>(a, st, ring[0], ring[1], G, 1, false, acc);  // flux (0, 1)
     auto step = [&](int u, int rr) {
-        ys[(2 + u + PF) % N] = u_load<1>(a, st, min(rr + PF, last), ring[(2 + u + PF) % N]);
-        u_use<1>(st, ys[(2 + u) % N], ring[(2 + u) % N]);
-        gc1_row<S, M>(a, st, ring[(1 + u) % N], ring[(2 + u) % N], G, rr, true, acc);
+        load((2 + u + PF) % N, rr + PF);
+        use((2 + u) % N);
+        gc1_row<S, M, C, Edge>(a, st, ring[(1 + u) % N], ring[(2 + u) % N], G, rr, true, acc);
     };
     int r = 2;
     for (; r + N <= st.r_end; r += N) {
@@ -460,41 +460,41 @@ __device__ __forceinline__ float march_gc1(const UnsplitArgs& a, const UStrip<1>
 // averaged and stored.  Only steps m >= 4 emit, so only their rows are read
 // (the rows of steps 0 and 1 would lie above the buffer for the first segment).
 template <class S, class M, bool Stage2>
-__device__ __forceinline__ float march_kp07u(const UnsplitArgs& a, const UStrip<2>& st) {
+__device__ __forceinline__ float march_kp07u(const UnsplitArgs& a, const Strip<1>& st) {
     constexpr int PF = kRowPrefetch;
     constexpr int N = PF + 3;
     static_assert(3 + PF >= 4, "rows loaded in the steps belong to emitting steps");
     float acc = M::exact ? __builtin_inff() : 0.0f;
-    float ring[N][3], old[N][3], P[3], G[3];
+    float ring[N][1][3], old[N][3], P[3], G[3];
     unsigned ys[N];  // y-momentum sign mask of each slot's row
     const int last = st.r_end - 1;  // r_end >= 5
     auto load = [&](int m, int slot) {  // m >= 4
-        ys[slot] = u_load<2>(a, st, min(m, last), ring[slot]);
-        if constexpr (Stage2) u_load_old<2>(a, st, st.row0 + min(m, last) - 2, old[slot]);
+        ys[slot] = load_row_raw<1, 3, true>(a, st, min(m, last), ring[slot]);
+        if constexpr (Stage2) u_load_old(a, st, st.row0 + min(m, last) - 2, old[slot]);
     };
 #pragma unroll
     for (int m = 0; m < N; ++m) {
         if (m >= 4)
             load(m, m);
         else
-            ys[m] = u_load<2>(a, st, min(m, last), ring[m]);
+            ys[m] = load_row_raw<1, 3, true>(a, st, min(m, last), ring[m]);
     }
 #pragma unroll
-    for (int m = 0; m < 3; ++m) u_use<2>(st, ys[m], ring[m]);
+    for (int m = 0; m < 3; ++m) use_row<1, 3, true>(st, ys[m], ring[m]);
 #pragma unroll
     for (int k = 0; k < 3; ++k) {  // top face of row 1
-        P[k] = ring[1][k] + half_slope<M>(ring[0][k], ring[1][k], ring[2][k], a);
+        P[k] = ring[1][0][k] + half_slope<M>(ring[0][0][k], ring[1][0][k], ring[2][0][k], a);
         G[k] = 0.0f;
     }
     load(3 + PF, (3 + PF) % N);
-    u_use<2>(st, ys[3 % N], ring[3 % N]);
-    kp07u_row<S, M, Stage2>(a, st, ring[1], ring[2], ring[3 % N], old[3 % N], P, G, 3, false, acc);  // flux (1, 2)
+    use_row<1, 3, true>(st, ys[3 % N], ring[3 % N]);
+    kp07u_row<S, M, Stage2>(a, st, ring[1][0], ring[2][0], ring[3 % N][0], old[3 % N], P, G, 3, false, acc);  // flux (1, 2)
     auto step = [&](int u, int rr) {
         load(rr + PF, (4 + u + PF) % N);
-        u_use<2>(st, ys[(4 + u) % N], ring[(4 + u) % N]);
+        use_row<1, 3, true>(st, ys[(4 + u) % N], ring[(4 + u) % N]);
         if constexpr (Stage2) u_pin(old[(4 + u) % N]);
-        kp07u_row<S, M, Stage2>(a, st, ring[(2 + u) % N], ring[(3 + u) % N], ring[(4 + u) % N], old[(4 + u) % N], P,
-                                G, rr, true, acc);
+        kp07u_row<S, M, Stage2>(a, st, ring[(2 + u) % N][0], ring[(3 + u) % N][0], ring[(4 + u) % N][0],
+                                old[(4 + u) % N], P, G, rr, true, acc);
     };
     int r = 4;
     for (; r + N <= st.r_end; r += N) {
@@ -520,17 +520,29 @@ __host__ __device__ inline bool unsplit_segment(const UnsplitArgs& a, int block,
         const int per = grid >> 3;
         lb = (block & 7) * per + (block >> 3);
     }
-    const int gw = lb * a.waves_per_block + wave;
-    if (lb >= a.num_blocks || gw >= a.num_waves) return false;
-    strip_x = gw / a.segs_per_strip;
-    row_in = (gw - strip_x * a.segs_per_strip) * a.seg_rows;
+    if (lb >= a.num_blocks) return false;
+    int seg;
+    if (a.cols == 2) {  // the waves of a workgroup take the same rows of adjacent strips
+        const int band = lb / a.segs_per_strip;
+        strip_x = band * a.waves_per_block + wave;
+        seg = lb - band * a.segs_per_strip;
+        if (strip_x >= a.strips_x) return false;
+    } else {
+        const int gw = lb * a.waves_per_block + wave;
+        if (gw >= a.num_waves) return false;
+        strip_x = gw / a.segs_per_strip;
+        seg = gw - strip_x * a.segs_per_strip;
+    }
+    row_in = seg * a.seg_rows;
     count = min(a.seg_rows, a.ny - row_in);
     return true;
 }
 
-template <class S, class M>
+// C: columns per lane (the two-ghost-cell scheme marches one)
+template <class S, class M, int C>
 __global__ void __launch_bounds__(256, 4) unsplit_kernel(UnsplitArgs a) {
     constexpr int GC = S::GC;
+    static_assert(GC == 1 || C == 1, "KP07 marches one column per lane");
     const int lane = threadIdx.x & (kLanes - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (a.cfl != nullptr && blockIdx.x == 0 && threadIdx.x == 0) a.cfl[1 - a.cfl_slot] = __builtin_inff();
@@ -539,13 +551,17 @@ __global__ void __launch_bounds__(256, 4) unsplit_kernel(UnsplitArgs a) {
     strip_x = __builtin_amdgcn_readfirstlane(strip_x);
     row_in = __builtin_amdgcn_readfirstlane(row_in);
     count = __builtin_amdgcn_readfirstlane(count);
-    UStrip<GC> st;
-    u_setup<GC>(a, st, lane, strip_x, row_in, count);
+    Strip<C> st;
+    u_setup<GC, C>(a, st, lane, strip_x, row_in, count);
     float acc;
-    if constexpr (GC == 1)
-        acc = march_gc1<S, M>(a, st);
-    else
+    if constexpr (GC == 1) {
+        if (C == 2 && (st.wave_fix || st.wave_single))
+            acc = march_gc1<S, M, C, C == 2>(a, st);
+        else
+            acc = march_gc1<S, M, C, false>(a, st);
+    } else {
         acc = a.stage2 ? march_kp07u<S, M, true>(a, st) : march_kp07u<S, M, false>(a, st);
+    }
     float dt_min = acc;
     if constexpr (!M::exact) dt_min = (acc > 0.0f) ? fast::rcp(acc) : __builtin_inff();
     if (a.cfl != nullptr) {
@@ -555,13 +571,18 @@ __global__ void __launch_bounds__(256, 4) unsplit_kernel(UnsplitArgs a) {
     }
 }
 
-// Strip-aligned segments (as plan_substep) for strips of 64 - 2*GC columns:
-// the round-weighted split where `round_ok` and it fits, else equal segments,
-// at most waves_per_simd waves on every SIMD.
+// Strip-aligned segments (as plan_substep) for a.cols columns per lane: the
+// round-weighted split where `round_ok` and it fits, else equal segments, at most
+// waves_per_simd waves on every SIMD.
 inline int plan_unsplit(UnsplitArgs& a, int gc, int cu_count, bool round_ok, int waves_per_simd = 4,
                         int min_seg = 24, int min_part = 16) {
-    const int W = kLanes - 2 * gc;
-    a.strips_x = (a.nx + W - 1) / W;
+    if (gc == 1 && a.cols == 2) {
+        constexpr int W = u_strip_cols<1, 2>();
+        a.strips_x = (a.nx + 1 + W - 1) / W;  // output columns from padded column 0 on
+    } else {
+        const int W = kLanes - 2 * gc;
+        a.strips_x = (a.nx + W - 1) / W;
+    }
     a.round_plan = 0;
     a.xcds = 8;
     a.cus_per_xcd = cu_count / 8;
@@ -583,7 +604,8 @@ inline int plan_unsplit(UnsplitArgs& a, int gc, int cu_count, bool round_ok, int
     if (a.seg_rows <= 0) a.seg_rows = balanced_segment_rows(a.ny, a.strips_x, cu_count, waves_per_simd, min_seg, 4);
     a.segs_per_strip = (a.ny + a.seg_rows - 1) / a.seg_rows;
     a.num_waves = a.strips_x * a.segs_per_strip;
-    a.num_blocks = (a.num_waves + a.waves_per_block - 1) / a.waves_per_block;
+    a.num_blocks = a.cols == 2 ? ((a.strips_x + a.waves_per_block - 1) / a.waves_per_block) * a.segs_per_strip
+                               : (a.num_waves + a.waves_per_block - 1) / a.waves_per_block;
     int grid = a.num_blocks;
     if (a.xcd_remap) grid = ((grid + 7) / 8) * 8;
     return grid;
@@ -591,25 +613,55 @@ inline int plan_unsplit(UnsplitArgs& a, int gc, int cu_count, bool round_ok, int
 
 enum UnsplitSchemeId : int { USCHEME_LXF = 0, USCHEME_HLL = 1, USCHEME_FORCE = 2, USCHEME_KP07 = 3 };
 
-// Schemes that take the round-weighted split.  Measured at 4096^2 against equal
-// segments: HLL 5 % and the unsplit KP07 1 % faster, LxF even, FORCE 3 % slower.
+// Schemes that take the round-weighted split with one column per lane.  Measured
+// at 4096^2 against equal segments: HLL 5 % and the unsplit KP07 1 % faster, LxF
+// even, FORCE 3 % slower.  With two columns per lane all take it where it fits
+// (adjacent strips per workgroup: 98 us at 4096^2 against 114 for equal segments
+// along a strip); elsewhere the equal segments of a workgroup are banded likewise
+// (2800^2: 50 -> 45 us).
 inline bool unsplit_round_ok(int scheme) { return scheme == USCHEME_HLL || scheme == USCHEME_KP07; }
+
+// Columns per lane of a launch.  Two (8-byte accesses, 124-column strips) for the
+// one-ghost-cell schemes, which are bound by memory: what a wave's row access
+// covers decides how near they come to a copy of their bytes (79 us at 4096^2).
+// Step of three simulators in turn at 4096^2: LxF 123 -> 98 us, FORCE 123 -> 98, HLL
+// 111 -> 98; 2800^2 59 -> 45, 2048^2 27.5 -> 24.  One where that leaves less than
+// a wave of `min_seg` rows per SIMD (1000^2: 7.7 us with one column, 11.3 with
+// two), for HLL in exact arithmetic (bound by VALU issue, 145 and 149 us), and for
+// fields that are not 8-byte aligned.
+inline int unsplit_cols(const UnsplitArgs& a, int scheme, bool exact, bool aligned8, int cu_count, int min_seg = 24) {
+    if (scheme == USCHEME_KP07 || !aligned8 || (exact && scheme == USCHEME_HLL)) return 1;
+    const long long strips = (a.nx + u_strip_cols<1, 2>()) / u_strip_cols<1, 2>();
+    const int seg = a.seg_rows > 0 ? a.seg_rows : min_seg;
+    return strips * ((a.ny + seg - 1) / seg) >= 4LL * cu_count ? 2 : 1;
+}
+
+template <class S, class M>
+void launch_unsplit_scheme(const UnsplitArgs& a, int grid, hipStream_t stream) {
+    const dim3 block(kLanes * a.waves_per_block);
+    if constexpr (S::GC == 1) {
+        if (a.cols == 2) {
+            hipLaunchKernelGGL((unsplit_kernel<S, M, 2>), dim3(grid), block, 0, stream, a);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((unsplit_kernel<S, M, 1>), dim3(grid), block, 0, stream, a);
+}
 
 template <class M>
 hipError_t launch_unsplit(int scheme, const UnsplitArgs& a, int grid, hipStream_t stream) {
-    const dim3 block(kLanes * a.waves_per_block);
     switch (scheme) {
         case USCHEME_LXF:
-            hipLaunchKernelGGL((unsplit_kernel<SweLxF<M>, M>), dim3(grid), block, 0, stream, a);
+            launch_unsplit_scheme<SweLxF<M>, M>(a, grid, stream);
             break;
         case USCHEME_HLL:
-            hipLaunchKernelGGL((unsplit_kernel<SweHLL1<M>, M>), dim3(grid), block, 0, stream, a);
+            launch_unsplit_scheme<SweHLL1<M>, M>(a, grid, stream);
             break;
         case USCHEME_FORCE:
-            hipLaunchKernelGGL((unsplit_kernel<SweFORCE<M>, M>), dim3(grid), block, 0, stream, a);
+            launch_unsplit_scheme<SweFORCE<M>, M>(a, grid, stream);
             break;
         case USCHEME_KP07:
-            hipLaunchKernelGGL((unsplit_kernel<SweKP07U<M>, M>), dim3(grid), block, 0, stream, a);
+            launch_unsplit_scheme<SweKP07U<M>, M>(a, grid, stream);
             break;
         default:
             return hipErrorInvalidValue;

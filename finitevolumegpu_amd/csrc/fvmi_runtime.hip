@@ -335,7 +335,13 @@ int run_unsplit(int scheme, UnsplitArgs& a, int gc, const fvmi_launch_t* launch,
         a.lw_kx = a.dt / (2.0f * a.dx);
         a.lw_ky = a.dt / (2.0f * a.dy);
     }
-    const int grid = plan_unsplit(a, gc, current_cu_count(), unsplit_round_ok(scheme));
+    bool aligned8 = true;
+    for (int k = 0; k < 3; ++k)
+        if (((uintptr_t)a.in[k] | (uintptr_t)a.out[k] | (unsigned)a.in_pitch[k] | (unsigned)a.out_pitch[k]) & 7)
+            aligned8 = false;
+    const int cus = current_cu_count();
+    a.cols = unsplit_cols(a, scheme, math == FVMI_MATH_EXACT, aligned8, cus);
+    const int grid = plan_unsplit(a, gc, cus, a.cols == 2 || unsplit_round_ok(scheme));
     hipError_t e = (math == FVMI_MATH_EXACT) ? launch_unsplit_exact(scheme, a, grid, (hipStream_t)stream)
                                              : launch_unsplit_fast(scheme, a, grid, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "unsplit launch");
@@ -355,6 +361,27 @@ UnsplitArgs first_order_args(int nx, int ny, float dx, float dy, float dt, float
     a.cfl = cfl;
     a.cfl_slot = cfl_slot;
     return a;
+}
+
+// The arguments of a launch that reads buffer `from` of a step and writes the other.
+SubstepArgs step_args(const fvmi_step_t* p, int nvars, int from, int step) {
+    SubstepArgs a{};
+    a.nx = p->nx, a.ny = p->ny, a.dx = p->dx, a.dy = p->dy, a.dt = p->dt;
+    a.g = p->g, a.theta = p->theta, a.gamma = p->gamma;
+    a.step = step, a.bc = p->boundary_conditions;
+    for (int k = 0; k < nvars; ++k) {
+        a.in[k] = p->state[from][k], a.in_pitch[k] = p->pitch[from][k];
+        a.out[k] = p->state[1 - from][k], a.out_pitch[k] = p->pitch[1 - from][k];
+    }
+    a.cfl = p->cfl;
+    return a;
+}
+
+// Plans a launch of a whole step; returns its grid.
+int plan_step(SubstepArgs& a, int cfl_slot, int cu_count) {
+    a.cfl_slot = cfl_slot;
+    a.strip_cols = strip_cols<1, kStepHalo>();
+    return plan_substep(a, cu_count, true, 4, kStepMinSeg);
 }
 
 }  // namespace
@@ -655,31 +682,6 @@ int fvmi_euler_kp07_dimsplit_substep(int nx, int ny, float dx, float dy, float d
     return run_substep(SCHEME_EULER, a, 4, launch, stream);
 }
 
-namespace {
-
-// The arguments of a launch that reads buffer `from` of a step and writes the other.
-SubstepArgs step_args(const fvmi_step_t* p, int nvars, int from, int step) {
-    SubstepArgs a{};
-    a.nx = p->nx, a.ny = p->ny, a.dx = p->dx, a.dy = p->dy, a.dt = p->dt;
-    a.g = p->g, a.theta = p->theta, a.gamma = p->gamma;
-    a.step = step, a.bc = p->boundary_conditions;
-    for (int k = 0; k < nvars; ++k) {
-        a.in[k] = p->state[from][k], a.in_pitch[k] = p->pitch[from][k];
-        a.out[k] = p->state[1 - from][k], a.out_pitch[k] = p->pitch[1 - from][k];
-    }
-    a.cfl = p->cfl;
-    return a;
-}
-
-// Plans a launch of a whole step; returns its grid.
-int plan_step(SubstepArgs& a, int cfl_slot) {
-    a.cfl_slot = cfl_slot;
-    a.strip_cols = strip_cols<1, kStepHalo>();
-    return plan_substep(a, current_cu_count(), true, 4, kStepMinSeg);
-}
-
-}  // namespace
-
 int fvmi_dimsplit_step(const fvmi_step_t* p, const fvmi_launch_t* launch, int* state_out, int* cfl_slot_out,
                        void* stream) {
     if (!p || !state_out || !cfl_slot_out) return fail(FVMI_ERR_INVALID, "NULL argument");
@@ -698,7 +700,7 @@ int fvmi_dimsplit_step(const fvmi_step_t* p, const fvmi_launch_t* launch, int* s
         *cfl_slot_out = 1;
         return FVMI_OK;
     }
-    const int grid = plan_step(a, p->cfl_slot);
+    const int grid = plan_step(a, p->cfl_slot, current_cu_count());
     hipError_t e = launch_step_fast(p->scheme, a, grid, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "step launch");
     *state_out = 1;
@@ -728,7 +730,7 @@ int fvmi_swe_kp07_rk2_step(const fvmi_step_t* p, const fvmi_launch_t* launch, in
         *cfl_slot_out = 1 - p->cfl_slot;
         return FVMI_OK;
     }
-    const int grid = plan_step(a, p->cfl_slot);
+    const int grid = plan_step(a, p->cfl_slot, current_cu_count());
     hipError_t e = launch_rk2_step(a, grid, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "step launch");
     *state_out = 1;
@@ -798,13 +800,16 @@ int fvmi_ensemble_prepare(fvmi_instance_t* table, int n, void* stream) {
 
 int fvmi_substep_plan(int scheme, int nx, int ny, int x0, int y0, int x1, int y1, const fvmi_launch_t* launch,
                       int cu_count, int* segs, int max_waves, int* n_waves) {
-    if (scheme < SCHEME_KP07 || scheme > SCHEME_EULER + 4) return fail(FVMI_ERR_INVALID, "unknown scheme %d", scheme);
+    const bool two_columns = scheme >= 12 && scheme <= 14, whole_step = scheme == 16;
+    if (two_columns) scheme -= 8;
+    if (!whole_step && (scheme < SCHEME_KP07 || scheme > SCHEME_EULER + 4))
+        return fail(FVMI_ERR_INVALID, "unknown scheme %d", scheme);
     if (nx < 2 || ny < 2 || cu_count < 1 || !n_waves || max_waves < 0 || (max_waves > 0 && !segs))
         return fail(FVMI_ERR_INVALID, "bad plan arguments");
-    if (scheme > SCHEME_EULER) {
-        // LxF, HLL, FORCE (one ghost cell) and the unsplit KP07 (two): the whole domain
-        if (x0 != 0 || y0 != 0 || (x1 != 0 && x1 != nx) || (y1 != 0 && y1 != ny))
-            return fail(FVMI_ERR_INVALID, "the unsplit schemes update the whole domain");
+    if (scheme > SCHEME_EULER && (x0 != 0 || y0 != 0 || (x1 != 0 && x1 != nx) || (y1 != 0 && y1 != ny)))
+        return fail(FVMI_ERR_INVALID, "the unsplit schemes and whole steps update the whole domain");
+    if (scheme > SCHEME_EULER && !whole_step) {
+        // LxF, HLL, FORCE (one ghost cell) and the unsplit KP07 (two)
         UnsplitArgs u{};
         u.nx = nx, u.ny = ny;
         SubstepArgs shape{};
@@ -813,8 +818,9 @@ int fvmi_substep_plan(int scheme, int nx, int ny, int x0, int y0, int x1, int y1
         u.seg_rows = shape.seg_rows;
         u.waves_per_block = shape.waves_per_block;
         u.xcd_remap = shape.xcd_remap;
+        u.cols = two_columns ? 2 : 1;
         const int grid = plan_unsplit(u, scheme == SCHEME_EULER + 4 ? 2 : 1, cu_count,
-                                      unsplit_round_ok(scheme - (SCHEME_EULER + 1)));
+                                      two_columns || unsplit_round_ok(scheme - (SCHEME_EULER + 1)));
         const long long total = (long long)grid * u.waves_per_block;
         if (total > (1LL << 30)) return fail(FVMI_ERR_INVALID, "plan too large");
         *n_waves = (int)total;
@@ -837,8 +843,9 @@ int fvmi_substep_plan(int scheme, int nx, int ny, int x0, int y0, int x1, int y1
         return fail(FVMI_ERR_INVALID, "sub-area outside the domain");
     int math = 0;
     if (int rc = fill_launch(launch, a, &math)) return rc;
-    a.strip_cols = scheme_strip_cols(scheme, math);
-    const int grid = plan_substep(a, cu_count, scheme != SCHEME_WAF);
+    a.strip_cols = whole_step ? strip_cols<1, kStepHalo>() : scheme_strip_cols(scheme, math);
+    const int grid =
+        whole_step ? plan_step(a, 0, cu_count) : plan_substep(a, cu_count, scheme != SCHEME_WAF);
     const long long total = (long long)grid * a.waves_per_block;
     if (total > (1LL << 30)) return fail(FVMI_ERR_INVALID, "plan too large");
     *n_waves = (int)total;

@@ -319,9 +319,12 @@ int fvmi_ensemble_substep(int scheme, fvmi_instance_t* table, const int* segs, c
  * points and of the unsplit ones, computed on the host with no device call:
  * the planner's choice for scheme (3 Euler in fast arithmetic: strips of 124
  * columns; 0 KP07_dimsplit, 1 HLL2, 2 WAF and 3 Euler in exact arithmetic: 60;
- * 4, 5, 6 LxF, HLL, FORCE: 62; 7 the unsplit KP07: 60), sub-area [x0,x1)x[y0,y1) of an nx x ny domain (x1 = y1 = 0: the
- * whole domain, the only one the unsplit schemes take), the launch shape and
- * a device of `cu_count` CUs.  For every wave of the grid, 3 ints in `segs`
+ * 4, 5, 6 LxF, HLL, FORCE with one column per lane: 62; 12, 13, 14 the same
+ * with two: 124, the first strip's first column being the ghost column beside
+ * the domain; 7 one stage of the unsplit KP07: 60; 16 a whole step in one
+ * launch: 56), sub-area [x0,x1)x[y0,y1) of an nx x ny domain (x1 = y1 = 0: the
+ * whole domain, the only one the unsplit schemes and whole steps take), the
+ * launch shape and a device of `cu_count` CUs.  For every wave of the grid, 3 ints in `segs`
  * (capacity `max_waves` waves): strip, first row and row count relative to
  * the sub-area, or (-1, 0, 0) for a wave with nothing to do; *n_waves receives
  * the grid's wave count.  No counterpart in the reference (its tile grid is

@@ -177,3 +177,27 @@ def test_mpi_step_equals_exchange_between_substeps(ctx, math):
         assert all(np.array_equal(x, y) for x, y in zip(*padded))
     assert sims[0].computeDt() == sims[1].computeDt()
     assert sims[0].profiling_data_mpi["n_time_steps"] == sims[1].profiling_data_mpi["n_time_steps"]
+
+
+@pytest.mark.parametrize("scheme", ["LxF", "HLL", "FORCE"])
+@pytest.mark.parametrize("bc", sorted(BOUNDARIES) + ["one-sided"])
+def test_first_order_with_two_columns_per_lane(ctx, scheme, bc):
+    """One-row segments make enough waves for two columns per lane, 64-row
+    segments leave one: the same fields, at the edges of 124-column strips."""
+    import importlib
+    from finitevolumegpu_amd.Simulator import BoundaryCondition
+    cls = getattr(importlib.import_module("finitevolumegpu_amd." + scheme), scheme)
+    code = O.pack_bc(P, R, R, P) if bc == "one-sided" else BOUNDARIES[bc]
+    edges = BoundaryCondition(BoundaryCondition.getTypes(code))
+    ny = 1100
+    for nx in (2, 61, 122, 123, 124, 125, 247, 248):
+        print("case two columns", scheme, bc, nx, flush=True)
+        fields = state("kp07_dimsplit", nx, ny, seed=nx)
+        sims = [cls(ctx, *fields, nx, ny, 1.0, 1.0, 9.81, boundary_conditions=edges, tile_rows=rows)
+                for rows in (1, 64)]
+        dt = np.float32(0.5 * sims[0].computeDt())
+        for _ in range(2):
+            for sim in sims:
+                sim.step(dt)
+        assert all(np.array_equal(x, y) for x, y in zip(*[s.download() for s in sims])), nx
+        assert sims[0].computeDt() == sims[1].computeDt()

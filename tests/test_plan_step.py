@@ -1,0 +1,70 @@
+"""Launch plans of a whole step (strips of 56 columns) and of the first-order
+schemes with two columns per lane (strips of 124, the first one starting at the
+ghost column beside the domain), on the host through fvmi_substep_plan: the
+segments cover every row of every strip once, at the edges of strips and row
+groups and on several CU counts."""
+
+import ctypes
+
+import numpy as np
+import pytest
+
+from finitevolumegpu_amd import _lib
+
+STEP, LXF2, HLL2, FORCE2 = 16, 12, 13, 14
+
+
+def plan(scheme, nx, ny, tile_rows=0, waves_per_block=4, xcd_remap=True, cu_count=256, sub=(0, 0, 0, 0)):
+    lib = _lib.lib()
+    launch = _lib.LaunchConfig(tile_rows, waves_per_block, _lib.FVMI_MATH_FAST, 1 if xcd_remap else 2)
+    n = ctypes.c_int()
+    rc = lib.fvmi_substep_plan(scheme, nx, ny, *sub, ctypes.byref(launch), cu_count, None, 0, ctypes.byref(n))
+    if n.value <= 0:
+        return rc
+    segs = np.zeros((n.value, 3), dtype=np.int32)
+    rc = lib.fvmi_substep_plan(scheme, nx, ny, *sub, ctypes.byref(launch), cu_count,
+                               segs.ctypes.data_as(ctypes.POINTER(ctypes.c_int)), n.value, ctypes.byref(n))
+    assert rc == 0, lib.fvmi_last_error().decode()
+    return segs
+
+
+@pytest.mark.parametrize("scheme", [STEP, LXF2, HLL2, FORCE2])
+@pytest.mark.parametrize("nx,ny,tile_rows,waves,remap,cus", [
+    (8, 8, 0, 4, True, 256), (55, 9, 0, 4, True, 256), (56, 40, 0, 4, True, 256), (57, 41, 0, 4, True, 256),
+    (123, 300, 0, 4, True, 256), (124, 300, 0, 4, True, 256), (125, 1100, 1, 4, True, 256),
+    (128, 128, 0, 4, True, 256), (2047, 2047, 0, 4, True, 256), (4096, 4096, 0, 4, True, 256),
+    (4096, 4096, 70, 3, False, 256), (6000, 777, 0, 2, True, 256), (3000, 2500, 0, 4, True, 80),
+])
+def test_segments_cover_the_domain_once(scheme, nx, ny, tile_rows, waves, remap, cus):
+    width, strip = (nx, 56) if scheme == STEP else (nx + 1, 124)
+    strips = -(-width // strip)
+    cover = np.zeros((strips, ny), dtype=np.int32)
+    for s, r, c in plan(scheme, nx, ny, tile_rows, waves, remap, cus):
+        if s < 0:
+            assert r == 0 and c == 0
+            continue
+        assert 0 <= s < strips and c >= 1 and 0 <= r and r + c <= ny
+        cover[s, r:r + c] += 1
+    assert (cover == 1).all()
+
+
+def test_second_segment_of_a_whole_step_starts_past_the_mirrored_rows():
+    """A segment's march mirrors ghost rows 0 and 1 from rows 2 and 3 of the
+    first segment only: every other segment starts at row 2 or later."""
+    for nx, ny in ((8, 8), (64, 64), (300, 100), (2047, 2047), (4096, 4096)):
+        rows = plan(STEP, nx, ny)
+        starts = rows[rows[:, 0] >= 0, 1]
+        assert not ((starts > 0) & (starts < 2)).any()
+
+
+def test_wide_strips_of_a_workgroup_are_adjacent():
+    segs = plan(LXF2, 3000, 3000)
+    for b in range(0, len(segs), 4):
+        live = segs[b:b + 4][segs[b:b + 4, 0] >= 0]
+        if len(live) > 1:
+            assert (live[:, 1:] == live[0, 1:]).all() and (np.diff(live[:, 0]) == 1).all()
+
+
+@pytest.mark.parametrize("scheme", [STEP, LXF2])
+def test_sub_areas_are_rejected(scheme):
+    assert plan(scheme, 64, 64, sub=(1, 0, 64, 64)) < 0
