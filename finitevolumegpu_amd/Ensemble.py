@@ -8,9 +8,12 @@ a device table (``fvmi_instance_t``) and advances all instances together:
 
 * one work list of wavefront segments covers every active instance, balanced
   so that small and large grids share the device;
-* a full step is four launches (prepare, substep 0, substep 1, advance), and
-  ``steps_per_graph`` steps are captured once in a hipGraph and replayed; the
-  substep kernels read the work list and its length on the device, so the
+* a full step is the two substeps and one launch that advances every instance
+  and prepares its next step; in fast arithmetic (KP07_dimsplit, HLL2, Euler) the
+  substeps are one launch too, if every instance allows it (``steppable``), and an
+  instance's state is then in buffer ``cur`` of its two;
+* ``steps_per_graph`` steps are captured once in a hipGraph and replayed; the
+  kernels read the work list and its length on the device, so the
   graph survives instances joining and leaving (it is captured again only when
   the list outgrows its buffer);
 * instance fields live in a ``DeviceArena`` (large device allocations carved
@@ -42,6 +45,19 @@ def strip_cols(scheme, math):
     fv_substep.h): 124 where it marches two columns per lane
     (EE2D_KP07_dimsplit in fast arithmetic), else 60."""
     return 124 if (scheme == "ee2d_kp07_dimsplit" and math == "fast") else 60
+
+
+# strips of the launch that takes a whole step (fv_step.h)
+STEP_STRIP_COLS = 56
+
+
+def steppable(nx, ny, bc):
+    """Whether an instance's whole step can be one launch: step_grid_fits of
+    fv_launch.h (no Dirichlet edge, periodic edges in opposite pairs)."""
+    T = BoundaryCondition.Type
+    west, east, south, north = (bc >> shift & 0xF for shift in (0, 8, 16, 24))
+    return (nx >= 8 and ny >= 8 and T.Dirichlet not in (west, east, south, north)
+            and (west == T.Periodic) == (east == T.Periodic) and (south == T.Periodic) == (north == T.Periodic))
 
 
 def _bc_code(bc):
@@ -263,6 +279,9 @@ class Ensemble:
         self.graph = None
         self.captures = 0
         self.planned_active = None
+        # whole steps in one launch; decided with each plan (_choose_steps)
+        self.whole_steps = False
+        self.table_fresh = True  # the host copy holds the device's times, steps and buffers
         self._sync()
 
     # ------------------------------------------------------------------
@@ -314,6 +333,7 @@ class Ensemble:
         I.t = 0.0
         I.t_end = float(spec["t_end"])
         I.nt = 0
+        I.cur = 0
         I.active = 1
         if spec.get("dt") is not None:
             I.fixed_dt = 1
@@ -332,6 +352,12 @@ class Ensemble:
         _lib.call("fvmi_memcpy_async", ctypes.addressof(self.host_table), self.table,
                   ctypes.sizeof(self.host_table), _lib.MEMCPY_DTOH, self.stream.handle)
         self._sync()
+        self.table_fresh = True
+
+    def _state(self, i, k):
+        """Address of variable k of instance i's current state (fresh table)."""
+        I = self.host_table[i]
+        return I.field[I.cur & 1][k]
 
     def _running(self):
         """Live slots whose instance is still active and short of t_end (host copy)."""
@@ -345,8 +371,33 @@ class Ensemble:
         """Rows of strips of the instances in ``mask`` (sum over them)."""
         nx = self.tab["nx"][mask].astype(np.int64)
         ny = self.tab["ny"][mask].astype(np.int64)
-        w = strip_cols(self.scheme, self.math)
+        w = self._strip_cols()
         return int(((nx + w - 1) // w * ny).sum())
+
+    def _strip_cols(self):
+        return STEP_STRIP_COLS if self.whole_steps else strip_cols(self.scheme, self.math)
+
+    def _choose_steps(self):
+        """Whole steps in one launch if the scheme has them and every live
+        instance allows them.  Substeps leave the state in buffer 0, so going
+        back to them puts every instance's current buffer first."""
+        whole = (self.math == "fast" and self.scheme != "waf" and not 0 < (self.seg_rows or 0) < 4
+                 and self.min_seg_rows >= 4
+                 and all(steppable(int(self.tab["nx"][i]), int(self.tab["ny"][i]), int(self.tab["bc"][i]))
+                         for i in np.flatnonzero(self.live)))
+        if whole == self.whole_steps:
+            return
+        if not whole:
+            self._download_table()
+            turned = np.flatnonzero(self.live & ((self.tab["cur"] & 1) != 0))
+            for i in turned:
+                self.tab["field"][i] = self.tab["field"][i][::-1].copy()
+                self.tab["cur"][i] = 0
+            _lib.call("fvmi_memcpy_async", self.table, ctypes.addressof(self.host_table),
+                      ctypes.sizeof(self.host_table), _lib.MEMCPY_HTOD, self.stream.handle)
+            self._sync()
+        self.whole_steps = whole
+        self._drop_graph()
 
     # ------------------------------------------------------------------
     # slots
@@ -400,6 +451,7 @@ class Ensemble:
         length are written to the device on the ensemble's stream; the graph
         is captured again only if the list outgrows its buffer."""
         active = np.asarray(active, dtype=bool) & self.live
+        self._choose_steps()
         total = self._strip_rows(active)
         if self.seg_rows:
             seg = int(self.seg_rows)
@@ -407,7 +459,7 @@ class Ensemble:
             slots = self.context.cu_count * 4 * self.waves_per_simd
             seg = max(self.min_seg_rows, -(-total // max(1, slots)))
         arr = plan_segments(np.flatnonzero(active), self.tab["nx"][active], self.tab["ny"][active], seg,
-                            strip_cols(self.scheme, self.math))
+                            self._strip_cols())
         need = len(arr)
         self._sync()  # the pinned staging buffer may still feed the previous upload
         if self.segs_dev is None or need > self.segs_cap:
@@ -443,12 +495,18 @@ class Ensemble:
 
     def _enqueue_steps(self, k):
         waves = self._waves()
-        for _ in range(k):
-            _lib.call("fvmi_ensemble_prepare", self.table, self.n, self.stream.handle)
-            for step in (0, 1):
-                _lib.call("fvmi_ensemble_substep", self.scheme_id, self.table, self.segs_dev, self.nsegs_dev, waves,
-                          step, self.launch, self.stream.handle)
-            _lib.call("fvmi_ensemble_advance", self.table, self.n, self.stream.handle)
+        whole = self.whole_steps
+        _lib.call("fvmi_ensemble_prepare", self.table, self.n, self.stream.handle)
+        for j in range(k):
+            if whole:
+                _lib.call("fvmi_ensemble_step", self.scheme_id, self.table, self.segs_dev, self.nsegs_dev, waves,
+                          self.launch, self.stream.handle)
+            else:
+                for step in (0, 1):
+                    _lib.call("fvmi_ensemble_substep", self.scheme_id, self.table, self.segs_dev, self.nsegs_dev,
+                              waves, step, self.launch, self.stream.handle)
+            # advance, and prepare the next step of the block
+            _lib.call("fvmi_ensemble_tick", self.table, self.n, int(whole), int(j + 1 < k), self.stream.handle)
 
     def _capture(self):
         _lib.call("fvmi_stream_begin_capture", self.stream.handle)
@@ -482,6 +540,7 @@ class Ensemble:
             self.plan(self._running())
         if self.num_segs == 0:
             return self.count_active() if wait else None
+        self.table_fresh = False
         if self.use_graph:
             if self.graph is None:
                 self._capture()
@@ -511,14 +570,20 @@ class Ensemble:
         self._download_table()
         return self.host_table[i].t, self.host_table[i].nt
 
+    def _refresh_buffers(self):
+        """Makes the host copy's ``cur`` the device's (substeps never change it)."""
+        if self.whole_steps and not self.table_fresh:
+            self._download_table()
+
     def download(self, i):
         """Interior of every field of instance i (float32 (ny, nx) arrays)."""
+        self._refresh_buffers()
         I = self.host_table[i]
         nx, ny, pitch = int(I.nx), int(I.ny), int(I.pitch)
         out = []
         for k in range(self.nvars):
             a = np.empty((ny, nx), dtype=np.float32)
-            _lib.call("fvmi_memcpy2d_async", a.ctypes.data, nx * 4, I.field[0][k] + 2 * pitch + 8, pitch, nx * 4, ny,
+            _lib.call("fvmi_memcpy2d_async", a.ctypes.data, nx * 4, self._state(i, k) + 2 * pitch + 8, pitch, nx * 4, ny,
                       _lib.MEMCPY_DTOH, self.stream.handle)
             out.append(a)
         self._sync()
@@ -539,13 +604,14 @@ class Ensemble:
             self.stats_dev = ctypes.c_void_p()
             _lib.call("fvmi_malloc", ctypes.byref(self.stats_dev), need)
             self.stats_cap = need
+        self._refresh_buffers()
         base = self.stats_dev.value
         _lib.call("fvmi_fill_f32", base, need, need // 4, 1, 0.0, self.stream.handle)
         for j, i in enumerate(slots):
             I = self.host_table[i]
             for k in range(self.nvars):
                 out = base + 16 * (j * self.nvars + k)
-                _lib.call("fvmi_field_stats", int(I.nx), int(I.ny), 2, 2, I.field[0][k], int(I.pitch), out, out + 8,
+                _lib.call("fvmi_field_stats", int(I.nx), int(I.ny), 2, 2, self._state(i, k), int(I.pitch), out, out + 8,
                           self.stream.handle)
         host = np.zeros(need // 8, dtype=np.float64)
         _lib.call("fvmi_memcpy_async", host.ctypes.data, base, need, _lib.MEMCPY_DTOH, self.stream.handle)

@@ -57,7 +57,7 @@ class Instance(ctypes.Structure):
                 ("dx", c_float), ("dy", c_float), ("g", c_float), ("theta", c_float),
                 ("gamma", c_float), ("sqrt_g", c_float), ("inv_g", c_float), ("inv_dx", c_float),
                 ("inv_dy", c_float), ("cfl", c_float * 2), ("dt_step", c_float),
-                ("nt", c_int), ("active", c_int), ("fixed_dt", c_int),
+                ("nt", c_int), ("active", c_int), ("fixed_dt", c_int), ("cur", c_int),
                 ("t", ctypes.c_double), ("t_end", ctypes.c_double), ("dt", ctypes.c_double),
                 ("cfl_scale", ctypes.c_double)]
 
@@ -145,6 +145,8 @@ SIGNATURES = {
     "fvmi_ensemble_prepare": (c_int, [c_void_p, c_int, c_void_p]),
     "fvmi_ensemble_substep": (c_int, [c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, P(LaunchConfig), c_void_p]),
     "fvmi_ensemble_advance": (c_int, [c_void_p, c_int, c_void_p]),
+    "fvmi_ensemble_tick": (c_int, [c_void_p, c_int, c_int, c_int, c_void_p]),
+    "fvmi_ensemble_step": (c_int, [c_int, c_void_p, c_void_p, c_void_p, c_int, P(LaunchConfig), c_void_p]),
     "fvmi_ensemble_count_active": (c_int, [c_void_p, c_int, c_void_p, c_void_p]),
     "fvmi_stream_begin_capture": (c_int, [c_void_p]),
     "fvmi_stream_end_capture": (c_int, [c_void_p, P(c_void_p)]),

@@ -21,6 +21,10 @@ hipError_t launch_step_fast(int scheme, const SubstepArgs& a, int grid, hipStrea
     if (scheme == SCHEME_EULER) return launch_step_scheme<StepEuler, MathFast>(a, grid, stream);
     return launch_step_fast_ilp(scheme, a, grid, stream);
 }
+hipError_t launch_ensemble_step_fast(int scheme, const EnsembleArgs& e, int grid, hipStream_t stream) {
+    if (scheme == SCHEME_EULER) return launch_ensemble_step_scheme<StepEuler, MathFast>(e, grid, stream);
+    return launch_ensemble_step_fast_ilp(scheme, e, grid, stream);
+}
 hipError_t launch_ensemble_fast(int scheme, const EnsembleArgs& e, int grid, hipStream_t stream) {
     switch (scheme) {
         case SCHEME_KP07:

@@ -30,6 +30,16 @@ hipError_t launch_step_fast_ilp(int scheme, const SubstepArgs& a, int grid, hipS
             return hipErrorInvalidValue;
     }
 }
+hipError_t launch_ensemble_step_fast_ilp(int scheme, const EnsembleArgs& e, int grid, hipStream_t stream) {
+    switch (scheme) {
+        case SCHEME_KP07:
+            return launch_ensemble_step_scheme<StepKP07, MathFast>(e, grid, stream);
+        case SCHEME_HLL2:
+            return launch_ensemble_step_scheme<StepHLL2, MathFast>(e, grid, stream);
+        default:
+            return hipErrorInvalidValue;
+    }
+}
 hipError_t launch_ensemble_fast_ilp(int scheme, const EnsembleArgs& e, int grid, hipStream_t stream) {
     switch (scheme) {
         case SCHEME_KP07:

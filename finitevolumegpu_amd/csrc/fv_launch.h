@@ -138,7 +138,13 @@ hipError_t launch_step_scheme(const SubstepArgs& a, int grid, hipStream_t stream
 
 template <class S, class M>
 hipError_t launch_ensemble_scheme(const EnsembleArgs& e, int grid, hipStream_t stream) {
-    hipLaunchKernelGGL((ensemble_substep_kernel<S, M>), dim3(grid), dim3(kLanes * e.waves_per_block), 0, stream, e);
+    hipLaunchKernelGGL((ensemble_kernel<S, M, false>), dim3(grid), dim3(kLanes * e.waves_per_block), 0, stream, e);
+    return hipGetLastError();
+}
+
+template <class S, class M>
+hipError_t launch_ensemble_step_scheme(const EnsembleArgs& e, int grid, hipStream_t stream) {
+    hipLaunchKernelGGL((ensemble_kernel<S, M, true>), dim3(grid), dim3(kLanes * e.waves_per_block), 0, stream, e);
     return hipGetLastError();
 }
 
@@ -147,16 +153,16 @@ hipError_t launch_ensemble_substep(int scheme, EnsembleArgs e, int grid, hipStre
     const dim3 block(kLanes * e.waves_per_block);
     switch (scheme) {
         case SCHEME_KP07:
-            hipLaunchKernelGGL((ensemble_substep_kernel<SweKP07<M>, M>), dim3(grid), block, 0, stream, e);
+            hipLaunchKernelGGL((ensemble_kernel<SweKP07<M>, M, false>), dim3(grid), block, 0, stream, e);
             break;
         case SCHEME_HLL2:
-            hipLaunchKernelGGL((ensemble_substep_kernel<SweHLL2<M>, M>), dim3(grid), block, 0, stream, e);
+            hipLaunchKernelGGL((ensemble_kernel<SweHLL2<M>, M, false>), dim3(grid), block, 0, stream, e);
             break;
         case SCHEME_WAF:
-            hipLaunchKernelGGL((ensemble_substep_kernel<SweWAF<M>, M>), dim3(grid), block, 0, stream, e);
+            hipLaunchKernelGGL((ensemble_kernel<SweWAF<M>, M, false>), dim3(grid), block, 0, stream, e);
             break;
         case SCHEME_EULER:
-            hipLaunchKernelGGL((ensemble_substep_kernel<EulerKP07<M>, M>), dim3(grid), block, 0, stream, e);
+            hipLaunchKernelGGL((ensemble_kernel<EulerKP07<M>, M, false>), dim3(grid), block, 0, stream, e);
             break;
         default:
             return hipErrorInvalidValue;
@@ -173,6 +179,8 @@ hipError_t launch_substep_fast(int scheme, const SubstepArgs& a, int grid, hipSt
 // (fv_kernels_fast_ilp.hip, built with the ILP-maximising scheduler)
 hipError_t launch_step_fast(int scheme, const SubstepArgs& a, int grid, hipStream_t stream);
 hipError_t launch_step_fast_ilp(int scheme, const SubstepArgs& a, int grid, hipStream_t stream);
+hipError_t launch_ensemble_step_fast(int scheme, const EnsembleArgs& e, int grid, hipStream_t stream);
+hipError_t launch_ensemble_step_fast_ilp(int scheme, const EnsembleArgs& e, int grid, hipStream_t stream);
 hipError_t launch_rk2_step(const SubstepArgs& a, int grid, hipStream_t stream);  // fast arithmetic
 hipError_t launch_substep_fast_ilp(int scheme, const SubstepArgs& a, int grid, hipStream_t stream);
 hipError_t launch_ensemble_fast_ilp(int scheme, const EnsembleArgs& e, int grid, hipStream_t stream);

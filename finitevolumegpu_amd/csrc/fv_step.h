@@ -349,6 +349,14 @@ __device__ __forceinline__ float march_step_paired(const SubstepArgs& a, const S
     return acc;
 }
 
+// The march of one segment; returns the CFL accumulator.
+template <class S, class M>
+__device__ __forceinline__ float march_step(const SubstepArgs& a, const Strip<1>& st, int row_in, int count) {
+    StepEdge e;
+    setup_edge(a, st, row_in, count, e);
+    return needs_edge(e) || count < 2 ? march_step_edge<S, M>(a, st, e) : march_step_paired<S, M>(a, st);
+}
+
 // Four waves fit on a SIMD (109 VGPRs for KP07_dimsplit, 120 for HLL2, 128 for
 // Euler, no scratch).  Measured per 4096^2 step with two columns per lane
 // (fewer halo lanes, 168 VGPRs with spills or 247): KP07_dimsplit 327 and 248
@@ -365,10 +373,7 @@ __global__ void __launch_bounds__(256, 4) step_kernel(SubstepArgs a) {
     count = __builtin_amdgcn_readfirstlane(count);
     Strip<1> st;
     setup_strip<S, M, kStepHalo>(a, st, lane, strip_x, row_in, count);
-    StepEdge e;
-    setup_edge(a, st, row_in, count, e);
-    const float acc =
-        needs_edge(e) || count < 2 ? march_step_edge<S, M>(a, st, e) : march_step_paired<S, M>(a, st);
+    const float acc = march_step<S, M>(a, st, row_in, count);
     if (a.cfl != nullptr) {
         float dt_min = acc;
         if constexpr (!M::exact) dt_min = (acc > 0.0f) ? fast::rcp(acc) : __builtin_inff();

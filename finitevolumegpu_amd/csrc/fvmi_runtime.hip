@@ -223,10 +223,7 @@ __global__ void halo_periodic_kernel(HaloArgs a) {
 }
 
 // Ensemble bookkeeping (one thread per instance); see fv_ensemble.h.
-__global__ void ensemble_prepare_kernel(fvmi_instance_t* table, int n) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    fvmi_instance_t& I = table[i];
+__device__ void instance_prepare(fvmi_instance_t& I) {
     if (!I.active) return;
     if (!(I.t < I.t_end)) {
         I.active = 0;
@@ -244,14 +241,24 @@ __global__ void ensemble_prepare_kernel(fvmi_instance_t* table, int n) {
     I.cfl[1] = __builtin_inff();
 }
 
-__global__ void ensemble_advance_kernel(fvmi_instance_t* table, int n) {
+// turn: the step left the state in the other buffer
+__device__ void instance_advance(fvmi_instance_t& I, int turn) {
+    if (!I.active) return;
+    I.t += (double)I.dt_step;
+    I.nt += 1;
+    if (turn) I.cur ^= 1;
+}
+
+__global__ void ensemble_prepare_kernel(fvmi_instance_t* table, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) instance_prepare(table[i]);
+}
+
+__global__ void ensemble_advance_kernel(fvmi_instance_t* table, int n, int turn, int prepare) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    fvmi_instance_t& I = table[i];
-    if (I.active) {
-        I.t += (double)I.dt_step;
-        I.nt += 1;
-    }
+    instance_advance(table[i], turn);
+    if (prepare) instance_prepare(table[i]);
 }
 
 __global__ void ensemble_count_kernel(const fvmi_instance_t* table, int n, int* out) {
@@ -361,6 +368,25 @@ UnsplitArgs first_order_args(int nx, int ny, float dx, float dy, float dt, float
     a.cfl = cfl;
     a.cfl_slot = cfl_slot;
     return a;
+}
+
+// Checks and launch shape of an ensemble launch.  The work list is sorted
+// longest first: dispatch order (block i on XCD i % 8) spreads it evenly over the
+// XCDs, whereas the contiguous remap of the single-grid kernel would give XCD 0
+// the longest segments and leave the last XCDs with the empty tail of the list.
+int fill_ensemble(int scheme, fvmi_instance_t* table, const int* segs, const int* num_segs_dev, int waves,
+                  const fvmi_launch_t* launch, EnsembleArgs& e, int& grid) {
+    if (!table || !segs || !num_segs_dev) return fail(FVMI_ERR_INVALID, "bad ensemble work list");
+    if (scheme < SCHEME_KP07 || scheme > SCHEME_EULER) return fail(FVMI_ERR_INVALID, "unknown scheme %d", scheme);
+    e.table = table;
+    e.segs = reinterpret_cast<const int4*>(segs);
+    e.num_segs = num_segs_dev;
+    e.waves_per_block = (launch && launch->waves_per_block > 0) ? launch->waves_per_block : 4;
+    if (e.waves_per_block > 4) return fail(FVMI_ERR_INVALID, "waves_per_block out of range [1, 4]");
+    if (waves <= 0) waves = current_cu_count() * 4 * 4;  // four waves per SIMD
+    e.num_blocks = (waves + e.waves_per_block - 1) / e.waves_per_block;
+    grid = e.num_blocks;
+    return FVMI_OK;
 }
 
 // The arguments of a launch that reads buffer `from` of a step and writes the other.
@@ -862,9 +888,14 @@ int fvmi_substep_plan(int scheme, int nx, int ny, int x0, int y0, int x1, int y1
 }
 
 int fvmi_ensemble_advance(fvmi_instance_t* table, int n, void* stream) {
+    return fvmi_ensemble_tick(table, n, 0, 0, stream);
+}
+
+int fvmi_ensemble_tick(fvmi_instance_t* table, int n, int turn, int prepare, void* stream) {
     if (!table || n < 0) return fail(FVMI_ERR_INVALID, "bad ensemble table");
     if (n == 0) return FVMI_OK;
-    hipLaunchKernelGGL(ensemble_advance_kernel, dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)stream, table, n);
+    hipLaunchKernelGGL(ensemble_advance_kernel, dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)stream, table, n,
+                       turn ? 1 : 0, prepare ? 1 : 0);
     FVMI_HIP(hipGetLastError());
     return FVMI_OK;
 }
@@ -878,29 +909,28 @@ int fvmi_ensemble_count_active(const fvmi_instance_t* table, int n, int* count_d
 
 int fvmi_ensemble_substep(int scheme, fvmi_instance_t* table, const int* segs, const int* num_segs_dev, int waves,
                           int step, const fvmi_launch_t* launch, void* stream) {
-    if (!table || !segs || !num_segs_dev) return fail(FVMI_ERR_INVALID, "bad ensemble work list");
-    if (scheme < SCHEME_KP07 || scheme > SCHEME_EULER) return fail(FVMI_ERR_INVALID, "unknown scheme %d", scheme);
-    if (step != 0 && step != 1) return fail(FVMI_ERR_INVALID, "step must be 0 or 1");
     EnsembleArgs e{};
-    e.table = table;
-    e.segs = reinterpret_cast<const int4*>(segs);
-    e.num_segs = num_segs_dev;
+    int grid = 0;
+    if (int rc = fill_ensemble(scheme, table, segs, num_segs_dev, waves, launch, e, grid)) return rc;
+    if (step != 0 && step != 1) return fail(FVMI_ERR_INVALID, "step must be 0 or 1");
     e.step = step;
-    e.waves_per_block = (launch && launch->waves_per_block > 0) ? launch->waves_per_block : 4;
-    if (e.waves_per_block > 4) return fail(FVMI_ERR_INVALID, "waves_per_block out of range [1, 4]");
-    // The work list is sorted longest first: dispatch order (block i on XCD
-    // i % 8) spreads it evenly over the XCDs, whereas the contiguous remap of
-    // the single-grid kernel would give XCD 0 the longest segments and leave
-    // the last XCDs with the empty tail of the list.
-    e.xcd_remap = 0;
     const int math = launch ? launch->math : FVMI_MATH_FAST;
-    if (waves <= 0) waves = current_cu_count() * 4 * 4;  // four waves per SIMD
-    e.num_blocks = (waves + e.waves_per_block - 1) / e.waves_per_block;
-    int grid = e.num_blocks;
-    if (e.xcd_remap) grid = ((grid + 7) / 8) * 8;
     hipError_t err = (math == FVMI_MATH_EXACT) ? launch_ensemble_exact(scheme, e, grid, (hipStream_t)stream)
                                                : launch_ensemble_fast(scheme, e, grid, (hipStream_t)stream);
     if (err != hipSuccess) return hip_fail(err, "ensemble substep launch");
+    return FVMI_OK;
+}
+
+int fvmi_ensemble_step(int scheme, fvmi_instance_t* table, const int* segs, const int* num_segs_dev, int waves,
+                       const fvmi_launch_t* launch, void* stream) {
+    EnsembleArgs e{};
+    int grid = 0;
+    if (int rc = fill_ensemble(scheme, table, segs, num_segs_dev, waves, launch, e, grid)) return rc;
+    const int math = launch ? launch->math : FVMI_MATH_FAST;
+    if (math == FVMI_MATH_EXACT || scheme == SCHEME_WAF)
+        return fail(FVMI_ERR_UNSUPPORTED, "no whole step in one launch for scheme %d in this arithmetic", scheme);
+    hipError_t err = launch_ensemble_step_fast(scheme, e, grid, (hipStream_t)stream);
+    if (err != hipSuccess) return hip_fail(err, "ensemble step launch");
     return FVMI_OK;
 }
 

@@ -282,9 +282,12 @@ int fvmi_field_stats(int nx, int ny, int x_halo, int y_halo, const float* field,
  * One full step of every instance = fvmi_ensemble_prepare, fvmi_ensemble_substep
  * (step 0), fvmi_ensemble_substep (step 1), fvmi_ensemble_advance, all on one
  * stream; the sequence may be captured in a graph (fvmi_stream_begin_capture).
+ * fvmi_ensemble_step takes both substeps in one launch where it applies, and
+ * fvmi_ensemble_tick the advance of a step and the prepare of the next.
  */
 typedef struct fvmi_instance {
-    float* field[2][4]; /* [buffer][variable]: padded fields; buffer 0 holds the state between steps */
+    float* field[2][4]; /* [buffer][variable]: padded fields; the state between steps is in buffer 0, or with
+                           fvmi_ensemble_step in buffer `cur` */
     int pitch;          /* bytes, shared by all fields of the instance */
     int nx, ny;
     int bc;             /* packed boundary conditions */
@@ -296,6 +299,7 @@ typedef struct fvmi_instance {
     int nt;             /* steps taken */
     int active;         /* 0 once t >= t_end */
     int fixed_dt;       /* 1: keep `dt`, no CFL refresh (simulate(t, dt=...)) */
+    int cur;            /* buffer of the state (0 or 1); read and turned only by fvmi_ensemble_step's sequence */
     double t, t_end, dt;
     double cfl_scale;
 } fvmi_instance_t;
@@ -315,6 +319,18 @@ int fvmi_ensemble_prepare(fvmi_instance_t* table, int n, void* stream);
  * evenly over the XCDs. */
 int fvmi_ensemble_substep(int scheme, fvmi_instance_t* table, const int* segs, const int* num_segs_dev, int waves,
                           int step, const fvmi_launch_t* launch, void* stream);
+/* Both substeps of every active instance in one launch (KP07_dimsplit, HLL2 and
+ * Euler in fast arithmetic; FVMI_ERR_UNSUPPORTED otherwise): reads buffer `cur`
+ * and writes the other, so the advance that follows has to turn `cur`.  As
+ * above, with strips of 56 columns.  Every instance has to meet
+ * fvmi_dimsplit_step's conditions for one launch (at least 8 x 8 cells, no
+ * Dirichlet edge, periodic edges in opposite pairs, segments of at least 4 rows
+ * but the last of a strip); results are those of the two substeps. */
+int fvmi_ensemble_step(int scheme, fvmi_instance_t* table, const int* segs, const int* num_segs_dev, int waves,
+                       const fvmi_launch_t* launch, void* stream);
+/* Time and step count of every active instance after a step (with `turn` also
+ * `cur`), then, with `prepare`, fvmi_ensemble_prepare for the next one. */
+int fvmi_ensemble_tick(fvmi_instance_t* table, int n, int turn, int prepare, void* stream);
 /* The work split of one substep launch of the four dimensionally split entry
  * points and of the unsplit ones, computed on the host with no device call:
  * the planner's choice for scheme (3 Euler in fast arithmetic: strips of 124

@@ -201,3 +201,57 @@ def test_first_order_with_two_columns_per_lane(ctx, scheme, bc):
                 sim.step(dt)
         assert all(np.array_equal(x, y) for x, y in zip(*[s.download() for s in sims])), nx
         assert sims[0].computeDt() == sims[1].computeDt()
+
+
+def _ensemble_specs(codes, sizes, seed):
+    specs = []
+    for j, ((nx, ny), code) in enumerate(zip(sizes, codes)):
+        specs.append({"fields": state("kp07_dimsplit", nx, ny, seed + j), "nx": nx, "ny": ny, "dx": 1.0, "dy": 1.0,
+                      "g": 9.81, "t_end": 1.3 + 0.4 * j, "bc": code})
+    return specs
+
+
+@pytest.mark.parametrize("scheme", ["kp07_dimsplit", "hll2"])
+@pytest.mark.parametrize("steps_per_graph,seg_rows", [(3, None), (4, 5)])
+def test_ensemble_of_whole_steps_equals_plain_runs(ctx, scheme, steps_per_graph, seg_rows):
+    """Instances that finish after odd and even step counts, in blocks of odd
+    and even length: each equals its plain run, also its non-finite count's
+    buffer.  An instance with a Dirichlet edge joining midway turns the whole
+    ensemble to substeps, with every instance's state where it was."""
+    from finitevolumegpu_amd.Ensemble import Ensemble
+    sizes = [(8, 8), (57, 33), (113, 65), (70, 120)]
+    codes = [BOUNDARIES[k] for k in ("reflective", "mixed", "periodic", "outflow")]
+    specs = _ensemble_specs(codes, sizes, 11)
+    late = _ensemble_specs([O.pack_bc(R, R, P, R)], [(40, 30)], 50)[0]  # one-sided periodic: substeps
+    late["t_end"] = 1.0
+    ens = Ensemble(ctx, scheme, specs, steps_per_graph=steps_per_graph, seg_rows=seg_rows, capacity=6)
+    ens.advance()
+    assert ens.whole_steps
+    slot = ens.add(late)
+    ens.advance()
+    assert not ens.whole_steps
+    ens.remove(slot) if slot in ens.finished() else None
+    ens.run()
+    for i, spec in list(enumerate(specs)) + [(slot, late)]:
+        if not ens.live[i]:
+            continue
+        sim = make(ctx, scheme, spec["fields"], spec["nx"], spec["ny"], spec["bc"])
+        sim.simulate(spec["t_end"])
+        t, nt = ens.state(i)
+        assert nt == sim.simSteps() and t == sim.simTime()
+        assert all(np.array_equal(x, y) for x, y in zip(ens.download(i), sim.download())), i
+    assert (ens.nonfinite_counts(range(len(specs))) == 0).all()
+    ens.close()
+    # and with whole steps to the end
+    ens = Ensemble(ctx, scheme, specs, steps_per_graph=steps_per_graph, seg_rows=seg_rows)
+    ens.run()
+    assert ens.whole_steps
+    parities = set()
+    for i, spec in enumerate(specs):
+        sim = make(ctx, scheme, spec["fields"], spec["nx"], spec["ny"], spec["bc"])
+        sim.simulate(spec["t_end"])
+        parities.add(sim.simSteps() % 2)
+        assert ens.state(i)[1] == sim.simSteps()
+        assert all(np.array_equal(x, y) for x, y in zip(ens.download(i), sim.download())), i
+    assert parities == {0, 1}
+    ens.close()
