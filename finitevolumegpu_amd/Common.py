@@ -84,6 +84,7 @@ class HipArray2D:
         pitch = ctypes.c_size_t()
         _lib.call("fvmi_malloc_pitch", ctypes.byref(ptr), ctypes.byref(pitch), nx_halo * 4, ny_halo)
         self.ptr = ptr
+        self.address = ptr.value  # 0 once freed
         self.pitch = int(pitch.value)
         _lib.call("fvmi_fill_f32", self.ptr, self.pitch, nx_halo, ny_halo, 0.0, _stream_handle(stream))
         if cpu_data is None:
@@ -150,6 +151,7 @@ class HipArray2D:
         if getattr(self, "ptr", None) is not None and self.ptr.value and _lib._lib is not None:
             _lib.lib().fvmi_free(self.ptr)
             self.ptr = ctypes.c_void_p()
+            self.address = 0
 
     def __del__(self):
         self.free()

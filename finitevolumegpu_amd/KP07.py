@@ -5,7 +5,8 @@ GPUSimulators/cuda/SWE2D_KP07.cu)."""
 import numpy as np
 
 from . import _lib
-from .Simulator import BoundaryCondition, UnsplitSimulator, _library_methods, _StepCall, swe_initial_cfl
+from .Simulator import (BoundaryCondition, UnsplitSimulator, _library_methods, _StepCall, _steps_in_library,
+                        swe_initial_cfl)
 
 
 def stepOrderToCodedInt(step, order):
@@ -34,7 +35,7 @@ class KP07(UnsplitSimulator):
         self._init_unsplit([h0, hu0, hv0], swe_initial_cfl(h0, hu0, hv0, self.dx, self.dy, g),
                            tile_rows, waves_per_block, math, xcd_remap)
         # a second-order step is one library call unless a subclass brings its own substeps
-        self._step_call = _StepCall()
+        self._step_call = _StepCall("fvmi_swe_kp07_rk2_step", _lib.RUN_KP07_RK2)
         self._whole_step = order == 2 and _library_methods(self, ("substep", "_launch", "_field_args", "cfl_pointer"))
 
     def step(self, dt):
@@ -43,12 +44,18 @@ class KP07(UnsplitSimulator):
         if not self._whole_step or self.num_substeps != 2 or "substep" in self.__dict__:
             super().step(dt)
             return
-        in_other, self.cfl_last = self._step_call("fvmi_swe_kp07_rk2_step", self, 0, dt, self.boundary_conditions,
-                                                  1 - self.cfl_last)
-        if in_other:
-            self.u0, self.u1 = self.u1, self.u0
+        self._take_step(*self._step_call.step(self, 0, np.float32(dt), self.boundary_conditions, 1 - self.cfl_last))
         self.t += float(dt)
         self.nt += 1
+
+    def _take_step(self, in_other, slot):
+        if in_other:
+            self.u0, self.u1 = self.u1, self.u0
+        self.cfl_last = slot
+
+    def _run_steps(self, t_end, max_steps):
+        return (self._whole_step and self.num_substeps == 2 and _steps_in_library(self)
+                and self._step_call.run(self, 0, t_end, max_steps, 1 - self.cfl_last))
 
     def substepRK(self, dt, substep):
         self.substep(dt, substep)

@@ -120,7 +120,8 @@ class BaseSimulator:
                 self.logger.warning("step %d: no time left to advance (dt %g), stopping", self.simSteps(),
                                     float(current_dt))
                 break
-            self.step(current_dt)
+            if not self._run_steps(t_end, 100 - self.simSteps() % 100):
+                self.step(current_dt)
             print_string = printer.getPrintString(self.simTime() - t_start)
             if print_string:
                 self.logger.info("%s: %s", self, print_string)
@@ -131,6 +132,11 @@ class BaseSimulator:
                     # reference read this suffix)
                     e.args = e.args + ("Step=%d, time=%f" % (self.simSteps(), self.simTime()),)
                     raise
+
+    def _run_steps(self, t_end, max_steps):
+        """Up to ``max_steps`` steps of length ``self.dt`` towards ``t_end`` in one
+        library call, where the simulator has one; returns whether it took any."""
+        return False
 
     def step(self, dt):
         """One full step of ``num_substeps`` substeps (Simulator.py:220-228)."""
@@ -200,33 +206,81 @@ def resolve_math(scheme, math):
 
 
 class _StepCall:
-    """Calls a whole-step entry point of the library (fvmi_step_t) for a
+    """Calls the whole-step entry points of the library (fvmi_step_t) for a
     simulator's current buffers and parameters."""
 
-    def __init__(self):
+    def __init__(self, name, run_kind):
+        self.name = name
+        self.run_kind = run_kind
         self.args = ctypes.create_string_buffer(ctypes.sizeof(_lib.StepArgs))
-        self.out = (ctypes.c_int * 2)()  # buffer of the new state, slot of its CFL minimum
+        # buffer of the new state, slot of its CFL minimum, steps taken; the time
+        self.out = (ctypes.c_int * 3)()
         self.out_ptr = ctypes.addressof(self.out)
+        self.time = ctypes.c_double()
+        self.time_ptr = ctypes.addressof(self.time)
 
-    def __call__(self, name, sim, scheme, dt, boundary_conditions, cfl_slot):
-        """Returns (state is in u1, CFL slot)."""
-        fields = []
-        pitches = []
-        for state in (sim.u0, sim.u1):
-            arrays = state.gpu_variables
-            fields += [v.ptr.value or 0 for v in arrays] + [0] * (4 - len(arrays))
-            pitches += [v.pitch for v in arrays] + [0] * (4 - len(arrays))
-        _lib.STEP_PACK.pack_into(self.args, 0, scheme, sim.nx, sim.ny, boundary_conditions, sim.dx, sim.dy,
-                                 np.float32(dt), sim.g, getattr(sim, "theta", 0.0), getattr(sim, "gamma", 0.0),
-                                 *fields, *pitches, sim.cfl_pointer() or 0, cfl_slot)
-        _lib.call(name, self.args, sim.launch, self.out_ptr, self.out_ptr + 4, sim.stream.handle)
-        return bool(self.out[0]), self.out[1]
+    def _pack(self, sim, scheme, dt, boundary_conditions, cfl_slot):
+        u, v = sim.u0.gpu_variables, sim.u1.gpu_variables
+        pad = (0,) * (4 - len(u))
+        _lib.STEP_PACK.pack_into(
+            self.args, 0, scheme, sim.nx, sim.ny, boundary_conditions, sim.dx, sim.dy, dt, sim.g,
+            getattr(sim, "theta", 0.0), getattr(sim, "gamma", 0.0), *[x.address for x in u], *pad,
+            *[x.address for x in v], *pad, *[x.pitch for x in u], *pad, *[x.pitch for x in v], *pad,
+            sim.cfl_pointer() or 0, cfl_slot)
+
+    def step(self, sim, scheme, dt, boundary_conditions, cfl_slot):
+        """One step; returns (state is in u1, CFL slot)."""
+        self._pack(sim, scheme, dt, boundary_conditions, cfl_slot)
+        _lib.call(self.name, self.args, sim.launch, self.out_ptr, self.out_ptr + 4, sim.stream.handle)
+        return self.out[0], self.out[1]
+
+    def run(self, sim, scheme, t_end, max_steps, cfl_slot):
+        """Steps of length sim.dt from sim.t towards ``t_end``; brings the
+        simulator's time, step count and state up to date with the steps taken,
+        also where one of them fails, and returns whether there was any.
+
+        Only for times in double precision: float32 ones are compared and
+        subtracted as such by the loop in Python, and that stays so.  Host time of
+        a KP07_dimsplit step 3.5 us against 6.5 through step(); three 256^2 runs in
+        turn 1909 -> 1782 us each, which then wait for the device."""
+        if not (isinstance(t_end, float) and isinstance(sim.t, float) and isinstance(sim.dt, (float, np.float32))):
+            return False
+        self._pack(sim, scheme, 0.0, sim.boundary_conditions, cfl_slot)
+        self.time.value = sim.t
+        self.out[2] = 0
+        try:
+            _lib.call("fvmi_run_steps", self.run_kind, self.args, sim.launch, self.time_ptr, t_end, sim.dt,
+                      max_steps, self.out_ptr + 8, self.out_ptr, self.out_ptr + 4, sim.stream.handle)
+        finally:
+            if self.out[2]:
+                sim.t = self.time.value
+                sim.nt += self.out[2]
+                sim._take_step(self.out[0], self.out[1])
+        return self.out[2] > 0
+
+
+# Methods that take part in a step and that a subclass, an instance or a
+# wrapper may replace: with its own version the simulator steps through it.
+_STEP_METHODS = ("step", "substep", "_launch", "_field_args", "cfl_pointer", "simTime", "simSteps")
+
+
+def _of_package(function):
+    """Whether the code of ``function`` is the package's own (a wrapper may carry
+    the name and module of what it wraps, so these do not tell)."""
+    module = getattr(function, "__globals__", {}).get("__name__", "")
+    return module.partition(".")[0] == __name__.partition(".")[0]
 
 
 def _library_methods(sim, names):
     """Whether the class of ``sim`` has the package's own methods of these names."""
-    package = __name__.partition(".")[0]
-    return all(getattr(type(sim), name).__module__.partition(".")[0] == package for name in names)
+    return all(_of_package(getattr(type(sim), name)) for name in names)
+
+
+def _steps_in_library(sim):
+    """Whether nothing stands between the steps of ``simulate``, progress
+    reports of a program's own included."""
+    return (sim.__dict__.keys().isdisjoint(_STEP_METHODS) and _library_methods(sim, _STEP_METHODS)
+            and _of_package(Common.ProgressPrinter.getPrintString))
 
 
 class DimsplitSimulator(BaseSimulator):
@@ -263,7 +317,7 @@ class DimsplitSimulator(BaseSimulator):
         init = np.array([np.inf, cfl_host], dtype=np.float32)
         _lib.call("fvmi_memcpy_async", self.cfl_data, init.ctypes.data, 8, _lib.MEMCPY_HTOD, self.stream.handle)
         self.stream.synchronize()
-        self._step_call = _StepCall()
+        self._step_call = _StepCall("fvmi_dimsplit_step", _lib.RUN_DIMSPLIT)
         # step() is one library call unless a subclass brings its own substeps
         self._whole_step = _library_methods(self, ("substep", "substepDimsplit", "_launch", "_field_args",
                                                    "cfl_pointer"))
@@ -274,7 +328,7 @@ class DimsplitSimulator(BaseSimulator):
     def step(self, dt):
         """One full step as one library call (fvmi_dimsplit_step), with the
         results of the two substeps of BaseSimulator.step."""
-        if not self._whole_step or "substep" in self.__dict__:
+        if not self._whole_step or self.num_substeps != 2 or "substep" in self.__dict__:
             super().step(dt)
             return
         self._step_both(dt, self.boundary_conditions)
@@ -283,13 +337,19 @@ class DimsplitSimulator(BaseSimulator):
 
     def _step_both(self, dt, boundary_conditions):
         """Both substeps of one step under ``boundary_conditions``."""
-        in_other, slot = self._step_call("fvmi_dimsplit_step", self, _lib.SCHEME_IDS[self.scheme], dt * 0.5,
-                                         boundary_conditions, self.cfl_free)
+        self._take_step(*self._step_call.step(self, _lib.SCHEME_IDS[self.scheme], np.float32(dt * 0.5),
+                                              boundary_conditions, self.cfl_free))
+
+    def _take_step(self, in_other, slot):
         if in_other:
             self.u0, self.u1 = self.u1, self.u0
         if self.cfl_pointer():
             self.cfl_last = slot
             self.cfl_free = 1 - slot
+
+    def _run_steps(self, t_end, max_steps):
+        return (self._whole_step and self.num_substeps == 2 and _steps_in_library(self)
+                and self._step_call.run(self, _lib.SCHEME_IDS[self.scheme], t_end, max_steps, self.cfl_free))
 
     def substep(self, dt, step_number):
         self.substepDimsplit(dt * 0.5, step_number)

@@ -139,6 +139,8 @@ SIGNATURES = {
                               + [c_void_p, c_int] * 6 + [c_void_p, c_int, P(LaunchConfig), c_void_p]),
     "fvmi_dimsplit_step": (c_int, [c_void_p, P(LaunchConfig), c_void_p, c_void_p, c_void_p]),
     "fvmi_swe_kp07_rk2_step": (c_int, [c_void_p, P(LaunchConfig), c_void_p, c_void_p, c_void_p]),
+    "fvmi_run_steps": (c_int, [c_int, c_void_p, P(LaunchConfig), c_void_p, ctypes.c_double, ctypes.c_double, c_int,
+                               c_void_p, c_void_p, c_void_p, c_void_p]),
     "fvmi_halo_copy_periodic_x": (c_int, [c_int, c_int, c_int, P(c_void_p), P(c_int), c_void_p]),
     "fvmi_halo_exchange_periodic": (c_int, [c_int, c_int, c_int, P(c_void_p), P(c_int), c_int, c_int, c_void_p]),
     "fvmi_field_stats": (c_int, [c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p]),
@@ -153,6 +155,9 @@ SIGNATURES = {
     "fvmi_graph_launch": (c_int, [c_void_p, c_void_p]),
     "fvmi_graph_destroy": (c_int, [c_void_p]),
 }
+
+RUN_DIMSPLIT = 0
+RUN_KP07_RK2 = 1
 
 _lib = None
 

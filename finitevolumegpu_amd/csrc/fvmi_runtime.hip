@@ -764,6 +764,42 @@ int fvmi_swe_kp07_rk2_step(const fvmi_step_t* p, const fvmi_launch_t* launch, in
     return FVMI_OK;
 }
 
+int fvmi_run_steps(int kind, const fvmi_step_t* p, const fvmi_launch_t* launch, double* t, double t_end, double dt,
+                   int max_steps, int* steps_out, int* state_out, int* cfl_slot_out, void* stream) {
+    if (!p || !t || !steps_out || !state_out || !cfl_slot_out) return fail(FVMI_ERR_INVALID, "NULL argument");
+    if (kind != FVMI_RUN_DIMSPLIT && kind != FVMI_RUN_KP07_RK2) return fail(FVMI_ERR_INVALID, "unknown run %d", kind);
+    fvmi_step_t s = *p;
+    int buffer = 0, slot = 1 - s.cfl_slot, n = 0;
+    int rc = FVMI_OK;
+    for (; n < max_steps && *t < t_end; ++n) {
+        const double left = t_end - *t;
+        const float cur = (float)(left < dt ? left : dt);
+        if (!(cur > 0.0f)) break;
+        s.dt = kind == FVMI_RUN_DIMSPLIT ? cur * 0.5f : cur;
+        int turned = 0;
+        rc = kind == FVMI_RUN_DIMSPLIT ? fvmi_dimsplit_step(&s, launch, &turned, &slot, stream)
+                                       : fvmi_swe_kp07_rk2_step(&s, launch, &turned, &slot, stream);
+        if (rc) break;
+        if (turned) {
+            for (int k = 0; k < 4; ++k) {
+                float* const f = s.state[0][k];
+                s.state[0][k] = s.state[1][k];
+                s.state[1][k] = f;
+                const int pitch = s.pitch[0][k];
+                s.pitch[0][k] = s.pitch[1][k];
+                s.pitch[1][k] = pitch;
+            }
+            buffer ^= 1;
+        }
+        s.cfl_slot = 1 - slot;
+        *t += (double)cur;
+    }
+    *steps_out = n;
+    *state_out = buffer;
+    *cfl_slot_out = slot;
+    return rc;
+}
+
 int fvmi_halo_exchange_periodic(int nx, int ny, int nvars, float* const* fields, const int* pitches, int wrap_x,
                                 int wrap_y, void* stream) {
     if (nx < 2 || ny < 2 || nvars < 1 || nvars > 4 || !fields || !pitches)

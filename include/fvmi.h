@@ -232,6 +232,19 @@ int fvmi_dimsplit_step(const fvmi_step_t* p, const fvmi_launch_t* launch, int* s
 int fvmi_swe_kp07_rk2_step(const fvmi_step_t* p, const fvmi_launch_t* launch, int* state_out, int* cfl_slot_out,
                            void* stream);
 
+/* The stepping loop of BaseSimulator.simulate (Simulator.py:176-217) between two
+ * refreshes of dt: up to `max_steps` steps of fvmi_dimsplit_step or
+ * fvmi_swe_kp07_rk2_step, each of float32 length min(dt, t_end - *t) (p->dt is
+ * not read), *t advanced in double precision; stops at t_end or where that
+ * length is not positive.  Queues the launches and returns; *steps_out is the
+ * number of steps, the other outputs as of the last step (of the step functions;
+ * with none, the state stays in buffer 0 and the slot is the one that is not
+ * free).  After an error they describe the steps before it. */
+#define FVMI_RUN_DIMSPLIT 0
+#define FVMI_RUN_KP07_RK2 1
+int fvmi_run_steps(int kind, const fvmi_step_t* p, const fvmi_launch_t* launch, double* t, double t_end, double dt,
+                   int max_steps, int* steps_out, int* state_out, int* cfl_slot_out, void* stream);
+
 /* One-rank stand-in for MPISimulator.full_exchange's east/west leg
  * (MPISimulator.py:283-295, 440-480) with a periodic-x neighbour: for each of
  * the `nvars` fields copy padded columns [nx, nx+2) -> [0, 2) and

@@ -255,3 +255,81 @@ def test_ensemble_of_whole_steps_equals_plain_runs(ctx, scheme, steps_per_graph,
         assert all(np.array_equal(x, y) for x, y in zip(ens.download(i), sim.download())), i
     assert parities == {0, 1}
     ens.close()
+
+
+RUNS = [("kp07_dimsplit", "fast"), ("hll2", "fast"), ("waf", "exact"), ("ee2d_kp07_dimsplit", "exact"),
+        ("kp07", "fast")]
+
+
+def step_loop(sim, t, dt=None):
+    """The loop of simulate(), a step at a time."""
+    t_end = sim.simTime() + t
+    sim.dt = sim.dt if dt is None else dt
+    while sim.simTime() < t_end:
+        if dt is None and sim.simSteps() % 100 == 0:
+            sim.dt = sim.computeDt() * sim.cfl_scale
+        sim.step(np.float32(min(sim.dt, t_end - sim.simTime())))
+
+
+@pytest.mark.parametrize("given", [None, float, np.float32])
+@pytest.mark.parametrize("scheme,math", RUNS)
+def test_simulate_equals_the_loop_of_steps(ctx, scheme, math, given):
+    """Runs of steps in one library call: across refreshes of dt, ending inside
+    one, on one (odd numbers of steps) and not at all, and with substeps between."""
+    nx, ny = 61, 34
+    fields = state(scheme, nx, ny, seed=8)
+    a, b = (make(ctx, scheme, fields, nx, ny, BOUNDARIES["channel"], math) for _ in range(2))
+    unit = 0.5 * a.computeDt()
+    dt = None if given is None else given(unit)
+    for length in (unit * 230.3, unit * 0.1, 0.0, unit * 31, np.float32(unit * 2.5), 3 * unit):
+        print("case simulate", scheme, math, length, flush=True)
+        a.simulate(length, dt)
+        step_loop(b, length, dt)
+        assert a.simTime() == b.simTime() and type(a.simTime()) is type(b.simTime())
+        assert a.simSteps() == b.simSteps() and a.computeDt() == b.computeDt() and a.dt == b.dt
+        assert all(np.array_equal(x, y) for x, y in zip(a.download(), b.download()))
+        for sim in (a, b):  # a substep pair changes the slots and buffers that the next run starts from
+            sim.substep(np.float32(unit), 0)
+            sim.substep(np.float32(unit), 1)
+    assert a.simSteps() > 100
+
+
+@pytest.mark.parametrize("scheme,math", [RUNS[0], RUNS[4]])
+def test_simulate_calls_replaced_methods(ctx, scheme, math, monkeypatch):
+    """A step or substep that a program wrapped is called for each step."""
+    import functools
+
+    sims = [make(ctx, scheme, state(scheme, 40, 30, seed=1), 40, 30, BOUNDARIES["reflective"], math)
+            for _ in range(3)]
+    cls = type(sims[0])
+    calls = []
+    dt = 0.1 * sims[0].computeDt()
+    sims[0].simulate(dt * 7.5, dt)
+    method = sims[1].step
+    sims[1].step = lambda *a: (calls.append(0), method(*a))
+    sims[1].simulate(dt * 7.5, dt)
+    assert len(calls) == sims[0].simSteps() == sims[1].simSteps() == 8
+    for name in ("step", "simTime"):
+        calls.clear()
+        inner = getattr(cls, name)
+        monkeypatch.setattr(cls, name, functools.wraps(inner)(lambda *a: (calls.append(0), inner(*a))[1]))
+        before = sims[2].simSteps()
+        sims[2].simulate(dt * 7.5, dt)
+        assert len(calls) >= sims[2].simSteps() - before >= 7
+        monkeypatch.undo()
+    assert all(np.array_equal(x, y) for x, y in zip(sims[0].download(), sims[1].download()))
+
+
+def test_run_of_steps_refuses_bad_arguments(ctx):
+    from finitevolumegpu_amd import _lib
+    sim = make(ctx, "kp07_dimsplit", state("kp07_dimsplit", 40, 30, seed=1), 40, 30, BOUNDARIES["reflective"])
+    out = sim._step_call.out_ptr
+    sim._step_call._pack(sim, _lib.SCHEME_IDS["kp07_dimsplit"], 0.0, sim.boundary_conditions, sim.cfl_free)
+    for kind, args, n in ((2, sim._step_call.args, out), (0, None, out), (0, sim._step_call.args, None)):
+        with pytest.raises(_lib.FvmiError):
+            _lib.call("fvmi_run_steps", kind, args, sim.launch, sim._step_call.time_ptr, 1.0, 0.1, 5, n, out, out,
+                      sim.stream.handle)
+    sim.nx = 1  # refused by the step, before anything is launched
+    with pytest.raises(_lib.FvmiError):
+        sim.simulate(0.1, 0.05)
+    assert sim.simSteps() == 0 and sim.simTime() == 0.0
