@@ -53,7 +53,8 @@ hipError_t launch_ensemble_fast_ilp(int scheme, const EnsembleArgs& e, int grid,
     }
 }
 hipError_t launch_rk2_step(const SubstepArgs& a, int grid, hipStream_t stream) {
-    hipLaunchKernelGGL((rk2_kernel<MathFast>), dim3(grid), dim3(kLanes * a.waves_per_block), 0, stream, a);
+    hipLaunchKernelGGL((rk2_kernel<MathFast>), dim3(grid), dim3(kLanes * a.waves_per_block),
+                       block_cfl_bytes(block_cfl(a.round_plan, a.cfl)), stream, a);
     return hipGetLastError();
 }
 hipError_t launch_unsplit_fast(int scheme, const UnsplitArgs& a, int grid, hipStream_t stream) {

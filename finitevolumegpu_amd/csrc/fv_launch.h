@@ -101,28 +101,33 @@ inline int plan_substep(SubstepArgs& a, int cu_count, bool round_ok = false, int
     return grid;
 }
 
+inline unsigned substep_lds(const SubstepArgs& a) {
+    return block_cfl_bytes(block_cfl(a.round_plan, a.step == 1 ? a.cfl : nullptr));
+}
+
 // One scheme's kernel (each translation unit instantiates the ones it owns).
 template <class S, class M>
 hipError_t launch_substep_scheme(const SubstepArgs& a, int grid, hipStream_t stream) {
-    hipLaunchKernelGGL((substep_kernel<S, M>), dim3(grid), dim3(kLanes * a.waves_per_block), 0, stream, a);
+    hipLaunchKernelGGL((substep_kernel<S, M>), dim3(grid), dim3(kLanes * a.waves_per_block), substep_lds(a), stream, a);
     return hipGetLastError();
 }
 
 template <class M>
 hipError_t launch_substep(int scheme, SubstepArgs a, int grid, hipStream_t stream) {
     const dim3 block(kLanes * a.waves_per_block);
+    const unsigned lds = substep_lds(a);
     switch (scheme) {
         case SCHEME_KP07:
-            hipLaunchKernelGGL((substep_kernel<SweKP07<M>, M>), dim3(grid), block, 0, stream, a);
+            hipLaunchKernelGGL((substep_kernel<SweKP07<M>, M>), dim3(grid), block, lds, stream, a);
             break;
         case SCHEME_HLL2:
-            hipLaunchKernelGGL((substep_kernel<SweHLL2<M>, M>), dim3(grid), block, 0, stream, a);
+            hipLaunchKernelGGL((substep_kernel<SweHLL2<M>, M>), dim3(grid), block, lds, stream, a);
             break;
         case SCHEME_WAF:
-            hipLaunchKernelGGL((substep_kernel<SweWAF<M>, M>), dim3(grid), block, 0, stream, a);
+            hipLaunchKernelGGL((substep_kernel<SweWAF<M>, M>), dim3(grid), block, lds, stream, a);
             break;
         case SCHEME_EULER:
-            hipLaunchKernelGGL((substep_kernel<EulerKP07<M>, M>), dim3(grid), block, 0, stream, a);
+            hipLaunchKernelGGL((substep_kernel<EulerKP07<M>, M>), dim3(grid), block, lds, stream, a);
             break;
         default:
             return hipErrorInvalidValue;
@@ -132,7 +137,8 @@ hipError_t launch_substep(int scheme, SubstepArgs a, int grid, hipStream_t strea
 
 template <class S, class M>
 hipError_t launch_step_scheme(const SubstepArgs& a, int grid, hipStream_t stream) {
-    hipLaunchKernelGGL((step_kernel<S, M>), dim3(grid), dim3(kLanes * a.waves_per_block), 0, stream, a);
+    hipLaunchKernelGGL((step_kernel<S, M>), dim3(grid), dim3(kLanes * a.waves_per_block),
+                       block_cfl_bytes(block_cfl(a.round_plan, a.cfl)), stream, a);
     return hipGetLastError();
 }
 

@@ -259,21 +259,21 @@ __global__ void __launch_bounds__(256, 4) rk2_kernel(SubstepArgs a) {
     const int lane = threadIdx.x & (kLanes - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (a.cfl != nullptr && blockIdx.x == 0 && threadIdx.x == 0) a.cfl[1 - a.cfl_slot] = __builtin_inff();
+    const bool shared = block_cfl(a.round_plan, a.cfl);
+    begin_cfl(shared);
     int strip_x, row_in, count;
-    if (!wave_segment(a, blockIdx.x, gridDim.x, wave, strip_x, row_in, count)) return;
-    strip_x = __builtin_amdgcn_readfirstlane(strip_x);
-    row_in = __builtin_amdgcn_readfirstlane(row_in);
-    count = __builtin_amdgcn_readfirstlane(count);
-    Strip<1> st;
-    setup_strip<SweKP07<M, 1>, M, kStepHalo>(a, st, lane, strip_x, row_in, count);
-    StepEdge e;
-    setup_edge(a, st, row_in, count, e);
-    const float acc = needs_edge(e) ? march_rk2<M, true>(a, st, e) : march_rk2<M, false>(a, st, e);
-    if (a.cfl != nullptr) {
-        const float m = wave_min((acc > 0.0f) ? fast::rcp(acc) : __builtin_inff());
-        if (lane == 0 && m < __builtin_inff())
-            atomicMin(reinterpret_cast<unsigned int*>(a.cfl + a.cfl_slot), __float_as_uint(m));
+    float acc = no_cfl<M>();
+    if (wave_segment(a, blockIdx.x, gridDim.x, wave, strip_x, row_in, count)) {
+        strip_x = __builtin_amdgcn_readfirstlane(strip_x);
+        row_in = __builtin_amdgcn_readfirstlane(row_in);
+        count = __builtin_amdgcn_readfirstlane(count);
+        Strip<1> st;
+        setup_strip<SweKP07<M, 1>, M, kStepHalo>(a, st, lane, strip_x, row_in, count);
+        StepEdge e;
+        setup_edge(a, st, row_in, count, e);
+        acc = needs_edge(e) ? march_rk2<M, true>(a, st, e) : march_rk2<M, false>(a, st, e);
     }
+    if (a.cfl != nullptr) reduce_cfl<M>(shared, a.cfl + a.cfl_slot, acc, lane);
 }
 
 }  // namespace fvmi

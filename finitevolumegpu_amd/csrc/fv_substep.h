@@ -316,6 +316,61 @@ __device__ __forceinline__ float wave_min(float v) {
     return v;
 }
 
+// A CFL accumulator that has seen no cell.
+template <class M>
+__device__ __forceinline__ float no_cfl() {
+    return M::exact ? __builtin_inff() : 0.0f;
+}
+
+// The CFL minimum of a workgroup and the number of its waves that have added
+// to it, in the launch's dynamic LDS.
+struct BlockCfl {
+    unsigned least, waves;
+};
+
+// Whether the waves of a workgroup take their CFL minimum to memory together.
+// Atomics on one address take about 10 ns each, one after the other, and where
+// the segments are of equal length they all come at the end: with one per wave,
+// and with one per workgroup, a step of one simulator: KP07_dimsplit 256^2 12.6
+// and 10.3 us, 512^2 20.6 and 14.3, 1000^2 31.7 and 23.8 (11.8 and 21.6 at the
+// last two without the minimum), Euler 512^2 exact 32.6 and 25.3, HLL2 2047^2 81
+// and 73, HLL 1000^2 20.8 and 15.4.  The parts of the round-weighted split end at
+// different times: KP07_dimsplit 4096^2 188 and 187 us, and with three simulators
+// on three streams 177 and 179 a step (a workgroup with LDS starts later beside
+// another launch's last ones).  The first-order schemes' shorter rows gain there
+// too, HLL 4096^2 120 and 102 us alone, 98 and 98 in turn (fv_unsplit.h shares
+// always; part of it is a row kept in registers, see store_row).
+__host__ __device__ inline bool block_cfl(bool round_plan, const float* cfl) { return !round_plan && cfl != nullptr; }
+
+inline unsigned block_cfl_bytes(bool shared) { return shared ? sizeof(BlockCfl) : 0; }
+
+__device__ __forceinline__ void begin_cfl(bool shared) {
+    extern __shared__ BlockCfl block[];
+    if (!shared) return;
+    if (threadIdx.x == 0) block->least = 0x7f800000u, block->waves = 0;  // +inf
+    __syncthreads();
+}
+
+// The accumulator of a wave (also of one without a segment) into the launch's
+// CFL minimum; the last wave of a workgroup with `shared` does it for all.
+template <class M>
+__device__ __forceinline__ void reduce_cfl(bool shared, float* slot, float acc, int lane) {
+    extern __shared__ BlockCfl block[];
+    float dt_min = acc;
+    if constexpr (!M::exact) dt_min = (acc > 0.0f) ? fast::rcp(acc) : __builtin_inff();
+    const float m = wave_min(dt_min);
+    if (lane != 0) return;
+    unsigned least = m < __builtin_inff() ? __float_as_uint(m) : 0x7f800000u;
+    if (shared) {
+        __hip_atomic_fetch_min(&block->least, least, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        const unsigned before =
+            __hip_atomic_fetch_add(&block->waves, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (before != blockDim.x / kLanes - 1) return;
+        least = __hip_atomic_load(&block->least, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    if (least < 0x7f800000u) atomicMin(reinterpret_cast<unsigned int*>(slot), least);
+}
+
 // Rows loaded ahead of the row being processed.  Each wave keeps a ring of
 // row slots in registers: the rows its y stencil still needs plus this many
 // rows in flight, so a load is issued kRowPrefetch rows of work before its
@@ -800,7 +855,11 @@ __device__ __forceinline__ void store_row(const Args& a, const Strip<C>& st, int
         if constexpr (C == 1) {
             __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(q[0][k]), st.rout[k], st.store_off, soff, 0);
         } else {
-            const fvmi_v2u x = {__float_as_uint(q[0][k]), __float_as_uint(q[1][k])};
+            // the optimiser widens a lone load of q[0][k] to a pair, which keeps q
+            // in memory (LDS or scratch) for the whole march: stop it here
+            unsigned lo = __float_as_uint(q[0][k]), hi = __float_as_uint(q[1][k]);
+            asm("" : "+v"(lo));
+            const fvmi_v2u x = {lo, hi};
             __builtin_amdgcn_raw_buffer_store_b64(x, st.rout[k], st.store_off, soff, 0);
         }
     }
@@ -1312,21 +1371,19 @@ __global__ void __launch_bounds__(256, FVMI_SUBSTEP_MIN_WAVES) substep_kernel(Su
     // wave index made scalar so that every row address is computed in SGPRs
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (a.cfl != nullptr && blockIdx.x == 0 && threadIdx.x == 0) a.cfl[1 - (a.step & 1)] = __builtin_inff();
+    const bool shared = block_cfl(a.round_plan, a.step == 1 ? a.cfl : nullptr);
+    begin_cfl(shared);
     int strip_x, row_in, count;
-    if (!wave_segment(a, blockIdx.x, gridDim.x, wave, strip_x, row_in, count)) return;
-    strip_x = __builtin_amdgcn_readfirstlane(strip_x);
-    row_in = __builtin_amdgcn_readfirstlane(row_in);
-    count = __builtin_amdgcn_readfirstlane(count);
-    Strip<S::kC> st;
-    setup_strip<S, M>(a, st, lane, strip_x, row_in, count);
-    const float acc = march<S, M>(a, st);
-    float dt_min = acc;
-    if constexpr (!M::exact) dt_min = (acc > 0.0f) ? fast::rcp(acc) : __builtin_inff();
-    if (a.cfl != nullptr && a.step == 1) {
-        const float m = wave_min(dt_min);
-        if (lane == 0 && m < __builtin_inff())
-            atomicMin(reinterpret_cast<unsigned int*>(a.cfl + 1), __float_as_uint(m));
+    float acc = no_cfl<M>();
+    if (wave_segment(a, blockIdx.x, gridDim.x, wave, strip_x, row_in, count)) {
+        strip_x = __builtin_amdgcn_readfirstlane(strip_x);
+        row_in = __builtin_amdgcn_readfirstlane(row_in);
+        count = __builtin_amdgcn_readfirstlane(count);
+        Strip<S::kC> st;
+        setup_strip<S, M>(a, st, lane, strip_x, row_in, count);
+        acc = march<S, M>(a, st);
     }
+    if (a.cfl != nullptr && a.step == 1) reduce_cfl<M>(shared, a.cfl + 1, acc, lane);
 }
 
 }  // namespace fvmi

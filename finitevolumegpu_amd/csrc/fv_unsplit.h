@@ -546,29 +546,25 @@ __global__ void __launch_bounds__(256, 4) unsplit_kernel(UnsplitArgs a) {
     const int lane = threadIdx.x & (kLanes - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (a.cfl != nullptr && blockIdx.x == 0 && threadIdx.x == 0) a.cfl[1 - a.cfl_slot] = __builtin_inff();
+    begin_cfl(a.cfl != nullptr);
     int strip_x, row_in, count;
-    if (!unsplit_segment(a, blockIdx.x, gridDim.x, wave, strip_x, row_in, count)) return;
-    strip_x = __builtin_amdgcn_readfirstlane(strip_x);
-    row_in = __builtin_amdgcn_readfirstlane(row_in);
-    count = __builtin_amdgcn_readfirstlane(count);
-    Strip<C> st;
-    u_setup<GC, C>(a, st, lane, strip_x, row_in, count);
-    float acc;
-    if constexpr (GC == 1) {
-        if (C == 2 && (st.wave_fix || st.wave_single))
-            acc = march_gc1<S, M, C, C == 2>(a, st);
-        else
-            acc = march_gc1<S, M, C, false>(a, st);
-    } else {
-        acc = a.stage2 ? march_kp07u<S, M, true>(a, st) : march_kp07u<S, M, false>(a, st);
+    float acc = no_cfl<M>();
+    if (unsplit_segment(a, blockIdx.x, gridDim.x, wave, strip_x, row_in, count)) {
+        strip_x = __builtin_amdgcn_readfirstlane(strip_x);
+        row_in = __builtin_amdgcn_readfirstlane(row_in);
+        count = __builtin_amdgcn_readfirstlane(count);
+        Strip<C> st;
+        u_setup<GC, C>(a, st, lane, strip_x, row_in, count);
+        if constexpr (GC == 1) {
+            if (C == 2 && (st.wave_fix || st.wave_single))
+                acc = march_gc1<S, M, C, C == 2>(a, st);
+            else
+                acc = march_gc1<S, M, C, false>(a, st);
+        } else {
+            acc = a.stage2 ? march_kp07u<S, M, true>(a, st) : march_kp07u<S, M, false>(a, st);
+        }
     }
-    float dt_min = acc;
-    if constexpr (!M::exact) dt_min = (acc > 0.0f) ? fast::rcp(acc) : __builtin_inff();
-    if (a.cfl != nullptr) {
-        const float m = wave_min(dt_min);
-        if (lane == 0 && m < __builtin_inff())
-            atomicMin(reinterpret_cast<unsigned int*>(a.cfl + a.cfl_slot), __float_as_uint(m));
-    }
+    if (a.cfl != nullptr) reduce_cfl<M>(true, a.cfl + a.cfl_slot, acc, lane);
 }
 
 // Strip-aligned segments (as plan_substep) for a.cols columns per lane: the
@@ -639,13 +635,14 @@ inline int unsplit_cols(const UnsplitArgs& a, int scheme, bool exact, bool align
 template <class S, class M>
 void launch_unsplit_scheme(const UnsplitArgs& a, int grid, hipStream_t stream) {
     const dim3 block(kLanes * a.waves_per_block);
+    const unsigned lds = block_cfl_bytes(a.cfl != nullptr);
     if constexpr (S::GC == 1) {
         if (a.cols == 2) {
-            hipLaunchKernelGGL((unsplit_kernel<S, M, 2>), dim3(grid), block, 0, stream, a);
+            hipLaunchKernelGGL((unsplit_kernel<S, M, 2>), dim3(grid), block, lds, stream, a);
             return;
         }
     }
-    hipLaunchKernelGGL((unsplit_kernel<S, M, 1>), dim3(grid), block, 0, stream, a);
+    hipLaunchKernelGGL((unsplit_kernel<S, M, 1>), dim3(grid), block, lds, stream, a);
 }
 
 template <class M>

@@ -333,3 +333,46 @@ def test_run_of_steps_refuses_bad_arguments(ctx):
     with pytest.raises(_lib.FvmiError):
         sim.simulate(0.1, 0.05)
     assert sim.simSteps() == 0 and sim.simTime() == 0.0
+
+
+def _host_cfl(sim):
+    h, hu, hv = (np.asarray(f, dtype=np.float64) for f in sim.download())
+    c = np.sqrt(9.81 * h)
+    return min((1.0 / (np.abs(hu / h) + c)).min(), (1.0 / (np.abs(hv / h) + c)).min())
+
+
+@pytest.mark.parametrize("scheme,math", [("kp07_dimsplit", "fast"), ("hll2", "exact"), ("waf", "exact")])
+@pytest.mark.parametrize("nx,ny", [(9, 8), (121, 33), (300, 251)])
+def test_cfl_minimum_of_every_launch_shape(ctx, scheme, math, nx, ny):
+    """The fastest cell, planted anywhere, gives the CFL minimum whichever wave
+    of whichever workgroup holds it, in workgroups of one to four waves, the last
+    of them partly without segments.  Bound: six roundings of 2^-23 (the sum,
+    quotient, root and reciprocal, at most one unit each)."""
+    rng = np.random.default_rng(nx)
+    for waves, tile in ((1, 4), (2, 5), (3, 7), (4, 4), (4, 9), (4, 0)):
+        h, hu, hv = (np.array(f) for f in state(scheme, nx, ny, seed=2))
+        y, x = rng.integers(ny), rng.integers(nx)
+        hv[y, x] = 6.0 * h[y, x]
+        print("case cfl", scheme, math, nx, ny, waves, tile, (y, x), flush=True)
+        sim = make(ctx, scheme, (h, hu, hv), nx, ny, BOUNDARIES["mixed"], math, waves_per_block=waves, tile_rows=tile)
+        for _ in range(3):
+            sim.step(np.float32(0.02))
+            assert abs(sim.computeDt() / 0.5 / _host_cfl(sim) - 1.0) < 6 * 2.0 ** -23
+
+
+@pytest.mark.parametrize("scheme", ["LxF", "HLL", "FORCE", "KP07"])
+def test_unsplit_cfl_minimum_of_every_launch_shape(ctx, scheme):
+    """Equal for every launch shape, one wave per workgroup included."""
+    import importlib
+    cls = getattr(importlib.import_module("finitevolumegpu_amd." + scheme), scheme)
+    rng = np.random.default_rng(7)
+    for nx, ny in ((9, 8), (121, 33), (300, 251)):
+        h, hu, hv = (np.array(f) for f in state("kp07_dimsplit", nx, ny, seed=2))
+        hv[rng.integers(ny), rng.integers(nx)] *= 40.0
+        print("case unsplit cfl", scheme, nx, ny, flush=True)
+        dts = set()
+        for waves, tile in ((1, 4), (2, 5), (3, 7), (4, 4), (4, 9), (4, 0)):
+            sim = cls(ctx, h, hu, hv, nx, ny, 1.0, 1.0, 9.81, waves_per_block=waves, tile_rows=tile)
+            sim.step(np.float32(0.02))
+            dts.add(sim.computeDt())
+        assert len(dts) == 1 and 0.0 < dts.pop() < 1.0
