@@ -50,22 +50,24 @@ inline bool step_is_fused(int scheme, int math, const SubstepArgs& a) {
     return math != FVMI_MATH_EXACT && scheme != SCHEME_WAF && step_grid_fits(a);
 }
 
-// Segments of a whole step re-sweep about 4 rows' worth of halo, twice a
-// substep's: at least 40 rows where the grid has them (HLL2 2047^2 step of one
-// simulator 93 us with 24, 81 with 40; of three in turn 57.7 and 55.0).
-constexpr int kStepMinSeg = 40;
+// Costs of the schemes' segments (fitted to steps of one simulator at 256^2 to
+// 2000^2 over segments of 2 to 40 rows).  Of a split step's two substeps one has
+// the CFL minimum.
+inline SegmentCost substep_cost(int math) {
+    return {4, 2, math == FVMI_MATH_EXACT ? 0.5f : 0.25f, 0.005f};
+}
+inline SegmentCost step_cost() { return {2 * kStepHalo, kStepMinSegRows, 0.45f, 0.01f}; }
 
 // Fills the decomposition fields of `a` (sub-area, launch shape, device size)
 // and returns the grid size to launch.  seg_rows == 0 picks the shape:
 //   * the round-weighted plan (round_segment) when `round_ok`, the workgroups
 //     have 4 waves, the XCD remap is on and every strip holds row groups long
 //     enough for their shortest part to have `min_part` rows;
-//   * otherwise the balanced segment length: at most `waves_per_simd` waves on
-//     every SIMD of the device, but no segment shorter than `min_seg` rows (the
-//     4-row prologue of a segment is then at most 1/6 of its work), except on
-//     small grids (balanced_segment_rows).
-inline int plan_substep(SubstepArgs& a, int cu_count, bool round_ok = false, int waves_per_simd = 4,
-                        int min_seg = 24, int min_part = 16) {
+//   * otherwise segments of equal length (balanced_segment_rows): at most
+//     `waves_per_simd` waves on every SIMD of the device (one more would run
+//     after all the others).
+inline int plan_substep(SubstepArgs& a, int cu_count, const SegmentCost& cost, bool round_ok = false,
+                        int waves_per_simd = 4, int min_part = 16) {
     const int wx = a.x1 - a.x0;
     a.rows_per_strip = a.y1 - a.y0;
     a.strips_x = (wx + a.strip_cols - 1) / a.strip_cols;
@@ -85,14 +87,7 @@ inline int plan_substep(SubstepArgs& a, int cu_count, bool round_ok = false, int
         a.num_blocks = kRounds * cu_count;
         return a.num_blocks;
     }
-    if (a.seg_rows <= 0) {
-        // at most waves_per_simd waves on every SIMD (one more would run after
-        // all the others), segments of at least min_seg rows; shorter ones on
-        // grids too small to fill one wave per SIMD with them
-        // (measured per full step: KP07_dimsplit 256^2 27.2 -> 14.8 us, 512^2
-        // 29.6 -> 23.3 us; EE2D 512^2 46.4 -> 31.5 us)
-        a.seg_rows = balanced_segment_rows(a.rows_per_strip, a.strips_x, cu_count, waves_per_simd, min_seg, min_seg);
-    }
+    if (a.seg_rows <= 0) a.seg_rows = balanced_segment_rows(a.rows_per_strip, a.strips_x, cu_count, waves_per_simd, cost);
     a.segs_per_strip = (a.rows_per_strip + a.seg_rows - 1) / a.seg_rows;
     a.num_waves = a.strips_x * a.segs_per_strip;
     a.num_blocks = (a.num_waves + a.waves_per_block - 1) / a.waves_per_block;

@@ -93,25 +93,44 @@ struct SubstepArgs {
     float g_theta;     // g theta
 };
 
-// Rows per segment of the equal-segment plan: at most waves_per_simd waves on
-// every SIMD (segments per strip rounded down) and no segment shorter than
-// min_seg rows, so that a segment's halo rows stay a small part of its work.
-// A grid too small for that, where one wave per SIMD would leave each wave at
-// most small_limit rows, is bound by the latency of one wave's march instead:
-// its strips are cut into segments of that length (at least kMinSegRowsSmall
-// rows), at most one wave per SIMD.
-constexpr int kMinSegRowsSmall = 4;
-__host__ __device__ inline int balanced_segment_rows(int rows, int strips, int cu_count, int waves_per_simd,
-                                                     int min_seg, int small_limit) {
-    int k = cu_count * 4 * waves_per_simd / strips;
-    if (k < 1) k = 1;
-    const int seg = (rows + k - 1) / k;
-    if (seg >= min_seg) return seg;
-    int k1 = cu_count * 4 / strips;
-    if (k1 < 1) k1 = 1;
-    const int seg1 = (rows + k1 - 1) / k1;
-    if (seg1 >= min_seg || seg1 > small_limit) return min_seg;
-    return seg1 < kMinSegRowsSmall ? kMinSegRowsSmall : seg1;
+// What a launch of equal segments costs, in us, with w waves on a SIMD:
+// row_us (rows + halo_rows) (1 + w) + block_us * workgroups.  A wave alone on its
+// SIMD waits for its own results; each further one adds about half that time to a
+// row of all of them (KP07_dimsplit whole steps, rows of 0.41 us: 5.4, 8.6, 11.2
+// and 13.9 cycles an instruction for one to four waves).  The second term is the
+// CFL minimum's atomics, one after the other (reduce_cfl).
+struct SegmentCost {
+    int halo_rows;   // rows a segment sweeps and does not store
+    int min_rows;    // shortest segment
+    float row_us;
+    float block_us;
+};
+
+// Rows per segment of the equal-segment plan: of the longest segments that put
+// one, two .. waves_per_simd waves on every SIMD, the cheapest; more waves only
+// for 3 % or more, since their halo rows are work that another stream's launches
+// would have to wait for.  A multiple of the device's SIMDs just exceeded is what
+// it avoids: KP07_dimsplit 1500^2 with 40 rows (1026 waves for 1024 SIMDs) and 20,
+// a step of one simulator: 57.9 and 35.8 us, KP07 2048x1500 51 and 44, Euler exact
+// 256^2 with 4 and 2 rows 19.9 and 16.5, HLL 512^2 with 24 and 6 13.9 and 8.8.
+inline int balanced_segment_rows(int rows, int strips, int cu_count, int waves_per_simd, const SegmentCost& c) {
+    int best = rows;  // also where there are more strips than waves
+    float best_cost = 0.0f;
+    for (int w = 1; w <= waves_per_simd; ++w) {
+        const int k = cu_count * 4 * w / strips;
+        if (k < 1) continue;
+        int seg = (rows + k - 1) / k;
+        if (seg < c.min_rows) seg = c.min_rows;
+        const long long waves = (long long)strips * ((rows + seg - 1) / seg);
+        const int per_simd = (int)((waves + 4LL * cu_count - 1) / (4LL * cu_count));
+        const float cost =
+            c.row_us * (float)(seg + c.halo_rows) * (float)(1 + per_simd) + c.block_us * 0.25f * (float)waves;
+        if (best_cost == 0.0f || cost < 0.97f * best_cost) {
+            best = seg;
+            best_cost = cost;
+        }
+    }
+    return best;
 }
 
 // the slope constants from g and theta

@@ -571,7 +571,7 @@ __global__ void __launch_bounds__(256, 4) unsplit_kernel(UnsplitArgs a) {
 // round-weighted split where `round_ok` and it fits, else equal segments, at most
 // waves_per_simd waves on every SIMD.
 inline int plan_unsplit(UnsplitArgs& a, int gc, int cu_count, bool round_ok, int waves_per_simd = 4,
-                        int min_seg = 24, int min_part = 16) {
+                        int min_part = 16) {
     if (gc == 1 && a.cols == 2) {
         constexpr int W = u_strip_cols<1, 2>();
         a.strips_x = (a.nx + 1 + W - 1) / W;  // output columns from padded column 0 on
@@ -595,9 +595,12 @@ inline int plan_unsplit(UnsplitArgs& a, int gc, int cu_count, bool round_ok, int
         a.num_blocks = kRounds * cu_count;
         return a.num_blocks;
     }
-    // short segments only where one wave per SIMD leaves at most 4 rows a wave:
-    // HLL 256^2 12.4 -> 8.5 us per step, but 512^2 (5 rows) 14.4 -> 16.0 us
-    if (a.seg_rows <= 0) a.seg_rows = balanced_segment_rows(a.ny, a.strips_x, cu_count, waves_per_simd, min_seg, 4);
+    if (a.seg_rows <= 0) {
+        const SegmentCost cost = {2 * gc, 2, gc == 2 ? 0.25f : 0.15f * a.cols, 0.01f};
+        const int band = a.cols == 2 ? a.waves_per_block : 1;  // strips are dealt out by workgroups
+        const int strips = (a.strips_x + band - 1) / band * band;
+        a.seg_rows = balanced_segment_rows(a.ny, strips, cu_count, waves_per_simd, cost);
+    }
     a.segs_per_strip = (a.ny + a.seg_rows - 1) / a.seg_rows;
     a.num_waves = a.strips_x * a.segs_per_strip;
     a.num_blocks = a.cols == 2 ? ((a.strips_x + a.waves_per_block - 1) / a.waves_per_block) * a.segs_per_strip

@@ -138,7 +138,7 @@ int run_substep(int scheme, SubstepArgs& a, int nvars, const fvmi_launch_t* laun
     if (int rc = check_substep(scheme, a, nvars, launch, &math)) return rc;
     a.strip_cols = scheme_strip_cols(scheme, math);
     // WAF keeps equal segments: the round-weighted plan made it 3 % slower
-    const int grid = plan_substep(a, current_cu_count(), scheme != SCHEME_WAF);
+    const int grid = plan_substep(a, current_cu_count(), substep_cost(math), scheme != SCHEME_WAF);
     hipError_t e = (math == FVMI_MATH_EXACT) ? launch_substep_exact(scheme, a, grid, (hipStream_t)stream)
                                              : launch_substep_fast(scheme, a, grid, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "substep launch");
@@ -407,7 +407,7 @@ SubstepArgs step_args(const fvmi_step_t* p, int nvars, int from, int step) {
 int plan_step(SubstepArgs& a, int cfl_slot, int cu_count) {
     a.cfl_slot = cfl_slot;
     a.strip_cols = strip_cols<1, kStepHalo>();
-    return plan_substep(a, cu_count, true, 4, kStepMinSeg);
+    return plan_substep(a, cu_count, step_cost(), true);
 }
 
 }  // namespace
@@ -906,8 +906,8 @@ int fvmi_substep_plan(int scheme, int nx, int ny, int x0, int y0, int x1, int y1
     int math = 0;
     if (int rc = fill_launch(launch, a, &math)) return rc;
     a.strip_cols = whole_step ? strip_cols<1, kStepHalo>() : scheme_strip_cols(scheme, math);
-    const int grid =
-        whole_step ? plan_step(a, 0, cu_count) : plan_substep(a, cu_count, scheme != SCHEME_WAF);
+    const int grid = whole_step ? plan_step(a, 0, cu_count)
+                                : plan_substep(a, cu_count, substep_cost(math), scheme != SCHEME_WAF);
     const long long total = (long long)grid * a.waves_per_block;
     if (total > (1LL << 30)) return fail(FVMI_ERR_INVALID, "plan too large");
     *n_waves = (int)total;

@@ -68,3 +68,35 @@ def test_wide_strips_of_a_workgroup_are_adjacent():
 @pytest.mark.parametrize("scheme", [STEP, LXF2])
 def test_sub_areas_are_rejected(scheme):
     assert plan(scheme, 64, 64, sub=(1, 0, 64, 64)) < 0
+
+
+@pytest.mark.parametrize("scheme,math,strip,extra", [(STEP, "fast", 56, 0), (0, "exact", 60, 0), (2, "exact", 60, 0),
+                                                     (5, "fast", 62, 0), (7, "fast", 60, 0), (HLL2, "fast", 124, 1)])
+@pytest.mark.parametrize("nx,ny,cus", [(8, 8, 256), (64, 3000, 256), (256, 256, 256), (1000, 1000, 256),
+                                       (1500, 1500, 256), (2048, 1500, 256), (4000, 100, 256), (1500, 1500, 80),
+                                       (300000, 60, 256)])
+def test_equal_segments_fill_whole_waves_per_simd(scheme, math, strip, extra, nx, ny, cus):
+    """Equal segments put no more than four waves on a SIMD (one workgroup of
+    four beside each other on a CU), and never just a few more than a whole
+    number of them: a shorter segment would not have fitted into as many."""
+    lib = _lib.lib()
+    launch = _lib.LaunchConfig(0, 4, _lib.FVMI_MATH_EXACT if math == "exact" else _lib.FVMI_MATH_FAST, 1)
+    n = ctypes.c_int()
+    lib.fvmi_substep_plan(scheme, nx, ny, 0, 0, 0, 0, ctypes.byref(launch), cus, None, 0, ctypes.byref(n))
+    segs = np.zeros((n.value, 3), dtype=np.int32)
+    assert lib.fvmi_substep_plan(scheme, nx, ny, 0, 0, 0, 0, ctypes.byref(launch), cus,
+                                 segs.ctypes.data_as(ctypes.POINTER(ctypes.c_int)), n.value, ctypes.byref(n)) == 0
+    live = segs[segs[:, 0] >= 0]
+    strips, rows = -(-(nx + extra) // strip), int(live[:, 2].max())
+    band = -(-strips // 4) * 4 if scheme == HLL2 else strips
+    simds = 4 * cus
+    least = 4 if scheme == STEP else 2
+    if len(np.unique(live[live[:, 1] + live[:, 2] < ny, 2])) > 1:
+        return  # the round-weighted split
+    if band > 4 * simds:
+        assert rows == ny
+        return
+    waves = -(-band * -(-ny // rows) // simds)  # per SIMD
+    assert waves <= 4 and rows >= min(least, ny)
+    shorter = -(-band * -(-ny // max(rows - 1, 1)) // simds)
+    assert shorter > waves or rows <= least or -(-ny // (rows - 1)) == -(-ny // rows)
