@@ -4,24 +4,25 @@
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--schemes kp07,hll2,waf,ee2d,lxf,hll,force,kp07u]
                     [--no-cpu-baseline] [--ensemble 512] [--serve 2000 --serve-rate 300]
 
-A "step" is one full time step of the plain Simulator API (two fused substep
-launches: x-y then y-x sweeps), on the seeded dam break with 16 Gaussian bumps,
+A "step" is one full time step of the plain Simulator API (x-y then y-x sweeps,
+both in one launch), on the seeded dam break with 16 Gaussian bumps,
 reflective walls, g = 9.81, theta = 1.3, at a dt pinned to 0.45 x the initial
 CFL.  The state stays resident in HBM; the timed region holds exactly K steps
 between device synchronisations, timed with HIP events on the simulator's
 stream.  One JSON line is printed:
 
 * value / unit      cell-updates per second (cells x full steps / s)
-* roofline          algorithmic HBM bytes of one substep launch (24 B per cell:
+* roofline          algorithmic HBM bytes of one step's launch (24 B per cell:
                     3 fields read + written) / average launch time, against
                     8 TB/s; `traffic` = measured HBM bytes per launch from the
                     rocprofv3 counter summary in profiles/ when present
 * cpu_baseline      the float32 NumPy oracle (one core) on a bounded sample of
                     the same workload (512x512 crop of the generator, a few steps)
-* schemes           the same measurement for HLL2 and WAF at 4096^2,
-                    EE2D_KP07_dimsplit at 8192^2 (64 B per cell-step) and the
-                    reference's other schemes LxF, HLL, FORCE (24 B per
-                    cell-step) and the unsplit KP07 with RK2 (60 B) at 4096^2
+* schemes           the same measurement for HLL2 and WAF (two launches, 48 B per
+                    cell-step) at 4096^2, EE2D_KP07_dimsplit at 8192^2 (64 B per
+                    cell-step; 32 in fast arithmetic, one launch) and the
+                    reference's other schemes LxF, HLL, FORCE and the unsplit
+                    KP07 with RK2 (one launch, 24 B per cell-step) at 4096^2
 * ensemble          512 dam breaks of uneven size in the batched engine against
                     the plain simulate() loop over the same instances
 * serving           the continuous-batching server on 2000 Poisson-arriving
@@ -148,11 +149,10 @@ def _swe_sim(ctx, scheme, n, args, math=None):
     return sim, dt
 
 
-# HBM bytes per cell of one full step as the algorithm needs them (fields read
-# once and written once per launch; the second RK2 stage of the unsplit KP07
-# also reads the output buffer), and launches per step
-STEP_BYTES = {"kp07": (48, 2), "hll2": (48, 2), "waf": (48, 2), "lxf": (24, 1), "hll": (24, 1), "force": (24, 1),
-              "kp07u": (60, 2), "ee2d": (64, 2)}
+# HBM bytes per cell of one full step as its launches need them (fields read
+# once and written once per launch), and launches per step
+STEP_BYTES = {"kp07": (24, 1), "hll2": (24, 1), "waf": (48, 2), "lxf": (24, 1), "hll": (24, 1), "force": (24, 1),
+              "kp07u": (24, 1), "ee2d": (64, 2), "ee2d_fast": (32, 1)}
 
 
 def _euler_sim(ctx, n, math=None):
@@ -186,7 +186,7 @@ def _measure(ctx, kind, args):
         n = args.n
         sim, dt = _swe_sim(ctx, scheme, n, args, math)
         steps = args.steps
-    step_bytes, per_step = STEP_BYTES[scheme]
+    step_bytes, per_step = STEP_BYTES.get(kind, STEP_BYTES[scheme])
     ms, wall = _time_steps(sim, dt, steps, args.warmup, ctx)
     steady = _steady_ms(sim, dt, 30 if scheme == "ee2d" else 100)
     out = sim.download()

@@ -43,9 +43,10 @@ inline bool step_grid_fits(const SubstepArgs& a) {
     return (w == BC_PERIODIC) == (e == BC_PERIODIC) && (s == BC_PERIODIC) == (n == BC_PERIODIC);
 }
 
-// Whether a dimensionally split step is.  Fast arithmetic only: the exact kernels and WAF are bound by VALU issue already as substeps
-// (4096^2: 184 us for KP07_dimsplit, 260 for WAF, against 79 us for their
-// bytes), so that the wider halo would cost more than the memory passes saved.
+// Whether a dimensionally split step is.  Fast arithmetic only: the exact kernels
+// and WAF are bound by VALU issue already as substeps (4096^2: 184 us for
+// KP07_dimsplit, 260 for WAF, against 79 us for their bytes), so that the wider
+// halo would cost more than the memory passes saved.
 inline bool step_is_fused(int scheme, int math, const SubstepArgs& a) {
     return math != FVMI_MATH_EXACT && scheme != SCHEME_WAF && step_grid_fits(a);
 }
@@ -56,6 +57,13 @@ inline bool step_is_fused(int scheme, int math, const SubstepArgs& a) {
 inline SegmentCost substep_cost(int math) {
     return {4, 2, math == FVMI_MATH_EXACT ? 0.5f : 0.25f, 0.005f};
 }
+// Percent of the equal segments' waves that the round-weighted split of a whole
+// step has to put to work.  8192^2 (24 of 27 segments a strip, 89 %), rounds and
+// equal segments, one simulator and three in turn: KP07_dimsplit 756 and 711 us,
+// 715 and 683, HLL2 949 and 883, 894 and 826, Euler 1239 and 1183, 1140 and 1049,
+// KP07 653 and 618, 621 and 622; 9500x7000 KP07_dimsplit 773 and 683; 7500^2 (93 %)
+// even; 5500^2 (98 %) 317 and 323.
+constexpr int kStepMinFill = 93;
 inline SegmentCost step_cost() { return {2 * kStepHalo, kStepMinSegRows, 0.45f, 0.01f}; }
 
 // Fills the decomposition fields of `a` (sub-area, launch shape, device size)
@@ -67,7 +75,7 @@ inline SegmentCost step_cost() { return {2 * kStepHalo, kStepMinSegRows, 0.45f, 
 //     `waves_per_simd` waves on every SIMD of the device (one more would run
 //     after all the others).
 inline int plan_substep(SubstepArgs& a, int cu_count, const SegmentCost& cost, bool round_ok = false,
-                        int waves_per_simd = 4, int min_part = 16) {
+                        int min_fill = 0, int waves_per_simd = 4, int min_part = 16) {
     const int wx = a.x1 - a.x0;
     a.rows_per_strip = a.y1 - a.y0;
     a.strips_x = (wx + a.strip_cols - 1) / a.strip_cols;
@@ -77,7 +85,7 @@ inline int plan_substep(SubstepArgs& a, int cu_count, const SegmentCost& cost, b
     a.gps = a.grows = 0;
     int gps = 0, grows = 0;
     if (round_ok && a.seg_rows <= 0 && a.xcd_remap &&
-        round_split_fits(a.strips_x, a.rows_per_strip, a.waves_per_block, cu_count, min_part, gps, grows)) {
+        round_split_fits(a.strips_x, a.rows_per_strip, a.waves_per_block, cu_count, min_part, min_fill, gps, grows)) {
         a.round_plan = 1;
         a.gps = gps;
         a.grows = grows;
@@ -87,7 +95,8 @@ inline int plan_substep(SubstepArgs& a, int cu_count, const SegmentCost& cost, b
         a.num_blocks = kRounds * cu_count;
         return a.num_blocks;
     }
-    if (a.seg_rows <= 0) a.seg_rows = balanced_segment_rows(a.rows_per_strip, a.strips_x, cu_count, waves_per_simd, cost);
+    if (a.seg_rows <= 0)
+        a.seg_rows = balanced_segment_rows(a.rows_per_strip, a.strips_x, cu_count, waves_per_simd, cost);
     a.segs_per_strip = (a.rows_per_strip + a.seg_rows - 1) / a.seg_rows;
     a.num_waves = a.strips_x * a.segs_per_strip;
     a.num_blocks = (a.num_waves + a.waves_per_block - 1) / a.waves_per_block;

@@ -1337,13 +1337,17 @@ __host__ __device__ inline bool round_segment_of(int block, int wave, int xcds, 
 }
 
 // Whether the round-weighted split fits: row groups (gps per strip, grows rows)
-// whose shortest part has at least `min_part` rows.
+// whose shortest part has at least `min_part` rows, and at least `min_fill` percent
+// of the waves that equal segments would have.  A group is a CU's, so that the
+// strips have to divide the CUs well: a whole step at 8192^2 gives 37 bands of
+// strips 6 groups each, 222 of 256 CUs.
 __host__ __device__ inline bool round_split_fits(int strips, int rows, int waves_per_block, int cu_count, int min_part,
-                                                 int& gps, int& grows) {
+                                                 int min_fill, int& gps, int& grows) {
     // one 4-wave workgroup per CU and round: a wave on every SIMD
     if (waves_per_block != 4 || cu_count <= 0 || cu_count % 8 != 0 || strips <= 0) return false;
     gps = cu_count / ((strips + waves_per_block - 1) / waves_per_block);
     if (gps <= 0) return false;
+    if (100LL * gps * kRounds < (long long)min_fill * (4 * kRounds * cu_count / strips)) return false;
     grows = (rows + gps - 1) / gps;
     const int last = rows - (gps - 1) * grows;  // the shortest (last) group
     return (last * kRoundWeights[kRounds - 1]) / kRoundWeightSum >= min_part;

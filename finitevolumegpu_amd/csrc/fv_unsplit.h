@@ -14,8 +14,9 @@
 // Work split and addressing as the dimensionally split kernel (fv_substep.h):
 // a wavefront owns a strip of 64 - 2*GC columns (lane c = padded column
 // 62*s + c for GC = 1, 60*s + c for GC = 2; the GC lanes at each edge are the
-// x halo), or for GC = 1 on large grids of 124 columns, two per lane, and marches down a segment of rows; x neighbours come through DPP
-// row moves, y neighbours from a register ring of rows.
+// x halo), or for GC = 1 on large grids of 124 columns, two per lane, and marches
+// down a segment of rows; x neighbours come through DPP row moves, y neighbours
+// from a register ring of rows.
 #pragma once
 
 #include "fv_substep.h"
@@ -585,7 +586,7 @@ inline int plan_unsplit(UnsplitArgs& a, int gc, int cu_count, bool round_ok, int
     a.gps = a.grows = 0;
     int gps = 0, grows = 0;
     if (round_ok && a.seg_rows <= 0 && a.xcd_remap &&
-        round_split_fits(a.strips_x, a.ny, a.waves_per_block, cu_count, min_part, gps, grows)) {
+        round_split_fits(a.strips_x, a.ny, a.waves_per_block, cu_count, min_part, 0, gps, grows)) {
         a.round_plan = 1;
         a.gps = gps;
         a.grows = grows;

@@ -407,7 +407,7 @@ SubstepArgs step_args(const fvmi_step_t* p, int nvars, int from, int step) {
 int plan_step(SubstepArgs& a, int cfl_slot, int cu_count) {
     a.cfl_slot = cfl_slot;
     a.strip_cols = strip_cols<1, kStepHalo>();
-    return plan_substep(a, cu_count, step_cost(), true);
+    return plan_substep(a, cu_count, step_cost(), true, kStepMinFill);
 }
 
 }  // namespace

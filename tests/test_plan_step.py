@@ -100,3 +100,16 @@ def test_equal_segments_fill_whole_waves_per_simd(scheme, math, strip, extra, nx
     assert waves <= 4 and rows >= min(least, ny)
     shorter = -(-band * -(-ny // max(rows - 1, 1)) // simds)
     assert shorter > waves or rows <= least or -(-ny // (rows - 1)) == -(-ny // rows)
+
+
+@pytest.mark.parametrize("nx,ny,rounds", [(4096, 4096, True), (5500, 5500, True), (8192, 8192, False),
+                                          (9500, 7000, False)])
+def test_rounds_only_where_the_strips_fill_the_device(nx, ny, rounds):
+    """The round-weighted split (parts in the ratio 14 : 6) where its row groups
+    put at least 93 % of the equal segments' waves to work."""
+    segs = plan(STEP, nx, ny)
+    counts = segs[(segs[:, 0] >= 0) & (segs[:, 1] + segs[:, 2] < ny), 2]
+    assert (counts.max() > 2 * counts.min()) == rounds
+    if not rounds:
+        assert len(np.unique(counts)) == 1
+        assert (segs[:, 0] >= 0).sum() > 0.95 * 4 * 1024
