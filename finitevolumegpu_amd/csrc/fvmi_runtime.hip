@@ -403,6 +403,15 @@ SubstepArgs step_args(const fvmi_step_t* p, int nvars, int from, int step) {
     return a;
 }
 
+// Whether launches on the stream are being recorded.  A recorded step has to end
+// in the buffer it began in, so that the graph can be replayed: it takes two
+// launches.
+bool is_capturing(void* stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    return stream != nullptr && hipStreamIsCapturing((hipStream_t)stream, &status) == hipSuccess &&
+           status == hipStreamCaptureStatusActive;
+}
+
 // Plans a launch of a whole step; returns its grid.
 int plan_step(SubstepArgs& a, int cfl_slot, int cu_count) {
     a.cfl_slot = cfl_slot;
@@ -718,7 +727,7 @@ int fvmi_dimsplit_step(const fvmi_step_t* p, const fvmi_launch_t* launch, int* s
     int math = 0;
     SubstepArgs a = step_args(p, nvars, 0, 0);
     if (int rc = check_substep(p->scheme, a, nvars, launch, &math)) return rc;
-    if (!step_is_fused(p->scheme, math, a)) {
+    if (!step_is_fused(p->scheme, math, a) || is_capturing(stream)) {
         if (int rc = run_substep(p->scheme, a, nvars, launch, stream)) return rc;
         SubstepArgs b = step_args(p, nvars, 1, 1);
         if (int rc = run_substep(p->scheme, b, nvars, launch, stream)) return rc;
@@ -741,7 +750,7 @@ int fvmi_swe_kp07_rk2_step(const fvmi_step_t* p, const fvmi_launch_t* launch, in
     int math = 0;
     SubstepArgs a = step_args(p, 3, 0, 0);
     if (int rc = check_substep(SCHEME_KP07, a, 3, launch, &math)) return rc;
-    if (math == FVMI_MATH_EXACT || !step_grid_fits(a)) {
+    if (math == FVMI_MATH_EXACT || !step_grid_fits(a) || is_capturing(stream)) {
         for (int stage = 0; stage < 2; ++stage) {
             const int slot = stage == 0 ? p->cfl_slot : 1 - p->cfl_slot;
             if (int rc = fvmi_swe_kp07_substep(

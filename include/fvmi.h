@@ -199,7 +199,9 @@ int fvmi_euler_kp07_dimsplit_substep(int nx, int ny, float dx, float dy, float d
  * The KP07_dimsplit, HLL2 and Euler steps in fast arithmetic are one launch
  * that reads and writes the state once (grids of at least 8 x 8 cells, no
  * Dirichlet edge, no periodic edge opposite to another kind, tile_rows 0 or at
- * least 4); every other step is the two substep launches.  The fields and the CFL minimum are the same either way.
+ * least 4); every other step is the two substep launches, and so is one that is
+ * being recorded for a graph, so that the graph ends in the buffer it begins in
+ * and can be replayed.  The fields and the CFL minimum are the same either way.
  *
  * cfl (may be NULL): two floats, of which slot `cfl_slot` holds +inf on entry.
  * On return the CFL minimum of the new state is in slot *cfl_slot_out and the

@@ -376,3 +376,32 @@ def test_unsplit_cfl_minimum_of_every_launch_shape(ctx, scheme):
             sim.step(np.float32(0.02))
             dts.add(sim.computeDt())
         assert len(dts) == 1 and 0.0 < dts.pop() < 1.0
+
+
+@pytest.mark.parametrize("scheme,math", [("kp07_dimsplit", "fast"), ("ee2d_kp07_dimsplit", "fast"), ("kp07", "fast"),
+                                         ("waf", "exact")])
+@pytest.mark.parametrize("steps", [1, 2])
+def test_recorded_steps_can_be_replayed(ctx, scheme, math, steps):
+    """A graph of a program's own recording (one step: an odd number) goes on from
+    its last replay, with eager work between."""
+    import ctypes
+    from finitevolumegpu_amd import _lib
+    nx, ny = 61, 34
+    fields = state(scheme, nx, ny, seed=5)
+    a, b = (make(ctx, scheme, fields, nx, ny, BOUNDARIES["channel"], math) for _ in range(2))
+    dt = np.float32(0.25 * a.computeDt())
+    for sim in (a, b):
+        sim.step(dt)
+    print("case replay", scheme, math, flush=True)
+    graph = ctypes.c_void_p()
+    _lib.call("fvmi_stream_begin_capture", a.stream.handle)
+    for _ in range(steps):
+        a.step(dt)
+    _lib.call("fvmi_stream_end_capture", a.stream.handle, ctypes.byref(graph))
+    for _ in range(4):
+        _lib.call("fvmi_graph_launch", graph, a.stream.handle)
+        for _ in range(steps):
+            b.step(dt)
+        assert all(np.array_equal(x, y) for x, y in zip(a.download(), b.download()))
+        assert a.computeDt() == b.computeDt()
+    _lib.call("fvmi_graph_destroy", graph)
