@@ -10,8 +10,9 @@ simulation time accumulated in double precision).
 
 ``DimsplitSimulator`` holds what the four scheme wrappers share
 (KP07_dimsplit.py:55-137 and its HLL2 / WAF / EE2D siblings): two padded states
-``u0``/``u1`` swapped after every substep, the device CFL slots, the initial
-CFL from the host arrays, and the ``substep(dt, i)`` launch with ``dt*0.5``.
+``u0``/``u1``, swapped after every substep or one-launch step, the device CFL
+slots, the initial CFL from the host arrays, the ``substep(dt, i)`` launch with
+``dt*0.5``, and the library calls for a whole step and for a run of steps.
 """
 
 import ctypes

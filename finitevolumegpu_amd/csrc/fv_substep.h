@@ -225,32 +225,10 @@ __device__ __forceinline__ int map_row(const RowMap& m, int k, unsigned& sign) {
     return __builtin_amdgcn_readfirstlane(row);
 }
 
-// Cross-lane moves: the value held by lane-1 / lane+1, as one DPP row move
-// (wave_shr:1 / wave_shl:1).  Lane 0 (resp. 63) receives 0; those lanes are
-// halo lanes whose results are never stored.
-__device__ __forceinline__ float from_left(float v) {
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x138, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float from_right(float v) {
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x130, 0xf, 0xf, true));
-}
-
-// the WafCell of lane+1
-__device__ __forceinline__ WafCell waf_shift_right(const WafCell& p) {
-    WafCell r;
-    r.h = from_right(p.h);
-    r.hu = from_right(p.hu);
-    r.hv = from_right(p.hv);
-    r.u = from_right(p.u);
-    r.v = from_right(p.v);
-    r.c = from_right(p.c);
-    r.ih = from_right(p.ih);
-    return r;
-}
-
-// Cross-lane operations on N values at once, as one run of DPP instructions: a
-// lone one among other VALU instructions costs several times its place in a
-// run (see FVMI_TRANS_RUN in fv_fast.h).  s_nop 1: a DPP operand that the
+// Cross-lane operations on N values at once (the value held by lane - 1 or
+// lane + 1: wave_shr:1, wave_shl:1), as one run of DPP instructions: a lone one
+// among other VALU instructions costs several times its place in a run (see
+// FVMI_TRANS_RUN in fv_math.h).  s_nop 1: a DPP operand that the
 // instruction before has written needs two wait states, which the compiler
 // does not see inside the block.  Lane 0 (63) takes 0 for its missing
 // neighbour.
