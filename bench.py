@@ -60,7 +60,7 @@ def _parse():
                     help="instances of the batched-ensemble leg (0 = skip the leg)")
     ap.add_argument("--serve", type=int, default=2000, help="requests of the serving leg (0 = skip the leg)")
     ap.add_argument("--serve-rate", type=float, default=300.0,
-                    help="Poisson arrival rate, requests/s (default just above the measured capacity, ~267/s)")
+                    help="Poisson arrival rate, requests/s (the measured capacity is ~340/s)")
     ap.add_argument("--sequential", type=int, default=-1,
                     help="requests of the sequential serving baseline (-1 = all; the first K by arrival)")
     return ap.parse_args()
