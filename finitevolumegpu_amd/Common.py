@@ -66,8 +66,44 @@ def _stream_handle(stream):
     return stream.handle if stream is not None else None
 
 
+class _DeviceMemory:
+    """A pitched device allocation, freed with its last holder."""
+
+    def __init__(self, row_bytes, rows):
+        ptr = ctypes.c_void_p()
+        pitch = ctypes.c_size_t()
+        _lib.call("fvmi_malloc_pitch", ctypes.byref(ptr), ctypes.byref(pitch), row_bytes, rows)
+        self.ptr = ptr
+        self.address = ptr.value  # 0 once freed
+        self.pitch = int(pitch.value)
+
+    def free(self):
+        if self.address and _lib._lib is not None:
+            _lib.lib().fvmi_free(self.ptr)
+            self.ptr = ctypes.c_void_p()
+            self.address = 0
+
+    def __del__(self):
+        if getattr(self, "address", None):
+            self.free()
+
+
+class Turn:
+    """Which of its two allocations each array of a pair of states holds (0 or 1).
+    A simulator turns it where a step leaves the new state in the allocations of
+    the other state, so that its arrays keep their roles."""
+
+    __slots__ = ("value",)
+
+    def __init__(self):
+        self.value = 0
+
+
 class HipArray2D:
-    """Pitched, zero-initialised 2-D float32 device buffer with ghost cells."""
+    """Pitched, zero-initialised 2-D float32 device buffer with ghost cells.
+
+    ``data_ptr`` and ``row_ptr`` are addresses as of now: an array of a
+    simulator's state may be in other memory after the next step."""
 
     def __init__(self, stream, nx, ny, x_halo, y_halo, cpu_data=None, dtype=np.float32):
         self.logger = logging.getLogger(__name__)
@@ -80,12 +116,9 @@ class HipArray2D:
         nx_halo = self.nx + 2 * self.x_halo
         ny_halo = self.ny + 2 * self.y_halo
         self.shape = (ny_halo, nx_halo)
-        ptr = ctypes.c_void_p()
-        pitch = ctypes.c_size_t()
-        _lib.call("fvmi_malloc_pitch", ctypes.byref(ptr), ctypes.byref(pitch), nx_halo * 4, ny_halo)
-        self.ptr = ptr
-        self.address = ptr.value  # 0 once freed
-        self.pitch = int(pitch.value)
+        memory = _DeviceMemory(nx_halo * 4, ny_halo)
+        self.memories = (memory, memory)  # by turn
+        self.turn = Turn()
         _lib.call("fvmi_fill_f32", self.ptr, self.pitch, nx_halo, ny_halo, 0.0, _stream_handle(stream))
         if cpu_data is None:
             return
@@ -102,6 +135,18 @@ class HipArray2D:
         self.upload(stream, cpu_data, extent=[x, y, cpu_data.shape[1], cpu_data.shape[0]])
         if stream is not None:
             stream.synchronize()
+
+    @property
+    def memory(self):
+        return self.memories[self.turn.value]
+
+    @property
+    def ptr(self):
+        return self.memory.ptr
+
+    @property
+    def pitch(self):
+        return self.memory.pitch
 
     @property
     def data_ptr(self):
@@ -148,13 +193,8 @@ class HipArray2D:
             stream.synchronize()
 
     def free(self):
-        if getattr(self, "ptr", None) is not None and self.ptr.value and _lib._lib is not None:
-            _lib.lib().fvmi_free(self.ptr)
-            self.ptr = ctypes.c_void_p()
-            self.address = 0
-
-    def __del__(self):
-        self.free()
+        if hasattr(self, "memories"):
+            self.memory.free()
 
 
 class ArakawaA2D:
@@ -173,6 +213,17 @@ class ArakawaA2D:
 
     def __len__(self):
         return len(self.gpu_variables)
+
+    def pair_with(self, other):
+        """Lets the arrays of two states of one shape exchange their memory; returns
+        the Turn that does it.  Both allocations of a variable live as long as
+        either of its arrays."""
+        turn = Turn()
+        for a, b in zip(self.gpu_variables, other.gpu_variables):
+            m, n = a.memory, b.memory
+            a.memories, b.memories = (m, n), (n, m)
+            a.turn = b.turn = turn
+        return turn
 
     def download(self, stream, variables=None):
         if variables is None:

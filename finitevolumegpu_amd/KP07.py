@@ -50,7 +50,7 @@ class KP07(UnsplitSimulator):
 
     def _take_step(self, in_other, slot):
         if in_other:
-            self.u0, self.u1 = self.u1, self.u0
+            self._turn_state()
         self.cfl_last = slot
 
     def _run_steps(self, t_end, max_steps):

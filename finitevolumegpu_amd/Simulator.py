@@ -10,9 +10,11 @@ simulation time accumulated in double precision).
 
 ``DimsplitSimulator`` holds what the four scheme wrappers share
 (KP07_dimsplit.py:55-137 and its HLL2 / WAF / EE2D siblings): two padded states
-``u0``/``u1``, swapped after every substep or one-launch step, the device CFL
-slots, the initial CFL from the host arrays, the ``substep(dt, i)`` launch with
-``dt*0.5``, and the library calls for a whole step and for a run of steps.
+``u0``/``u1``, swapped after every substep (a one-launch step exchanges their
+memory instead, so that ``u0`` stays the state's object as it does over two
+substeps), the device CFL slots, the initial CFL from the host arrays, the
+``substep(dt, i)`` launch with ``dt*0.5``, and the library calls for a whole step
+and for a run of steps.
 """
 
 import ctypes
@@ -139,6 +141,16 @@ class BaseSimulator:
         library call, where the simulator has one; returns whether it took any."""
         return False
 
+    def _turn_state(self):
+        """Exchanges the memory of u0 and u1 after a step that left the state in u1's
+        (also where a program has put arrays of its own into them)."""
+        turn = self.turn
+        for a, b in zip(self.u0.gpu_variables, self.u1.gpu_variables):
+            if a.turn is not turn or b.turn is not turn:
+                turn = self.turn = self.u0.pair_with(self.u1)
+                break
+        turn.value ^= 1
+
     def step(self, dt):
         """One full step of ``num_substeps`` substeps (Simulator.py:220-228)."""
         for i in range(self.num_substeps):
@@ -221,7 +233,8 @@ class _StepCall:
         self.time_ptr = ctypes.addressof(self.time)
 
     def _pack(self, sim, scheme, dt, boundary_conditions, cfl_slot):
-        u, v = sim.u0.gpu_variables, sim.u1.gpu_variables
+        u = [x.memories[x.turn.value] for x in sim.u0.gpu_variables]
+        v = [x.memories[x.turn.value] for x in sim.u1.gpu_variables]
         pad = (0,) * (4 - len(u))
         _lib.STEP_PACK.pack_into(
             self.args, 0, scheme, sim.nx, sim.ny, boundary_conditions, sim.dx, sim.dy, dt, sim.g,
@@ -309,6 +322,7 @@ class DimsplitSimulator(BaseSimulator):
         self.gc_y = 2
         self.u0 = Common.ArakawaA2D(self.stream, self.nx, self.ny, 2, 2, fields)
         self.u1 = Common.ArakawaA2D(self.stream, self.nx, self.ny, 2, 2, [None] * len(fields))
+        self.turn = self.u0.pair_with(self.u1)
         # Two-slot device CFL minimum (see fvmi.h): slot 0 = +inf, slot 1 = initial value.
         ptr = ctypes.c_void_p()
         _lib.call("fvmi_malloc", ctypes.byref(ptr), 8)
@@ -343,7 +357,7 @@ class DimsplitSimulator(BaseSimulator):
 
     def _take_step(self, in_other, slot):
         if in_other:
-            self.u0, self.u1 = self.u1, self.u0
+            self._turn_state()
         if self.cfl_pointer():
             self.cfl_last = slot
             self.cfl_free = 1 - slot
@@ -420,6 +434,7 @@ class UnsplitSimulator(BaseSimulator):
         self.gc_y = self.gc
         self.u0 = Common.ArakawaA2D(self.stream, self.nx, self.ny, self.gc, self.gc, fields)
         self.u1 = Common.ArakawaA2D(self.stream, self.nx, self.ny, self.gc, self.gc, [None] * len(fields))
+        self.turn = self.u0.pair_with(self.u1)
         ptr = ctypes.c_void_p()
         _lib.call("fvmi_malloc", ctypes.byref(ptr), 8)
         self.cfl_data = ptr

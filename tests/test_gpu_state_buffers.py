@@ -1,0 +1,86 @@
+"""Where a simulator's state is between steps, as a program sees it: objects that
+it holds, graphs that it recorded, ghost cells that it wrote and the table of an
+ensemble.  Two simulators of the same state, one through whole steps and one
+through its substeps, in which the state is back in its buffer after each step;
+their results are equal."""
+
+import numpy as np
+import pytest
+
+from oracle import fv_oracle as O
+from tests._cases import make_gpu_sim, state
+from tests.test_gpu_step import BOUNDARIES, make
+
+pytestmark = pytest.mark.gpu
+
+R, P, F, D = O.REFLECTIVE, O.PERIODIC, O.OUTFLOW, O.DIRICHLET
+
+# one launch a step, and two
+SCHEMES = [("kp07_dimsplit", "fast"), ("hll2", "fast"), ("ee2d_kp07_dimsplit", "fast"), ("kp07", "fast"),
+           ("waf", "exact")]
+DT = np.float32(2.0 ** -5)  # sums of a few are exact
+
+
+def pair(ctx, scheme, math="fast", bc="channel", nx=61, ny=34):
+    code = BOUNDARIES[bc] if isinstance(bc, str) else bc
+    fields = state(scheme, nx, ny, seed=5)
+    return [make(ctx, scheme, fields, nx, ny, code, math) for _ in range(2)]
+
+
+def by_substeps(sim, steps=1):
+    for _ in range(steps):
+        for i in range(2):
+            sim.substep(DT, i)
+
+
+def assert_same(a, b):
+    assert all(np.array_equal(x, y) for x, y in zip(a.download(), b.download()))
+    assert a.computeDt() == b.computeDt()
+
+
+@pytest.mark.parametrize("scheme,math", SCHEMES)
+@pytest.mark.parametrize("steps", [1, 2, 3])
+def test_held_state_stays_current(ctx, scheme, math, steps):
+    a, b = pair(ctx, scheme, math)
+    print("case held", scheme, math, steps, flush=True)
+    out, fields = a.getOutput(), list(a.getOutput().gpu_variables)
+    for advance in (lambda: [a.step(DT) for _ in range(steps)], lambda: a.simulate(float(steps * DT), DT)):
+        advance()
+        by_substeps(b, steps)
+        assert a.getOutput() is out and all(x is y for x, y in zip(out.gpu_variables, fields))
+        assert_same(a, b)
+        assert all(np.array_equal(x, f.download(a.stream)) for x, f in zip(b.download(), fields))
+
+
+def test_memory_outlives_the_simulator_with_either_field(ctx):
+    """Both buffers of a variable live as long as one of its arrays, since a
+    program's view of the array's memory may be of either."""
+    import gc
+    sim = pair(ctx, "kp07_dimsplit")[0]
+    held = sim.u0[0]
+    addresses = [held.data_ptr]
+    sim.step(DT)
+    addresses.append(held.data_ptr)
+    state_now = sim.download()[0]
+    sim.synchronize()
+    del sim
+    gc.collect()
+    others = pair(ctx, "kp07_dimsplit")  # would be given freed memory
+    assert not {x.data_ptr for s in others for u in (s.u0, s.u1) for x in u.gpu_variables} & set(addresses)
+    assert np.array_equal(held.download(others[0].stream), state_now)
+
+
+def test_arrays_that_a_program_put_into_a_state(ctx):
+    from finitevolumegpu_amd import Common
+    a, b = pair(ctx, "kp07_dimsplit")
+    a.step(DT)
+    by_substeps(b)
+    nx, ny = int(a.nx), int(a.ny)
+    print("case own arrays", flush=True)
+    a.u1 = Common.ArakawaA2D(a.stream, nx, ny, 2, 2, [None] * 3)
+    own = a.u0.gpu_variables[1] = Common.HipArray2D(a.stream, nx, ny, 2, 2, a.download()[1])
+    for _ in range(3):
+        a.step(DT)
+        by_substeps(b)
+        assert a.u0[1] is own
+        assert_same(a, b)
