@@ -53,6 +53,7 @@ class EE2D_KP07_dimsplit(DimsplitSimulator):
         dt = np.float32(dt)
         cfl = self.cfl_pointer()
         nx, ny = int(self.nx), int(self.ny)
+        self._note_recording()
         self._note_substep(substep)
         if external and internal:
             self._launch(dt, substep, self.u0, self.u1, cfl, 0, 0, nx, ny)

@@ -41,7 +41,7 @@ class KP07(UnsplitSimulator):
     def step(self, dt):
         """One full step; with two stages as one library call
         (fvmi_swe_kp07_rk2_step) with the results of the two substeps."""
-        if not self._whole_step or self.num_substeps != 2 or "substep" in self.__dict__:
+        if self._recorded or not self._whole_step or self.num_substeps != 2 or "substep" in self.__dict__:
             super().step(dt)
             return
         self._take_step(*self._step_call.step(self, 0, np.float32(dt), self.boundary_conditions, 1 - self.cfl_last))
@@ -51,11 +51,18 @@ class KP07(UnsplitSimulator):
     def _take_step(self, in_other, slot):
         if in_other:
             self._turn_state()
+        else:
+            self._note_recording()
         self.cfl_last = slot
 
     def _run_steps(self, t_end, max_steps):
-        return (self._whole_step and self.num_substeps == 2 and _steps_in_library(self)
+        self._note_recording()
+        return (not self._recorded and self._whole_step and self.num_substeps == 2 and _steps_in_library(self)
                 and self._step_call.run(self, 0, t_end, max_steps, 1 - self.cfl_last))
+
+    def substep(self, dt, step_number):
+        self._note_recording()
+        super().substep(dt, step_number)
 
     def substepRK(self, dt, substep):
         self.substep(dt, substep)

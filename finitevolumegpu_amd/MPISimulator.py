@@ -118,6 +118,7 @@ class MPISimulator(BaseSimulator):
     def full_exchange(self):
         """On-device exchange of the current state's ghost cells (MPISimulator.py:371-480)."""
         t0 = time.time()
+        self.sim._note_recording()
         state = self.sim.getOutput()
         ptrs = (ctypes.c_void_p * self.nvars)(*[state[k].data_ptr for k in range(self.nvars)])
         pitches = (ctypes.c_int * self.nvars)(*[state[k].pitch for k in range(self.nvars)])
@@ -132,7 +133,7 @@ class MPISimulator(BaseSimulator):
         the rank is its own neighbour) in place of the exchange between them;
         the exchange after the step fills the new state's ghost cells."""
         sim = self.sim
-        if (not isinstance(sim, DimsplitSimulator) or not sim._whole_step
+        if (not isinstance(sim, DimsplitSimulator) or sim._recorded or not sim._whole_step
                 or "substep" in sim.__dict__ or "substep" in self.__dict__ or "full_exchange" in self.__dict__
                 or type(self).substep is not MPISimulator.substep
                 or type(self).full_exchange is not MPISimulator.full_exchange):

@@ -81,6 +81,9 @@ class BoundaryCondition:
 class BaseSimulator:
     """Stepping loop and dt policy (Simulator.py:109-266)."""
 
+    # work on the state has been recorded for a graph (see _note_recording)
+    _recorded = False
+
     def __init__(self, context, nx, ny, dx, dy, boundary_conditions, cfl_scale, num_substeps,
                  block_width, block_height):
         self.logger = logging.getLogger(__name__ + "." + self.__class__.__name__)
@@ -140,6 +143,14 @@ class BaseSimulator:
         """Up to ``max_steps`` steps of length ``self.dt`` towards ``t_end`` in one
         library call, where the simulator has one; returns whether it took any."""
         return False
+
+    def _note_recording(self):
+        """A graph's replays read and write the buffers that its work was recorded
+        with.  From the first recording on, the steps of a simulator are therefore
+        two launches each, which leave the state in the buffer that it was in, as
+        the recorded ones do: replays and steps go on from each other."""
+        if not self._recorded and self.launch.math == _lib.FVMI_MATH_FAST and self.stream.capturing():
+            self._recorded = True
 
     def _turn_state(self):
         """Exchanges the memory of u0 and u1 after a step that left the state in u1's
@@ -343,7 +354,7 @@ class DimsplitSimulator(BaseSimulator):
     def step(self, dt):
         """One full step as one library call (fvmi_dimsplit_step), with the
         results of the two substeps of BaseSimulator.step."""
-        if not self._whole_step or self.num_substeps != 2 or "substep" in self.__dict__:
+        if self._recorded or not self._whole_step or self.num_substeps != 2 or "substep" in self.__dict__:
             super().step(dt)
             return
         self._step_both(dt, self.boundary_conditions)
@@ -358,18 +369,22 @@ class DimsplitSimulator(BaseSimulator):
     def _take_step(self, in_other, slot):
         if in_other:
             self._turn_state()
+        else:
+            self._note_recording()
         if self.cfl_pointer():
             self.cfl_last = slot
             self.cfl_free = 1 - slot
 
     def _run_steps(self, t_end, max_steps):
-        return (self._whole_step and self.num_substeps == 2 and _steps_in_library(self)
+        self._note_recording()
+        return (not self._recorded and self._whole_step and self.num_substeps == 2 and _steps_in_library(self)
                 and self._step_call.run(self, _lib.SCHEME_IDS[self.scheme], t_end, max_steps, self.cfl_free))
 
     def substep(self, dt, step_number):
         self.substepDimsplit(dt * 0.5, step_number)
 
     def substepDimsplit(self, dt, substep):
+        self._note_recording()
         self._launch(np.float32(dt), int(substep), self.u0, self.u1, self.cfl_pointer())
         self._note_substep(substep)
         self.u0, self.u1 = self.u1, self.u0

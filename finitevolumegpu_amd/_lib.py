@@ -151,6 +151,7 @@ SIGNATURES = {
     "fvmi_ensemble_step": (c_int, [c_int, c_void_p, c_void_p, c_void_p, c_int, P(LaunchConfig), c_void_p]),
     "fvmi_ensemble_count_active": (c_int, [c_void_p, c_int, c_void_p, c_void_p]),
     "fvmi_stream_begin_capture": (c_int, [c_void_p]),
+    "fvmi_stream_is_capturing": (c_int, [c_void_p, P(c_int)]),
     "fvmi_stream_end_capture": (c_int, [c_void_p, P(c_void_p)]),
     "fvmi_graph_launch": (c_int, [c_void_p, c_void_p]),
     "fvmi_graph_destroy": (c_int, [c_void_p]),

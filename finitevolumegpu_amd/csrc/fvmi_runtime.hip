@@ -984,6 +984,12 @@ int fvmi_stream_begin_capture(void* stream) {
     return FVMI_OK;
 }
 
+int fvmi_stream_is_capturing(void* stream, int* capturing) {
+    if (!capturing) return fail(FVMI_ERR_INVALID, "capturing is NULL");
+    *capturing = is_capturing(stream) ? 1 : 0;
+    return FVMI_OK;
+}
+
 int fvmi_stream_end_capture(void* stream, void** graph_exec) {
     if (!graph_exec) return fail(FVMI_ERR_INVALID, "graph_exec is NULL");
     hipGraph_t g = nullptr;

@@ -202,6 +202,9 @@ int fvmi_euler_kp07_dimsplit_substep(int nx, int ny, float dx, float dy, float d
  * least 4); every other step is the two substep launches, and so is one that is
  * being recorded for a graph, so that the graph ends in the buffer it begins in
  * and can be replayed.  The fields and the CFL minimum are the same either way.
+ * A caller who steps between replays has to find the state in the recorded buffer
+ * each time: it takes those steps with the substep entry points (the Python
+ * simulators do so from the first recording on).
  *
  * cfl (may be NULL): two floats, of which slot `cfl_slot` holds +inf on entry.
  * On return the CFL minimum of the new state is in slot *cfl_slot_out and the
@@ -375,6 +378,8 @@ int fvmi_ensemble_count_active(const fvmi_instance_t* table, int n, int* count_d
 
 /* ---- stream capture (hipGraph) -------------------------------------------- */
 int fvmi_stream_begin_capture(void* stream);
+/* Whether launches on the stream are being recorded for a graph, whoever began it. */
+int fvmi_stream_is_capturing(void* stream, int* capturing);
 /* Ends the capture and instantiates the graph. */
 int fvmi_stream_end_capture(void* stream, void** graph_exec);
 int fvmi_graph_launch(void* graph_exec, void* stream);

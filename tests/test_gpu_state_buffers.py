@@ -4,6 +4,8 @@ ensemble.  Two simulators of the same state, one through whole steps and one
 through its substeps, in which the state is back in its buffer after each step;
 their results are equal."""
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -84,3 +86,67 @@ def test_arrays_that_a_program_put_into_a_state(ctx):
         by_substeps(b)
         assert a.u0[1] is own
         assert_same(a, b)
+
+
+def record(sim, enqueue):
+    from finitevolumegpu_amd import _lib
+    graph = ctypes.c_void_p()
+    _lib.call("fvmi_stream_begin_capture", sim.stream.handle)
+    try:
+        enqueue()
+    finally:
+        _lib.call("fvmi_stream_end_capture", sim.stream.handle, ctypes.byref(graph))
+    return graph
+
+
+@pytest.mark.parametrize("how", ["step", "substep", "simulate"])
+@pytest.mark.parametrize("scheme,math", SCHEMES)
+def test_replays_and_eager_steps_in_turn(ctx, scheme, math, how):
+    """A recorded step goes on from the latest state, whatever was stepped
+    between its replays, and the other way round."""
+    from finitevolumegpu_amd import _lib
+    a, b = pair(ctx, scheme, math)
+    a.step(DT)  # an odd number of steps before the recording
+    by_substeps(b)
+    print("case replays in turn", scheme, math, how, flush=True)
+    graph = record(a, {"step": lambda: a.step(DT), "substep": lambda: by_substeps(a),
+                       "simulate": lambda: a.simulate(float(DT), DT)}[how])
+    for steps, run in ((1, 0), (0, 1), (0, 0), (3, 2), (2, 3), (1, 1)):
+        _lib.call("fvmi_graph_launch", graph, a.stream.handle)
+        by_substeps(b)
+        assert_same(a, b)
+        for _ in range(steps):
+            a.step(DT)
+        by_substeps(b, steps)
+        assert_same(a, b)
+        a.simulate(float(run * DT), DT)
+        by_substeps(b, run)
+        assert_same(a, b)
+    _lib.call("fvmi_graph_destroy", graph)
+
+
+@pytest.mark.parametrize("how", ["step", "exchange"])
+@pytest.mark.parametrize("math", ["fast", "exact"])
+def test_mpi_replays_and_eager_steps_in_turn(ctx, math, how):
+    from finitevolumegpu_amd import _lib
+    from finitevolumegpu_amd.MPISimulator import MPISimulator
+    a, b = (MPISimulator(s) for s in pair(ctx, "ee2d_kp07_dimsplit", math))
+    a.step(DT)
+    by_substeps(b)
+    print("case mpi replays", math, how, flush=True)
+    graph = record(a, (lambda: a.step(DT)) if how == "step" else a.full_exchange)
+    for steps in (1, 0, 3, 2):
+        _lib.call("fvmi_graph_launch", graph, a.stream.handle)
+        if how == "step":
+            by_substeps(b)
+        else:
+            b.full_exchange()
+        for _ in range(steps):
+            a.step(DT)
+        by_substeps(b, steps)
+        assert_same(a, b)
+        nx, ny = int(a.nx), int(a.ny)
+        padded = [[v.download(s.stream, extent=[0, 0, nx + 4, ny + 4]) for v in s.getOutput().gpu_variables]
+                  for s in (a, b)]
+        assert all(np.array_equal(x, y) for x, y in zip(*padded))
+    _lib.call("fvmi_graph_destroy", graph)
