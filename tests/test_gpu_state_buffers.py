@@ -150,3 +150,31 @@ def test_mpi_replays_and_eager_steps_in_turn(ctx, math, how):
                   for s in (a, b)]
         assert all(np.array_equal(x, y) for x, y in zip(*padded))
     _lib.call("fvmi_graph_destroy", graph)
+
+
+def write_ghosts(sim, seed):
+    """Ghost cells of both buffers, others in each, around their interiors."""
+    rng = np.random.default_rng(seed)
+    ny, nx = sim.download()[0].shape
+    for buf in (sim.u0, sim.u1):
+        for k, v in enumerate(buf.gpu_variables):
+            pad = (np.array([1.05, 0.01, -0.01, 6.5])[k] * rng.uniform(0.9, 1.1, (ny + 4, nx + 4))).astype(np.float32)
+            pad[2:-2, 2:-2] = v.download(sim.stream)
+            v.upload(sim.stream, pad, extent=[0, 0, nx + 4, ny + 4])
+
+
+@pytest.mark.parametrize("math", ["fast", "exact"])
+@pytest.mark.parametrize("edges", [(D, D, P, P), (P, P, D, R), (F, D, P, P)])
+def test_mpi_step_with_a_dirichlet_edge(ctx, math, edges):
+    """Beside an exchanged edge, the corners of a Dirichlet edge are memory that
+    the exchange does not write."""
+    from finitevolumegpu_amd.MPISimulator import MPISimulator
+    sims = []
+    for sim in pair(ctx, "ee2d_kp07_dimsplit", math, O.pack_bc(*edges)):
+        write_ghosts(sim, seed=9)
+        sims.append(MPISimulator(sim))
+    print("case mpi dirichlet", math, edges, flush=True)
+    for _ in range(3):
+        sims[0].step(DT)
+        by_substeps(sims[1])
+        assert_same(*sims)
