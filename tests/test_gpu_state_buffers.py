@@ -178,3 +178,24 @@ def test_mpi_step_with_a_dirichlet_edge(ctx, math, edges):
         sims[0].step(DT)
         by_substeps(sims[1])
         assert_same(*sims)
+
+
+@pytest.mark.parametrize("scheme", ["kp07_dimsplit", "ee2d_kp07_dimsplit", "kp07"])
+@pytest.mark.parametrize("before", [1, 2, 3])
+def test_ghost_cells_written_before_a_dirichlet_edge(ctx, scheme, before):
+    """A substep under Dirichlet edges reads the ghost cells that its input
+    buffer was given, also those given while other edges were in force."""
+    from finitevolumegpu_amd.Simulator import BoundaryCondition
+    a, b = pair(ctx, scheme)
+    print("case ghosts", scheme, before, flush=True)
+    for sim in (a, b):
+        write_ghosts(sim, seed=3)
+    for _ in range(before):
+        a.step(DT)
+    by_substeps(b, before)
+    for sim in (a, b):
+        sim.setBoundaryConditions(BoundaryCondition(BoundaryCondition.getTypes(O.pack_bc(D, D, R, D))))
+    for _ in range(3):
+        a.step(DT)
+        by_substeps(b)
+        assert_same(a, b)
