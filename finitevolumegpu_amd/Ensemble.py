@@ -281,7 +281,6 @@ class Ensemble:
         self.planned_active = None
         # whole steps in one launch; decided with each plan (_choose_steps)
         self.whole_steps = False
-        self.table_fresh = True  # the host copy holds the device's times, steps and buffers
         self._sync()
 
     # ------------------------------------------------------------------
@@ -352,10 +351,10 @@ class Ensemble:
         _lib.call("fvmi_memcpy_async", ctypes.addressof(self.host_table), self.table,
                   ctypes.sizeof(self.host_table), _lib.MEMCPY_DTOH, self.stream.handle)
         self._sync()
-        self.table_fresh = True
 
     def _state(self, i, k):
-        """Address of variable k of instance i's current state (fresh table)."""
+        """Address of variable k of instance i's current state (after
+        _refresh_buffers)."""
         I = self.host_table[i]
         return I.field[I.cur & 1][k]
 
@@ -540,7 +539,6 @@ class Ensemble:
             self.plan(self._running())
         if self.num_segs == 0:
             return self.count_active() if wait else None
-        self.table_fresh = False
         if self.use_graph:
             if self.graph is None:
                 self._capture()
@@ -571,8 +569,9 @@ class Ensemble:
         return self.host_table[i].t, self.host_table[i].nt
 
     def _refresh_buffers(self):
-        """Makes the host copy's ``cur`` the device's (substeps never change it)."""
-        if self.whole_steps and not self.table_fresh:
+        """Makes the host copy's ``cur`` the device's, which any launch on the table
+        may have turned, a program's own replay too (substeps never do)."""
+        if self.whole_steps:
             self._download_table()
 
     def download(self, i):

@@ -199,3 +199,27 @@ def test_ghost_cells_written_before_a_dirichlet_edge(ctx, scheme, before):
         a.step(DT)
         by_substeps(b)
         assert_same(a, b)
+
+
+@pytest.mark.parametrize("steps", [1, 2])
+def test_ensemble_after_replays_of_a_recorded_block(ctx, steps):
+    """download() and nonfinite_counts() show the state after a program's own
+    replays of a block that it recorded."""
+    from finitevolumegpu_amd import _lib
+    from finitevolumegpu_amd.Ensemble import Ensemble
+    nx, ny = 57, 33
+    fields = state("kp07_dimsplit", nx, ny, 3)
+    spec = {"fields": fields, "nx": nx, "ny": ny, "dx": 1.0, "dy": 1.0, "g": 9.81, "t_end": 1e9,
+            "bc": BOUNDARIES["reflective"], "dt": float(DT)}
+    ens = Ensemble(ctx, "kp07_dimsplit", [spec], steps_per_graph=steps, use_graph=False)
+    sim = make_gpu_sim(ctx, "kp07_dimsplit", fields, nx, ny, 1.0, 1.0, BOUNDARIES["reflective"])
+    ens.advance()
+    by_substeps(sim, steps)
+    print("case ensemble replays", steps, flush=True)
+    graph = record(ens, lambda: ens.advance(wait=False))
+    for _ in range(3):
+        _lib.call("fvmi_graph_launch", graph, ens.stream.handle)
+        by_substeps(sim, steps)
+        assert all(np.array_equal(x, y) for x, y in zip(ens.download(0), sim.download()))
+    _lib.call("fvmi_graph_destroy", graph)
+    ens.close()
