@@ -5,7 +5,7 @@ GPUSimulators/cuda/SWE2D_KP07.cu)."""
 import numpy as np
 
 from . import _lib
-from .Simulator import (BoundaryCondition, UnsplitSimulator, _library_methods, _StepCall, _steps_in_library,
+from .Simulator import (BoundaryCondition, UnsplitSimulator, _StepCall, _steps_in_library, _SubstepMethods,
                         swe_initial_cfl)
 
 
@@ -21,6 +21,7 @@ class KP07(UnsplitSimulator):
     scheme = "kp07"
     gc = 2
     nvars = 3
+    _substep_methods = _SubstepMethods("substep", "_launch", "_field_args", "cfl_pointer")
 
     def __init__(self, context, h0, hu0, hv0, nx, ny, dx, dy, g, theta=1.3, cfl_scale=0.9, order=2,
                  boundary_conditions=BoundaryCondition(), block_width=16, block_height=16,
@@ -34,14 +35,14 @@ class KP07(UnsplitSimulator):
         self.dt_factor = 0.5 ** (order - 1)
         self._init_unsplit([h0, hu0, hv0], swe_initial_cfl(h0, hu0, hv0, self.dx, self.dy, g),
                            tile_rows, waves_per_block, math, xcd_remap)
-        # a second-order step is one library call unless a subclass brings its own substeps
+        # a second-order step is one library call
         self._step_call = _StepCall("fvmi_swe_kp07_rk2_step", _lib.RUN_KP07_RK2)
-        self._whole_step = order == 2 and _library_methods(self, ("substep", "_launch", "_field_args", "cfl_pointer"))
+        self._library = self._substep_methods.library(self) if order == 2 else None
 
     def step(self, dt):
         """One full step; with two stages as one library call
         (fvmi_swe_kp07_rk2_step) with the results of the two substeps."""
-        if self._recorded or not self._whole_step or self.num_substeps != 2 or "substep" in self.__dict__:
+        if not self._one_call():
             super().step(dt)
             return
         self._take_step(*self._step_call.step(self, 0, np.float32(dt), self.boundary_conditions, 1 - self.cfl_last))
@@ -57,7 +58,7 @@ class KP07(UnsplitSimulator):
 
     def _run_steps(self, t_end, max_steps):
         self._note_recording()
-        return (not self._recorded and self._whole_step and self.num_substeps == 2 and _steps_in_library(self)
+        return (self._one_call() and _steps_in_library(self)
                 and self._step_call.run(self, 0, t_end, max_steps, 1 - self.cfl_last))
 
     def substep(self, dt, step_number):

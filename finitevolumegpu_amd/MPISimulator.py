@@ -21,7 +21,7 @@ import time
 import numpy as np
 
 from . import _lib
-from .Simulator import BaseSimulator, BoundaryCondition, DimsplitSimulator
+from .Simulator import BaseSimulator, BoundaryCondition, DimsplitSimulator, _library_methods
 
 
 class SingleRankComm:
@@ -135,10 +135,9 @@ class MPISimulator(BaseSimulator):
         Dirichlet edge that is not exchanged: the corners between it and an
         exchanged edge are memory that no exchange writes."""
         sim = self.sim
-        if (not isinstance(sim, DimsplitSimulator) or sim._recorded or not sim._whole_step
-                or "substep" in sim.__dict__ or "substep" in self.__dict__ or "full_exchange" in self.__dict__
-                or type(self).substep is not MPISimulator.substep
-                or type(self).full_exchange is not MPISimulator.full_exchange):
+        own = ("substep", "full_exchange")
+        if (not isinstance(sim, DimsplitSimulator) or not sim._one_call() or not self.__dict__.keys().isdisjoint(own)
+                or not _library_methods(self, own)):
             super().step(dt)
             return
         t0 = time.time()

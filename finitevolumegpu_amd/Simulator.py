@@ -19,6 +19,7 @@ and for a run of steps.
 
 import ctypes
 import logging
+import operator
 from enum import IntEnum
 
 import numpy as np
@@ -162,6 +163,11 @@ class BaseSimulator:
                 break
         turn.value ^= 1
 
+    def _one_call(self):
+        """Whether a full step of two substeps may be one call of the library."""
+        return (not self._recorded and self.num_substeps == 2
+                and self._substep_methods.unchanged(self, self._library))
+
     def _return_state(self):
         """After an odd number of one-launch steps, copies the state back into the
         memory that two launches a step would have it in: under Dirichlet edges each
@@ -300,11 +306,6 @@ class _StepCall:
         return self.out[2] > 0
 
 
-# Methods that take part in a step and that a subclass, an instance or a
-# wrapper may replace: with its own version the simulator steps through it.
-_STEP_METHODS = ("step", "substep", "_launch", "_field_args", "cfl_pointer", "simTime", "simSteps")
-
-
 def _of_package(function):
     """Whether the code of ``function`` is the package's own (a wrapper may carry
     the name and module of what it wraps, so these do not tell)."""
@@ -317,10 +318,34 @@ def _library_methods(sim, names):
     return all(_of_package(getattr(type(sim), name)) for name in names)
 
 
+class _SubstepMethods:
+    """The methods between ``step`` and the launches of a simulator, any of which a
+    subclass, a wrapper on the class or the simulator itself may replace, before or
+    after the simulator was made: with a version that is not the package's own, the
+    step goes through them."""
+
+    def __init__(self, *names):
+        self.names = names
+        self._of_class = operator.attrgetter(*names)
+
+    def library(self, sim):
+        """The methods of the class of ``sim`` if they are the package's own, else None."""
+        return self._of_class(type(sim)) if _library_methods(sim, self.names) else None
+
+    def unchanged(self, sim, library):
+        """Whether they are still those that ``library`` gave; asked at every step."""
+        return (library is not None and self._of_class(type(sim)) == library
+                and sim.__dict__.keys().isdisjoint(self.names))
+
+
+# what simulate() calls besides, once a step
+_LOOP_METHODS = ("step", "simTime", "simSteps")
+
+
 def _steps_in_library(sim):
     """Whether nothing stands between the steps of ``simulate``, progress
     reports of a program's own included."""
-    return (sim.__dict__.keys().isdisjoint(_STEP_METHODS) and _library_methods(sim, _STEP_METHODS)
+    return (sim.__dict__.keys().isdisjoint(_LOOP_METHODS) and _library_methods(sim, _LOOP_METHODS)
             and _of_package(Common.ProgressPrinter.getPrintString))
 
 
@@ -331,6 +356,7 @@ class DimsplitSimulator(BaseSimulator):
     nvars = 3
     # default launch shape when neither the caller nor the autotuner gives one
     default_waves_per_block = 4
+    _substep_methods = _SubstepMethods("substep", "substepDimsplit", "_launch", "_field_args", "cfl_pointer")
 
     def _init_dimsplit(self, fields, cfl_host, tile_rows, waves_per_block, math, xcd_remap):
         if self.context.autotuner is not None and tile_rows is None and waves_per_block is None:
@@ -360,9 +386,7 @@ class DimsplitSimulator(BaseSimulator):
         _lib.call("fvmi_memcpy_async", self.cfl_data, init.ctypes.data, 8, _lib.MEMCPY_HTOD, self.stream.handle)
         self.stream.synchronize()
         self._step_call = _StepCall("fvmi_dimsplit_step", _lib.RUN_DIMSPLIT)
-        # step() is one library call unless a subclass brings its own substeps
-        self._whole_step = _library_methods(self, ("substep", "substepDimsplit", "_launch", "_field_args",
-                                                   "cfl_pointer"))
+        self._library = self._substep_methods.library(self)
 
     def cfl_pointer(self):
         return self.cfl_data.value
@@ -370,7 +394,7 @@ class DimsplitSimulator(BaseSimulator):
     def step(self, dt):
         """One full step as one library call (fvmi_dimsplit_step), with the
         results of the two substeps of BaseSimulator.step."""
-        if self._recorded or not self._whole_step or self.num_substeps != 2 or "substep" in self.__dict__:
+        if not self._one_call():
             super().step(dt)
             return
         self._step_both(dt, self.boundary_conditions)
@@ -393,7 +417,7 @@ class DimsplitSimulator(BaseSimulator):
 
     def _run_steps(self, t_end, max_steps):
         self._note_recording()
-        return (not self._recorded and self._whole_step and self.num_substeps == 2 and _steps_in_library(self)
+        return (self._one_call() and _steps_in_library(self)
                 and self._step_call.run(self, _lib.SCHEME_IDS[self.scheme], t_end, max_steps, self.cfl_free))
 
     def substep(self, dt, step_number):
