@@ -520,6 +520,7 @@ class Ensemble:
 
     def _drop_graph(self):
         if self.graph is not None:
+            self._sync()  # a launch of it may still run
             _lib.call("fvmi_graph_destroy", self.graph)
             self.graph = None
 
@@ -625,11 +626,11 @@ class Ensemble:
         return int((self.tab["nx"][m].astype(np.int64) * self.tab["ny"][m] * self.tab["nt"][m]).sum())
 
     def close(self):
+        if getattr(self, "stream", None) is not None:
+            self.stream.synchronize()
         if getattr(self, "graph", None) is not None:
             _lib.lib().fvmi_graph_destroy(self.graph)
             self.graph = None
-        if getattr(self, "stream", None) is not None:
-            self.stream.synchronize()
         for p in ("segs_dev", "nsegs_dev", "table", "count_dev", "stats_dev"):
             ptr = getattr(self, p, None)
             if ptr is not None and ptr.value:
