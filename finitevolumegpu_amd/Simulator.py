@@ -111,7 +111,9 @@ class BaseSimulator:
         return "{:s} [{:d}x{:d}]".format(self.__class__.__name__, int(self.nx), int(self.ny))
 
     def simulate(self, t, dt=None):
-        """Advances ``t`` time units (Simulator.py:176-217)."""
+        """Advances ``t`` time units (Simulator.py:176-217).  The progress printer,
+        and check() with it, is asked after each step or each library call of
+        several (_run_steps)."""
         printer = Common.ProgressPrinter(t)
         t_start = self.simTime()
         t_end = t_start + t
@@ -284,7 +286,9 @@ class _StepCall:
     def run(self, sim, scheme, t_end, max_steps, cfl_slot):
         """Steps of length sim.dt from sim.t towards ``t_end``; brings the
         simulator's time, step count and state up to date with the steps taken,
-        also where one of them fails, and returns whether there was any.
+        also where one of them fails, and returns whether there was any.  At most
+        2^27 cells (1 to 2 ms of work) in one call, so that progress is reported as
+        often as by single steps.
 
         Only for times in double precision: float32 ones are compared and
         subtracted as such by the loop in Python, and that stays so.  Host time of
@@ -292,6 +296,7 @@ class _StepCall:
         turn 1909 -> 1782 us each, which then wait for the device."""
         if not (isinstance(t_end, float) and isinstance(sim.t, float) and isinstance(sim.dt, (float, np.float32))):
             return False
+        max_steps = min(max_steps, max(1, 2 ** 27 // (int(sim.nx) * int(sim.ny))))
         self._pack(sim, scheme, 0.0, sim.boundary_conditions, cfl_slot)
         self.time.value = sim.t
         self.out[2] = 0
