@@ -296,7 +296,7 @@ class _StepCall:
         turn 1909 -> 1782 us each, which then wait for the device."""
         if not (isinstance(t_end, float) and isinstance(sim.t, float) and isinstance(sim.dt, (float, np.float32))):
             return False
-        max_steps = min(max_steps, max(1, 2 ** 27 // (int(sim.nx) * int(sim.ny))))
+        max_steps = min(max_steps, max(1, 2 ** 27 // max(1, int(sim.nx) * int(sim.ny))))
         self._pack(sim, scheme, 0.0, sim.boundary_conditions, cfl_slot)
         self.time.value = sim.t
         self.out[2] = 0

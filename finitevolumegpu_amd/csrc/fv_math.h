@@ -67,18 +67,24 @@ FVMI_TRANS_RUN(sqrt_all, __builtin_amdgcn_sqrtf, "v_sqrt_f32")
 //    from -0 into +0: div_rn puts it back with one v_bfi (the sign of a zero
 //    reaches copysign in the WAF limiter), quot_rn leaves it (no other scheme
 //    reads a zero's sign, and its values are equal either way);
-//  * square root: s = x y with y = v_rsq_f32(x), and s + (x - s^2) y/2 with
-//    both products in FMAs.  The argument of v_rsq is x + 2^-126, x itself for
-//    every x above 2^-101, so that the square root of a zero is zero.
+//  * square root: v_sqrt_f32 (1 ulp) and its two neighbours, the one whose
+//    residual x - s s' changes sign chosen by two FMAs (exact from x = 2^-101 on,
+//    within 2 ulp below; 0 and infinity give themselves).  Newton's correction
+//    s + (x - s^2) y/2 from y = v_rsq_f32(x) takes 6 instructions for 9 and equals
+//    it from 2^-101 up to the largest finite number only: y is infinite at 0, the
+//    residual underflows below, and infinity gives NaN.  A branch to the
+//    compiler's sequence for those cost small grids more than the neighbours do
+//    (a step of one simulator: WAF 1023x777 48.1 us without it, 50.3 with the
+//    neighbours, 52.6 with the branch, KP07 2048x1500 68.6, 72.3 and 77.8; three
+//    simulators in turn, WAF 4096^2 476, 486 and 472, Euler 8192^2 1800, 1824 and
+//    1824).
 // Checked against the IEEE sequences on every mantissa of [1, 2) (reciprocal)
 // and [1, 4) (square root) and on random quotients, and in every exact-
 // arithmetic test, which compare the fields with the float32 oracle for
 // equality.  The exact kernels are bound by VALU issue, so their time follows
-// the instruction count: with the quotient at 6 and the square root at 6
-// instructions (8 and 9 before, signs and neighbours chosen by compares) and
-// the limiter of minmod_slope, KP07_dimsplit went from 480 to 343
-// instructions a row and from 222 to 184 us per 4096^2 substep, HLL2 from 274
-// to 219, Euler from 275 to 231 and WAF (no limited slopes) from 315 to 298.
+// the instruction count: with the quotient at 6 instructions (8 before, its sign
+// chosen by a compare) and the limiter of minmod_slope, KP07_dimsplit has 358
+// instructions a row (480 before).
 __device__ __forceinline__ float rcp_rn(float b) {
     const float y = __builtin_amdgcn_rcpf(b);
     return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
@@ -94,11 +100,14 @@ __device__ __forceinline__ float div_rn(float a, float b, float y) {
 }
 __device__ __forceinline__ float quot_rn(float a, float b) { return quot_rn(a, b, rcp_rn(b)); }
 __device__ __forceinline__ float div_rn(float a, float b) { return div_rn(a, b, rcp_rn(b)); }
-__device__ __forceinline__ float sqrt_rn(float x) {
-    const float y = __builtin_amdgcn_rsqf(x + 0x1p-126f);
-    const float s = x * y;
-    return __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
+// the square root of x from s = v_sqrt_f32(x)
+__device__ __forceinline__ float sqrt_rn(float x, float s) {
+    const float dn = __uint_as_float(__float_as_uint(s) - 1u);
+    const float up = __uint_as_float(__float_as_uint(s) + 1u);
+    const float r = (__builtin_fmaf(-dn, s, x) <= 0.0f) ? dn : s;
+    return (__builtin_fmaf(-up, s, x) > 0.0f) ? up : r;
 }
+__device__ __forceinline__ float sqrt_rn(float x) { return sqrt_rn(x, __builtin_amdgcn_sqrtf(x)); }
 // the same of N values, their v_rcp / v_rsq in one run
 template <int N>
 __device__ __forceinline__ void rcp_rn_all(const float (&b)[N], float (&r)[N]) {
@@ -109,15 +118,10 @@ __device__ __forceinline__ void rcp_rn_all(const float (&b)[N], float (&r)[N]) {
 }
 template <int N>
 __device__ __forceinline__ void sqrt_rn_all(const float (&x)[N], float (&r)[N]) {
-    float b[N], y[N];
+    float s[N];
+    sqrt_all<N>(x, s);
 #pragma unroll
-    for (int i = 0; i < N; ++i) b[i] = x[i] + 0x1p-126f;
-    rsq_all<N>(b, y);
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        const float s = x[i] * y[i];
-        r[i] = __builtin_fmaf(__builtin_fmaf(-s, s, x[i]), 0.5f * y[i], s);
-    }
+    for (int i = 0; i < N; ++i) r[i] = sqrt_rn(x[i], s[i]);
 }
 
 struct MathExact {
