@@ -158,7 +158,9 @@ __device__ __forceinline__ AxisMap map_axis_gc(int k, int n, int bc_lo, int bc_h
         if (bc_lo == BC_PERIODIC) return {k + n, false};
         if (bc_lo == BC_REFLECTIVE) return {2 * GC - 1 - k, true};
         if (bc_lo == BC_OUTFLOW) return {GC, false};
-        return {k, false};
+        // the two columns before a strip that starts at padded column 0 (u_first_col
+        // in fv_unsplit.h) read those after it
+        return {k < 0 ? k + 2 * GC : k, false};
     }
     if (k >= n + GC) {
         const int k_max = n + 2 * GC - 1 + (Deep && bc_hi == BC_PERIODIC ? 2 : 0);
