@@ -105,6 +105,22 @@ inline int plan_substep(SubstepArgs& a, int cu_count, const SegmentCost& cost, b
     return grid;
 }
 
+// The plan of a whole step.  Equal segments of a large grid fill the device once,
+// so that a lone launch ends with SIMDs at one wave; for Euler, whose rows cost most,
+// segments above this length are halved.  One simulator, and three in turn, as they
+// are, halved, and the two substep launches: 7300^2 920, 872 and 907 us, 835, 855
+// and 953; 8192^2 1180, 1117 and 1134, 1061, 1110 and 1227; 10000^2 1783, 1658 and
+// 1684, 1561, 1583 and 1846.  KP07_dimsplit and HLL2 8192^2 gain 2 and 3 % alone and
+// lose 4 and 2 % in turn: theirs stay.
+constexpr int kEulerMaxRows = 200;
+inline int plan_whole_step(SubstepArgs& a, int scheme, int cu_count) {
+    const bool chosen = a.seg_rows <= 0;
+    const int grid = plan_substep(a, cu_count, step_cost(), true, kStepMinFill);
+    if (!chosen || scheme != SCHEME_EULER || a.round_plan || a.seg_rows <= kEulerMaxRows) return grid;
+    a.seg_rows = (a.seg_rows + 1) / 2;
+    return plan_substep(a, cu_count, step_cost());
+}
+
 inline unsigned substep_lds(const SubstepArgs& a) {
     return block_cfl_bytes(block_cfl(a.round_plan, a.step == 1 ? a.cfl : nullptr));
 }

@@ -413,10 +413,10 @@ bool is_capturing(void* stream) {
 }
 
 // Plans a launch of a whole step; returns its grid.
-int plan_step(SubstepArgs& a, int cfl_slot, int cu_count) {
+int plan_step(SubstepArgs& a, int scheme, int cfl_slot, int cu_count) {
     a.cfl_slot = cfl_slot;
     a.strip_cols = strip_cols<1, kStepHalo>();
-    return plan_substep(a, cu_count, step_cost(), true, kStepMinFill);
+    return plan_whole_step(a, scheme, cu_count);
 }
 
 }  // namespace
@@ -735,7 +735,7 @@ int fvmi_dimsplit_step(const fvmi_step_t* p, const fvmi_launch_t* launch, int* s
         *cfl_slot_out = 1;
         return FVMI_OK;
     }
-    const int grid = plan_step(a, p->cfl_slot, current_cu_count());
+    const int grid = plan_step(a, p->scheme, p->cfl_slot, current_cu_count());
     hipError_t e = launch_step_fast(p->scheme, a, grid, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "step launch");
     *state_out = 1;
@@ -765,7 +765,7 @@ int fvmi_swe_kp07_rk2_step(const fvmi_step_t* p, const fvmi_launch_t* launch, in
         *cfl_slot_out = 1 - p->cfl_slot;
         return FVMI_OK;
     }
-    const int grid = plan_step(a, p->cfl_slot, current_cu_count());
+    const int grid = plan_step(a, SCHEME_KP07, p->cfl_slot, current_cu_count());
     hipError_t e = launch_rk2_step(a, grid, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "step launch");
     *state_out = 1;
@@ -871,7 +871,7 @@ int fvmi_ensemble_prepare(fvmi_instance_t* table, int n, void* stream) {
 
 int fvmi_substep_plan(int scheme, int nx, int ny, int x0, int y0, int x1, int y1, const fvmi_launch_t* launch,
                       int cu_count, int* segs, int max_waves, int* n_waves) {
-    const bool two_columns = scheme >= 12 && scheme <= 14, whole_step = scheme == 16;
+    const bool two_columns = scheme >= 12 && scheme <= 14, whole_step = scheme == 16 || scheme == 16 + SCHEME_EULER;
     if (two_columns) scheme -= 8;
     if (!whole_step && (scheme < SCHEME_KP07 || scheme > SCHEME_EULER + 4))
         return fail(FVMI_ERR_INVALID, "unknown scheme %d", scheme);
@@ -915,7 +915,7 @@ int fvmi_substep_plan(int scheme, int nx, int ny, int x0, int y0, int x1, int y1
     int math = 0;
     if (int rc = fill_launch(launch, a, &math)) return rc;
     a.strip_cols = whole_step ? strip_cols<1, kStepHalo>() : scheme_strip_cols(scheme, math);
-    const int grid = whole_step ? plan_step(a, 0, cu_count)
+    const int grid = whole_step ? plan_step(a, scheme - 16, 0, cu_count)
                                 : plan_substep(a, cu_count, substep_cost(math), scheme != SCHEME_WAF);
     const long long total = (long long)grid * a.waves_per_block;
     if (total > (1LL << 30)) return fail(FVMI_ERR_INVALID, "plan too large");

@@ -356,7 +356,7 @@ int fvmi_ensemble_tick(fvmi_instance_t* table, int n, int turn, int prepare, voi
  * 4, 5, 6 LxF, HLL, FORCE with one column per lane: 62; 12, 13, 14 the same
  * with two: 124, the first strip's first column being the ghost column beside
  * the domain; 7 one stage of the unsplit KP07: 60; 16 a whole step in one
- * launch: 56), sub-area [x0,x1)x[y0,y1) of an nx x ny domain (x1 = y1 = 0: the
+ * launch: 56, 19 that of Euler), sub-area [x0,x1)x[y0,y1) of an nx x ny domain (x1 = y1 = 0: the
  * whole domain, the only one the unsplit schemes and whole steps take), the
  * launch shape and a device of `cu_count` CUs.  For every wave of the grid, 3 ints in `segs`
  * (capacity `max_waves` waves): strip, first row and row count relative to
