@@ -89,14 +89,37 @@ class _DeviceMemory:
 
 
 class Turn:
-    """Which of its two allocations each array of a pair of states holds (0 or 1).
-    A simulator turns it where a step leaves the new state in the allocations of
-    the other state, so that its arrays keep their roles."""
+    """Which of its two allocations each array of a pair of states holds: ``value``
+    is 0 or 1.  A simulator turns it where a step leaves the new state in the
+    allocations of the other state, so that its arrays keep their roles."""
 
-    __slots__ = ("value",)
+    __slots__ = ("value", "first", "second", "places")
 
-    def __init__(self):
+    def __init__(self, first=None, second=None):
         self.value = 0
+        self.first, self.second = first, second  # the two states' arrays
+        if first is None:
+            return
+        # addresses and pitches of both states as fvmi_step_t has them, for either
+        # state first and either turn
+        pad = (0,) * (4 - len(first))
+
+        def place(a, b):
+            return tuple(x.address for x in a) + pad + tuple(x.address for x in b) + pad, \
+                tuple(x.pitch for x in a) + pad + tuple(x.pitch for x in b) + pad
+
+        a, b = [x.memory for x in first], [x.memory for x in second]
+        ab, ba = place(a, b), place(b, a)
+        self.places = (ab[0] + ab[1], ba[0] + ba[1])
+
+    def places_of(self, u, v):
+        """The 8 addresses and 8 pitches of the states ``u`` and ``v`` (lists of
+        arrays), or None if they are not this pair's two."""
+        if u == self.first and v == self.second:
+            return self.places[self.value]
+        if u == self.second and v == self.first:
+            return self.places[1 - self.value]
+        return None
 
 
 class HipArray2D:
@@ -150,10 +173,10 @@ class HipArray2D:
 
     @property
     def data_ptr(self):
-        return self.ptr.value
+        return self.memories[self.turn.value].address or None
 
     def row_ptr(self, row, col=0):
-        return self.ptr.value + row * self.pitch + col * 4
+        return self.data_ptr + row * self.pitch + col * 4
 
     def download(self, stream, cpu_data=None, asynch=False, extent=None):
         if extent is None:
@@ -195,6 +218,7 @@ class HipArray2D:
     def free(self):
         if hasattr(self, "memories"):
             self.memory.free()
+            self.turn.first = self.turn.second = None  # its addresses are no longer good
 
 
 class ArakawaA2D:
@@ -218,8 +242,8 @@ class ArakawaA2D:
         """Lets the arrays of two states of one shape exchange their memory; returns
         the Turn that does it.  Both allocations of a variable live as long as
         either of its arrays."""
-        turn = Turn()
-        for a, b in zip(self.gpu_variables, other.gpu_variables):
+        turn = Turn(list(self.gpu_variables), list(other.gpu_variables))
+        for a, b in zip(turn.first, turn.second):
             m, n = a.memory, b.memory
             a.memories, b.memories = (m, n), (n, m)
             a.turn = b.turn = turn

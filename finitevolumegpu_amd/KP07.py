@@ -2,11 +2,12 @@
 Runge-Kutta time stepping (GPUSimulators/KP07.py; kernel
 GPUSimulators/cuda/SWE2D_KP07.cu)."""
 
+import operator
+
 import numpy as np
 
 from . import _lib
-from .Simulator import (BoundaryCondition, UnsplitSimulator, _StepCall, _steps_in_library, _SubstepMethods,
-                        swe_initial_cfl)
+from .Simulator import BoundaryCondition, UnsplitSimulator, _StepCall, _steps_in_library, swe_initial_cfl
 
 
 def stepOrderToCodedInt(step, order):
@@ -21,7 +22,8 @@ class KP07(UnsplitSimulator):
     scheme = "kp07"
     gc = 2
     nvars = 3
-    _substep_methods = _SubstepMethods("substep", "_launch", "_field_args", "cfl_pointer")
+    _substep_names = ("substep", "_launch", "_field_args", "cfl_pointer")
+    _methods_of = operator.attrgetter(*_substep_names)
 
     def __init__(self, context, h0, hu0, hv0, nx, ny, dx, dy, g, theta=1.3, cfl_scale=0.9, order=2,
                  boundary_conditions=BoundaryCondition(), block_width=16, block_height=16,
@@ -37,7 +39,8 @@ class KP07(UnsplitSimulator):
                            tile_rows, waves_per_block, math, xcd_remap)
         # a second-order step is one library call
         self._step_call = _StepCall("fvmi_swe_kp07_rk2_step", _lib.RUN_KP07_RK2)
-        self._library = self._substep_methods.library(self) if order == 2 else None
+        if order == 2:
+            self._find_own_methods()
 
     def step(self, dt):
         """One full step; with two stages as one library call
@@ -51,8 +54,8 @@ class KP07(UnsplitSimulator):
 
     def _take_step(self, in_other, slot):
         if in_other:
-            self._turn_state()
-        else:
+            self.turn.value ^= 1
+        elif self.math == "fast":
             self._note_recording()
         self.cfl_last = slot
 

@@ -118,7 +118,8 @@ class MPISimulator(BaseSimulator):
     def full_exchange(self):
         """On-device exchange of the current state's ghost cells (MPISimulator.py:371-480)."""
         t0 = time.time()
-        self.sim._note_recording()
+        if isinstance(self.sim, BaseSimulator):
+            self.sim._note_recording()
         state = self.sim.getOutput()
         ptrs = (ctypes.c_void_p * self.nvars)(*[state[k].data_ptr for k in range(self.nvars)])
         pitches = (ctypes.c_int * self.nvars)(*[state[k].pitch for k in range(self.nvars)])

@@ -152,29 +152,31 @@ class BaseSimulator:
         with.  From the first recording on, the steps of a simulator are therefore
         two launches each, which leave the state in the buffer that it was in, as
         the recorded ones do: replays and steps go on from each other."""
-        if not self._recorded and self.launch.math == _lib.FVMI_MATH_FAST and self.stream.capturing():
+        if getattr(self, "math", None) == "fast" and not self._recorded and self.stream.capturing():
             self._recorded = True
 
-    def _turn_state(self):
-        """Exchanges the memory of u0 and u1 after a step that left the state in u1's
-        (also where a program has put arrays of its own into them)."""
-        turn = self.turn
-        for a, b in zip(self.u0.gpu_variables, self.u1.gpu_variables):
-            if a.turn is not turn or b.turn is not turn:
-                turn = self.turn = self.u0.pair_with(self.u1)
-                break
-        turn.value ^= 1
+    # Methods between step() and the launches.  A subclass, a wrapper on the class
+    # or the simulator itself may replace any of them, before or after the simulator
+    # was made: a step then goes through them.
+    _substep_names = ()
+    _own_methods = None  # those of the class, if all are the package's
+
+    def _find_own_methods(self):
+        if _library_methods(self, self._substep_names):
+            self._own_methods = self._methods_of(type(self))
 
     def _one_call(self):
         """Whether a full step of two substeps may be one call of the library."""
-        return (not self._recorded and self.num_substeps == 2
-                and self._substep_methods.unchanged(self, self._library))
+        return (self._own_methods is not None and not self._recorded and self.num_substeps == 2
+                and self._methods_of(type(self)) == self._own_methods
+                and self.__dict__.keys().isdisjoint(self._substep_names))
 
     def _return_state(self):
         """After an odd number of one-launch steps, copies the state back into the
         memory that two launches a step would have it in: under Dirichlet edges each
         substep reads the ghost cells that a program wrote into its input buffer."""
-        if getattr(self, "turn", None) is None or self.turn.value == 0:
+        turn = getattr(self, "turn", None)
+        if turn is None or turn.value == 0 or turn.places_of(self.u0.gpu_variables, self.u1.gpu_variables) is None:
             return
         self._note_recording()
         if self._recorded:  # the recorded work stays where it is
@@ -182,7 +184,7 @@ class BaseSimulator:
         for a, b in zip(self.u0.gpu_variables, self.u1.gpu_variables):
             _lib.call("fvmi_memcpy2d_async", b.row_ptr(b.y_halo, b.x_halo), b.pitch, a.row_ptr(a.y_halo, a.x_halo),
                       a.pitch, 4 * a.nx, a.ny, _lib.MEMCPY_DTOD, self.stream.handle)
-        self._turn_state()
+        self.turn.value = 0
 
     def step(self, dt):
         """One full step of ``num_substeps`` substeps (Simulator.py:220-228)."""
@@ -268,14 +270,14 @@ class _StepCall:
         self.time_ptr = ctypes.addressof(self.time)
 
     def _pack(self, sim, scheme, dt, boundary_conditions, cfl_slot):
-        u = [x.memories[x.turn.value] for x in sim.u0.gpu_variables]
-        v = [x.memories[x.turn.value] for x in sim.u1.gpu_variables]
-        pad = (0,) * (4 - len(u))
+        u, v = sim.u0.gpu_variables, sim.u1.gpu_variables
+        places = sim.turn.places_of(u, v)
+        if places is None:  # a program has put arrays of its own into them, or freed some
+            sim.turn = sim.u0.pair_with(sim.u1)
+            places = sim.turn.places[0]
         _lib.STEP_PACK.pack_into(
             self.args, 0, scheme, sim.nx, sim.ny, boundary_conditions, sim.dx, sim.dy, dt, sim.g,
-            getattr(sim, "theta", 0.0), getattr(sim, "gamma", 0.0), *[x.address for x in u], *pad,
-            *[x.address for x in v], *pad, *[x.pitch for x in u], *pad, *[x.pitch for x in v], *pad,
-            sim.cfl_pointer() or 0, cfl_slot)
+            getattr(sim, "theta", 0.0), getattr(sim, "gamma", 0.0), *places, sim.cfl_pointer() or 0, cfl_slot)
 
     def step(self, sim, scheme, dt, boundary_conditions, cfl_slot):
         """One step; returns (state is in u1, CFL slot)."""
@@ -323,26 +325,6 @@ def _library_methods(sim, names):
     return all(_of_package(getattr(type(sim), name)) for name in names)
 
 
-class _SubstepMethods:
-    """The methods between ``step`` and the launches of a simulator, any of which a
-    subclass, a wrapper on the class or the simulator itself may replace, before or
-    after the simulator was made: with a version that is not the package's own, the
-    step goes through them."""
-
-    def __init__(self, *names):
-        self.names = names
-        self._of_class = operator.attrgetter(*names)
-
-    def library(self, sim):
-        """The methods of the class of ``sim`` if they are the package's own, else None."""
-        return self._of_class(type(sim)) if _library_methods(sim, self.names) else None
-
-    def unchanged(self, sim, library):
-        """Whether they are still those that ``library`` gave; asked at every step."""
-        return (library is not None and self._of_class(type(sim)) == library
-                and sim.__dict__.keys().isdisjoint(self.names))
-
-
 # what simulate() calls besides, once a step
 _LOOP_METHODS = ("step", "simTime", "simSteps")
 
@@ -361,7 +343,8 @@ class DimsplitSimulator(BaseSimulator):
     nvars = 3
     # default launch shape when neither the caller nor the autotuner gives one
     default_waves_per_block = 4
-    _substep_methods = _SubstepMethods("substep", "substepDimsplit", "_launch", "_field_args", "cfl_pointer")
+    _substep_names = ("substep", "substepDimsplit", "_launch", "_field_args", "cfl_pointer")
+    _methods_of = operator.attrgetter(*_substep_names)
 
     def _init_dimsplit(self, fields, cfl_host, tile_rows, waves_per_block, math, xcd_remap):
         if self.context.autotuner is not None and tile_rows is None and waves_per_block is None:
@@ -391,7 +374,7 @@ class DimsplitSimulator(BaseSimulator):
         _lib.call("fvmi_memcpy_async", self.cfl_data, init.ctypes.data, 8, _lib.MEMCPY_HTOD, self.stream.handle)
         self.stream.synchronize()
         self._step_call = _StepCall("fvmi_dimsplit_step", _lib.RUN_DIMSPLIT)
-        self._library = self._substep_methods.library(self)
+        self._find_own_methods()
 
     def cfl_pointer(self):
         return self.cfl_data.value
@@ -413,8 +396,8 @@ class DimsplitSimulator(BaseSimulator):
 
     def _take_step(self, in_other, slot):
         if in_other:
-            self._turn_state()
-        else:
+            self.turn.value ^= 1
+        elif self.math == "fast":
             self._note_recording()
         if self.cfl_pointer():
             self.cfl_last = slot

@@ -88,6 +88,23 @@ def test_arrays_that_a_program_put_into_a_state(ctx):
         assert_same(a, b)
 
 
+@pytest.mark.parametrize("scheme,math", SCHEMES)
+@pytest.mark.parametrize("which", ["u0", "u1"])
+def test_step_of_a_freed_array_is_refused(ctx, scheme, math, which):
+    from finitevolumegpu_amd import _lib
+    sim = pair(ctx, scheme, math)[0]
+    sim.step(DT)
+    sim.synchronize()
+    print("case freed", scheme, math, which, flush=True)
+    array = getattr(sim, which)[1]
+    array.free()
+    assert array.data_ptr is None
+    with pytest.raises(_lib.FvmiError):
+        sim.step(DT)
+    with pytest.raises(_lib.FvmiError):
+        sim.simulate(float(DT), DT)
+
+
 def record(sim, enqueue):
     from finitevolumegpu_amd import _lib
     graph = ctypes.c_void_p()
