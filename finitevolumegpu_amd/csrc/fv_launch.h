@@ -44,9 +44,10 @@ inline bool step_grid_fits(const SubstepArgs& a) {
 }
 
 // Whether a dimensionally split step is.  Fast arithmetic only: the exact kernels
-// and WAF are bound by VALU issue already as substeps (4096^2: 184 us for
-// KP07_dimsplit, 260 for WAF, against 79 us for their bytes), so that the wider
-// halo would cost more than the memory passes saved.
+// and WAF are bound by VALU issue already as substeps (4096^2: 177 us for
+// KP07_dimsplit, 262 for WAF, against 79 us for their bytes), so that the wider
+// halo is expected to cost more than the memory passes saved (a whole exact step has
+// not been built and timed).
 inline bool step_is_fused(int scheme, int math, const SubstepArgs& a) {
     return math != FVMI_MATH_EXACT && scheme != SCHEME_WAF && step_grid_fits(a);
 }
@@ -62,7 +63,8 @@ inline SegmentCost substep_cost(int math) {
 // equal segments, one simulator and three in turn: KP07_dimsplit 756 and 711 us,
 // 715 and 683, HLL2 949 and 883, 894 and 826, Euler 1239 and 1183, 1140 and 1049,
 // KP07 653 and 618, 621 and 622; 9500x7000 KP07_dimsplit 773 and 683; 7500^2 (93 %)
-// even; 5500^2 (98 %) 317 and 323.
+// even; 5500^2 (98 %) 317 and 323.  The weights and the shortest part are those of
+// the substep kernel; at 3000^2 equal segments were 4 % faster than these rounds.
 constexpr int kStepMinFill = 93;
 inline SegmentCost step_cost() { return {2 * kStepHalo, kStepMinSegRows, 0.45f, 0.01f}; }
 
@@ -196,18 +198,19 @@ hipError_t launch_ensemble_substep(int scheme, EnsembleArgs e, int grid, hipStre
     return hipGetLastError();
 }
 
-// Defined in fv_kernels_exact.hip / fv_kernels_fast.hip.
+// Defined in fv_kernels_exact.hip and fv_kernels_fast.hip (whole steps: KP07_dimsplit,
+// HLL2 and Euler in fast arithmetic).
 hipError_t launch_ensemble_exact(int scheme, const EnsembleArgs& e, int grid, hipStream_t stream);
 hipError_t launch_ensemble_fast(int scheme, const EnsembleArgs& e, int grid, hipStream_t stream);
 hipError_t launch_substep_exact(int scheme, const SubstepArgs& a, int grid, hipStream_t stream);
 hipError_t launch_substep_fast(int scheme, const SubstepArgs& a, int grid, hipStream_t stream);
-// KP07_dimsplit and HLL2 in fast arithmetic, single grid and ensemble
-// (fv_kernels_fast_ilp.hip, built with the ILP-maximising scheduler)
 hipError_t launch_step_fast(int scheme, const SubstepArgs& a, int grid, hipStream_t stream);
-hipError_t launch_step_fast_ilp(int scheme, const SubstepArgs& a, int grid, hipStream_t stream);
 hipError_t launch_ensemble_step_fast(int scheme, const EnsembleArgs& e, int grid, hipStream_t stream);
+// Defined in fv_kernels_fast_ilp.hip: the shallow-water schemes of the above, and the
+// two Runge-Kutta stages of KP07 in fast arithmetic.
+hipError_t launch_step_fast_ilp(int scheme, const SubstepArgs& a, int grid, hipStream_t stream);
 hipError_t launch_ensemble_step_fast_ilp(int scheme, const EnsembleArgs& e, int grid, hipStream_t stream);
-hipError_t launch_rk2_step(const SubstepArgs& a, int grid, hipStream_t stream);  // fast arithmetic
+hipError_t launch_rk2_step(const SubstepArgs& a, int grid, hipStream_t stream);
 hipError_t launch_substep_fast_ilp(int scheme, const SubstepArgs& a, int grid, hipStream_t stream);
 hipError_t launch_ensemble_fast_ilp(int scheme, const EnsembleArgs& e, int grid, hipStream_t stream);
 

@@ -66,7 +66,8 @@ FVMI_TRANS_RUN(sqrt_all, __builtin_amdgcn_sqrtf, "v_sqrt_f32")
 //    quotient needs care only for its sign, which q0 has and q0 + r y may turn
 //    from -0 into +0: div_rn puts it back with one v_bfi (the sign of a zero
 //    reaches copysign in the WAF limiter), quot_rn leaves it (no other scheme
-//    reads a zero's sign, and its values are equal either way);
+//    reads a zero's sign, and its values are equal either way; exact runs from
+//    momenta of +0 and -0 keep the oracle's signs too);
 //  * square root: v_sqrt_f32 (1 ulp) and its two neighbours, the one whose
 //    residual x - s s' changes sign chosen by two FMAs (exact from x = 2^-101 on,
 //    within 2 ulp below; 0 and infinity give themselves).  Newton's correction
@@ -108,7 +109,7 @@ __device__ __forceinline__ float sqrt_rn(float x, float s) {
     return (__builtin_fmaf(-up, s, x) > 0.0f) ? up : r;
 }
 __device__ __forceinline__ float sqrt_rn(float x) { return sqrt_rn(x, __builtin_amdgcn_sqrtf(x)); }
-// the same of N values, their v_rcp / v_rsq in one run
+// the same of N values, their v_rcp / v_sqrt in one run
 template <int N>
 __device__ __forceinline__ void rcp_rn_all(const float (&b)[N], float (&r)[N]) {
     float y[N];

@@ -357,8 +357,12 @@ __device__ __forceinline__ float march_step(const SubstepArgs& a, const Strip<1>
     return needs_edge(e) || count < 2 ? march_step_edge<S, M>(a, st, e) : march_step_paired<S, M>(a, st);
 }
 
-// Four waves fit on a SIMD (109 VGPRs for KP07_dimsplit, 120 for HLL2, 128 for
-// Euler, no scratch).  Measured per 4096^2 step with two columns per lane
+// Four waves fit on a SIMD: 112 VGPRs for KP07_dimsplit and 123 for HLL2, no
+// scratch; for Euler 128 and 64 bytes of scratch a lane (ensemble kernel: 128 bytes),
+// where the edge march keeps its middle rows: fill_ghost_row takes one of three by
+// branch, which becomes a load through a selected address.  The kernels are large (60
+// and 72 KB against 38 and 46 for a substep, two marches with their prologues), which
+// the first launch of a program pays for.  Measured per 4096^2 step with two columns per lane
 // (fewer halo lanes, 168 VGPRs with spills or 247): KP07_dimsplit 327 and 248
 // us against 182; five and six waves (96 and 80 VGPRs): 178 and 176 against 172.
 template <class S, class M>

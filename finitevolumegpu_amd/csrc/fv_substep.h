@@ -873,8 +873,8 @@ __device__ __forceinline__ void store_row(const Args& a, const Strip<C>& st, int
 }
 
 // CFL accumulator: the exact policy keeps min(dt) as the reference's writeCfl
-// does; the fast policy keeps max(1/dt) (one reciprocal per strip, taken in
-// finish_cfl).
+// does; the fast policy keeps max(1/dt) (one reciprocal per segment, taken in
+// reduce_cfl).
 template <class S, class M>
 __device__ __forceinline__ void accumulate_cfl(const float (&q)[S::kC][S::NV], const SubstepArgs& a,
                                                const Strip<S::kC>& st, float& acc) {
