@@ -53,11 +53,15 @@ STEP_STRIP_COLS = 56
 
 def steppable(nx, ny, bc):
     """Whether an instance's whole step can be one launch: step_grid_fits of
-    fv_launch.h (no Dirichlet edge, periodic edges in opposite pairs)."""
-    T = BoundaryCondition.Type
+    fv_launch.h (no Dirichlet edge, periodic edges in opposite pairs).  Of integers,
+    or of arrays of instances."""
+    dirichlet, periodic = int(BoundaryCondition.Type.Dirichlet), int(BoundaryCondition.Type.Periodic)
     west, east, south, north = (bc >> shift & 0xF for shift in (0, 8, 16, 24))
-    return (nx >= 8 and ny >= 8 and T.Dirichlet not in (west, east, south, north)
-            and (west == T.Periodic) == (east == T.Periodic) and (south == T.Periodic) == (north == T.Periodic))
+    ok = (nx >= 8) & (ny >= 8)
+    for edge in (west, east, south, north):
+        ok = ok & (edge != dirichlet)
+    return (ok & ((west == periodic) == (east == periodic))
+            & ((south == periodic) == (north == periodic)))
 
 
 def _bc_code(bc):
@@ -382,8 +386,7 @@ class Ensemble:
         back to them puts every instance's current buffer first."""
         whole = (self.math == "fast" and self.scheme != "waf" and not 0 < (self.seg_rows or 0) < 4
                  and self.min_seg_rows >= 4
-                 and all(steppable(int(self.tab["nx"][i]), int(self.tab["ny"][i]), int(self.tab["bc"][i]))
-                         for i in np.flatnonzero(self.live)))
+                 and bool(steppable(*(self.tab[k][self.live] for k in ("nx", "ny", "bc"))).all()))
         if whole == self.whole_steps:
             return
         if not whole:
