@@ -24,12 +24,6 @@ class Stream:
     def synchronize(self):
         _lib.call("fvmi_stream_synchronize", self.handle)
 
-    def capturing(self):
-        """Whether the work queued now is being recorded for a graph."""
-        out = ctypes.c_int()
-        _lib.call("fvmi_stream_is_capturing", self.handle, ctypes.byref(out))
-        return out.value != 0
-
     def wait_for_event(self, event):
         """Work queued after this call waits for ``event``."""
         _lib.call("fvmi_stream_wait_event", self.handle, event.handle)

@@ -152,8 +152,10 @@ class BaseSimulator:
         with.  From the first recording on, the steps of a simulator are therefore
         two launches each, which leave the state in the buffer that it was in, as
         the recorded ones do: replays and steps go on from each other."""
-        if getattr(self, "math", None) == "fast" and not self._recorded and self.stream.capturing():
-            self._recorded = True
+        if getattr(self, "math", None) == "fast" and not self._recorded:
+            capturing = ctypes.c_int()
+            _lib.call("fvmi_stream_is_capturing", self.stream.handle, ctypes.byref(capturing))
+            self._recorded = capturing.value != 0
 
     # Methods between step() and the launches.  A subclass, a wrapper on the class
     # or the simulator itself may replace any of them, before or after the simulator
