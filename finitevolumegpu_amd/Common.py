@@ -169,7 +169,7 @@ class HipArray2D:
 
     @property
     def pitch(self):
-        return self.memory.pitch
+        return self.memories[self.turn.value].pitch
 
     @property
     def data_ptr(self):

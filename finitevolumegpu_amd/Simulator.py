@@ -427,7 +427,8 @@ class DimsplitSimulator(BaseSimulator):
     def _field_args(self, state):
         args = []
         for k in range(self.nvars):
-            args += [state[k].data_ptr, state[k].pitch]
+            memory = state[k].memory
+            args += [memory.address or None, memory.pitch]
         return args
 
     def getOutput(self):
@@ -500,7 +501,8 @@ class UnsplitSimulator(BaseSimulator):
     def _field_args(self, state):
         args = []
         for k in range(self.nvars):
-            args += [state[k].data_ptr, state[k].pitch]
+            memory = state[k].memory
+            args += [memory.address or None, memory.pitch]
         return args
 
     def getOutput(self):
