@@ -93,32 +93,43 @@ class Turn:
     is 0 or 1.  A simulator turns it where a step leaves the new state in the
     allocations of the other state, so that its arrays keep their roles."""
 
-    __slots__ = ("value", "first", "second", "places")
+    __slots__ = ("value", "valid")
 
-    def __init__(self, first=None, second=None):
+    def __init__(self):
         self.value = 0
-        self.first, self.second = first, second  # the two states' arrays
-        if first is None:
-            return
-        # addresses and pitches of both states as fvmi_step_t has them, for either
-        # state first and either turn
-        pad = (0,) * (4 - len(first))
+        self.valid = True  # none of the arrays has been freed
+
+
+class StatePair:
+    """Two states of one shape whose arrays exchange their memory.  Both allocations
+    of a variable live as long as either of its arrays (which know the Turn, but not
+    the pair: they and their memory go with the last reference)."""
+
+    def __init__(self, u, v):
+        self.first, self.second = list(u.gpu_variables), list(v.gpu_variables)
+        self.turn = Turn()
+        m, n = [x.memory for x in self.first], [x.memory for x in self.second]
+        for arrays, memories in ((self.first, zip(m, n)), (self.second, zip(n, m))):
+            for x, pair in zip(arrays, memories):
+                x.memories, x.turn = pair, self.turn
+        # addresses and pitches of both states as fvmi_step_t has them, with the
+        # first or the second of the allocations in front
+        pad = (0,) * (4 - len(m))
 
         def place(a, b):
-            return tuple(x.address for x in a) + pad + tuple(x.address for x in b) + pad, \
-                tuple(x.pitch for x in a) + pad + tuple(x.pitch for x in b) + pad
+            return (tuple(x.address for x in a) + pad + tuple(x.address for x in b) + pad
+                    + tuple(x.pitch for x in a) + pad + tuple(x.pitch for x in b) + pad)
 
-        a, b = [x.memory for x in first], [x.memory for x in second]
-        ab, ba = place(a, b), place(b, a)
-        self.places = (ab[0] + ab[1], ba[0] + ba[1])
+        self.places = (place(m, n), place(n, m))
 
     def places_of(self, u, v):
         """The 8 addresses and 8 pitches of the states ``u`` and ``v`` (lists of
-        arrays), or None if they are not this pair's two."""
-        if u == self.first and v == self.second:
-            return self.places[self.value]
-        if u == self.second and v == self.first:
-            return self.places[1 - self.value]
+        arrays), or None if they are not this pair's two or one of them is freed."""
+        if self.turn.valid:
+            if u == self.first and v == self.second:
+                return self.places[self.turn.value]
+            if u == self.second and v == self.first:
+                return self.places[1 - self.turn.value]
         return None
 
 
@@ -218,7 +229,7 @@ class HipArray2D:
     def free(self):
         if hasattr(self, "memories"):
             self.memory.free()
-            self.turn.first = self.turn.second = None  # its addresses are no longer good
+            self.turn.valid = False
 
 
 class ArakawaA2D:
@@ -237,17 +248,6 @@ class ArakawaA2D:
 
     def __len__(self):
         return len(self.gpu_variables)
-
-    def pair_with(self, other):
-        """Lets the arrays of two states of one shape exchange their memory; returns
-        the Turn that does it.  Both allocations of a variable live as long as
-        either of its arrays."""
-        turn = Turn(list(self.gpu_variables), list(other.gpu_variables))
-        for a, b in zip(turn.first, turn.second):
-            m, n = a.memory, b.memory
-            a.memories, b.memories = (m, n), (n, m)
-            a.turn = b.turn = turn
-        return turn
 
     def download(self, stream, variables=None):
         if variables is None:

@@ -54,7 +54,7 @@ class KP07(UnsplitSimulator):
 
     def _take_step(self, in_other, slot):
         if in_other:
-            self.turn.value ^= 1
+            self.pair.turn.value ^= 1
         elif self.math == "fast":
             self._note_recording()
         self.cfl_last = slot

@@ -177,8 +177,9 @@ class BaseSimulator:
         """After an odd number of one-launch steps, copies the state back into the
         memory that two launches a step would have it in: under Dirichlet edges each
         substep reads the ghost cells that a program wrote into its input buffer."""
-        turn = getattr(self, "turn", None)
-        if turn is None or turn.value == 0 or turn.places_of(self.u0.gpu_variables, self.u1.gpu_variables) is None:
+        pair = getattr(self, "pair", None)
+        if pair is None or pair.turn.value == 0 or pair.places_of(self.u0.gpu_variables,
+                                                                  self.u1.gpu_variables) is None:
             return
         self._note_recording()
         if self._recorded:  # the recorded work stays where it is
@@ -186,7 +187,7 @@ class BaseSimulator:
         for a, b in zip(self.u0.gpu_variables, self.u1.gpu_variables):
             _lib.call("fvmi_memcpy2d_async", b.row_ptr(b.y_halo, b.x_halo), b.pitch, a.row_ptr(a.y_halo, a.x_halo),
                       a.pitch, 4 * a.nx, a.ny, _lib.MEMCPY_DTOD, self.stream.handle)
-        self.turn.value = 0
+        pair.turn.value = 0
 
     def step(self, dt):
         """One full step of ``num_substeps`` substeps (Simulator.py:220-228)."""
@@ -273,10 +274,10 @@ class _StepCall:
 
     def _pack(self, sim, scheme, dt, boundary_conditions, cfl_slot):
         u, v = sim.u0.gpu_variables, sim.u1.gpu_variables
-        places = sim.turn.places_of(u, v)
+        places = sim.pair.places_of(u, v)
         if places is None:  # a program has put arrays of its own into them, or freed some
-            sim.turn = sim.u0.pair_with(sim.u1)
-            places = sim.turn.places[0]
+            sim.pair = Common.StatePair(sim.u0, sim.u1)
+            places = sim.pair.places[0]
         _lib.STEP_PACK.pack_into(
             self.args, 0, scheme, sim.nx, sim.ny, boundary_conditions, sim.dx, sim.dy, dt, sim.g,
             getattr(sim, "theta", 0.0), getattr(sim, "gamma", 0.0), *places, sim.cfl_pointer() or 0, cfl_slot)
@@ -365,7 +366,7 @@ class DimsplitSimulator(BaseSimulator):
         self.gc_y = 2
         self.u0 = Common.ArakawaA2D(self.stream, self.nx, self.ny, 2, 2, fields)
         self.u1 = Common.ArakawaA2D(self.stream, self.nx, self.ny, 2, 2, [None] * len(fields))
-        self.turn = self.u0.pair_with(self.u1)
+        self.pair = Common.StatePair(self.u0, self.u1)
         # Two-slot device CFL minimum (see fvmi.h): slot 0 = +inf, slot 1 = initial value.
         ptr = ctypes.c_void_p()
         _lib.call("fvmi_malloc", ctypes.byref(ptr), 8)
@@ -398,7 +399,7 @@ class DimsplitSimulator(BaseSimulator):
 
     def _take_step(self, in_other, slot):
         if in_other:
-            self.turn.value ^= 1
+            self.pair.turn.value ^= 1
         elif self.math == "fast":
             self._note_recording()
         if self.cfl_pointer():
@@ -480,7 +481,7 @@ class UnsplitSimulator(BaseSimulator):
         self.gc_y = self.gc
         self.u0 = Common.ArakawaA2D(self.stream, self.nx, self.ny, self.gc, self.gc, fields)
         self.u1 = Common.ArakawaA2D(self.stream, self.nx, self.ny, self.gc, self.gc, [None] * len(fields))
-        self.turn = self.u0.pair_with(self.u1)
+        self.pair = Common.StatePair(self.u0, self.u1)
         ptr = ctypes.c_void_p()
         _lib.call("fvmi_malloc", ctypes.byref(ptr), 8)
         self.cfl_data = ptr

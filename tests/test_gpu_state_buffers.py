@@ -72,6 +72,29 @@ def test_memory_outlives_the_simulator_with_either_field(ctx):
     assert np.array_equal(held.download(others[0].stream), state_now)
 
 
+@pytest.mark.parametrize("scheme,math", SCHEMES)
+def test_memory_goes_with_the_simulator(ctx, scheme, math):
+    """Without the cycle collector, as large states are dropped in loops."""
+    import gc
+    import weakref
+    gc.collect()
+    gc.disable()
+    try:
+        sim = pair(ctx, scheme, math)[0]
+        sim.step(DT)
+        sim.simulate(float(DT), DT)
+        sim.synchronize()
+        memory = [weakref.ref(x.memory) for u in (sim.u0, sim.u1) for x in u.gpu_variables]
+        held = sim.u0[0]
+        del sim
+        alive = [m() is not None for m in memory]
+        assert sum(alive) == 2  # the held array's two
+        del held
+        assert all(m() is None for m in memory)
+    finally:
+        gc.enable()
+
+
 def test_arrays_that_a_program_put_into_a_state(ctx):
     from finitevolumegpu_amd import Common
     a, b = pair(ctx, "kp07_dimsplit")

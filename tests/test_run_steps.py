@@ -15,8 +15,8 @@ def test_steps_of_one_library_call(monkeypatch, nx, ny):
     asked = []
     monkeypatch.setattr(_lib, "call", lambda name, *args: asked.append(args[6]))
     state = SimpleNamespace(gpu_variables=[])
-    turn = SimpleNamespace(places_of=lambda u, v: (0,) * 16)
-    sim = SimpleNamespace(nx=np.int32(nx), ny=np.int32(ny), dx=1.0, dy=1.0, g=9.81, u0=state, u1=state, turn=turn, t=0.0,
+    pair = SimpleNamespace(places_of=lambda u, v: (0,) * 16)
+    sim = SimpleNamespace(nx=np.int32(nx), ny=np.int32(ny), dx=1.0, dy=1.0, g=9.81, u0=state, u1=state, pair=pair, t=0.0,
                           dt=0.5, boundary_conditions=0, cfl_pointer=lambda: 0, launch=None,
                           stream=SimpleNamespace(handle=None))
     for left in (100, 7, 1):
